@@ -510,6 +510,20 @@ int matpl_nep_feat(int f64, int angular, int mode, const void *c, const void *Ri
                    void *gc, void *ggfeat, void *stream);
 
 /*
+ * The descriptor kernels of matpl_nep_feat with each derivative on its own (a model that knows which it
+ * needs): arguments as there, save [N][nm*24] the angular sums s or [N][T*nb] the radial basis sums.
+ *  mode 0: feats and save (radial: save may be null);
+ *  mode 1: gRi only, for gfeat (angular: reads save);
+ *  mode 2: second order: ggfeat and gc; angular: the gradient of s goes to gsave [N][nm*24] instead of
+ *          into gc, for the caller's mode 3 to add (gs there);
+ *  mode 3: gc only, from gfeat and save (angular: gs, if not null, is added to dL/ds; gfeat may then be null).
+ */
+int matpl_nep_descriptor(int f64, int angular, int mode, const void *c, const void *Ri, const int64_t *NL,
+                         const int64_t *atom_map, int64_t N, int S, int T, int nm, int nb, int ld, int col0, int l3,
+                         int l4, int l5, double rc, void *feats, void *save, const void *gfeat, const void *gs,
+                         const void *gg, void *gRi, void *gc, void *ggfeat, void *gsave, void *stream);
+
+/*
  * Neighbor scatter F[NL[i][k]] += dE[i][k] . Ri_d[i][k] (a 4x3 contraction)
  * into F [N][3], which holds the centre terms -sum_k dE[i][k] . Ri_d[i][k]
  * on entry. dE [N][S][4], Ri_d [N][S][4][3]. Replaces

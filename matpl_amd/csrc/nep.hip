@@ -1,26 +1,12 @@
-// NEP descriptor path on gfx950: neighbor search, radial and angular
-// (3/4/5-body) features, their first and second derivatives, and the NEP
-// force / virial scatter. FP64 and FP32 instantiations.
+// NEP neighbor search and force / virial scatter on gfx950, FP64 and FP32 (the descriptor's kernels are in
+// nep_feat.hip).
 //
-// Semantics (the reference's src/op contract, with the maths restated):
 //   neighbor  : calculateNepNeighbor.cu:166-281 / cpu_calculate_nepneighbor.cpp:97-203
 //               every atom of a frame against every atom of the frame in every
 //               replica (ia,ib,ic) < num_cell, self excluded in replica 0,
 //               minimum image in the expanded box; lists ordered (n2, ia, ib, ic),
 //               global indices, -1 padded; Ri = [r, x, y, z] (or [x, y, z])
-//   f_k(r)    : (T_k(x)+1)/2 fc(r), x = 2(r/rc-1)^2-1, fc = (1+cos(pi r/rc))/2 (r < rc)
-//   radial    : q_n = sum_j sum_k c2[ti,tj,n,k] f_k(r_ij)         (calculateNepFeat.cu:5-96)
-//   angular   : s_nlm = sum_j g_n(r_ij) b_lm(r_ij/r), g_n = sum_k c3[ti,tj,n,k] f_k
-//               q = C3B-weighted s^2 per L, 4-body, 5-body         (nep3_small_box.cuh:68-146)
-// Derivatives are taken with r and (x, y, z) as independent inputs, the
-// reference's convention for the [N, S, 4] gradient of the descriptor ops.
 // Neighbor loops stop at the first -1 entry as the reference's do.
-//
-// Layout: one wavefront per atom, lanes over neighbor slots for the per-pair
-// work; sums over slots (s_nlm, their tangents, coefficient gradients) run
-// transposed with lanes over outputs, so lanes never add to one address; the
-// per-type coefficient gradients are accumulated per block in LDS and added
-// to global memory once per block (persistent grid).
 #include "common.h"
 
 #pragma clang fp contract(off)
@@ -29,165 +15,6 @@ namespace matpl {
 namespace {
 
 constexpr int WAVE = 64;
-constexpr int NEP_WAVES = 4;
-constexpr int NB_MAX = 20;      // basis functions
-constexpr int NM_MAX = 8;       // radial functions per descriptor part
-constexpr int NLM = 24;
-constexpr int WS = NLM + 1;     // LDS row stride of a slot's harmonics (odd: lanes writing their rows hit distinct banks)
-constexpr double PI_D = 3.14159265358979323846;
-
-// f_k(r) and f_k'(r) for k = 0, 1, 2, ... in order, one per next() call
-// (Chebyshev recursion, nothing stored per k).
-template <typename T>
-struct Basis {
-    T x, xp, fc, fcp, t0, t1, tp0, tp1;
-    int k;
-    __device__ __forceinline__ Basis(T r, T rc) {
-        const T rcinv = T(1) / rc;
-        fc = T(0);
-        fcp = T(0);
-        if (r < rc) {
-            const T a = T(PI_D) * r * rcinv;
-            fc = T(0.5) * cos(a) + T(0.5);
-            fcp = -T(0.5 * PI_D) * sin(a) * rcinv;
-        }
-        const T d = r * rcinv - T(1);
-        x = T(2) * d * d - T(1);
-        xp = T(4) * d * rcinv;
-        t0 = T(1); t1 = x; tp0 = T(0); tp1 = T(1);
-        k = 0;
-    }
-    __device__ __forceinline__ void next(T &f, T &fp) {
-        T t, tp;
-        if (k == 0) { t = t0; tp = tp0; }
-        else if (k == 1) { t = t1; tp = tp1; }
-        else {
-            t = T(2) * x * t1 - t0;
-            tp = T(2) * t1 + T(2) * x * tp1 - tp0;
-            t0 = t1; t1 = t; tp0 = tp1; tp1 = tp;
-        }
-        k++;
-        f = (t + T(1)) * T(0.5) * fc;
-        fp = T(0.5) * (tp * xp * fc + (t + T(1)) * fcp);
-    }
-};
-
-// The 24 real harmonics b_k(u) of a unit vector u (accumulate_s order): calls
-// fn(k, b_k, db_k/dux, db_k/duy, db_k/duz) for k = 0..23. With r and (x, y, z)
-// as independent inputs and u = (x, y, z)/r:
-//   db_k/dx_w = (db_k/du_w) / r,   db_k/dr = -(u . db_k/du) / r.
-template <typename T, typename Fn>
-__device__ __forceinline__ void blm_each(T x, T y, T z, Fn &&fn) {
-    const T x2 = x * x, y2 = y * y, z2 = z * z, xy2 = x2 - y2;
-    fn(0, z, T(0), T(0), T(1));
-    fn(1, x, T(1), T(0), T(0));
-    fn(2, y, T(0), T(1), T(0));
-    fn(3, T(3) * z2 - T(1), T(0), T(0), T(6) * z);
-    fn(4, x * z, z, T(0), x);
-    fn(5, y * z, T(0), z, y);
-    fn(6, xy2, T(2) * x, -T(2) * y, T(0));
-    fn(7, T(2) * x * y, T(2) * y, T(2) * x, T(0));
-    fn(8, (T(5) * z2 - T(3)) * z, T(0), T(0), T(15) * z2 - T(3));
-    fn(9, (T(5) * z2 - T(1)) * x, T(5) * z2 - T(1), T(0), T(10) * x * z);
-    fn(10, (T(5) * z2 - T(1)) * y, T(0), T(5) * z2 - T(1), T(10) * y * z);
-    fn(11, xy2 * z, T(2) * x * z, -T(2) * y * z, xy2);
-    fn(12, T(2) * x * y * z, T(2) * y * z, T(2) * x * z, T(2) * x * y);
-    fn(13, (x2 - T(3) * y2) * x, T(3) * x2 - T(3) * y2, -T(6) * x * y, T(0));
-    fn(14, (T(3) * x2 - y2) * y, T(6) * x * y, T(3) * x2 - T(3) * y2, T(0));
-    fn(15, (T(35) * z2 - T(30)) * z2 + T(3), T(0), T(0), T(140) * z2 * z - T(60) * z);
-    fn(16, (T(7) * z2 - T(3)) * x * z, (T(7) * z2 - T(3)) * z, T(0), T(21) * x * z2 - T(3) * x);
-    fn(17, (T(7) * z2 - T(3)) * y * z, T(0), (T(7) * z2 - T(3)) * z, T(21) * y * z2 - T(3) * y);
-    fn(18, (T(7) * z2 - T(1)) * xy2, T(2) * x * (T(7) * z2 - T(1)), -T(2) * y * (T(7) * z2 - T(1)),
-       T(14) * z * xy2);
-    fn(19, (T(7) * z2 - T(1)) * x * y * T(2), T(2) * y * (T(7) * z2 - T(1)), T(2) * x * (T(7) * z2 - T(1)),
-       T(28) * x * y * z);
-    fn(20, (x2 - T(3) * y2) * x * z, (T(3) * x2 - T(3) * y2) * z, -T(6) * x * y * z, (x2 - T(3) * y2) * x);
-    fn(21, (T(3) * x2 - y2) * y * z, T(6) * x * y * z, (T(3) * x2 - T(3) * y2) * z, (T(3) * x2 - y2) * y);
-    fn(22, xy2 * xy2 - T(4) * x2 * y2, T(4) * x2 * x - T(12) * x * y2, T(4) * y2 * y - T(12) * x2 * y, T(0));
-    fn(23, T(4) * x * y * xy2, T(12) * x2 * y - T(4) * y2 * y, T(4) * x2 * x - T(12) * x * y2, T(0));
-}
-
-// ------------------------------------------------------------ q(s) and its gradient
-// Weighted C3B (factor 2 on m != 0, nep_cpu.cpp:93-107), C4B, C5B (nep_cpu.h:8-16).
-__constant__ double kC3B[NLM] = {
-    0.238732414637843, 0.238732414637844, 0.238732414637844, 0.099471839432435, 1.193662073189216,
-    1.193662073189216, 0.298415518297304, 0.298415518297304, 0.139260575205408, 0.208890862808112,
-    0.208890862808112, 2.088908628081126, 2.088908628081126, 0.348151438013522, 0.348151438013522,
-    0.011190581936149, 0.447623277445956, 0.447623277445956, 0.223811638722978, 0.223811638722978,
-    3.133362942121690, 3.133362942121690, 0.391670367765212, 0.391670367765212};
-__constant__ double kC4B[5] = {-0.007499480826664, -0.134990654879954, 0.067495327439977, 0.404971964639861,
-                               -0.809943929279723};
-__constant__ double kC5B[3] = {0.026596810706114, 0.053193621412227, 0.026596810706114};
-
-// Forward-mode dual number (value, tangent) for Hessian-vector products.
-template <typename T>
-struct Dual {
-    T v, e;
-    __device__ Dual() {}
-    __device__ Dual(T a) : v(a), e(T(0)) {}
-    __device__ Dual(T a, T b) : v(a), e(b) {}
-};
-template <typename T> __device__ __forceinline__ Dual<T> operator+(Dual<T> a, Dual<T> b) { return {a.v + b.v, a.e + b.e}; }
-template <typename T> __device__ __forceinline__ Dual<T> operator-(Dual<T> a, Dual<T> b) { return {a.v - b.v, a.e - b.e}; }
-template <typename T> __device__ __forceinline__ Dual<T> operator*(Dual<T> a, Dual<T> b) { return {a.v * b.v, a.v * b.e + a.e * b.v}; }
-template <typename T> __device__ __forceinline__ Dual<T> operator*(T a, Dual<T> b) { return {a * b.v, a * b.e}; }
-
-// q for one radial index: q3[l] (l < l3), then 4-body, then 5-body (nq outputs).
-// The 4/5-body terms need l3 = 4, so their slots are q[4] and q[5]. Every index
-// below is a compile-time constant once unrolled, keeping s, q and D in registers.
-constexpr int LSTART[5] = {0, 3, 8, 15, 24};
-template <typename T, typename S>
-__device__ __forceinline__ int q_of_s(const S s[NLM], int l3, int l4, int l5, S q[6]) {
-#pragma unroll
-    for (int l = 0; l < 4; l++) {
-        S acc(T(0));
-#pragma unroll
-        for (int m = LSTART[l]; m < LSTART[l + 1]; m++) acc = acc + T(kC3B[m]) * (s[m] * s[m]);
-        q[l] = acc;
-    }
-    if (l4 > 0) {
-        q[4] = T(kC4B[0]) * (s[3] * s[3] * s[3]) + T(kC4B[1]) * (s[3] * (s[4] * s[4] + s[5] * s[5])) +
-                  T(kC4B[2]) * (s[3] * (s[6] * s[6] + s[7] * s[7])) + T(kC4B[3]) * (s[6] * (s[5] * s[5] - s[4] * s[4])) +
-                  T(kC4B[4]) * (s[4] * s[5] * s[7]);
-    }
-    if (l5 > 0) {
-        const S s0 = s[0] * s[0], s12 = s[1] * s[1] + s[2] * s[2];
-        q[5] = T(kC5B[0]) * (s0 * s0) + T(kC5B[1]) * (s0 * s12) + T(kC5B[2]) * (s12 * s12);
-    }
-    return l3 + (l4 > 0) + (l5 > 0);
-}
-
-// D[m] = sum_F gq[F] dq_F/ds_m (gq in q_of_s order).
-template <typename T, typename S>
-__device__ __forceinline__ void dq_ds(const S s[NLM], const T *gq, int l3, int l4, int l5, S D[NLM]) {
-#pragma unroll
-    for (int m = 0; m < NLM; m++) D[m] = S(T(0));
-#pragma unroll
-    for (int l = 0; l < 4; l++)
-        if (l < l3)
-#pragma unroll
-            for (int m = LSTART[l]; m < LSTART[l + 1]; m++) D[m] = D[m] + (T(2) * T(kC3B[m]) * gq[l]) * s[m];
-    if (l4 > 0) {
-        const T g = gq[4];
-        const T c0 = T(kC4B[0]), c1 = T(kC4B[1]), c2 = T(kC4B[2]), c3 = T(kC4B[3]), c4 = T(kC4B[4]);
-        D[3] = D[3] + g * (T(3) * c0 * (s[3] * s[3]) + c1 * (s[4] * s[4] + s[5] * s[5]) + c2 * (s[6] * s[6] + s[7] * s[7]));
-        D[4] = D[4] + g * (T(2) * c1 * (s[3] * s[4]) - T(2) * c3 * (s[6] * s[4]) + c4 * (s[5] * s[7]));
-        D[5] = D[5] + g * (T(2) * c1 * (s[3] * s[5]) + T(2) * c3 * (s[6] * s[5]) + c4 * (s[4] * s[7]));
-        D[6] = D[6] + g * (T(2) * c2 * (s[3] * s[6]) + c3 * (s[5] * s[5] - s[4] * s[4]));
-        D[7] = D[7] + g * (T(2) * c2 * (s[3] * s[7]) + c4 * (s[4] * s[5]));
-    }
-    if (l5 > 0) {
-        const T g = gq[5];
-        const T c0 = T(kC5B[0]), c1 = T(kC5B[1]), c2 = T(kC5B[2]);
-        const S s12 = s[1] * s[1] + s[2] * s[2];
-        D[0] = D[0] + g * (T(4) * c0 * (s[0] * s[0] * s[0]) + T(2) * c1 * (s[0] * s12));
-        D[1] = D[1] + g * (T(2) * c1 * (s[0] * s[0] * s[1]) + T(4) * c2 * (s12 * s[1]));
-        D[2] = D[2] + g * (T(2) * c1 * (s[0] * s[0] * s[2]) + T(4) * c2 * (s12 * s[2]));
-    }
-}
-
-// position of feature (group f, radial index n) in the angular feature vector
-__device__ __forceinline__ int aidx(int f, int n, int na) { return f * na + n; }
 
 // ------------------------------------------------------------------ neighbor search
 struct NepGeo {
@@ -382,290 +209,6 @@ nep_neighbor_kernel(NepGeo g, const int64_t *__restrict__ frame_start, const int
     for (int64_t k = (basea < maxa ? basea : maxa) + lane; k < maxa; k += WAVE) {
         NL_a[n1 * maxa + k] = -1;
         for (int q = 0; q < w; q++) Ri_a[(n1 * maxa + k) * w + q] = R(0);
-    }
-}
-
-// ------------------------------------------------------------------ feature kernels
-struct FeatArgs {
-    const void *c;          // [T][T][nm][nb]
-    const void *Ri;         // [N][S][4]
-    const int64_t *NL;      // [N][S]
-    const int64_t *atom_map;
-    void *feats;            // [N][ld] (written at column offset col0)
-    void *s_save;           // [N][nm][24] angular sums (angular only)
-    const void *gfeat;      // [N][ld] upstream gradient of feats
-    const void *gg;         // [N][S][4] upstream gradient of the position gradient (2nd order)
-    void *gRi;              // [N][S][4] out
-    void *gc;               // [T][T][nm][nb] out (accumulated)
-    void *ggfeat;           // [N][ld] out (2nd order)
-    int64_t N;
-    int pw;                 // coefficient-gradient tables per wavefront (plain adds) instead of per block (LDS atomics)
-    int S, T, nm, nb, ld, col0, l3, l4, l5;
-    double rc;
-};
-
-// first used slot count (loop stops at the first -1)
-__device__ __forceinline__ int slot_count(const int64_t *NL, int64_t i, int S) {
-    int lo = 0, hi = S;   // NL entries are a valid prefix followed by -1
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (NL[i * S + mid] >= 0) lo = mid + 1; else hi = mid;
-    }
-    return lo;
-}
-
-// The block's coefficient-gradient tables (ntab of count entries: one per wavefront, or one shared)
-// summed and added to global memory, one atomic per entry.
-template <typename T>
-__device__ __forceinline__ void block_flush_add(T *lds, T *glob, int count, int ntab) {
-    __syncthreads();
-    for (int x = threadIdx.x; x < count; x += blockDim.x) {
-        T v = lds[x];
-        for (int w = 1; w < ntab; w++) v += lds[w * count + x];
-        if (v != T(0)) atomic_add(glob + x, v);
-    }
-}
-
-// Feature kernels. Radial: one wavefront per centre atom; angular: a wavefront
-// walks a contiguous range of atoms, several atoms' slots to a chunk (below).
-// Per-neighbor work runs with lanes over the list entries (slots) and writes
-// per-slot factors to a per-wave LDS chunk. Every sum over slots then runs transposed, with lanes
-// over its outputs reading the chunk as broadcasts, so no two lanes of a
-// wavefront ever add to the same address:
-//   radial  q_n                  lanes over slots, wave sums (registers)
-//   radial  dL/dc[ti][tj][n][q]  = g_n sum_{k: tj} v_k[q]: lanes over (tj, q)
-//   angular s_nm, P_nm           = sum_k u_k[n] w_k[m]: lanes over (n, m)
-//   angular dL/dc                = sum_k u_k[n] v_k[q]: lanes over (n, q), one
-//                                  LDS add per lane per slot into the block's table
-// The block's coefficient-gradient table goes to global memory with one atomic
-// per entry at the end.
-// mode: 0 = forward features, 1 = backward (gRi, gc), 2 = second order (ggfeat, gc)
-constexpr int RCH = WAVE;        // radial slots per chunk
-constexpr int ANG_WAVES = 2;     // wavefronts per angular block (LDS per wave is large)
-
-template <typename T, int MODE>
-__global__ void __launch_bounds__(NEP_WAVES * WAVE)
-nep_radial_kernel(FeatArgs a) {
-    extern __shared__ unsigned char smem_raw[];
-    const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
-    const int ncoef = a.T * a.T * a.nm * a.nb;
-    const int ntab = (MODE > 0 && a.pw) ? NEP_WAVES : 1;
-    T *gcl = reinterpret_cast<T *>(smem_raw);                    // [ntab][T*T*nm*nb] tables (MODE > 0)
-    T *gtab = gcl + (ntab > 1 ? wid : 0) * ncoef;                // this wave's table
-    // per-wave chunk: v[RCH][nb] and the neighbor type of each slot (MODE > 0)
-    T *vch = gcl + (size_t)ntab * ncoef + (size_t)wid * RCH * a.nb;
-    int *tch = reinterpret_cast<int *>(gcl + (size_t)ntab * ncoef + (size_t)NEP_WAVES * RCH * a.nb) + wid * RCH;
-    if (MODE > 0) {
-        for (int x = threadIdx.x; x < ntab * ncoef; x += blockDim.x) gcl[x] = T(0);
-        __syncthreads();
-    }
-    const T *c = reinterpret_cast<const T *>(a.c);
-    const T *Ri = reinterpret_cast<const T *>(a.Ri);
-    for (int64_t i = (int64_t)blockIdx.x * NEP_WAVES + wid; i < a.N; i += (int64_t)gridDim.x * NEP_WAVES) {
-        const int ti = (int)a.atom_map[i];
-        const int cnt = slot_count(a.NL, i, a.S);
-        T acc[NM_MAX], g[NM_MAX];
-#pragma unroll
-        for (int n = 0; n < NM_MAX; n++) {
-            acc[n] = T(0);
-            g[n] = (MODE > 0 && n < a.nm) ? reinterpret_cast<const T *>(a.gfeat)[i * a.ld + a.col0 + n] : T(0);
-        }
-        if (MODE == 1)
-            for (int k = cnt + lane; k < a.S; k += WAVE) {
-                T *gRi = reinterpret_cast<T *>(a.gRi) + (i * a.S + k) * 4;
-                gRi[0] = gRi[1] = gRi[2] = gRi[3] = T(0);
-            }
-        for (int k0 = 0; k0 < cnt; k0 += RCH) {
-            const int k = k0 + lane;
-            if (k < cnt) {
-                const int tj = (int)a.atom_map[a.NL[i * a.S + k]];
-                const T r = Ri[(i * a.S + k) * 4];
-                const T gg = MODE == 2 ? reinterpret_cast<const T *>(a.gg)[(i * a.S + k) * 4] : T(0);
-                const T *cij = c + ((int64_t)(ti * a.T + tj) * a.nm) * a.nb;
-                Basis<T> bs(r, (T)a.rc);
-                T sn[NM_MAX];
-#pragma unroll
-                for (int n = 0; n < NM_MAX; n++) sn[n] = T(0);
-                for (int q = 0; q < a.nb; q++) {
-                    T f, fp;
-                    bs.next(f, fp);
-                    const T fq = MODE == 0 ? f : fp;
-#pragma unroll
-                    for (int n = 0; n < NM_MAX; n++)
-                        if (n < a.nm) sn[n] += cij[n * a.nb + q] * fq;
-                    if (MODE == 1) vch[lane * a.nb + q] = f;            // dc = g_n f_q
-                    if (MODE == 2) vch[lane * a.nb + q] = gg * fp;      // dc = g_n gg fp_q
-                }
-                if (MODE == 1) {
-                    T d = T(0);
-#pragma unroll
-                    for (int n = 0; n < NM_MAX; n++)
-                        if (n < a.nm) d += g[n] * sn[n];
-                    T *gRi = reinterpret_cast<T *>(a.gRi) + (i * a.S + k) * 4;
-                    gRi[0] = d; gRi[1] = gRi[2] = gRi[3] = T(0);
-                } else {
-#pragma unroll
-                    for (int n = 0; n < NM_MAX; n++) acc[n] += MODE == 0 ? sn[n] : gg * sn[n];
-                }
-                if (MODE > 0) tch[lane] = tj;
-            }
-            if (MODE > 0) {
-                // dc[ti][tj][n][q] += g_n sum_{slots of type tj} v[q]: lanes over (tj, q)
-                __builtin_amdgcn_wave_barrier();
-                const int nk = cnt - k0 < RCH ? cnt - k0 : RCH;
-                for (int o = lane; o < a.T * a.nb; o += WAVE) {
-                    const int tj = o / a.nb, q = o - tj * a.nb;
-                    T sv = T(0);
-                    for (int kk = 0; kk < nk; kk++)
-                        if (tch[kk] == tj) sv += vch[kk * a.nb + q];
-                    if (sv != T(0)) {
-                        T *gcp = gtab + ((ti * a.T + tj) * a.nm) * a.nb + q;
-                        // lanes own distinct (tj, q): a wave's own table needs no atomics
-#pragma unroll
-                        for (int n = 0; n < NM_MAX; n++)
-                            if (n < a.nm) {
-                                if (ntab > 1) gcp[n * a.nb] += g[n] * sv;
-                                else atomicAdd(gcp + n * a.nb, g[n] * sv);
-                            }
-                    }
-                }
-                __builtin_amdgcn_wave_barrier();
-            }
-        }
-        if (MODE == 0 || MODE == 2) {
-            T *out = reinterpret_cast<T *>(MODE == 0 ? a.feats : a.ggfeat);
-#pragma unroll
-            for (int n = 0; n < NM_MAX; n++) {
-                if (n < a.nm) {
-                    const T v = wave_sum(acc[n]);
-                    if (lane == 0) out[i * a.ld + a.col0 + n] = v;
-                }
-            }
-        }
-    }
-    if (MODE > 0) block_flush_add(gcl, reinterpret_cast<T *>(a.gc), ncoef, ntab);
-}
-
-// Angular features (mode 0): s_nm = sum over an atom's slots of g_n(r) b_m(u), with the slots of up
-// to AB_ATOMS atoms in one 64-lane chunk (an atom has ~16 angular neighbors at rc = 4 A). Lanes take
-// slots for g_n and b_m (written to per-wave LDS rows), then lanes own (n, m) outputs and sum each
-// atom's rows; s goes to s_save (the derivative passes read it) and q_of_s(s) to the features.
-constexpr int AB_ATOMS = 4;      // atoms whose angular slots share one chunk
-
-__host__ __device__ inline int angf_wave_elems(int nm) { return AB_ATOMS * nm * NLM + WAVE * (nm + WS); }
-
-template <typename T>
-__global__ void __launch_bounds__(ANG_WAVES * WAVE)
-nep_angular_fwd_kernel(FeatArgs a) {
-    constexpr int NRED = (NM_MAX * NLM + WAVE - 1) / WAVE;
-    extern __shared__ unsigned char smem_raw[];
-    const int lane = threadIdx.x & (WAVE - 1);
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int per = a.nm * NLM;
-    const int nm = a.nm, nb = a.nb;
-    T *Sq = reinterpret_cast<T *>(smem_raw) + (size_t)wid * angf_wave_elems(nm);   // [AB_ATOMS][nm][24]
-    T *u1 = Sq + AB_ATOMS * per;                                                    // [WAVE][nm] g_n
-    T *w1 = u1 + WAVE * nm;                                                         // [WAVE][WS] b_m
-    const T *c = reinterpret_cast<const T *>(a.c);
-    const T *Ri = reinterpret_cast<const T *>(a.Ri);
-    T *fo = reinterpret_cast<T *>(a.feats);
-    T *so = reinterpret_cast<T *>(a.s_save);
-    const int64_t nw = (int64_t)gridDim.x * ANG_WAVES, gw = (int64_t)blockIdx.x * ANG_WAVES + wid;
-    const int64_t i1 = a.N * (gw + 1) / nw;
-    for (int64_t i = a.N * gw / nw; i < i1;) {
-        const int64_t il = i + (lane < AB_ATOMS ? lane : 0);
-        const int c_l = (lane < AB_ATOMS && il < i1) ? slot_count(a.NL, il, a.S) : -1;
-        int off[AB_ATOMS + 1];
-        off[0] = 0;
-        int na = 0;
-        bool open = true;
-#pragma unroll
-        for (int q = 0; q < AB_ATOMS; q++) {
-            const int cq = __builtin_amdgcn_readlane(c_l, q);
-            open = open && (q == 0 || (cq >= 0 && off[q] + cq <= WAVE));
-            if (open) na = q + 1;
-            off[q + 1] = off[q] + (open ? cq : 0);
-        }
-        const int tot = off[AB_ATOMS];
-        T red[AB_ATOMS][NRED];
-#pragma unroll
-        for (int q = 0; q < AB_ATOMS; q++)
-#pragma unroll
-            for (int j = 0; j < NRED; j++) red[q][j] = T(0);
-        for (int e0 = 0; e0 < tot; e0 += WAVE) {
-            const int nk = tot - e0 < WAVE ? tot - e0 : WAVE;
-            if (lane < nk) {
-                const int e = e0 + lane;
-                int q = 0;
-#pragma unroll
-                for (int qq = 1; qq < AB_ATOMS; qq++) q += (e >= off[qq]) ? 1 : 0;
-                const int64_t ia = i + q;
-                const int k = e - off[q];
-                const int ti = (int)a.atom_map[ia];
-                const int tj = (int)a.atom_map[a.NL[ia * a.S + k]];
-                const T *er = Ri + (ia * a.S + k) * 4;
-                const T r = er[0], ir = T(1) / r;
-                const T *cij = c + ((int64_t)(ti * a.T + tj) * nm) * nb;
-                T gn[NM_MAX];
-                {
-                    Basis<T> bs(r, (T)a.rc);
-#pragma unroll
-                    for (int n = 0; n < NM_MAX; n++) gn[n] = T(0);
-                    for (int qb = 0; qb < nb; qb++) {
-                        T f, fp;
-                        bs.next(f, fp);
-#pragma unroll
-                        for (int n = 0; n < NM_MAX; n++)
-                            if (n < nm) gn[n] += cij[n * nb + qb] * f;
-                    }
-                }
-#pragma unroll
-                for (int n = 0; n < NM_MAX; n++)
-                    if (n < nm) u1[lane * nm + n] = gn[n];
-                blm_each<T>(er[1] * ir, er[2] * ir, er[3] * ir, [&](int m, T bv, T, T, T) { w1[lane * WS + m] = bv; });
-            }
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int q = 0; q < AB_ATOMS; q++) {
-                if (q >= na) break;
-                const int k0 = off[q] - e0 > 0 ? off[q] - e0 : 0;
-                const int k1 = off[q + 1] - e0 < nk ? off[q + 1] - e0 : nk;
-#pragma unroll
-                for (int j = 0; j < NRED; j++) {
-                    const int o = lane + j * WAVE;
-                    if (o < per) {
-                        const int n = o / NLM, m = o - n * NLM;
-                        T sacc = T(0);
-                        for (int kk = k0; kk < k1; kk++) sacc += u1[kk * nm + n] * w1[kk * WS + m];
-                        red[q][j] += sacc;
-                    }
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-#pragma unroll
-        for (int q = 0; q < AB_ATOMS; q++) {
-            if (q >= na) break;
-#pragma unroll
-            for (int j = 0; j < NRED; j++) {
-                const int o = lane + j * WAVE;
-                if (o < per) {
-                    Sq[q * per + o] = red[q][j];
-                    so[(i + q) * per + o] = red[q][j];
-                }
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (lane < na * nm) {
-            const int q = lane / nm, n = lane - q * nm;
-            T qv[6];
-            const int nq = q_of_s<T, T>(Sq + q * per + n * NLM, a.l3, a.l4, a.l5, qv);
-#pragma unroll
-            for (int f = 0; f < 6; f++)
-                if (f < nq) fo[(i + q) * a.ld + a.col0 + aidx(f, n, nm)] = qv[f];
-        }
-        __builtin_amdgcn_wave_barrier();
-        i += na;
     }
 }
 
@@ -1026,462 +569,6 @@ __global__ void nep_virial_grad_kernel(const int64_t *__restrict__ NL, const T *
     }
 }
 
-// The angular descriptor's first derivative (mode 1: gRi and dL/dc), batched like the features: per
-// batch the dE/ds rows (B) of its atoms in LDS, then per slot (lanes) gRi = sum_nm D_nm d(g_n b_m)/dRi
-// and the rows of dc[n][q] = f_q (D b)_n, added with lanes over (n, q) into the table row of each
-// slot's (centre type, neighbor type).
-__host__ __device__ inline int angb_wave_elems(int nm, int nb) { return AB_ATOMS * nm * NLM + WAVE * (nm + nb); }
-
-template <typename T>
-__global__ void __launch_bounds__(ANG_WAVES * WAVE)
-nep_angular_bwd_kernel(FeatArgs a) {
-    extern __shared__ unsigned char smem_raw[];
-    const int lane = threadIdx.x & (WAVE - 1);
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int ncoef = a.T * a.T * a.nm * a.nb;
-    const int per = a.nm * NLM;
-    const int nm = a.nm, nb = a.nb, nmb = nm * nb;
-    const int ntab = a.pw ? ANG_WAVES : 1;
-    T *gcl = reinterpret_cast<T *>(smem_raw);                                  // [ntab][ncoef]
-    T *gtab = gcl + (ntab > 1 ? wid : 0) * ncoef;                             // this wave's table
-    T *Bq = gcl + (size_t)ntab * ncoef + (size_t)wid * angb_wave_elems(nm, nb);   // [AB_ATOMS][nm][24]
-    T *u1 = Bq + AB_ATOMS * per;                                               // [WAVE][nm]
-    T *v1 = u1 + WAVE * nm;                                                    // [WAVE][nb]
-    int *trow = reinterpret_cast<int *>(gcl + (size_t)ntab * ncoef + (size_t)ANG_WAVES * angb_wave_elems(nm, nb)) +
-                wid * WAVE;                                                    // [WAVE] table row per slot
-    for (int x = threadIdx.x; x < ntab * ncoef; x += blockDim.x) gcl[x] = T(0);
-    __syncthreads();
-    const T *c = reinterpret_cast<const T *>(a.c);
-    const T *Ri = reinterpret_cast<const T *>(a.Ri);
-    const T *gfe = reinterpret_cast<const T *>(a.gfeat);
-    T *gRiA = reinterpret_cast<T *>(a.gRi);
-    const int nf = a.l3 + (a.l4 > 0) + (a.l5 > 0);
-    // this wavefront's contiguous range of atoms
-    const int64_t nw = (int64_t)gridDim.x * ANG_WAVES, gw = (int64_t)blockIdx.x * ANG_WAVES + wid;
-    const int64_t i1 = a.N * (gw + 1) / nw;
-    for (int64_t i = a.N * gw / nw; i < i1;) {
-        const int64_t il = i + (lane < AB_ATOMS ? lane : 0);
-        const int c_l = (lane < AB_ATOMS && il < i1) ? slot_count(a.NL, il, a.S) : -1;
-        int off[AB_ATOMS + 1];
-        off[0] = 0;
-        int na = 0;
-        bool open = true;
-#pragma unroll
-        for (int q = 0; q < AB_ATOMS; q++) {
-            const int cq = __builtin_amdgcn_readlane(c_l, q);
-            open = open && (q == 0 || (cq >= 0 && off[q] + cq <= WAVE));
-            if (open) na = q + 1;
-            off[q + 1] = off[q] + (open ? cq : 0);
-        }
-        const int tot = off[AB_ATOMS];
-        // unused slots of each atom get gRi = 0
-        for (int q = 0; q < na; q++) {
-            const int64_t ia = i + q;
-            for (int k = off[q + 1] - off[q] + lane; k < a.S; k += WAVE) {
-                T *g = gRiA + (ia * a.S + k) * 4;
-                g[0] = g[1] = g[2] = g[3] = T(0);
-            }
-        }
-        // B = D = dE/ds of each atom of the batch (lanes over (atom, n))
-        if (lane < na * nm) {
-            const int q = lane / nm, n = lane - q * nm;
-            const int64_t ia = i + q;
-            T gq[6];
-#pragma unroll
-            for (int f = 0; f < 6; f++) gq[f] = f < nf ? gfe[ia * a.ld + a.col0 + aidx(f, n, nm)] : T(0);
-            T D[NLM];
-            dq_ds<T, T>(reinterpret_cast<const T *>(a.s_save) + ia * per + n * NLM, gq, a.l3, a.l4, a.l5, D);
-            for (int m = 0; m < NLM; m++) Bq[q * per + n * NLM + m] = D[m];
-        }
-        __builtin_amdgcn_wave_barrier();
-        for (int e0 = 0; e0 < tot; e0 += WAVE) {
-            const int nk = tot - e0 < WAVE ? tot - e0 : WAVE;
-            const int e = e0 + lane;
-            if (lane < nk) {
-                int q = 0;
-#pragma unroll
-                for (int qq = 1; qq < AB_ATOMS; qq++) q += (e >= off[qq]) ? 1 : 0;
-                const int64_t ia = i + q;
-                const int k = e - off[q];
-                const int ti = (int)a.atom_map[ia];
-                const int tj = (int)a.atom_map[a.NL[ia * a.S + k]];
-                const T *er = Ri + (ia * a.S + k) * 4;
-                const T r = er[0], ir = T(1) / r;
-                const T ux = er[1] * ir, uy = er[2] * ir, uz = er[3] * ir;
-                const T *cij = c + ((int64_t)(ti * a.T + tj) * nm) * nb;
-                trow[lane] = ti * a.T + tj;
-                // g_n, g'_n over the streamed basis, f_q to this slot's v1 row
-                T gn[NM_MAX], gnp[NM_MAX];
-                {
-                    Basis<T> bs(r, (T)a.rc);
-#pragma unroll
-                    for (int n = 0; n < NM_MAX; n++) { gn[n] = T(0); gnp[n] = T(0); }
-                    for (int qb = 0; qb < nb; qb++) {
-                        T f, fp;
-                        bs.next(f, fp);
-#pragma unroll
-                        for (int n = 0; n < NM_MAX; n++)
-                            if (n < nm) { gn[n] += cij[n * nb + qb] * f; gnp[n] += cij[n * nb + qb] * fp; }
-                        v1[lane * nb + qb] = f;
-                    }
-                }
-                // gRi = sum_nm D_nm d(g_n b_m)/dRi; dc[n][q] = f_q (D b)_n
-                const T *B = Bq + q * per;
-                T b[NLM];
-                blm_each<T>(ux, uy, uz, [&](int m, T bv, T, T, T) { b[m] = bv; });
-                T Dg[NLM], Db[NM_MAX];
-#pragma unroll
-                for (int n = 0; n < NM_MAX; n++) Db[n] = T(0);
-                T gr0 = T(0);
-#pragma unroll
-                for (int m = 0; m < NLM; m++) {
-                    T dg = T(0), dgp = T(0);
-#pragma unroll
-                    for (int n = 0; n < NM_MAX; n++)
-                        if (n < nm) {
-                            const T Bv = B[n * NLM + m];
-                            dg += Bv * gn[n];
-                            dgp += Bv * gnp[n];
-                            Db[n] += Bv * b[m];
-                        }
-                    Dg[m] = dg;
-                    gr0 += dgp * b[m];
-                }
-#pragma unroll
-                for (int n = 0; n < NM_MAX; n++)
-                    if (n < nm) u1[lane * nm + n] = Db[n];
-                T V0 = T(0), V1 = T(0), V2 = T(0);
-                blm_each<T>(ux, uy, uz, [&](int m, T, T d0, T d1, T d2) {
-                    V0 += Dg[m] * d0; V1 += Dg[m] * d1; V2 += Dg[m] * d2;
-                });
-                T *g = gRiA + (ia * a.S + k) * 4;
-                g[0] = gr0 - (ux * V0 + uy * V1 + uz * V2) * ir;
-                g[1] = V0 * ir;
-                g[2] = V1 * ir;
-                g[3] = V2 * ir;
-            }
-            __builtin_amdgcn_wave_barrier();
-            // dc[row of slot kk][n][q] += u1[kk][n] v1[kk][q]: lanes over (n, q), no two lanes on one entry
-            for (int o = lane; o < nmb; o += WAVE) {
-                const int n = o / nb, qb = o - n * nb;
-                for (int kk = 0; kk < nk; kk++) {
-                    const T d = u1[kk * nm + n] * v1[kk * nb + qb];
-                    if (ntab > 1) gtab[trow[kk] * nmb + o] += d;
-                    else atomicAdd(gtab + trow[kk] * nmb + o, d);
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-        i += na;
-    }
-    block_flush_add(gcl, reinterpret_cast<T *>(a.gc), ncoef, ntab);
-}
-
-// The angular descriptor's second-order pass (mode 2: ggfeat and dL/dc) with the slots of up to AB
-// atoms in one chunk of CHB lanes, as nep_angular_bwd_kernel does for mode 1: per batch the dE/ds
-// rows (B) of its atoms, a first pass over the slots (the directional derivative P of each atom's
-// s, summed per atom with lanes over (n, m), and the explicit coefficient gradient), then per atom
-// ggfeat = J P and E = H P, and a second pass (the coefficient gradient through s). Float takes 48
-// slots of up to 4 atoms; double keeps 16 slots of one atom (its per-slot rows, 96 values of 8
-// bytes, leave no room for more in LDS).
-template <typename T>
-struct Ang2Shape {
-    static constexpr int CHB = sizeof(T) == 4 ? 48 : 16;
-    static constexpr int AB = sizeof(T) == 4 ? 4 : 1;
-};
-
-template <typename T>
-__host__ __device__ inline int angb2_wave_elems(int nm, int nb) {
-    return Ang2Shape<T>::AB * 2 * nm * NLM + Ang2Shape<T>::CHB * (4 * nm + 2 * WS + 2 * nb);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(ANG_WAVES * WAVE)
-nep_angular_bwd2_kernel(FeatArgs a) {
-    constexpr int CHB = Ang2Shape<T>::CHB, AB = Ang2Shape<T>::AB;
-    constexpr int NRED = (NM_MAX * NLM + WAVE - 1) / WAVE;
-    extern __shared__ unsigned char smem_raw[];
-    const int lane = threadIdx.x & (WAVE - 1);
-    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int ncoef = a.T * a.T * a.nm * a.nb;
-    const int per = a.nm * NLM;
-    const int nm = a.nm, nb = a.nb, nmb = nm * nb;
-    const int ntab = a.pw ? ANG_WAVES : 1;
-    T *gcl = reinterpret_cast<T *>(smem_raw);                                  // [ntab][ncoef]
-    T *gtab = gcl + (ntab > 1 ? wid : 0) * ncoef;                             // this wave's table
-    T *Bq = gcl + (size_t)ntab * ncoef + (size_t)wid * angb2_wave_elems<T>(nm, nb);   // [AB][nm][24] D
-    T *Cq = Bq + AB * per;                                                    // [AB][nm][24] P, then E
-    T *u1 = Cq + AB * per, *u2 = u1 + CHB * nm;                                // g'_n, g_n (pass 2: (E b)_n)
-    T *w1 = u2 + CHB * nm, *w2 = w1 + CHB * WS;                                // beta_m, delta_m
-    T *z1 = w2 + CHB * WS, *z2 = z1 + CHB * nm;                                // (B beta)_n, (B delta)_n
-    T *v1 = z2 + CHB * nm, *v2 = v1 + CHB * nb;                                // f'_q, f_q (pass 2: f_q)
-    int *trow = reinterpret_cast<int *>(gcl + (size_t)ntab * ncoef + (size_t)ANG_WAVES * angb2_wave_elems<T>(nm, nb)) +
-                wid * CHB;                                                     // [CHB] table row per slot
-    for (int x = threadIdx.x; x < ntab * ncoef; x += blockDim.x) gcl[x] = T(0);
-    __syncthreads();
-    const T *c = reinterpret_cast<const T *>(a.c);
-    const T *Ri = reinterpret_cast<const T *>(a.Ri);
-    const T *gfe = reinterpret_cast<const T *>(a.gfeat);
-    const T *sv = reinterpret_cast<const T *>(a.s_save);
-    T *go = reinterpret_cast<T *>(a.ggfeat);
-    const int nf = a.l3 + (a.l4 > 0) + (a.l5 > 0);
-    // dc[row of slot kk][n][q] += p1[kk][n] q1[kk][q] (+ p2 q2): lanes over (n, q)
-    auto add_dc_rows = [&](int nk, const T *p1, const T *q1, const T *p2, const T *q2) {
-        for (int o = lane; o < nmb; o += WAVE) {
-            const int n = o / nb, qb = o - n * nb;
-            for (int kk = 0; kk < nk; kk++) {
-                T d = p1[kk * nm + n] * q1[kk * nb + qb];
-                if (p2) d += p2[kk * nm + n] * q2[kk * nb + qb];
-                if (ntab > 1) gtab[trow[kk] * nmb + o] += d;
-                else atomicAdd(gtab + trow[kk] * nmb + o, d);
-            }
-        }
-    };
-    const int64_t nw = (int64_t)gridDim.x * ANG_WAVES, gw = (int64_t)blockIdx.x * ANG_WAVES + wid;
-    const int64_t i1 = a.N * (gw + 1) / nw;
-    for (int64_t i = a.N * gw / nw; i < i1;) {
-        const int64_t il = i + (lane < AB ? lane : 0);
-        const int c_l = (lane < AB && il < i1) ? slot_count(a.NL, il, a.S) : -1;
-        int off[AB + 1];
-        off[0] = 0;
-        int na = 0;
-        bool open = true;
-#pragma unroll
-        for (int q = 0; q < AB; q++) {
-            const int cq = __builtin_amdgcn_readlane(c_l, q);
-            open = open && (q == 0 || (cq >= 0 && off[q] + cq <= CHB));
-            if (open) na = q + 1;
-            off[q + 1] = off[q] + (open ? cq : 0);
-        }
-        const int tot = off[AB];
-        auto atom_of = [&](int e) {
-            int q = 0;
-#pragma unroll
-            for (int qq = 1; qq < AB; qq++) q += (e >= off[qq]) ? 1 : 0;
-            return q;
-        };
-        // B = D = dE/ds of each atom (lanes over (atom, n))
-        if (lane < na * nm) {
-            const int q = lane / nm, n = lane - q * nm;
-            const int64_t ia = i + q;
-            T gq[6];
-#pragma unroll
-            for (int f = 0; f < 6; f++) gq[f] = f < nf ? gfe[ia * a.ld + a.col0 + aidx(f, n, nm)] : T(0);
-            T D[NLM];
-            dq_ds<T, T>(sv + ia * per + n * NLM, gq, a.l3, a.l4, a.l5, D);
-            for (int m = 0; m < NLM; m++) Bq[q * per + n * NLM + m] = D[m];
-        }
-        __builtin_amdgcn_wave_barrier();
-        T red[AB][NRED];
-#pragma unroll
-        for (int q = 0; q < AB; q++)
-#pragma unroll
-            for (int j = 0; j < NRED; j++) red[q][j] = T(0);
-        // pass 1: P_nm = sum_slots gg . d(g_n b_m)/dRi = g'_n beta_m + g_n delta_m with beta_m = gg0 b_m,
-        // delta_m = (db_m/du . (gg_xyz - gg0 u)) / r; explicit c-gradient
-        // sum_m B_nm dP_nm/dc[n][q] = f'_q (B beta)_n + f_q (B delta)_n
-        for (int e0 = 0; e0 < tot; e0 += CHB) {
-            const int nk = tot - e0 < CHB ? tot - e0 : CHB;
-            if (lane < nk) {
-                const int e = e0 + lane, q = atom_of(e);
-                const int64_t ia = i + q;
-                const int k = e - off[q];
-                const int ti = (int)a.atom_map[ia];
-                const int tj = (int)a.atom_map[a.NL[ia * a.S + k]];
-                const T *er = Ri + (ia * a.S + k) * 4;
-                const T r = er[0], ir = T(1) / r;
-                const T ux = er[1] * ir, uy = er[2] * ir, uz = er[3] * ir;
-                const T *cij = c + ((int64_t)(ti * a.T + tj) * nm) * nb;
-                trow[lane] = ti * a.T + tj;
-                const T *gg = reinterpret_cast<const T *>(a.gg) + (ia * a.S + k) * 4;
-                const T g0 = gg[0];
-                const T gx = gg[1] - g0 * ux, gy = gg[2] - g0 * uy, gz = gg[3] - g0 * uz;
-                T gn[NM_MAX], gnp[NM_MAX];
-                {
-                    Basis<T> bs(r, (T)a.rc);
-#pragma unroll
-                    for (int n = 0; n < NM_MAX; n++) { gn[n] = T(0); gnp[n] = T(0); }
-                    for (int qb = 0; qb < nb; qb++) {
-                        T f, fp;
-                        bs.next(f, fp);
-#pragma unroll
-                        for (int n = 0; n < NM_MAX; n++)
-                            if (n < nm) { gn[n] += cij[n * nb + qb] * f; gnp[n] += cij[n * nb + qb] * fp; }
-                        v2[lane * nb + qb] = f;
-                        v1[lane * nb + qb] = fp;
-                    }
-                }
-                T be[NLM], de[NLM];
-                blm_each<T>(ux, uy, uz, [&](int m, T bv, T d0, T d1, T d2) {
-                    be[m] = g0 * bv;
-                    de[m] = (d0 * gx + d1 * gy + d2 * gz) * ir;
-                });
-#pragma unroll
-                for (int m = 0; m < NLM; m++) {
-                    w1[lane * WS + m] = be[m];
-                    w2[lane * WS + m] = de[m];
-                }
-                const T *B = Bq + q * per;
-#pragma unroll
-                for (int n = 0; n < NM_MAX; n++)
-                    if (n < nm) {
-                        u1[lane * nm + n] = gnp[n];
-                        u2[lane * nm + n] = gn[n];
-                        T sb = T(0), sd = T(0);
-#pragma unroll
-                        for (int m = 0; m < NLM; m++) {
-                            sb += B[n * NLM + m] * be[m];
-                            sd += B[n * NLM + m] * de[m];
-                        }
-                        z1[lane * nm + n] = sb;
-                        z2[lane * nm + n] = sd;
-                    }
-            }
-            __builtin_amdgcn_wave_barrier();
-            // P of each atom over its slots of this chunk: lanes own (n, m) outputs
-#pragma unroll
-            for (int q = 0; q < AB; q++) {
-                if (q >= na) break;
-                const int k0 = off[q] - e0 > 0 ? off[q] - e0 : 0;
-                const int k1 = off[q + 1] - e0 < nk ? off[q + 1] - e0 : nk;
-#pragma unroll
-                for (int j = 0; j < NRED; j++) {
-                    const int o = lane + j * WAVE;
-                    if (o < per) {
-                        const int n = o / NLM, m = o - n * NLM;
-                        T sacc = T(0);
-                        for (int kk = k0; kk < k1; kk++)
-                            sacc += u1[kk * nm + n] * w1[kk * WS + m] + u2[kk * nm + n] * w2[kk * WS + m];
-                        red[q][j] += sacc;
-                    }
-                }
-            }
-            add_dc_rows(nk, z1, v1, z2, v2);
-            __builtin_amdgcn_wave_barrier();
-        }
-        // per atom: ggfeat = J P (directional derivative of q along P); E = H(gq) P
-#pragma unroll
-        for (int q = 0; q < AB; q++) {
-            if (q >= na) break;
-#pragma unroll
-            for (int j = 0; j < NRED; j++)
-                if (lane + j * WAVE < per) Cq[q * per + lane + j * WAVE] = red[q][j];
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (lane < na * nm) {
-            const int q = lane / nm, n = lane - q * nm;
-            const int64_t ia = i + q;
-            Dual<T> sd[NLM];
-            for (int m = 0; m < NLM; m++) sd[m] = Dual<T>(sv[ia * per + n * NLM + m], Cq[q * per + n * NLM + m]);
-            Dual<T> qv[6];
-            const int nq = q_of_s<T, Dual<T>>(sd, a.l3, a.l4, a.l5, qv);
-#pragma unroll
-            for (int f = 0; f < 6; f++)
-                if (f < nq) go[ia * a.ld + a.col0 + aidx(f, n, nm)] = qv[f].e;
-            T gq[6];
-#pragma unroll
-            for (int f = 0; f < 6; f++) gq[f] = f < nf ? gfe[ia * a.ld + a.col0 + aidx(f, n, nm)] : T(0);
-            Dual<T> D[NLM];
-            dq_ds<T, Dual<T>>(sd, gq, a.l3, a.l4, a.l5, D);
-            for (int m = 0; m < NLM; m++) Cq[q * per + n * NLM + m] = D[m].e;     // E = (H P)_m
-        }
-        __builtin_amdgcn_wave_barrier();
-        // pass 2: c-gradient through s, dc[ti][tj][n][q] += (E b)_n f_q over the slots
-        for (int e0 = 0; e0 < tot; e0 += CHB) {
-            const int nk = tot - e0 < CHB ? tot - e0 : CHB;
-            if (lane < nk) {
-                const int e = e0 + lane, q = atom_of(e);
-                const int64_t ia = i + q;
-                const int k = e - off[q];
-                const int ti = (int)a.atom_map[ia];
-                trow[lane] = ti * a.T + (int)a.atom_map[a.NL[ia * a.S + k]];
-                const T *er = Ri + (ia * a.S + k) * 4;
-                const T ir = T(1) / er[0];
-                Basis<T> bs(er[0], (T)a.rc);
-                for (int qb = 0; qb < nb; qb++) {
-                    T f, fp;
-                    bs.next(f, fp);
-                    v1[lane * nb + qb] = f;
-                }
-                T b[NLM];
-                blm_each<T>(er[1] * ir, er[2] * ir, er[3] * ir, [&](int m, T bv, T, T, T) { b[m] = bv; });
-                const T *E = Cq + q * per;
-#pragma unroll
-                for (int n = 0; n < NM_MAX; n++)
-                    if (n < nm) {
-                        T Eb = T(0);
-#pragma unroll
-                        for (int m = 0; m < NLM; m++) Eb += E[n * NLM + m] * b[m];
-                        u1[lane * nm + n] = Eb;
-                    }
-            }
-            __builtin_amdgcn_wave_barrier();
-            add_dc_rows(nk, u1, v1, nullptr, nullptr);
-            __builtin_amdgcn_wave_barrier();
-        }
-        i += na;
-    }
-    block_flush_add(gcl, reinterpret_cast<T *>(a.gc), ncoef, ntab);
-}
-
-template <typename T>
-int feat_launch(FeatArgs &a, int angular, int mode, hipStream_t st) {
-    MATPL_CHECK_ARG(a.nb >= 1 && a.nb <= NB_MAX && a.nm >= 1 && a.nm <= NM_MAX, "nep_feat: basis sizes out of range");
-    MATPL_CHECK_ARG(a.T >= 1 && a.T <= 16, "nep_feat: ntypes out of range");
-    MATPL_CHECK_ARG(!angular || (a.l3 >= 0 && a.l3 <= 4 && (a.l3 == 4 || (a.l4 == 0 && a.l5 == 0))),
-                    "nep_feat: l_max_3 must be 4 when 4/5-body terms are on");
-    MATPL_CHECK_ARG(!angular || a.l5 == 0 || a.l4 > 0, "nep_feat: the 5-body term needs the 4-body term");
-    if (a.N == 0) return OK;
-    const size_t ncoef = (size_t)a.T * a.T * a.nm * a.nb;
-    // LDS of the block for ntab coefficient-gradient tables
-    auto lds_of = [&](size_t ntab) -> size_t {
-        if (!angular)
-            return mode > 0 ? (ntab * ncoef + (size_t)NEP_WAVES * RCH * a.nb) * sizeof(T) +
-                                  (size_t)NEP_WAVES * RCH * sizeof(int)
-                            : 0;
-        if (mode == 1)
-            return (ntab * ncoef + (size_t)ANG_WAVES * angb_wave_elems(a.nm, a.nb)) * sizeof(T) +
-                   (size_t)ANG_WAVES * WAVE * sizeof(int);
-        if (mode == 2)
-            return (ntab * ncoef + (size_t)ANG_WAVES * angb2_wave_elems<T>(a.nm, a.nb)) * sizeof(T) +
-                   (size_t)ANG_WAVES * Ang2Shape<T>::CHB * sizeof(int);
-        return (size_t)ANG_WAVES * angf_wave_elems(a.nm) * sizeof(T);
-    };
-    // float: a table per wavefront (plain adds) when they fit, else one per block (LDS atomics).
-    // Measured on the NEP training batch: float LDS atomic adds keep the LDS busy 3-4x longer than
-    // double ones for the same instruction count (the per-wave tables take the float step from
-    // 9.46 to 9.05 ms), while for double the larger tables cost occupancy (10.3 -> 11.8 ms).
-    const size_t nw = angular ? ANG_WAVES : NEP_WAVES;
-    a.pw = (mode > 0 && sizeof(T) == 4 && lds_of(nw) <= 64 * 1024) ? 1 : 0;
-    const size_t lds = lds_of(a.pw ? nw : 1);
-    MATPL_CHECK_ARG(lds <= 64 * 1024, "nep_feat: LDS %zu too large", lds);
-    const int waves = angular ? ANG_WAVES : NEP_WAVES;
-    int64_t blocks = (a.N + waves - 1) / waves;
-    // gradient modes: a bounded grid (4,096 wavefronts, 16 per CU) keeps the global coefficient
-    // atomics few (one per table entry and block) while hiding the kernels' memory waits (on the
-    // NEP training batch 2,048 wavefronts left them waiting ~65 % of their cycles: float step 8.9
-    // -> 8.3 ms at 4,096; 8,192 gives the same time with twice the atomics)
-    if (mode > 0 && blocks > 4096 / waves) blocks = 4096 / waves;
-    if (blocks > 8192) blocks = 8192;
-    dim3 grid((unsigned)blocks), block(waves * WAVE);
-    if (!angular) {
-        if (mode == 0) hipLaunchKernelGGL((nep_radial_kernel<T, 0>), grid, block, lds, st, a);
-        else if (mode == 1) hipLaunchKernelGGL((nep_radial_kernel<T, 1>), grid, block, lds, st, a);
-        else hipLaunchKernelGGL((nep_radial_kernel<T, 2>), grid, block, lds, st, a);
-        return check_launch("nep_radial_kernel");
-    }
-    if (mode == 1) {
-        hipLaunchKernelGGL((nep_angular_bwd_kernel<T>), grid, block, lds, st, a);
-        return check_launch("nep_angular_bwd_kernel");
-    }
-    if (mode == 2) {
-        hipLaunchKernelGGL((nep_angular_bwd2_kernel<T>), grid, block, lds, st, a);
-        return check_launch("nep_angular_bwd2_kernel");
-    }
-    hipLaunchKernelGGL((nep_angular_fwd_kernel<T>), grid, block, lds, st, a);
-    return check_launch("nep_angular_fwd_kernel");
-}
-
 template <typename T, int NV>
 int scatter_launch(const int64_t *NL, const T *dE, const T *Ri_d, const T *Rij, T *out, int64_t N, int S,
                    hipStream_t st) {
@@ -1602,25 +689,6 @@ MATPL_EXPORT int matpl_nep_neighbor_ri32(const double *box, const double *box_or
                        frame_start, atom_frame, nullptr, pos, rc_r, rc_a, maxr, maxa, n, 0, rij4, NN_r, NL_r, NN_a,
                        NL_a, Ri_r, Ri_a, status);
     return check_launch("nep_neighbor_kernel");
-}
-
-MATPL_EXPORT int matpl_nep_feat(int f64, int angular, int mode, const void *c, const void *Ri, const int64_t *NL,
-                                const int64_t *atom_map, int64_t N, int S, int T, int nm, int nb, int ld, int col0,
-                                int l3, int l4, int l5, double rc, void *feats, void *s_save, const void *gfeat,
-                                const void *gg, void *gRi, void *gc, void *ggfeat, void *stream) {
-    FeatArgs a{};
-    a.c = c; a.Ri = Ri; a.NL = NL; a.atom_map = atom_map; a.feats = feats; a.s_save = s_save; a.gfeat = gfeat;
-    a.gg = gg; a.gRi = gRi; a.gc = gc; a.ggfeat = ggfeat;
-    a.N = N; a.S = S; a.T = T; a.nm = nm; a.nb = nb; a.ld = ld; a.col0 = col0; a.l3 = l3; a.l4 = l4; a.l5 = l5;
-    a.rc = rc;
-    MATPL_CHECK_ARG(mode >= 0 && mode <= 2, "nep_feat: bad mode");
-    MATPL_CHECK_ARG(N == 0 || (c && Ri && NL && atom_map), "nep_feat: null input");
-    MATPL_CHECK_ARG(mode != 0 || N == 0 || (feats && (!angular || s_save)), "nep_feat: null output");
-    MATPL_CHECK_ARG(mode != 1 || N == 0 || (gfeat && gRi && gc && (!angular || s_save)), "nep_feat: null grad io");
-    MATPL_CHECK_ARG(mode != 2 || N == 0 || (gfeat && gg && gc && ggfeat && (!angular || s_save)),
-                    "nep_feat: null 2nd-order io");
-    hipStream_t st = (hipStream_t)stream;
-    return f64 ? feat_launch<double>(a, angular, mode, st) : feat_launch<float>(a, angular, mode, st);
 }
 
 MATPL_EXPORT int matpl_nep_force(int f64, const int64_t *NL, const void *dE, const void *Ri_d, void *F, int64_t N, int S,
