@@ -514,14 +514,33 @@ int matpl_nep_feat(int f64, int angular, int mode, const void *c, const void *Ri
  * needs): arguments as there, save [N][nm*24] the angular sums s or [N][T*nb] the radial basis sums.
  *  mode 0: feats and save (radial: save may be null);
  *  mode 1: gRi only, for gfeat (angular: reads save);
- *  mode 2: second order: ggfeat and gc; angular: the gradient of s goes to gsave [N][nm*24] instead of
- *          into gc, for the caller's mode 3 to add (gs there);
+ *  mode 2: second order: ggfeat and gc, for gg or, if gg is null, for the upstream gradients gF [N][3] and
+ *          gV [frames][9] (either may be null) of matpl_nep_model_forces' outputs; angular: the gradient of s
+ *          goes to gsave [N][nm*24] instead of into gc, for the caller's mode 3 to add (gs there);
  *  mode 3: gc only, from gfeat and save (angular: gs, if not null, is added to dL/ds; gfeat may then be null).
  */
 int matpl_nep_descriptor(int f64, int angular, int mode, const void *c, const void *Ri, const int64_t *NL,
                          const int64_t *atom_map, int64_t N, int S, int T, int nm, int nb, int ld, int col0, int l3,
                          int l4, int l5, double rc, void *feats, void *save, const void *gfeat, const void *gs,
-                         const void *gg, void *gRi, void *gc, void *ggfeat, void *gsave, void *stream);
+                         const void *gg, const void *gF, const void *gV, const int32_t *atom_frame, void *gRi,
+                         void *gc, void *ggfeat, void *gsave, void *stream);
+
+/*
+ * Forces F [N][3] and frame virials V [frames][9] of the NEP model (its own signs, src/model/nep_net.py:600-648)
+ * from gfeat = dEtot/dq [N][ld] (radial features first, then the angular ones) and the angular sums s_save: the
+ * descriptor's position gradient and the force terms of both lists in one kernel. frame_start [frames + 1] and
+ * atom_frame [N] give each atom's frame, max_frame the largest frame's atoms; every list entry should name an
+ * atom of its own frame (others are added atomically). l3 = 0: no angular part. work:
+ * matpl_nep_model_forces_work bytes.
+ */
+int64_t matpl_nep_model_forces_work(int f64, int64_t N, int64_t nframes, int64_t max_frame, int ntypes, int na,
+                                    int nbr);
+int matpl_nep_model_forces(int f64, const void *c2, const void *c3, const void *Ri_r, const int64_t *NL_r,
+                           const void *Ri_a, const int64_t *NL_a, const int64_t *atom_map, const int64_t *frame_start,
+                           const int32_t *atom_frame, int64_t nframes, int64_t max_frame, int64_t N, int S_r, int S_a,
+                           int T, int nr, int nbr, int na, int nba, int ld, int l3, int l4, int l5, double rc_r,
+                           double rc_a, const void *gfeat, const void *s_save, void *F, void *V, void *work,
+                           int64_t work_bytes, void *stream);
 
 /*
  * Neighbor scatter F[NL[i][k]] += dE[i][k] . Ri_d[i][k] (a 4x3 contraction)

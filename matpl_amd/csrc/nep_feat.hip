@@ -192,6 +192,8 @@ struct FeatArgs {
     void *gc;               // [T][T][nm][nb] out (accumulated)
     void *ggfeat;           // [N][ld] out (2nd order)
     void *gsave;            // angular 2nd order: [N][nm][24] gradient of s out (null: its coefficient gradient is taken here)
+    const void *gF, *gV;    // 2nd order without gg: upstream gradients of the forces [N][3] and frame virials [F][9]
+    const int32_t *atom_frame;
     int64_t N;
     int pw;                 // coefficient-gradient tables per wavefront (plain adds) instead of per block (LDS atomics)
     int S, T, nm, nb, ld, col0, l3, l4, l5;
@@ -216,6 +218,31 @@ __device__ __forceinline__ Row4<T> load4(const T *p) { return *reinterpret_cast<
 template <typename T>
 __device__ __forceinline__ void store4(T *p, T a, T b, T c, T d) {
     *reinterpret_cast<Row4<T> *>(p) = Row4<T>{{a, b, c, d}};
+}
+
+// The second-order pass's gg of slot s (atom i -> j, row er = [r, x, y, z]): read, or formed from the upstream
+// gradients of the model's forces F and frame virials V (either may be null). With f(s) = dE[s][0] u +
+// dE[s][1:4], F[j] -= f, F[i] += f and V -= f (x) x, so dL/df = q = gF[i] - gF[j] - gV x and gg = [q . u, q].
+template <typename T>
+__device__ __forceinline__ Row4<T> slot_gg(const FeatArgs &a, int64_t s, int64_t i, int64_t j, const Row4<T> &er) {
+    if (a.gg) return load4(reinterpret_cast<const T *>(a.gg) + s * 4);
+    Row4<T> g{{T(0), T(0), T(0), T(0)}};
+    if (fabs(er.v[0]) > T(1e-5)) {
+        const T *gF = reinterpret_cast<const T *>(a.gF), *gV = reinterpret_cast<const T *>(a.gV);
+        T q[3] = {T(0), T(0), T(0)};
+        if (gF) {
+#pragma unroll
+            for (int x = 0; x < 3; x++) q[x] = gF[3 * i + x] - gF[3 * j + x];
+        }
+        if (gV) {
+            const T *v = gV + 9 * (int64_t)a.atom_frame[i];
+#pragma unroll
+            for (int x = 0; x < 3; x++) q[x] -= v[3 * x] * er.v[1] + v[3 * x + 1] * er.v[2] + v[3 * x + 2] * er.v[3];
+        }
+        const T ir = T(1) / er.v[0];
+        g = Row4<T>{{(q[0] * er.v[1] + q[1] * er.v[2] + q[2] * er.v[3]) * ir, q[0], q[1], q[2]}};
+    }
+    return g;
 }
 
 // NL rows are a valid prefix followed by -1: its length, for rows whose first 64 entries are all valid.
@@ -340,7 +367,8 @@ nep_radial_kernel(FeatArgs a) {
                 int start = 0, pos = 0;
                 if constexpr (SUM) pos = sort_by_type(live, tj, a.T, lane, start);
                 if (live) {
-                    const T gg = (WHAT & R_2ND) ? reinterpret_cast<const T *>(a.gg)[s * 4] : T(0);
+                    T gg = T(0);
+                    if constexpr ((WHAT & R_2ND) != 0) gg = slot_gg<T>(a, s, i, j, load4(Ri + s * 4)).v[0];
                     Basis<T> bs(Ri[s * 4], (T)a.rc);
                     T d = T(0);
                     T *row = rows + pos * st;
@@ -611,6 +639,38 @@ __device__ __forceinline__ void radial_fn(const T *cij, T r, T rc, int nm, int n
     }
 }
 
+// The first derivative of one angular slot: (D b)_n for every n and, with GRI, dE/d[r, x, y, z]; B the atom's D
+// rows [nm][24], u the slot's unit vector. With (D b)_n at hand the radial part of dE/dr is sum_n g'_n (D b)_n.
+template <typename T, int NMC, bool GRI>
+__device__ __forceinline__ void angular_slot(const T *B, int nm, T ux, T uy, T uz, T ir, const T gn[NM_MAX],
+                                             const T gp[NM_MAX], T Db[NM_MAX], T d[4]) {
+    T bm[NLM], Dg[NLM];
+    blm_each<T>(ux, uy, uz, [&](int m, T bv, T, T, T) { bm[m] = bv; Dg[m] = T(0); });
+#pragma unroll
+    for (int n = 0; n < (NMC ? NMC : NM_MAX); n++) {
+        Db[n] = T(0);
+        if (n < nm) {
+#pragma unroll
+            for (int m = 0; m < NLM; m++) {
+                const T Bv = B[n * NLM + m];
+                Db[n] += Bv * bm[m];
+                if constexpr (GRI) Dg[m] += Bv * gn[n];
+            }
+        }
+    }
+    if constexpr (GRI) {
+        T gr = T(0), V0 = T(0), V1 = T(0), V2 = T(0);
+#pragma unroll
+        for (int n = 0; n < (NMC ? NMC : NM_MAX); n++)
+            if (n < nm) gr += gp[n] * Db[n];
+        blm_each<T>(ux, uy, uz, [&](int m, T, T d0, T d1, T d2) {
+            V0 += Dg[m] * d0; V1 += Dg[m] * d1; V2 += Dg[m] * d2;
+        });
+        d[0] = gr - (ux * V0 + uy * V1 + uz * V2) * ir;
+        d[1] = V0 * ir; d[2] = V1 * ir; d[3] = V2 * ir;
+    }
+}
+
 // ------------------------------------------------------------------ angular features (mode 0)
 constexpr int ANG_WAVES = 2;     // wavefronts per angular block (LDS per wave is large)
 
@@ -690,8 +750,7 @@ nep_angular_fwd_kernel(FeatArgs a) {
 // ------------------------------------------------------------------ angular first derivative
 // GRI: gRi = sum_nm D_nm d(g_n b_m)/dRi of every slot; GC: dc[ti][tj][n][q] = f_q (D b)_n (mode 1: both;
 // alone: the position gradient of a force pass, or the coefficient gradient of a training step with gs, the
-// second-order pass's gradient of s, added to D). With (D b)_n at hand the radial part of dE/dr is
-// sum_n g'_n (D b)_n.
+// second-order pass's gradient of s, added to D).
 __host__ __device__ inline int angb_wave_elems(int nm, int nb, bool gc) {
     return ANG_AB * nm * NLM + (gc ? WAVE * ((nm + nb) | 1) : 0);
 }
@@ -759,32 +818,14 @@ nep_angular_bwd_kernel(FeatArgs a) {
                         bs.step();
                     }
                 }
-                const T *B = Bq + q * per;
-                T bm[NLM], Dg[NLM], Db[NM_MAX];
-                blm_each<T>(ux, uy, uz, [&](int m, T bv, T, T, T) { bm[m] = bv; Dg[m] = T(0); });
-#pragma unroll
-                for (int n = 0; n < (NMC ? NMC : NM_MAX); n++) {
-                    Db[n] = T(0);
-                    if (n < nm) {
-#pragma unroll
-                        for (int m = 0; m < NLM; m++) {
-                            const T Bv = B[n * NLM + m];
-                            Db[n] += Bv * bm[m];
-                            if constexpr (GRI) Dg[m] += Bv * gn[n];
-                        }
-                        if constexpr (GC) row[n] = Db[n];
-                    }
-                }
-                if constexpr (GRI) {
-                    T gr = T(0), V0 = T(0), V1 = T(0), V2 = T(0);
+                T Db[NM_MAX], d[4];
+                angular_slot<T, NMC, GRI>(Bq + q * per, nm, ux, uy, uz, ir, gn, gp, Db, d);
+                if constexpr (GC) {
 #pragma unroll
                     for (int n = 0; n < (NMC ? NMC : NM_MAX); n++)
-                        if (n < nm) gr += gp[n] * Db[n];
-                    blm_each<T>(ux, uy, uz, [&](int m, T, T d0, T d1, T d2) {
-                        V0 += Dg[m] * d0; V1 += Dg[m] * d1; V2 += Dg[m] * d2;
-                    });
-                    store4<T>(gRiA + s * 4, gr - (ux * V0 + uy * V1 + uz * V2) * ir, V0 * ir, V1 * ir, V2 * ir);
+                        if (n < nm) row[n] = Db[n];
                 }
+                if constexpr (GRI) store4<T>(gRiA + s * 4, d[0], d[1], d[2], d[3]);
             }
             if constexpr (GC) {
                 wave_sync();
@@ -842,7 +883,6 @@ nep_angular_bwd2_kernel(FeatArgs a) {
     __syncthreads();
     const T *c = reinterpret_cast<const T *>(a.c);
     const T *Ri = reinterpret_cast<const T *>(a.Ri);
-    const T *gga = reinterpret_cast<const T *>(a.gg);
     const T *gfe = reinterpret_cast<const T *>(a.gfeat);
     const T *sv = reinterpret_cast<const T *>(a.save);
     T *go = reinterpret_cast<T *>(a.ggfeat);
@@ -870,7 +910,7 @@ nep_angular_bwd2_kernel(FeatArgs a) {
             T f[NBM], fp[NBM], zb[NM_MAX], zd[NM_MAX];
             if (live) {
                 // rows for P, in the slots' own order: g'_n, g_n | beta_m, delta_m
-                const Row4<T> er = load4(Ri + s * 4), gg = load4(gga + s * 4);
+                const Row4<T> er = load4(Ri + s * 4), gg = slot_gg<T>(a, s, i + q, a.NL[s], er);
                 const T ir = T(1) / er.v[0];
                 const T ux = er.v[1] * ir, uy = er.v[2] * ir, uz = er.v[3] * ir;
                 const T g0 = gg.v[0], gx = (gg.v[1] - g0 * ux) * ir, gy = (gg.v[2] - g0 * uy) * ir,
@@ -999,6 +1039,279 @@ nep_angular_bwd2_kernel(FeatArgs a) {
     block_flush_add(gcl, reinterpret_cast<T *>(a.gc), ncoef, ntab);
 }
 
+// ------------------------------------------------------------------ model forces
+// F [N][3] and the frame virials V [F][9] of the NEP model straight from dE/dq: the radial and angular slot
+// derivatives (nep_radial_kernel R_GRI, nep_angular_bwd_kernel GRI) and the force terms of each slot,
+// f = dE[s][0] (x, y, z)/r + dE[s][1:4] (src/model/nep_net.py:440-468 and :608; calculateNepForce,
+// CalcOps.cpp:75-158; the frame sum of calculateNepVirial, CalcOps.cpp:239-328), with the model's signs
+// (nep_net.py negates both): F[i] += f, F[j] -= f, V[frame] -= f (x) x. No [N][S][4] gradient is written or read.
+// A block takes windows of `ch` consecutive atoms, frame by frame (a segment); neighbor terms go to an LDS copy
+// of F over the segment's frame (n <= rcap atoms), written once to the segment's row of `part`, since device
+// atomics are carried out beyond the per-XCD L2 caches here; nep_force_final_kernel adds the rows. Segment
+// (window b, frame f) has row b + f: consecutive segments advance b or f. Larger frames (rcap = 0), and any
+// entry naming an atom of another frame, use global atomics.
+struct ForceArgs {
+    FeatArgs r, a;                // radial / angular: c, Ri, NL, atom_map, gfeat, save, sizes
+    const int64_t *frame_start;   // [F + 1]
+    const int32_t *atom_frame;    // [N]
+    void *F, *part;               // [N][3] (zeroed), [segments][3 rcap]
+    double *vpart;                // [segments][9]
+    int64_t rcap;
+    int ch;
+};
+
+// Sum over the wavefront of up to 16 values per lane at once: lane l returns the total of v[l % 16]. Each step
+// exchanges half of the values still held (17 exchanges, not 6 per value).
+template <typename T>
+__device__ __forceinline__ T fold16(T v[16], int lane) {
+#pragma unroll
+    for (int b = 0, n = 8; b < 4; b++, n >>= 1)
+#pragma unroll
+        for (int k = 0; k < n; k++) {
+            const bool hi = (lane >> b) & 1;
+            const T keep = hi ? v[2 * k + 1] : v[2 * k], send = hi ? v[2 * k] : v[2 * k + 1];
+            v[k] = keep + __shfl_xor(send, 1 << b, WAVE);
+        }
+    T x = v[0];
+    x += __shfl_xor(x, 16, WAVE);
+    x += __shfl_xor(x, 32, WAVE);
+    return x;
+}
+
+// (141 float and 256 double VGPRs: 3 and 2 wavefronts per SIMD, which blocks of 4 wavefronts fill; of 8, one
+// float block fits a CU)
+constexpr int FORCE_WAVES = 4;
+
+template <typename T>
+inline size_t force_fixed_lds(int T_, int na, int nbr) {
+    return (size_t)FORCE_WAVES * (((size_t)ANG_AB * na * NLM + (size_t)T_ * nbr) * sizeof(T) + 9 * sizeof(double));
+}
+
+template <typename T, int NMC, int NBC>
+__global__ void __launch_bounds__(FORCE_WAVES * WAVE, sizeof(T) == 4 ? 3 : 2)
+nep_force_kernel(ForceArgs p) {
+    extern __shared__ unsigned char smem_raw[];
+    constexpr int W = FORCE_WAVES;
+    const FeatArgs &R = p.r, &A = p.a;
+    const int lane = threadIdx.x & (WAVE - 1), wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int nr = NMC ? NMC : R.nm, nbr = NBC ? NBC : R.nb, na = NMC ? NMC : A.nm, nba = NBC ? NBC : A.nb;
+    const int per = A.l3 > 0 ? na * NLM : 0, tb = R.T * nbr;       // as force_fixed_lds counts (na = 0 without angular part)
+    double *vred = reinterpret_cast<double *>(smem_raw);                          // [W][9]
+    T *Bq = reinterpret_cast<T *>(vred + W * 9) + (size_t)wid * ANG_AB * per;     // [AB][na][24]
+    T *wt = reinterpret_cast<T *>(vred + W * 9) + (size_t)W * ANG_AB * per + (size_t)wid * tb;   // [T][nbr]
+    T *acc = reinterpret_cast<T *>(vred + W * 9) + (size_t)W * (ANG_AB * per + tb);               // [3 rcap]
+    T *F = reinterpret_cast<T *>(p.F);
+    const int64_t i0 = (int64_t)blockIdx.x * p.ch, i1 = i0 + p.ch < R.N ? i0 + p.ch : R.N;
+    const int f1 = p.atom_frame[i1 - 1];
+    for (int f = p.atom_frame[i0]; f <= f1; f++) {
+        const int64_t fs = p.frame_start[f], fe = p.frame_start[f + 1];
+        const int64_t s0 = i0 > fs ? i0 : fs, s1 = i1 < fe ? i1 : fe;
+        if (s0 >= s1) continue;
+        const bool lds = fe - fs <= p.rcap;
+        if (lds)
+            for (int64_t x = threadIdx.x; x < 3 * (fe - fs); x += blockDim.x) acc[x] = T(0);
+        __syncthreads();
+        auto add = [&](int64_t j, int c, T v) {
+            if (lds && j >= fs && j < fe) atomicAdd(acc + 3 * (j - fs) + c, v);
+            else atomic_add(F + 3 * j + c, v);
+        };
+        T vir[9];
+#pragma unroll
+        for (int x = 0; x < 9; x++) vir[x] = T(0);
+        // radial list: one wavefront per atom, lanes over slots
+        const T *Rr = reinterpret_cast<const T *>(R.Ri), *Ra = reinterpret_cast<const T *>(A.Ri);
+        for (int64_t i = s0 + wid; i < s1; i += W) {
+            const T *ci = reinterpret_cast<const T *>(R.c) + (int64_t)R.atom_map[i] * R.T * nr * nbr;
+            const T *gi = reinterpret_cast<const T *>(R.gfeat) + i * R.ld + R.col0;
+            for (int o = lane; o < tb; o += WAVE) {
+                const int t = o / nbr, q = o - t * nbr;
+                T w = T(0);
+#pragma unroll
+                for (int n = 0; n < (NMC ? NMC : NM_MAX); n++)
+                    if (n < nr) w += gi[n] * ci[(t * nr + n) * nbr + q];
+                wt[o] = w;
+            }
+            wave_sync();
+            T cen[3] = {T(0), T(0), T(0)};
+            for (int k0 = 0; k0 < R.S; k0 += WAVE) {
+                const int k = k0 + lane;
+                const int64_t s = i * R.S + k;
+                const int64_t j = k < R.S ? R.NL[s] : -1;
+                const uint64_t end = __ballot(j < 0);
+                if (lane < (end ? __builtin_ctzll(end) : WAVE)) {
+                    const Row4<T> er = load4(Rr + s * 4);
+                    const T *w = wt + (int)R.atom_map[j] * nbr;
+                    Basis<T> bs(er.v[0], (T)R.rc);
+                    T d = T(0);
+#pragma unroll
+                    for (int q = 0; q < (NBC ? NBC : NB_MAX); q++) {
+                        if (NBC == 0 && q >= nbr) continue;
+                        d += w[q] * bs.slope();
+                        bs.step();
+                    }
+                    if (fabs(er.v[0]) > T(1e-5)) {
+                        const T dr = d / er.v[0];
+#pragma unroll
+                        for (int x = 0; x < 3; x++) {
+                            const T fx = dr * er.v[1 + x];
+                            cen[x] += fx;
+                            add(j, x, -fx);
+#pragma unroll
+                            for (int y = 0; y < 3; y++) vir[3 * x + y] -= fx * er.v[1 + y];
+                        }
+                    }
+                }
+                if (end) break;
+            }
+#pragma unroll
+            for (int x = 0; x < 3; x++) {
+                const T c = wave_sum(cen[x]);
+                if (lane == x) add(i, x, c);
+            }
+            wave_sync();
+        }
+        // angular list: a contiguous part of the segment's atoms per wavefront, several atoms to a pass
+        if (A.l3 > 0) {
+            int64_t i = s0 + (s1 - s0) * wid / W;
+            const int64_t e1 = s0 + (s1 - s0) * (wid + 1) / W;
+            while (i < e1) {
+                const Batch<ANG_AB> b = next_batch<ANG_AB, WAVE>(A, i, e1, lane);
+                batch_dq<T, ANG_AB>(A, b, i, na, lane, Bq, nullptr);
+                wave_sync();
+                T cen[16];
+#pragma unroll
+                for (int x = 0; x < 16; x++) cen[x] = T(0);
+                for (int e0 = 0; e0 < b.tot; e0 += WAVE) {
+                    if (lane < b.tot - e0) {
+                        const int e = e0 + lane, q = b.atom(e);
+                        const int64_t s = (i + q) * A.S + (e - b.first(q)), j = A.NL[s];
+                        const Row4<T> er = load4(Ra + s * 4);
+                        const T ir = T(1) / er.v[0];
+                        const T ux = er.v[1] * ir, uy = er.v[2] * ir, uz = er.v[3] * ir;
+                        T gn[NM_MAX], gp[NM_MAX];
+                        radial_fn<T, NMC, NBC, true>(
+                            reinterpret_cast<const T *>(A.c) + (int64_t)(b.ti * A.T + (int)A.atom_map[j]) * na * nba,
+                            er.v[0], (T)A.rc, na, nba, gn, gp, [](int, T, T) {});
+                        T Db[NM_MAX], d[4];
+                        angular_slot<T, NMC, true>(Bq + q * per, na, ux, uy, uz, ir, gn, gp, Db, d);
+                        // (selects, not a branch: the compiler would move the slot's work behind it and spill)
+                        const bool far = fabs(er.v[0]) > T(1e-5);
+                        const T fx[3] = {far ? d[0] * ux + d[1] : T(0), far ? d[0] * uy + d[2] : T(0),
+                                         far ? d[0] * uz + d[3] : T(0)};
+#pragma unroll
+                        for (int x = 0; x < 3; x++) {
+                            add(j, x, -fx[x]);
+#pragma unroll
+                            for (int y = 0; y < 3; y++) vir[3 * x + y] -= fx[x] * er.v[1 + y];
+#pragma unroll
+                            for (int u = 0; u < ANG_AB; u++) cen[3 * u + x] += q == u ? fx[x] : T(0);
+                        }
+                    }
+                }
+                const T c = fold16<T>(cen, lane);
+                if (lane < 3 * b.na) add(i + lane / 3, lane % 3, c);
+                wave_sync();
+                i += b.na;
+            }
+        }
+        T vf[16];
+#pragma unroll
+        for (int x = 0; x < 16; x++) vf[x] = x < 9 ? vir[x] : T(0);
+        const T vs = fold16<T>(vf, lane);
+        if (lane < 9) vred[wid * 9 + lane] = (double)vs;
+        __syncthreads();
+        const int64_t seg = (int64_t)blockIdx.x + f;
+        if (threadIdx.x < 9) {
+            double v = 0.0;
+            for (int w = 0; w < W; w++) v += vred[w * 9 + threadIdx.x];
+            p.vpart[seg * 9 + threadIdx.x] = v;
+        }
+        if (lds) {
+            T *o = reinterpret_cast<T *>(p.part) + seg * 3 * p.rcap;
+            for (int64_t x = threadIdx.x; x < 3 * (fe - fs); x += blockDim.x) o[x] = acc[x];
+        }
+        __syncthreads();
+    }
+}
+
+// F += the segments' LDS copies (blocks [0, fblocks): 64 entries, the segments of their frame in 4 groups), and
+// each frame's virial from its segments' sums (one block per frame after them).
+template <typename T>
+__global__ void __launch_bounds__(256)
+nep_force_final_kernel(const int64_t *__restrict__ frame_start, const int32_t *__restrict__ atom_frame, int64_t N,
+                       int ch, int64_t rcap, const T *__restrict__ part, const double *__restrict__ vpart,
+                       T *__restrict__ F, T *__restrict__ V, int64_t fblocks) {
+    __shared__ double red[256];
+    if ((int64_t)blockIdx.x >= fblocks) {
+        const int64_t f = (int64_t)blockIdx.x - fblocks, fs = frame_start[f], fe = frame_start[f + 1];
+        const int c = threadIdx.x % 9, g = threadIdx.x / 9;          // 28 groups of 9 components
+        double s = 0.0;
+        if (fs < fe && g < 28)
+            for (int64_t b = fs / ch + g; b <= (fe - 1) / ch; b += 28) s += vpart[(b + f) * 9 + c];
+        red[threadIdx.x] = s;
+        __syncthreads();
+        if (threadIdx.x < 9) {
+            s = 0.0;
+            for (int q = 0; q < 28; q++) s += red[9 * q + threadIdx.x];
+            V[9 * f + threadIdx.x] = (T)s;
+        }
+        return;
+    }
+    T *redT = reinterpret_cast<T *>(red);
+    const int el = threadIdx.x & 63, g = threadIdx.x >> 6;
+    const int64_t e = (int64_t)blockIdx.x * 64 + el;
+    T s = T(0);
+    bool any = false;
+    if (e < 3 * N) {
+        const int64_t j = e / 3;
+        const int f = atom_frame[j];
+        const int64_t fs = frame_start[f], fe = frame_start[f + 1];
+        any = fe - fs <= rcap;
+        if (any) {
+            const T *q = part + (e - 3 * fs);
+            const int64_t b1 = (fe - 1) / ch;
+#pragma unroll 4
+            for (int64_t b = fs / ch + g; b <= b1; b += 4) s += q[(b + f) * 3 * rcap];
+        }
+    }
+    redT[threadIdx.x] = s;
+    __syncthreads();
+    if (g == 0 && any) F[e] += ((redT[el] + redT[el + 64]) + (redT[el + 128] + redT[el + 192]));
+}
+
+// The window, and the LDS copy of F: frames of at most rcap atoms within the block's 64 KB. Windows shrink with
+// the atom count, down to 8, so that a small system still fills the chip.
+struct ForcePlan {
+    int ch;
+    int64_t rcap;
+    size_t lds;
+};
+template <typename T>
+inline ForcePlan force_plan(int64_t N, int64_t max_frame, int ntypes, int na, int nbr) {
+    const size_t fixed = force_fixed_lds<T>(ntypes, na, nbr);
+    int64_t ch = (N + 511) / 512;
+    ch = ch < 8 ? 8 : (ch > 64 ? 64 : ch);
+    const int64_t cap = fixed < 64 * 1024 ? (int64_t)((64 * 1024 - fixed) / (3 * sizeof(T))) : 0;
+    const int64_t rcap = max_frame <= cap ? max_frame : 0;
+    return {(int)ch, rcap, fixed + 3 * rcap * sizeof(T)};
+}
+
+template <typename T, int NMC, int NBC>
+int force_launch(ForceArgs &p, const ForcePlan &pl, int64_t nframes, T *V, hipStream_t st) {
+    const int64_t N = p.r.N, blocks = ceil_div(N, pl.ch);
+    p.ch = pl.ch;
+    p.rcap = pl.rcap;
+    hipLaunchKernelGGL((nep_force_kernel<T, NMC, NBC>), dim3((unsigned)blocks), dim3(FORCE_WAVES * WAVE), pl.lds, st,
+                       p);
+    int rc = check_launch("nep_force_kernel");
+    if (rc) return rc;
+    const int64_t fblocks = pl.rcap > 0 ? ceil_div(3 * N, 64) : 0;
+    hipLaunchKernelGGL(nep_force_final_kernel<T>, dim3((unsigned)(fblocks + nframes)), dim3(256), 0, st, p.frame_start,
+                       p.atom_frame, N, pl.ch, pl.rcap, reinterpret_cast<const T *>(p.part), p.vpart,
+                       reinterpret_cast<T *>(p.F), V, fblocks);
+    return check_launch("nep_force_final_kernel");
+}
+
 // ------------------------------------------------------------------ launch
 enum FeatWhat { W_FEAT, W_GRI, W_GRI_GC, W_GC, W_2ND, W_2ND_GS };
 
@@ -1108,11 +1421,13 @@ MATPL_EXPORT int matpl_nep_feat(int f64, int angular, int mode, const void *c, c
 MATPL_EXPORT int matpl_nep_descriptor(int f64, int angular, int mode, const void *c, const void *Ri, const int64_t *NL,
                                       const int64_t *atom_map, int64_t N, int S, int T, int nm, int nb, int ld,
                                       int col0, int l3, int l4, int l5, double rc, void *feats, void *save,
-                                      const void *gfeat, const void *gs, const void *gg, void *gRi, void *gc,
-                                      void *ggfeat, void *gsave, void *stream) {
+                                      const void *gfeat, const void *gs, const void *gg, const void *gF,
+                                      const void *gV, const int32_t *atom_frame, void *gRi, void *gc, void *ggfeat,
+                                      void *gsave, void *stream) {
     FeatArgs a{};
     a.c = c; a.Ri = Ri; a.NL = NL; a.atom_map = atom_map; a.feats = feats; a.save = save;
     a.gfeat = gfeat; a.gs = angular ? gs : nullptr; a.gg = gg; a.gRi = gRi; a.gc = gc; a.ggfeat = ggfeat; a.gsave = gsave;
+    a.gF = gF; a.gV = gV; a.atom_frame = atom_frame;
     a.N = N; a.S = S; a.T = T; a.nm = nm; a.nb = nb; a.ld = ld; a.col0 = col0; a.l3 = l3; a.l4 = l4; a.l5 = l5;
     a.rc = rc;
     MATPL_CHECK_ARG(mode >= 0 && mode <= 3, "nep_descriptor: bad mode");
@@ -1120,10 +1435,65 @@ MATPL_EXPORT int matpl_nep_descriptor(int f64, int angular, int mode, const void
     MATPL_CHECK_ARG(N == 0 || (c && Ri && NL && atom_map), "nep_descriptor: null input");
     MATPL_CHECK_ARG(mode != 0 || N == 0 || (feats && (!angular || save)), "nep_descriptor: null output");
     MATPL_CHECK_ARG(mode != 1 || N == 0 || (gfeat && gRi && (!angular || save)), "nep_descriptor: null gradient io");
-    MATPL_CHECK_ARG(mode != 2 || N == 0 || (gfeat && gg && gc && ggfeat && (!angular || (save && gsave))),
+    MATPL_CHECK_ARG(mode != 2 || N == 0 || (gfeat && gc && ggfeat && (!angular || (save && gsave))),
                     "nep_descriptor: null 2nd-order io");
+    MATPL_CHECK_ARG(mode != 2 || N == 0 || gg || ((gF || gV) && (!gV || atom_frame)),
+                    "nep_descriptor: second order needs gg, or gF / gV with atom_frame");
     MATPL_CHECK_ARG(mode != 3 || N == 0 || (gc && save && (gfeat || (angular && gs))),
                     "nep_descriptor: null coefficient-gradient io");
     static const FeatWhat what[4] = {W_FEAT, W_GRI, W_2ND_GS, W_GC};
     return feat_run(a, f64, angular != 0, what[mode], (hipStream_t)stream);
+}
+
+// Bytes of the work buffer of matpl_nep_model_forces (segment rows of F, then of the virial).
+MATPL_EXPORT int64_t matpl_nep_model_forces_work(int f64, int64_t N, int64_t nframes, int64_t max_frame, int ntypes,
+                                                 int na, int nbr) {
+    if (N <= 0 || nframes < 1 || max_frame < 1 || ntypes < 1 || na < 0 || nbr < 1) return 0;
+    const ForcePlan pl = f64 ? force_plan<double>(N, max_frame, ntypes, na, nbr)
+                             : force_plan<float>(N, max_frame, ntypes, na, nbr);
+    const int64_t seg = ceil_div(N, pl.ch) + nframes;
+    return seg * (9 * (int64_t)sizeof(double) + 3 * pl.rcap * (f64 ? 8 : 4));
+}
+
+MATPL_EXPORT int matpl_nep_model_forces(int f64, const void *c2, const void *c3, const void *Ri_r, const int64_t *NL_r,
+                                        const void *Ri_a, const int64_t *NL_a, const int64_t *atom_map,
+                                        const int64_t *frame_start, const int32_t *atom_frame, int64_t nframes,
+                                        int64_t max_frame, int64_t N, int S_r, int S_a, int T, int nr, int nbr, int na,
+                                        int nba, int ld, int l3, int l4, int l5, double rc_r, double rc_a,
+                                        const void *gfeat, const void *s_save, void *F, void *V, void *work,
+                                        int64_t work_bytes, void *stream) {
+    MATPL_CHECK_ARG(N >= 0 && S_r >= 0 && S_a >= 0 && nframes >= 1 && max_frame >= 1 && ld >= 1,
+                    "nep_model_forces: bad sizes");
+    MATPL_CHECK_ARG(F && V && frame_start, "nep_model_forces: null output");
+    hipStream_t st = (hipStream_t)stream;
+    int rc = f64 ? fill_async<double>((double *)F, 0.0, 3 * N, st) : fill_async<float>((float *)F, 0.0f, 3 * N, st);
+    if (rc) return rc;
+    if (N == 0)
+        return f64 ? fill_async<double>((double *)V, 0.0, 9 * nframes, st)
+                   : fill_async<float>((float *)V, 0.0f, 9 * nframes, st);
+    MATPL_CHECK_ARG(c2 && Ri_r && NL_r && atom_map && atom_frame && gfeat && work, "nep_model_forces: null input");
+    MATPL_CHECK_ARG(l3 == 0 || (c3 && Ri_a && NL_a && s_save), "nep_model_forces: null angular input");
+    if (l3 == 0) na = 0;
+    MATPL_CHECK_ARG(work_bytes >= matpl_nep_model_forces_work(f64, N, nframes, max_frame, T, na, nbr) &&
+                        ((uintptr_t)work & 7u) == 0,
+                    "nep_model_forces: work buffer too small or not 8-byte aligned");
+    ForceArgs p{};
+    p.r.c = c2; p.r.Ri = Ri_r; p.r.NL = NL_r; p.r.atom_map = atom_map; p.r.gfeat = gfeat; p.r.N = N; p.r.S = S_r;
+    p.r.T = T; p.r.nm = nr; p.r.nb = nbr; p.r.ld = ld; p.r.col0 = 0; p.r.rc = rc_r;
+    p.a = p.r;
+    p.a.c = c3; p.a.Ri = Ri_a; p.a.NL = NL_a; p.a.S = S_a; p.a.nm = na; p.a.nb = nba; p.a.col0 = nr; p.a.rc = rc_a;
+    p.a.l3 = l3; p.a.l4 = l4; p.a.l5 = l5;
+    p.a.save = const_cast<void *>(s_save);
+    p.frame_start = frame_start; p.atom_frame = atom_frame; p.F = F;
+    if ((rc = feat_check(p.r, false)) || (l3 > 0 && (rc = feat_check(p.a, true)))) return rc;
+    const ForcePlan pl = f64 ? force_plan<double>(N, max_frame, T, na, nbr) : force_plan<float>(N, max_frame, T, na, nbr);
+    MATPL_CHECK_ARG(pl.lds <= 64 * 1024, "nep_model_forces: LDS %zu too large", pl.lds);
+    p.vpart = (double *)work;
+    p.part = (double *)work + 9 * (ceil_div(N, pl.ch) + nframes);
+    const bool std_sizes = nr == 5 && nbr == 13 && (l3 == 0 || (na == 5 && nba == 13));
+    if (f64)
+        return std_sizes ? force_launch<double, 5, 13>(p, pl, nframes, (double *)V, st)
+                         : force_launch<double, 0, 0>(p, pl, nframes, (double *)V, st);
+    return std_sizes ? force_launch<float, 5, 13>(p, pl, nframes, (float *)V, st)
+                     : force_launch<float, 0, 0>(p, pl, nframes, (float *)V, st);
 }

@@ -299,32 +299,33 @@ class NEPTorch(torch.nn.Module):
 
     def forward(self, NN_r, NL_r, Ri_r, NN_a, NL_a, Ri_a, num_atom, atom_type_map, is_calc_f=True,
                 create_graph=None, type_index=None):
-        Ri_r = Ri_r.to(self.dtype).detach().requires_grad_()
-        Ri_a = Ri_a.to(self.dtype).detach().requires_grad_()
-        l3 = self.cfg.l_max[0]
-        feats = self.features(Ri_r, NL_r, Ri_a, NL_a, atom_type_map)
-        gq = None
-        if self.fit_kernel:
-            Ei, gq = self.energies_and_grad(feats, atom_type_map, type_index)
-        else:
-            Ei = self.energies(feats, atom_type_map, type_index)
-        nf = num_atom.numel()
-        frame = nep_ops._frame_index(num_atom, Ei.device)[1]
-        if nf == 1:
-            # one frame: a plain reduction (index_add would send every atom's atomic add to one address)
-            Etot = Ei.sum().reshape(1, 1)
-        else:
-            Etot = torch.zeros(nf, dtype=Ei.dtype, device=Ei.device).index_add(0, frame, Ei).unsqueeze(-1)
-        if not is_calc_f:
-            return Etot, Ei, None, None
+        cfg = self.cfg
+        l3 = cfg.l_max[0]
         if create_graph is None:
             create_graph = torch.is_grad_enabled() and any(p.requires_grad for p in self.parameters())
+        Ri_r = Ri_r.to(self.dtype).detach()
+        Ri_a = Ri_a.to(self.dtype).detach()
+        if self.fit_kernel:
+            lists = nep_ops.nep_lists(self.c2, self.c3, Ri_r, NL_r, Ri_a, NL_a, atom_type_map, num_atom,
+                                      cfg.rcut_radial, cfg.rcut_angular, cfg.l_max)
+            q, s = nep_ops.NepDescriptor.apply(self.c2, self.c3, lists)
+            Ei, gq = self.energies_and_grad(q, atom_type_map, type_index)
+            Etot = self._frame_sum(Ei, num_atom)
+            if not is_calc_f:
+                return Etot, Ei, None, None
+            # dEtot/dRi = (dEi/dq) dq/dRi with the fitting kernel's gq, and the forces of both lists, in one kernel
+            with torch.set_grad_enabled(create_graph):
+                Force, Virial = nep_ops.NepModelForces.apply(gq, s, self.c2, self.c3, lists)
+            return Etot, Ei, Force, Virial
+        Ri_r.requires_grad_()
+        Ri_a.requires_grad_()
+        feats = self.features(Ri_r, NL_r, Ri_a, NL_a, atom_type_map)
+        Ei = self.energies(feats, atom_type_map, type_index)
+        Etot = self._frame_sum(Ei, num_atom)
+        if not is_calc_f:
+            return Etot, Ei, None, None
         ins = [Ri_r, Ri_a] if l3 > 0 else [Ri_r]
-        if gq is not None:
-            # dEtot/dRi = (dEi/dq) dq/dRi: the fitting kernel's g through the feature ops only
-            g = torch.autograd.grad([feats], ins, grad_outputs=[gq], create_graph=create_graph, allow_unused=True)
-        else:
-            g = torch.autograd.grad([Etot.sum()], ins, create_graph=create_graph, allow_unused=True)
+        g = torch.autograd.grad([Etot.sum()], ins, create_graph=create_graph, allow_unused=True)
         Force = Virial = None
         for Ri, NL, dE in zip(ins, (NL_r, NL_a), g):
             if dE is None:
@@ -335,6 +336,15 @@ class NEPTorch(torch.nn.Module):
             Force = F if Force is None else Force + F
             Virial = V if Virial is None else Virial + V
         return Etot, Ei, -Force, -Virial
+
+    @staticmethod
+    def _frame_sum(Ei, num_atom):
+        nf = num_atom.numel()
+        if nf == 1:
+            # one frame: a plain reduction (index_add would send every atom's atomic add to one address)
+            return Ei.sum().reshape(1, 1)
+        frame = nep_ops._frame_index(num_atom, Ei.device)[1]
+        return torch.zeros(nf, dtype=Ei.dtype, device=Ei.device).index_add(0, frame, Ei).unsqueeze(-1)
 
 
 class NEPGraph:

@@ -22,7 +22,7 @@ the coefficient-gradient output (zero in force-loss training).
 from __future__ import annotations
 
 from contextlib import contextmanager
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 
 import numpy as np
 import torch
@@ -397,6 +397,154 @@ class NepForceVirialRi(torch.autograd.Function):
 def nep_force_virial(NL, dE, Ri, num_atom):
     """(F, V) of one neighbor list from dE and Ri; see NepForceVirialRi."""
     return NepForceVirialRi.apply(NL, dE, Ri, num_atom)
+
+
+# ------------------------------------------------------------------ the model's descriptor and forces
+def _desc_call(mode, angular, a, feats=None, save=None, gfeat=None, gs=None, gF=None, gV=None, gc=None, ggfeat=None,
+               gsave=None, width=0):
+    """matpl_nep_descriptor for one of the two lists of ``a`` (NepLists); the feature arrays are [N, width]."""
+    c, Ri, NL, rc, col0, l = ((a.c3, a.Ri_a, a.NL_a, a.rc_a, a.c2.shape[2], a.l) if angular else
+                              (a.c2, a.Ri_r, a.NL_r, a.rc_r, 0, (0, 0, 0)))
+    N, S = NL.shape
+    T, _, nm, nb = c.shape
+    _lib.call("matpl_nep_descriptor", _f64(Ri), int(angular), mode, _ptr(c), _ptr(Ri), _ptr(NL), _ptr(a.atom_map), N, S,
+              T, nm, nb, width, col0, *l, rc, _ptr(feats), _ptr(save), _ptr(gfeat), _ptr(gs), None, _ptr(gF), _ptr(gV),
+              _ptr(a.af), None, _ptr(gc), _ptr(ggfeat), _ptr(gsave), _stream())
+
+
+@dataclass
+class NepLists:
+    """Both neighbor lists of a batch as the NEP model's kernels take them (checked, contiguous)."""
+    c2: torch.Tensor
+    c3: torch.Tensor
+    Ri_r: torch.Tensor
+    NL_r: torch.Tensor
+    Ri_a: torch.Tensor
+    NL_a: torch.Tensor
+    atom_map: torch.Tensor
+    rc_r: float
+    rc_a: float
+    l: tuple
+    start: torch.Tensor
+    af: torch.Tensor
+    max_frame: int
+
+    @property
+    def width(self):
+        return self.c2.shape[2] + _nangular(self.c3.shape[2], *self.l)
+
+    def with_tensors(self, c2, c3, Ri_r, NL_r, Ri_a, NL_a, atom_map, af):
+        return replace(self, c2=c2, c3=c3, Ri_r=Ri_r, NL_r=NL_r, Ri_a=Ri_a, NL_a=NL_a, atom_map=atom_map, af=af)
+
+    @property
+    def tensors(self):
+        return self.c2, self.c3, self.Ri_r, self.NL_r, self.Ri_a, self.NL_a, self.atom_map, self.af
+
+
+def nep_lists(c2, c3, Ri_r, NL_r, Ri_a, NL_a, atom_map, num_atom, rc_r, rc_a, l) -> NepLists:
+    c2, Ri_r, NL_r, am = _prep(c2.detach(), Ri_r, NL_r, atom_map)
+    if l[0] > 0:
+        c3, Ri_a, NL_a, am = _prep(c3.detach(), Ri_a, NL_a, atom_map)
+        if NL_a.shape[0] != NL_r.shape[0]:
+            raise ValueError("NEP model: the radial and angular lists have different atom counts")
+    N = NL_r.shape[0]
+    if _STATIC is not None and num_atom is _STATIC.num_atom:
+        maxf = _STATIC.max_frame
+    else:
+        if _int_sum(num_atom) != N:
+            raise ValueError(f"NEP model: num_atom sums to {_int_sum(num_atom)}, list has {N} atoms")
+        maxf = max(_int_max(num_atom), 1)
+    start, af = _frame_index(num_atom, Ri_r.device)
+    return NepLists(c2, c3.detach(), Ri_r, NL_r, Ri_a, NL_a, am, float(rc_r), float(rc_a), tuple(int(x) for x in l),
+                    start, af, maxf)
+
+
+class NepDescriptor(torch.autograd.Function):
+    """(q [N, features], s [N, na * 24]): all features of the model and the angular sums they are formed from. s is
+    an output of its own so that the second-order pass of NepModelForces can return its gradient here: one pass
+    over the slots then takes the coefficient gradient of both orders."""
+
+    @staticmethod
+    def forward(ctx, c2, c3, a: NepLists):
+        N, dt, dev = a.NL_r.shape[0], a.Ri_r.dtype, a.Ri_r.device
+        T, _, nr, nbr = a.c2.shape
+        q = torch.empty((N, a.width), dtype=dt, device=dev)
+        keep = ctx.needs_input_grad[0]
+        F = torch.empty((N, T * nbr), dtype=dt, device=dev) if keep else None
+        _desc_call(0, False, a, feats=q, save=F, width=a.width)
+        if a.l[0] > 0:
+            s = torch.empty((N, a.c3.shape[2] * 24), dtype=dt, device=dev)
+            _desc_call(0, True, a, feats=q, save=s, width=a.width)
+        else:
+            s = torch.empty((N, 0), dtype=dt, device=dev)
+        ctx.set_materialize_grads(False)
+        ctx.lists = replace(a, **{k: None for k in _NEP_TENSORS})
+        ctx.save_for_backward(*a.tensors, s, F)
+        return q, s
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, gq, gs):
+        *ts, s, F = ctx.saved_tensors
+        a = ctx.lists.with_tensors(*ts)
+        gq = None if gq is None else gq.contiguous()
+        gs = None if gs is None else gs.contiguous()
+        g2 = g3 = None
+        if ctx.needs_input_grad[0] and gq is not None:
+            g2 = torch.zeros_like(a.c2)
+            _desc_call(3, False, a, save=F, gfeat=gq, gc=g2, width=a.width)
+        if ctx.needs_input_grad[1] and a.l[0] > 0 and (gq is not None or gs is not None):
+            g3 = torch.zeros_like(a.c3)
+            _desc_call(3, True, a, save=s, gfeat=gq, gs=gs, gc=g3, width=a.width)
+        return g2, g3, None
+
+
+class NepModelForces(torch.autograd.Function):
+    """(F [N, 3], V [frames, 9]) of the NEP model from g = dEtot/dq: the descriptor's position gradient and the
+    force and frame-virial terms of both lists in one kernel, signs as the model returns them
+    (src/model/nep_net.py:600-648). The backward is the second-order pass (gradients of g, s, c2 and c3)."""
+
+    @staticmethod
+    def forward(ctx, g, s, c2, c3, a: NepLists):
+        g = g.contiguous()
+        N, dt, dev = a.NL_r.shape[0], a.Ri_r.dtype, a.Ri_r.device
+        T, _, nr, nbr = a.c2.shape
+        na, nba = (a.c3.shape[2], a.c3.shape[3]) if a.l[0] > 0 else (0, 1)
+        nf = a.start.numel() - 1
+        F = torch.empty((N, 3), dtype=dt, device=dev)
+        V = torch.empty((nf, 9), dtype=dt, device=dev)
+        nbytes = _lib.query("matpl_nep_model_forces_work", _f64(a.Ri_r), N, nf, a.max_frame, T, na, nbr)
+        work = torch.empty(max(nbytes, 8), dtype=torch.uint8, device=dev)
+        _lib.call("matpl_nep_model_forces", _f64(a.Ri_r), _ptr(a.c2), _ptr(a.c3), _ptr(a.Ri_r), _ptr(a.NL_r),
+                  _ptr(a.Ri_a), _ptr(a.NL_a), _ptr(a.atom_map), _ptr(a.start), _ptr(a.af), nf, a.max_frame, N,
+                  a.NL_r.shape[1], a.NL_a.shape[1] if a.l[0] > 0 else 0, T, nr, nbr, na, nba, a.width, *a.l, a.rc_r,
+                  a.rc_a, _ptr(g), _ptr(s), _ptr(F), _ptr(V), _ptr(work), work.numel(), _stream())
+        ctx.set_materialize_grads(False)
+        ctx.lists = replace(a, **{k: None for k in _NEP_TENSORS})
+        ctx.save_for_backward(*a.tensors, g, s)
+        return F, V
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, gF, gV):
+        *ts, g, s = ctx.saved_tensors
+        a = ctx.lists.with_tensors(*ts)
+        if gF is None and gV is None:
+            return None, None, None, None, None
+        dt = a.Ri_r.dtype
+        gF = None if gF is None else gF.to(dt).contiguous()
+        gV = None if gV is None else gV.to(dt).contiguous()
+        ggq = torch.empty_like(g)
+        g2 = torch.zeros_like(a.c2)
+        _desc_call(2, False, a, gfeat=g, gF=gF, gV=gV, gc=g2, ggfeat=ggq, width=a.width)
+        g3 = gs = None
+        if a.l[0] > 0:
+            g3, gs = torch.zeros_like(a.c3), torch.empty_like(s)
+            _desc_call(2, True, a, save=s, gfeat=g, gF=gF, gV=gV, gc=g3, ggfeat=ggq, gsave=gs, width=a.width)
+        return ggq, gs, g2, g3, None
+
+
+_NEP_TENSORS = ("c2", "c3", "Ri_r", "NL_r", "Ri_a", "NL_a", "atom_map", "af")
 
 
 def nep_centre_force(dE, Ri_d):

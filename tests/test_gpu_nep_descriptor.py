@@ -106,21 +106,21 @@ def test_descriptor_modes(dev, dtype, angular, T, nm, nb, l, S, counts):
             _close(cut(ggf), ggq, dtype, "ggfeat")
             _close(gc, gc2, dtype, "gc second order")
         else:
-            call(name, 0, feats, save, None, None, None, None, None, None, None)
+            call(name, 0, feats, save, *[None] * 10)
             _close(cut(feats), q, dtype, "feats")
             assert torch.isnan(feats[:, :col0]).all() and torch.isnan(feats[:, col0 + nf:]).all()
             g = new(N, S, 4)
-            call(name, 1, None, save, gqd, None, None, g, None, None, None)
+            call(name, 1, None, save, gqd, *[None] * 5, g, None, None, None)
             _close(g, gRi, dtype, "gRi")
             gc, ggf, gs = torch.zeros_like(cd), new(N, ld), new(N, nm * 24)
-            call(name, 2, None, save, gqd, None, ggd, None, gc, ggf, gs if angular else None)
+            call(name, 2, None, save, gqd, None, ggd, *[None] * 4, gc, ggf, gs if angular else None)
             _close(cut(ggf), ggq, dtype, "ggfeat")
             # the second order's rest and the first order in one coefficient pass
-            call(name, 3, None, save, gqd, gs if angular else None, None, None, gc, None, None)
+            call(name, 3, None, save, gqd, gs if angular else None, *[None] * 5, gc, None, None)
             _close(gc, gc1 + gc2, dtype, "gc of both orders")
             if angular:
                 gc = torch.zeros_like(cd)
-                call(name, 3, None, save, None, gs, None, None, gc, None, None)
+                call(name, 3, None, save, None, gs, *[None] * 5, gc, None, None)
                 gc3 = torch.zeros_like(cd)
-                call(name, 3, None, save, gqd, gs, None, None, gc3, None, None)
+                call(name, 3, None, save, gqd, gs, *[None] * 5, gc3, None, None)
                 _close(gc3 - gc, gc1, dtype, "gc without gs")

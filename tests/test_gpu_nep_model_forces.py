@@ -1,0 +1,89 @@
+"""The NEP model's fused descriptor, force and virial path (matpl_nep_descriptor, matpl_nep_model_forces and their
+backward) against the operators' sequence it stands for (calculateNepFeat / calculateNepMbFeat, autograd for dE/dRi,
+nep_force_virial) in double, at the edges of its windows: frames of 1 atom, several frames in a window, frames above
+the LDS copy of F (device atomics), sizes other than the default, no angular part.
+
+Tolerances: outputs and gradients are sums of at most ~1e5 terms; 1e-11 (double, about 5e4 eps) and 2e-4 (float) of
+the largest entry bound any order of summation and are far above what is measured."""
+import numpy as np
+import pytest
+import torch
+
+from matpl_amd import nep as mn
+from matpl_amd import nep_ops
+from matpl_amd.nepnet import NEPConfig, NEPWeights
+from matpl_amd.structures import Frame
+
+pytestmark = pytest.mark.gpu
+
+
+def _frames(sizes, T, seed):
+    rng = np.random.default_rng(seed)
+    out = []
+    for n in sizes:
+        side = int(np.ceil(n ** (1 / 3)))
+        L = side * 2.6
+        site = rng.permutation(side ** 3)[:n]
+        pos = np.stack([site // (side * side), site // side % side, site % side], -1) * 2.6
+        out.append(Frame(np.diag([L] * 3), pos + rng.uniform(0, 0.3, (n, 3)), rng.integers(0, T, n).astype(np.int32)))
+    return out
+
+
+def _by_ops(model, nb, p):
+    """(E, F, V) through the operators, differentiable in the parameters."""
+    cfg = model.cfg
+    ins = [nb["Ri_r"].detach().requires_grad_(), nb["Ri_a"].detach().requires_grad_()]
+    q = model.features(ins[0], nb["NL_r"], ins[1], nb["NL_a"], p["atom_type_map"])
+    Ei, gq = model.energies_and_grad(q, p["atom_type_map"])      # gq = dEi/dq, differentiable
+    E = model._frame_sum(Ei, p["num_atoms"])
+    ins = ins[:1] if cfg.l_max[0] == 0 else ins
+    F = V = 0
+    for Ri, NL, dE in zip(ins, (nb["NL_r"], nb["NL_a"]), torch.autograd.grad([q], ins, [gq], create_graph=True)):
+        f, v = nep_ops.nep_force_virial(NL, dE, Ri, p["num_atoms"])
+        F, V = F - f, V - v
+    return E, F, V
+
+
+CASES = [([1, 2, 3, 70, 64, 5, 1, 130], 3, 4, 12, [4, 2, 0]),       # many frames in a window
+         ([2500], 2, 4, 12, [4, 2, 0]),                              # above the LDS copy in double
+         ([40, 9, 300], 2, 3, 7, [4, 2, 1]),                         # other sizes, 5-body
+         ([50, 20], 5, 4, 12, [0, 0, 0])]                            # radial only
+
+
+@pytest.mark.parametrize("sizes,T,n_max,basis,l_max", CASES)
+def test_model_path_equals_operator_sequence(dev, sizes, T, n_max, basis, l_max):
+    print(f"case nep model path sizes={sizes} T={T} n_max={n_max} basis={basis} l_max={l_max}", flush=True)
+    cfg = NEPConfig(ntypes=T, n_max_radial=n_max, n_max_angular=n_max, basis_radial=basis, basis_angular=basis,
+                    l_max=l_max)
+    w = NEPWeights.random(cfg, seed=31, q_scaler=np.full(cfg.nfeat, 0.3))
+    p = mn.pack_frames(_frames(sizes, T, 5), cfg.rcut_radial, dev)
+    nb = mn.neighbors(p, cfg.rcut_radial, cfg.rcut_angular, T)
+    g = torch.Generator(device=dev).manual_seed(3)
+    n, nf = sum(sizes), len(sizes)
+    wE, wF, wV = (torch.randn(*s, dtype=torch.float64, device=dev, generator=g) for s in ((nf, 1), (n, 3), (nf, 9)))
+    ref = mn.NEPTorch(w, torch.float64, dev)
+    want = _by_ops(ref, nb, p)
+    params = [q for q in ref.parameters() if l_max[0] > 0 or q is not ref.c3]
+    want += torch.autograd.grad((want[0] * wE).sum() + (want[1] * wF).sum() + 0.1 * (want[2] * wV).sum(), params)
+    for dtype, tol in ((torch.float64, 1e-11), (torch.float32, 2e-4)):
+        model = mn.NEPTorch(w, dtype, dev)
+        args = (nb["NN_r"], nb["NL_r"], nb["Ri_r"], nb["NN_a"], nb["NL_a"], nb["Ri_a"], p["num_atoms"],
+                p["atom_type_map"])
+        E, _, F, V = model(*args, create_graph=True)
+        loss = (E * wE).sum() + (F * wF).sum() + 0.1 * (V * wV).sum()
+        params = [q for q in model.parameters() if l_max[0] > 0 or q is not model.c3]
+        got = (E, F, V) + torch.autograd.grad(loss, params)
+        for k, (a, b) in enumerate(zip(got, want)):
+            a, b = a.detach().double(), b.detach()
+            err = float((a - b).abs().max())
+            assert err <= tol * max(float(b.abs().max()), 1e-2), (dtype, k, err, float(b.abs().max()))
+        # without a graph: the same values, detached forces
+        E1, _, F1, V1 = model(*args, create_graph=False)
+        assert not F1.requires_grad and not V1.requires_grad
+        assert float((F1 - F.detach()).abs().max()) <= tol * float(F.detach().abs().max().clamp_min(1e-2))
+        # only the forces, or only the virials, in the loss
+        for x, wx in ((F, wF), (V, wV)):
+            E, _, F, V = model(*args, create_graph=True)
+            x = F if wx is wF else V
+            gs = torch.autograd.grad((x * wx).sum(), params, allow_unused=True)
+            assert all(torch.isfinite(q).all() for q in gs if q is not None)
