@@ -1047,7 +1047,10 @@ nep_angular_bwd2_kernel(FeatArgs a) {
 // (nep_net.py negates both): F[i] += f, F[j] -= f, V[frame] -= f (x) x. No [N][S][4] gradient is written or read.
 // A block takes windows of `ch` consecutive atoms, frame by frame (a segment); neighbor terms go to an LDS copy
 // of F over the segment's frame (n <= rcap atoms), written once to the segment's row of `part`, since device
-// atomics are carried out beyond the per-XCD L2 caches here; nep_force_final_kernel adds the rows. Segment
+// atomics are carried out beyond the per-XCD L2 caches here; nep_force_final_kernel adds the rows. The copy is in
+// double in both precisions: LDS adds of floats take several times those of doubles here (62,713-atom float
+// batch: 276 us with a float copy, 181 with this one; the position gradients, two force kernels and their
+// reductions that this kernel stands for took 590 us). Segment
 // (window b, frame f) has row b + f: consecutive segments advance b or f. Larger frames (rcap = 0), and any
 // entry naming an atom of another frame, use global atomics.
 struct ForceArgs {
@@ -1097,9 +1100,10 @@ nep_force_kernel(ForceArgs p) {
     const int nr = NMC ? NMC : R.nm, nbr = NBC ? NBC : R.nb, na = NMC ? NMC : A.nm, nba = NBC ? NBC : A.nb;
     const int per = A.l3 > 0 ? na * NLM : 0, tb = R.T * nbr;       // as force_fixed_lds counts (na = 0 without angular part)
     double *vred = reinterpret_cast<double *>(smem_raw);                          // [W][9]
-    T *Bq = reinterpret_cast<T *>(vred + W * 9) + (size_t)wid * ANG_AB * per;     // [AB][na][24]
-    T *wt = reinterpret_cast<T *>(vred + W * 9) + (size_t)W * ANG_AB * per + (size_t)wid * tb;   // [T][nbr]
-    T *acc = reinterpret_cast<T *>(vred + W * 9) + (size_t)W * (ANG_AB * per + tb);               // [3 rcap]
+    double *acc = vred + W * 9;                                                    // [3 rcap]
+    T *wv = reinterpret_cast<T *>(acc + 3 * p.rcap);
+    T *Bq = wv + (size_t)wid * ANG_AB * per;                                      // [AB][na][24]
+    T *wt = wv + (size_t)W * ANG_AB * per + (size_t)wid * tb;                      // [T][nbr]
     T *F = reinterpret_cast<T *>(p.F);
     const int64_t i0 = (int64_t)blockIdx.x * p.ch, i1 = i0 + p.ch < R.N ? i0 + p.ch : R.N;
     const int f1 = p.atom_frame[i1 - 1];
@@ -1109,10 +1113,10 @@ nep_force_kernel(ForceArgs p) {
         if (s0 >= s1) continue;
         const bool lds = fe - fs <= p.rcap;
         if (lds)
-            for (int64_t x = threadIdx.x; x < 3 * (fe - fs); x += blockDim.x) acc[x] = T(0);
+            for (int64_t x = threadIdx.x; x < 3 * (fe - fs); x += blockDim.x) acc[x] = 0.0;
         __syncthreads();
         auto add = [&](int64_t j, int c, T v) {
-            if (lds && j >= fs && j < fe) atomicAdd(acc + 3 * (j - fs) + c, v);
+            if (lds && j >= fs && j < fe) atomicAdd(acc + 3 * (j - fs) + c, (double)v);
             else atomic_add(F + 3 * j + c, v);
         };
         T vir[9];
@@ -1228,7 +1232,7 @@ nep_force_kernel(ForceArgs p) {
         }
         if (lds) {
             T *o = reinterpret_cast<T *>(p.part) + seg * 3 * p.rcap;
-            for (int64_t x = threadIdx.x; x < 3 * (fe - fs); x += blockDim.x) o[x] = acc[x];
+            for (int64_t x = threadIdx.x; x < 3 * (fe - fs); x += blockDim.x) o[x] = (T)acc[x];
         }
         __syncthreads();
     }
@@ -1291,9 +1295,9 @@ inline ForcePlan force_plan(int64_t N, int64_t max_frame, int ntypes, int na, in
     const size_t fixed = force_fixed_lds<T>(ntypes, na, nbr);
     int64_t ch = (N + 511) / 512;
     ch = ch < 8 ? 8 : (ch > 64 ? 64 : ch);
-    const int64_t cap = fixed < 64 * 1024 ? (int64_t)((64 * 1024 - fixed) / (3 * sizeof(T))) : 0;
+    const int64_t cap = fixed < 64 * 1024 ? (int64_t)((64 * 1024 - fixed) / (3 * sizeof(double))) : 0;
     const int64_t rcap = max_frame <= cap ? max_frame : 0;
-    return {(int)ch, rcap, fixed + 3 * rcap * sizeof(T)};
+    return {(int)ch, rcap, fixed + 3 * rcap * sizeof(double)};
 }
 
 template <typename T, int NMC, int NBC>
