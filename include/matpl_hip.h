@@ -657,11 +657,22 @@ int matpl_nep_fit_part_width(int D, int H);
 int matpl_nep_fit_forward(int f64, const void *q, const void *qs, const int32_t *perm, const int32_t *tiles,
                           int ntiles, int tile_atoms, const void *W0, const void *b0, const void *w1, const void *b1,
                           int D, int H, void *Ei, void *g, void *stream);
+/* The same with one weight pointer per type (host tables of ntypes <= 16 device pointers). */
+int matpl_nep_fit_forward_nets(int f64, const void *q, const void *qs, const int32_t *perm, const int32_t *tiles,
+                               int ntiles, int tile_atoms, int ntypes, const void *const *W0, const void *const *b0,
+                               const void *const *w1, const void *const *b1, int D, int H, void *Ei, void *g,
+                               void *stream);
 int matpl_nep_fit_backward(int f64, const void *q, const void *qs, const int32_t *perm, const int32_t *tiles,
                            int ntiles, int tile_atoms, const int32_t *tstart, int ntypes, const void *W0,
                            const void *b0, const void *w1, const void *b1, int D, int H, const void *gE,
                            const void *gg, void *dq, void *part, void *dW0, void *db0, void *dw1, void *db1,
                            void *stream);
+/* The same with one weight pointer per type; the gradients stay stacked [ntypes]. */
+int matpl_nep_fit_backward_nets(int f64, const void *q, const void *qs, const int32_t *perm, const int32_t *tiles,
+                                int ntiles, int tile_atoms, const int32_t *tstart, int ntypes, const void *const *W0,
+                                const void *const *b0, const void *const *w1, const void *const *b1, int D, int H,
+                                const void *gE, const void *gg, void *dq, void *part, void *dW0, void *db0, void *dw1,
+                                void *db1, void *stream);
 
 /* ------------------------------------------------------------ MD helpers */
 /*

@@ -91,6 +91,9 @@ SIGNATURES = {
     "matpl_nep_fit_tile_atoms": (I32, [I32, I32, I32]),
     "matpl_nep_fit_part_width": (I32, [I32, I32]),
     "matpl_nep_fit_forward": (I32, [I32, P, P, P, P, I32, I32, P, P, P, P, I32, I32, P, P, P]),
+    "matpl_nep_fit_forward_nets": (I32, [I32, P, P, P, P, I32, I32, I32, P, P, P, P, I32, I32, P, P, P]),
+    "matpl_nep_fit_backward_nets": (I32, [I32, P, P, P, P, I32, I32, P, I32, P, P, P, P, I32, I32, P, P, P, P, P, P, P, P,
+                                          P]),
     "matpl_nep_fit_backward": (I32, [I32, P, P, P, P, I32, I32, P, I32, P, P, P, P, I32, I32, P, P, P, P, P, P, P, P,
                                      P]),
     # MD helpers

@@ -28,15 +28,30 @@ namespace {
 
 constexpr int FIT_THREADS = 256;
 
+// Each type's weights: W0 [D][H], b0 [H], w1 [H], b1 [1], from stacked arrays ([T] of them) or, when `tables`,
+// from one pointer per type, so that a model's own parameters need no stacking.
+constexpr int FIT_TYPES = 16;
+struct FitWeights {
+    const void *W0[FIT_TYPES], *b0[FIT_TYPES], *w1[FIT_TYPES], *b1[FIT_TYPES];
+    int tables;
+    template <typename T>
+    __device__ __forceinline__ void of(int ty, int D, int H, const T *&w0_, const T *&b0_, const T *&w1_,
+                                       const T *&b1_) const {
+        const int e = tables ? ty : 0;
+        const size_t s = tables ? 0 : (size_t)ty;
+        w0_ = reinterpret_cast<const T *>(W0[e]) + s * D * H;
+        b0_ = reinterpret_cast<const T *>(b0[e]) + s * H;
+        w1_ = reinterpret_cast<const T *>(w1[e]) + s * H;
+        b1_ = reinterpret_cast<const T *>(b1[e]) + s;
+    }
+};
+
 struct FitArgs {
     const void *q;           // [N][D] unscaled features
     const void *qs;          // [D]
     const int32_t *perm;     // [N] atoms grouped by type
     const int32_t *tiles;    // [ntiles][3]: type, first position in perm, count (<= TA)
-    const void *W0;          // [T][D][H]
-    const void *b0;          // [T][H]
-    const void *w1;          // [T][H]
-    const void *b1;          // [T]
+    FitWeights w;
     void *Ei;                // [N]              forward
     void *g;                 // [N][D] dEi/dq    forward (may be null)
     const void *gE;          // [N]              backward (may be null)
@@ -44,7 +59,15 @@ struct FitArgs {
     void *dq;                // [N][D]           backward (may be null)
     void *part;              // [ntiles][PW]     backward: per-tile parameter-gradient rows
     int D, H, TA;
+    int per;                 // forward: atoms per block (divides TA)
 };
+
+// Orders a wavefront's own LDS writes before its lanes' reads of each other's values.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 __host__ __device__ inline int odd(int n) { return n | 1; }     // LDS row stride (odd: fewer bank conflicts)
 
@@ -55,62 +78,64 @@ __device__ __forceinline__ float tanh_t<float>(float z) { return tanhf(z); }
 template <>
 __device__ __forceinline__ double tanh_t<double>(double z) { return tanh(z); }
 
-template <typename T>
+// Forward: 32 lanes per atom, 8 atoms of a block at a time; lanes over the hidden units, then over the features.
+// With WL the type's W0 sits in LDS (rows of odd stride, read along both axes without conflicts), otherwise it is
+// read from global memory. Each half-wave only reads the rows it wrote, so no block barrier follows the staging.
+// What bounds it: at thousands of atoms the serial chain of two D x H products on few wavefronts (a block per 64
+// atoms, a thread per atom and strided units: 1,728 atoms 23 us, with a block per 8 atoms 5 us); at 62,713
+// atoms LDS reads (37 -> 34 us).
+constexpr int FIT_GROUP = 32, FIT_ATOMS = FIT_THREADS / FIT_GROUP;
+
+template <typename T, bool WL>
 __global__ void __launch_bounds__(FIT_THREADS) nep_fit_fwd_kernel(FitArgs a) {
     extern __shared__ unsigned char smem_raw[];
-    const int D = a.D, H = a.H, TA = a.TA;
+    const int D = a.D, H = a.H, nsub = a.TA / a.per;
     const int sd = odd(D), sh = odd(H);
-    const int NG = FIT_THREADS / TA;                      // thread groups per atom
-    T *xs = reinterpret_cast<T *>(smem_raw);              // [TA][sd]  x, then g
-    T *us = xs + TA * sd;                                 // [TA][sh]  u
-    T *ep = us + TA * sh;                                 // [NG][TA]  energy partials
-    const int *tile = a.tiles + 3 * blockIdx.x;
-    const int ty = tile[0], first = tile[1], cnt = tile[2];
+    const int l = threadIdx.x % FIT_GROUP, grp = threadIdx.x / FIT_GROUP;
+    T *x = reinterpret_cast<T *>(smem_raw) + grp * (sd + sh);      // [D] this atom's x
+    T *u = x + sd;                                                 // [H]
+    T *ws = reinterpret_cast<T *>(smem_raw) + FIT_ATOMS * (sd + sh);   // [D][sh] (WL)
+    const int *tile = a.tiles + 3 * (blockIdx.x / nsub);
+    const int ty = tile[0], r0 = (blockIdx.x % nsub) * a.per;
+    const int first = tile[1] + r0, cnt = tile[2] - r0 < a.per ? tile[2] - r0 : a.per;
+    if (cnt <= 0) return;
     const T *q = reinterpret_cast<const T *>(a.q);
     const T *qs = reinterpret_cast<const T *>(a.qs);
-    const T *W0 = reinterpret_cast<const T *>(a.W0) + (size_t)ty * D * H;
-    const T *b0 = reinterpret_cast<const T *>(a.b0) + (size_t)ty * H;
-    const T *w1 = reinterpret_cast<const T *>(a.w1) + (size_t)ty * H;
-    for (int e = threadIdx.x; e < cnt * D; e += FIT_THREADS) {
-        const int at = e / D, d = e - at * D;
-        xs[at * sd + d] = q[(size_t)a.perm[first + at] * D + d] * qs[d];
+    const T *W0, *b0, *w1, *b1;
+    a.w.of<T>(ty, D, H, W0, b0, w1, b1);
+    if constexpr (WL) {
+        for (int e = threadIdx.x; e < D * H; e += FIT_THREADS) ws[(e / H) * sh + e % H] = W0[e];
+        __syncthreads();
     }
-    __syncthreads();
-    const int at = threadIdx.x % TA, grp = threadIdx.x / TA;
-    T epart = T(0);
-    if (at < cnt) {
-        const T *x = xs + at * sd;
-        for (int j = grp; j < H; j += NG) {
+    const T *W = WL ? ws : W0;
+    const int sw = WL ? sh : H;
+    for (int r = grp; r < cnt; r += FIT_ATOMS) {
+        const size_t at = (size_t)a.perm[first + r];
+        for (int d = l; d < D; d += FIT_GROUP) x[d] = q[at * D + d] * qs[d];
+        wave_sync();
+        T e = T(0);
+        for (int j = l; j < H; j += FIT_GROUP) {
             T z = b0[j];
-            for (int d = 0; d < D; d++) z += x[d] * W0[d * H + j];
+#pragma unroll 10
+            for (int d = 0; d < D; d++) z += x[d] * W[d * sw + j];
             const T h = tanh_t(z);
-            epart += w1[j] * h;
-            us[at * sh + j] = w1[j] * (T(1) - h * h);
+            e += w1[j] * h;
+            u[j] = w1[j] * (T(1) - h * h);
         }
-    }
-    ep[grp * TA + at] = epart;
-    __syncthreads();
-    // g_x[d] = sum_j W0[d][j] u[j], written over x (no longer needed)
-    if (at < cnt) {
-        const T *u = us + at * sh;
-        for (int d = grp; d < D; d += NG) {
-            T s = T(0);
-            for (int j = 0; j < H; j++) s += W0[d * H + j] * u[j];
-            xs[at * sd + d] = s * qs[d];
+        wave_sync();
+#pragma unroll
+        for (int o = FIT_GROUP / 2; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
+        if (l == 0) reinterpret_cast<T *>(a.Ei)[at] = e + b1[0];
+        if (a.g) {
+            T *g = reinterpret_cast<T *>(a.g);
+            for (int d = l; d < D; d += FIT_GROUP) {
+                T s = T(0);
+#pragma unroll 10
+                for (int j = 0; j < H; j++) s += W[d * sw + j] * u[j];
+                g[at * D + d] = s * qs[d];
+            }
         }
-    }
-    __syncthreads();
-    if (threadIdx.x < cnt) {
-        T e = reinterpret_cast<const T *>(a.b1)[ty];
-        for (int k = 0; k < NG; k++) e += ep[k * TA + threadIdx.x];
-        reinterpret_cast<T *>(a.Ei)[a.perm[first + threadIdx.x]] = e;
-    }
-    if (a.g) {
-        T *g = reinterpret_cast<T *>(a.g);
-        for (int e = threadIdx.x; e < cnt * D; e += FIT_THREADS) {
-            const int r = e / D, d = e - r * D;
-            g[(size_t)a.perm[first + r] * D + d] = xs[r * sd + d];
-        }
+        wave_sync();
     }
 }
 
@@ -135,9 +160,8 @@ __global__ void __launch_bounds__(FIT_THREADS) nep_fit_bwd_kernel(FitArgs a) {
     const T *qs = reinterpret_cast<const T *>(a.qs);
     const T *gg = reinterpret_cast<const T *>(a.gg);
     const T *gE = reinterpret_cast<const T *>(a.gE);
-    const T *W0 = reinterpret_cast<const T *>(a.W0) + (size_t)ty * D * H;
-    const T *b0 = reinterpret_cast<const T *>(a.b0) + (size_t)ty * H;
-    const T *w1 = reinterpret_cast<const T *>(a.w1) + (size_t)ty * H;
+    const T *W0, *b0, *w1, *b1;
+    a.w.of<T>(ty, D, H, W0, b0, w1, b1);
     for (int e = threadIdx.x; e < cnt * D; e += FIT_THREADS) {
         const int at = e / D, d = e - at * D;
         const size_t src = (size_t)a.perm[first + at] * D + d;
@@ -220,11 +244,78 @@ nep_fit_reduce_kernel(const T *part, const int32_t *tstart, int PW, int D, int H
     else db1[t] = s;
 }
 
-size_t fwd_lds(int D, int H, int TA, size_t es) {
-    return es * ((size_t)TA * odd(D) + (size_t)TA * odd(H) + (size_t)FIT_THREADS);
+size_t fwd_lds(int D, int H, bool wl, size_t es) {
+    return es * ((size_t)FIT_ATOMS * (odd(D) + odd(H)) + (wl ? (size_t)D * odd(H) : 0));
 }
 size_t bwd_lds(int D, int H, int TA, size_t es) {
     return es * (2 * (size_t)TA * odd(D) + 3 * (size_t)TA * odd(H) + (size_t)TA);
+}
+
+template <typename T>
+int fwd_launch(FitArgs &a, int ntiles, hipStream_t st) {
+    // fewer atoms per block while that leaves the chip short of blocks (four per CU), down to one per half-wave
+    a.per = a.TA;
+    while (a.per > FIT_ATOMS && (int64_t)ntiles * (a.TA / a.per) < 1024) a.per /= 2;
+    const dim3 grid((unsigned)ntiles * (unsigned)(a.TA / a.per)), block(FIT_THREADS);
+    // W0 in LDS up to 24 KB: blocks of several types share a CU's 160 KB
+    if ((size_t)a.D * odd(a.H) * sizeof(T) <= 24 * 1024)
+        hipLaunchKernelGGL((nep_fit_fwd_kernel<T, true>), grid, block, fwd_lds(a.D, a.H, true, sizeof(T)), st, a);
+    else
+        hipLaunchKernelGGL((nep_fit_fwd_kernel<T, false>), grid, block, fwd_lds(a.D, a.H, false, sizeof(T)), st, a);
+    return check_launch("nep_fit_fwd_kernel");
+}
+
+int set_stacked(FitArgs &a, const void *W0, const void *b0, const void *w1, const void *b1) {
+    a.w.tables = 0;
+    a.w.W0[0] = W0; a.w.b0[0] = b0; a.w.w1[0] = w1; a.w.b1[0] = b1;
+    return OK;
+}
+
+int set_tables(FitArgs &a, int ntypes, const void *const *W0, const void *const *b0, const void *const *w1,
+               const void *const *b1) {
+    MATPL_CHECK_ARG(ntypes >= 1 && ntypes <= FIT_TYPES, "nep_fit: ntypes must be in [1,%d]", FIT_TYPES);
+    MATPL_CHECK_ARG(W0 && b0 && w1 && b1, "nep_fit: null weight table");
+    a.w.tables = 1;
+    for (int t = 0; t < ntypes; t++) {
+        MATPL_CHECK_ARG(W0[t] && b0[t] && w1[t] && b1[t], "nep_fit: null weights of type %d", t);
+        a.w.W0[t] = W0[t]; a.w.b0[t] = b0[t]; a.w.w1[t] = w1[t]; a.w.b1[t] = b1[t];
+    }
+    return OK;
+}
+
+int forward_run(FitArgs &a, int f64, const void *q, const void *qs, const int32_t *perm, const int32_t *tiles, int ntiles,
+                int tile_atoms, int D, int H, void *Ei, void *g, hipStream_t st) {
+    a.q = q; a.qs = qs; a.perm = perm; a.tiles = tiles; a.Ei = Ei; a.g = g; a.D = D; a.H = H; a.TA = tile_atoms;
+    return f64 ? fwd_launch<double>(a, ntiles, st) : fwd_launch<float>(a, ntiles, st);
+}
+
+int backward_run(FitArgs &a, int f64, const void *q, const void *qs, const int32_t *perm, const int32_t *tiles,
+                 int ntiles, int tile_atoms, const int32_t *tstart, int ntypes, int D, int H, const void *gE,
+                 const void *gg, void *dq, void *part, void *dW0, void *db0, void *dw1, void *db1, hipStream_t st) {
+    const int PW = part_width(D, H);
+    if (ntiles > 0) {
+        a.q = q; a.qs = qs; a.perm = perm; a.tiles = tiles;
+        a.gE = gE; a.gg = gg; a.dq = dq; a.part = part; a.D = D; a.H = H; a.TA = tile_atoms;
+        if (f64)
+            hipLaunchKernelGGL(nep_fit_bwd_kernel<double>, dim3(ntiles), dim3(FIT_THREADS), bwd_lds(D, H, a.TA, 8), st,
+                               a);
+        else
+            hipLaunchKernelGGL(nep_fit_bwd_kernel<float>, dim3(ntiles), dim3(FIT_THREADS), bwd_lds(D, H, a.TA, 4), st,
+                               a);
+        int rc = check_launch("nep_fit_bwd_kernel");
+        if (rc) return rc;
+    }
+    const dim3 grid((PW + RED_ENTRIES - 1) / RED_ENTRIES, ntypes);
+    const dim3 block(RED_ENTRIES * RED_GROUPS);
+    if (f64)
+        hipLaunchKernelGGL(nep_fit_reduce_kernel<double>, grid, block, 0, st, static_cast<const double *>(part),
+                           tstart, PW, D, H, static_cast<double *>(dW0), static_cast<double *>(db0),
+                           static_cast<double *>(dw1), static_cast<double *>(db1));
+    else
+        hipLaunchKernelGGL(nep_fit_reduce_kernel<float>, grid, block, 0, st, static_cast<const float *>(part),
+                           tstart, PW, D, H, static_cast<float *>(dW0), static_cast<float *>(db0),
+                           static_cast<float *>(dw1), static_cast<float *>(db1));
+    return check_launch("nep_fit_reduce_kernel");
 }
 
 }  // namespace
@@ -255,14 +346,24 @@ MATPL_EXPORT int matpl_nep_fit_forward(int f64, const void *q, const void *qs, c
     if (ntiles == 0) return OK;
     MATPL_CHECK_ARG(q && qs && perm && tiles && W0 && b0 && w1 && b1 && Ei, "nep_fit_forward: null pointer");
     FitArgs a{};
-    a.q = q; a.qs = qs; a.perm = perm; a.tiles = tiles; a.W0 = W0; a.b0 = b0; a.w1 = w1; a.b1 = b1;
-    a.Ei = Ei; a.g = g; a.D = D; a.H = H; a.TA = tile_atoms;
-    hipStream_t st = (hipStream_t)stream;
-    if (f64)
-        hipLaunchKernelGGL(nep_fit_fwd_kernel<double>, dim3(ntiles), dim3(FIT_THREADS), fwd_lds(D, H, a.TA, 8), st, a);
-    else
-        hipLaunchKernelGGL(nep_fit_fwd_kernel<float>, dim3(ntiles), dim3(FIT_THREADS), fwd_lds(D, H, a.TA, 4), st, a);
-    return check_launch("nep_fit_fwd_kernel");
+    set_stacked(a, W0, b0, w1, b1);
+    return forward_run(a, f64, q, qs, perm, tiles, ntiles, tile_atoms, D, H, Ei, g, (hipStream_t)stream);
+}
+
+// matpl_nep_fit_forward with one weight pointer per type (host tables of ntypes device pointers).
+MATPL_EXPORT int matpl_nep_fit_forward_nets(int f64, const void *q, const void *qs, const int32_t *perm,
+                                            const int32_t *tiles, int ntiles, int tile_atoms, int ntypes,
+                                            const void *const *W0, const void *const *b0, const void *const *w1,
+                                            const void *const *b1, int D, int H, void *Ei, void *g, void *stream) {
+    MATPL_CHECK_ARG(D >= 1 && H >= 1 && ntiles >= 0, "nep_fit_forward_nets: bad sizes D=%d H=%d", D, H);
+    MATPL_CHECK_ARG(tile_atoms == matpl_nep_fit_tile_atoms(f64, D, H),
+                    "nep_fit_forward_nets: tile_atoms %d is not matpl_nep_fit_tile_atoms", tile_atoms);
+    if (ntiles == 0) return OK;
+    MATPL_CHECK_ARG(q && qs && perm && tiles && Ei, "nep_fit_forward_nets: null pointer");
+    FitArgs a{};
+    const int rc = set_tables(a, ntypes, W0, b0, w1, b1);
+    if (rc) return rc;
+    return forward_run(a, f64, q, qs, perm, tiles, ntiles, tile_atoms, D, H, Ei, g, (hipStream_t)stream);
 }
 
 MATPL_EXPORT int matpl_nep_fit_backward(int f64, const void *q, const void *qs, const int32_t *perm,
@@ -275,31 +376,29 @@ MATPL_EXPORT int matpl_nep_fit_backward(int f64, const void *q, const void *qs, 
                     "nep_fit_backward: tile_atoms %d is not matpl_nep_fit_tile_atoms (%d)", tile_atoms,
                     matpl_nep_fit_tile_atoms(f64, D, H));
     MATPL_CHECK_ARG(tstart && dW0 && db0 && dw1 && db1, "nep_fit_backward: null pointer");
-    hipStream_t st = (hipStream_t)stream;
-    const int PW = part_width(D, H);
-    if (ntiles > 0) {
-        MATPL_CHECK_ARG(q && qs && perm && tiles && W0 && b0 && w1 && b1 && part, "nep_fit_backward: null pointer");
-        FitArgs a{};
-        a.q = q; a.qs = qs; a.perm = perm; a.tiles = tiles; a.W0 = W0; a.b0 = b0; a.w1 = w1; a.b1 = b1;
-        a.gE = gE; a.gg = gg; a.dq = dq; a.part = part; a.D = D; a.H = H; a.TA = tile_atoms;
-        if (f64)
-            hipLaunchKernelGGL(nep_fit_bwd_kernel<double>, dim3(ntiles), dim3(FIT_THREADS), bwd_lds(D, H, a.TA, 8), st,
-                               a);
-        else
-            hipLaunchKernelGGL(nep_fit_bwd_kernel<float>, dim3(ntiles), dim3(FIT_THREADS), bwd_lds(D, H, a.TA, 4), st,
-                               a);
-        int rc = check_launch("nep_fit_bwd_kernel");
-        if (rc) return rc;
-    }
-    const dim3 grid((PW + RED_ENTRIES - 1) / RED_ENTRIES, ntypes);
-    const dim3 block(RED_ENTRIES * RED_GROUPS);
-    if (f64)
-        hipLaunchKernelGGL(nep_fit_reduce_kernel<double>, grid, block, 0, st, static_cast<const double *>(part),
-                           tstart, PW, D, H, static_cast<double *>(dW0), static_cast<double *>(db0),
-                           static_cast<double *>(dw1), static_cast<double *>(db1));
-    else
-        hipLaunchKernelGGL(nep_fit_reduce_kernel<float>, grid, block, 0, st, static_cast<const float *>(part),
-                           tstart, PW, D, H, static_cast<float *>(dW0), static_cast<float *>(db0),
-                           static_cast<float *>(dw1), static_cast<float *>(db1));
-    return check_launch("nep_fit_reduce_kernel");
+    MATPL_CHECK_ARG(ntiles == 0 || (q && qs && perm && tiles && W0 && b0 && w1 && b1 && part),
+                    "nep_fit_backward: null pointer");
+    FitArgs a{};
+    set_stacked(a, W0, b0, w1, b1);
+    return backward_run(a, f64, q, qs, perm, tiles, ntiles, tile_atoms, tstart, ntypes, D, H, gE, gg, dq, part, dW0, db0,
+                        dw1, db1, (hipStream_t)stream);
+}
+
+// matpl_nep_fit_backward with one weight pointer per type; the gradients stay stacked.
+MATPL_EXPORT int matpl_nep_fit_backward_nets(int f64, const void *q, const void *qs, const int32_t *perm,
+                                             const int32_t *tiles, int ntiles, int tile_atoms, const int32_t *tstart,
+                                             int ntypes, const void *const *W0, const void *const *b0,
+                                             const void *const *w1, const void *const *b1, int D, int H,
+                                             const void *gE, const void *gg, void *dq, void *part, void *dW0,
+                                             void *db0, void *dw1, void *db1, void *stream) {
+    MATPL_CHECK_ARG(D >= 1 && H >= 1 && ntiles >= 0, "nep_fit_backward_nets: bad sizes D=%d H=%d", D, H);
+    MATPL_CHECK_ARG(tile_atoms == matpl_nep_fit_tile_atoms(f64, D, H),
+                    "nep_fit_backward_nets: tile_atoms %d is not matpl_nep_fit_tile_atoms", tile_atoms);
+    MATPL_CHECK_ARG(tstart && dW0 && db0 && dw1 && db1 && (ntiles == 0 || (q && qs && perm && tiles && part)),
+                    "nep_fit_backward_nets: null pointer");
+    FitArgs a{};
+    const int rc = set_tables(a, ntypes, W0, b0, w1, b1);
+    if (rc) return rc;
+    return backward_run(a, f64, q, qs, perm, tiles, ntiles, tile_atoms, tstart, ntypes, D, H, gE, gg, dq, part, dW0, db0,
+                        dw1, db1, (hipStream_t)stream);
 }

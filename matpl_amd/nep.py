@@ -224,6 +224,53 @@ class _NepFitFn(torch.autograd.Function):
         return dq, None, dW0, db0, dw1, db1, None
 
 
+class _NepFitNetsFn(torch.autograd.Function):
+    """_NepFitFn with every type's own parameter tensors (W0 [D, H], b0 [H], w1 [H, 1], b1 [1] per type, in that
+    order) instead of stacked ones: no launches to stack them, and gradients that are views of the stacked sums."""
+
+    @staticmethod
+    def forward(ctx, q, qs, plan, *params):
+        q = q.contiguous()
+        N, D = q.shape
+        H = params[0].shape[1]
+        params = [w.detach().to(q.dtype).contiguous() for w in params]
+        Ei = torch.empty(N, dtype=q.dtype, device=q.device)
+        g = torch.empty_like(q)
+        tabs = _NepFitNetsFn._tables(params)
+        _lib.call("matpl_nep_fit_forward_nets", int(q.dtype == torch.float64), _ptr(q), _ptr(qs), _ptr(plan.perm),
+                  _ptr(plan.tiles), plan.ntiles, plan.tile_atoms, len(params) // 4, *[t.ctypes.data for t in tabs], D, H,
+                  _ptr(Ei), _ptr(g), _stream())
+        ctx.save_for_backward(q, qs, *params)
+        ctx.plan = plan
+        return Ei, g
+
+    @staticmethod
+    def _tables(params):
+        """The pointer tables of W0, b0, w1 and b1 (host arrays, one entry per type)."""
+        ptrs = np.array([w.data_ptr() for w in params], np.uint64).reshape(-1, 4)
+        return [np.ascontiguousarray(ptrs[:, k]) for k in range(4)]
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, gE, gg):
+        q, qs, *params = ctx.saved_tensors
+        plan = ctx.plan
+        N, D = q.shape
+        T, H = len(params) // 4, params[0].shape[1]
+        f64 = int(q.dtype == torch.float64)
+        gE = None if gE is None else gE.contiguous()
+        gg = None if gg is None else gg.contiguous()
+        new = lambda *s: torch.empty(s, dtype=q.dtype, device=q.device)
+        dq = torch.empty_like(q) if ctx.needs_input_grad[0] else None
+        part = new(max(plan.ntiles, 1) * _lib.query("matpl_nep_fit_part_width", D, H))
+        dW0, db0, dw1, db1 = new(T, D, H), new(T, H), new(T, H, 1), new(T, 1)
+        tabs = _NepFitNetsFn._tables(params)
+        _lib.call("matpl_nep_fit_backward_nets", f64, _ptr(q), _ptr(qs), _ptr(plan.perm), _ptr(plan.tiles), plan.ntiles,
+                  plan.tile_atoms, _ptr(plan.tstart), T, *[t.ctypes.data for t in tabs], D, H, _ptr(gE), _ptr(gg),
+                  _ptr(dq), _ptr(part), _ptr(dW0), _ptr(db0), _ptr(dw1), _ptr(db1), _stream())
+        return (dq, None, None) + tuple(x[t] for t in range(T) for x in (dW0, db0, dw1, db1))
+
+
 class NEPTorch(torch.nn.Module):
     """NEP.forward on the HIP operators: (Etot [F,1], Ei [N], Force [N,3], Virial [F,9])."""
 
@@ -279,11 +326,13 @@ class NEPTorch(torch.nn.Module):
     def energies_and_grad(self, feats, atom_type_map, type_index=None):
         """(Ei [N], dEi/dfeats [N, D]) from the fitting kernels (fit_kernel nets only)."""
         plan = self.fit_plan(atom_type_map, type_index)
-        W0 = torch.stack([n.W[0] for n in self.fit])
-        b0 = torch.stack([n.b[0] for n in self.fit])
-        w1 = torch.stack([n.W[1][:, 0] for n in self.fit])
-        b1 = torch.stack([n.b[1].reshape(()) for n in self.fit])
-        return _NepFitFn.apply(feats, self.q_scaler, W0, b0, w1, b1, plan)
+        if len(self.fit) > 16:          # more types than the kernels' pointer tables hold
+            return _NepFitFn.apply(feats, self.q_scaler, torch.stack([n.W[0] for n in self.fit]),
+                                   torch.stack([n.b[0] for n in self.fit]),
+                                   torch.stack([n.W[1][:, 0] for n in self.fit]),
+                                   torch.stack([n.b[1].reshape(()) for n in self.fit]), plan)
+        return _NepFitNetsFn.apply(feats, self.q_scaler, plan,
+                                   *[x for n in self.fit for x in (n.W[0], n.b[0], n.W[1], n.b[1])])
 
     def energies(self, feats, atom_type_map, type_index=None):
         """type_index: the atoms of each type (precomputed, e.g. for graph capture); else found here."""
