@@ -44,7 +44,7 @@
 // pre-permuted per lane (fwd[l][r] = W[f(r,h)][l%32], bwd[l][r] =
 // W[l%32][f(r,h)]) so no data moves between layers. The FP32 variant uses
 // v_mfma_f32_32x32x2_f32 with K-chunk r = registers r of both halves.
-#include "dp_fused_common.h"
+#include "dp_group.h"
 
 namespace matpl {
 namespace {
@@ -455,6 +455,316 @@ dp_fused_bwd_kernel(FusedParams p) {
     }
 }
 
+// ------------------------------------------------------------------ group passes (dp_group.h)
+// The forward of up to GA atoms at once: the same tiles and net as dp_fused_fwd_kernel over the group's neighbors;
+// the contraction's rows are (atom, component), of which a neighbor fills its own atom's four (BF16 as there, FP32
+// by contract_group). Measured against an atom per wavefront: 73,742 atoms of four types in BF16 395 -> 248 us,
+// 7,000 in FP32 151 -> 106.
+template <int E, bool BF16, bool GST>
+__global__ void __launch_bounds__(FUSED_WAVES * WAVE)
+dp_group_fwd_kernel(FusedParams p) {
+    constexpr int NR = NReg<E>::value;
+    extern __shared__ float4 smem[];
+    const int lane = threadIdx.x & (WAVE - 1), wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int h = lane >> 5, n = lane & 31, nbw = group_nbw(p);
+    const GroupLds L = group_lds(reinterpret_cast<unsigned char *>(smem), wid, nbw, BF16 ? GROUP_BF16_BYTES : GROUP_F32_BYTES);
+    const unsigned char *mat = reinterpret_cast<const unsigned char *>(p.mat);
+    const int64_t i0 = ((int64_t)blockIdx.x * FUSED_WAVES + wid) * p.gchunk;
+    const int64_t i1 = i0 + p.gchunk < p.natoms ? i0 + p.gchunk : p.natoms;
+    for (int64_t i = i0; i < i1;) {
+        int first;
+        const Group g = group_at(p, i, i1, p.ga, nbw, lane, first);
+        group_begin(p.T, first, lane, L.cnt, L.seg);
+        const float *tinfo = p.tinfo + g.ti * NTI;
+        floatx16 D;
+        floatx4 D4[2];
+#pragma unroll
+        for (int r = 0; r < 16; r++) D[r] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) D4[c][r] = 0.0f;
+        int s0 = 0, tb = 0;
+        for (int t = 0; t < p.T; t++) {
+            if (t == tb) {
+                tb = group_range(p.T, t, nbw, L.seg);
+                const int bad = compact_group<false>(p, i, t, tb, lane, nbw, L.nb, L.cnt, L.seg, nullptr);
+                if (bad >= 0 && lane == 0) atomicCAS(p.status, 0, (int)(i + bad + 1));
+                s0 = 0;
+            }
+            const int nv = group_type(L.cnt, t), pair = g.ti * p.T + t;
+            for (int k0 = 0; k0 < nv; k0 += TILE) {
+                const bool live = k0 + n < nv && s0 + k0 + n < nbw;
+                int tp = pair;
+                asm volatile("" : "+v"(tp));
+                float Ri[4] = {0.f, 0.f, 0.f, 0.f};
+                float r, s, ds;
+                int q = 0;
+                if (live) {
+                    const float4 e = L.nb[s0 + k0 + n];
+                    q = __float_as_int(e.w) >> QSHIFT;
+                    ri_of(e, tinfo, p.rmin, p.rmax, p.iw, Ri, r, s, ds);
+                }
+                float G[16];
+                if constexpr (GST) {
+                    // store mode: G and dG/ds at the entry's index among its atom's neighbors of this type
+                    float Gd[16];
+                    embed_fwd_tan<E, BF16, false>(p.vec, mat, tp, lane, Ri[0], G, Gd);
+                    int k = k0 + n;
+                    for (int x = 0; x < GA - 1; x++) k -= x < q ? L.cnt[t * GA + x] : 0;
+                    if (live && k < p.cap) store_g<E, BF16>(p, i + q, t, k, h, G, Gd);
+                } else {
+                    float h1[16], t2[16], t3[16];
+                    embed_fwd<E, BF16, false>(p.vec, mat, tp, lane, Ri[0], h1, t2, t3, G);
+                }
+                if (!live) Ri[0] = Ri[1] = Ri[2] = Ri[3] = 0.0f;
+                if constexpr (BF16) {
+                    __bf16 *rit = reinterpret_cast<__bf16 *>(L.rest), *gt = rit + 32 * 32;
+                    reinterpret_cast<uint4 *>(rit)[lane] = make_uint4(0, 0, 0, 0);      // rows of the four atoms
+                    __builtin_amdgcn_wave_barrier();
+                    if (h == 0) {
+#pragma unroll
+                        for (int w = 0; w < 4; w++) rit[(4 * q + w) * 32 + n] = (__bf16)Ri[w];
+                    }
+#pragma unroll
+                    for (int rr = 0; rr < NR; rr++) {
+                        const int f = feat(rr, h);
+                        if (f < E) gt[f * 32 + n] = (__bf16)G[rr];
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                    // rows >= 4 GA and columns >= E of D are never read: their lanes read row 0
+                    const int ia = n < 4 * GA ? n : 0, jb = n < E ? n : 0;
+                    const bf16x8 a0 = *reinterpret_cast<const bf16x8 *>(rit + ia * 32 + 8 * h);
+                    const bf16x8 a1 = *reinterpret_cast<const bf16x8 *>(rit + ia * 32 + 16 + 8 * h);
+                    const bf16x8 b0 = *reinterpret_cast<const bf16x8 *>(gt + jb * 32 + 8 * h);
+                    const bf16x8 b1 = *reinterpret_cast<const bf16x8 *>(gt + jb * 32 + 16 + 8 * h);
+                    D = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b0, D, 0, 0, 0);
+                    D = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, D, 0, 0, 0);
+                    __builtin_amdgcn_wave_barrier();
+                } else {
+                    float *xs = reinterpret_cast<float *>(L.rest);
+                    contract_group<E>(Ri, q, G, lane, xs, xs + 32 * 5, D4);
+                }
+            }
+            s0 += nv;
+        }
+        // lane (h, f = n) holds atoms h and 2 + h (BF16, registers 0-3 and 4-7), lane (q, f % 16) atom q for
+        // features f % 16 and 16 + f % 16 (FP32)
+        float scale;
+        const uint32_t tmask = frame_type_mask(p, i, scale);
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int q = BF16 ? 2 * u + h : lane >> 4, f = BF16 ? n : 16 * u + (lane & 15);
+            if (q < g.na && f < E) {
+                float pad = 0.0f;
+                for (int t = 0; t < p.T; t++) {
+                    if (!((tmask >> t) & 1u)) continue;     // the bucket of a type outside the frame's list
+                    pad += (float)(p.m - L.cnt[t * GA + q]) *
+                           vec_ptr(p.vec, g.ti * p.T + t, V_GPAD, (f >> 2) & 1)[4 * (f >> 3) + (f & 3)];
+                }
+                float *Ao = p.A + (size_t)(i + q) * 4 * E + f;
+#pragma unroll
+                for (int w = 0; w < 4; w++) {
+                    const float x = BF16 ? D[4 * u + w] : D4[u][w];
+                    Ao[w * E] = (x + tinfo[TI_SPAD + w] * pad) * scale;
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        i += g.na;
+    }
+}
+
+// The backward of up to GA atoms at once: dp_fused_bwd_kernel's tile with the dA rows of the lane's own atom (read
+// once for dG and dRi), centre forces summed per atom of the tile. Measured against an
+// atom per wavefront: 73,742 atoms of four types in BF16 786 -> 495 us, 7,000 in FP32 212 -> 184.
+template <int E, bool BF16>
+__global__ void __launch_bounds__(FUSED_WAVES * WAVE)
+dp_group_bwd_kernel(FusedParams p) {
+    constexpr int NR = NReg<E>::value;
+    extern __shared__ float4 smem[];
+    __shared__ double vsum[FUSED_WAVES][9];
+    __shared__ int vfr[FUSED_WAVES];
+    const int lane = threadIdx.x & (WAVE - 1), wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int h = lane >> 5, n = lane & 31, nbw = group_nbw(p);
+    const GroupLds L = group_lds(reinterpret_cast<unsigned char *>(smem), wid, nbw, GROUP_DA_BYTES);
+    float4 *das = reinterpret_cast<float4 *>(L.rest);                 // [GA][DA_STRIDE] dA of each atom, scaled
+    float *cen = reinterpret_cast<float *>(das + GA * DA_STRIDE);     // [GA][3] centre forces
+    const unsigned char *mat = reinterpret_cast<const unsigned char *>(p.mat);
+    int vframe = -1;
+    // virial: an FP32 partial per group and lane, added to FP64 lane sums of the frame (as dp_fused_bwd_kernel)
+    float vf[9];
+    double vd[9];
+#pragma unroll
+    for (int v = 0; v < 9; v++) { vf[v] = 0.0f; vd[v] = 0.0; }
+    const int64_t i0 = ((int64_t)blockIdx.x * FUSED_WAVES + wid) * p.gchunk;
+    const int64_t i1 = i0 + p.gchunk < p.natoms ? i0 + p.gchunk : p.natoms;
+    for (int64_t i = i0; i < i1;) {
+        int first;
+        const Group g = group_at(p, i, i1, p.ga, nbw, lane, first);
+        if (g.frame != vframe) {
+#pragma unroll
+            for (int v = 0; v < 9; v++) {
+                const double x = wave_sum(vd[v]);
+                if (vframe >= 0 && lane == v && x != 0.0) atomic_add(p.virial + 9 * vframe + v, x);
+                vd[v] = 0.0;
+            }
+            vframe = g.frame;
+        }
+        float scale;
+        frame_type_mask(p, i, scale);
+        float dav[GA][2];
+#pragma unroll
+        for (int q = 0; q < GA; q++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int x = lane + u * WAVE, f = x >> 2, w = x & 3;
+                dav[q][u] = (q < g.na && f < E) ? p.dA[(size_t)(i + q) * 4 * E + w * E + f] : 0.0f;
+            }
+        group_begin(p.T, first, lane, L.cnt, L.seg);
+#pragma unroll
+        for (int q = 0; q < GA; q++)
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+                reinterpret_cast<float *>(das + q * DA_STRIDE)[lane + u * WAVE] = dav[q][u] * scale;
+        if (lane < 3 * GA) cen[lane] = 0.0f;
+        __builtin_amdgcn_wave_barrier();
+        const float *tinfo = p.tinfo + g.ti * NTI;
+        int s0 = 0, tb = 0;
+        for (int t = 0; t < p.T; t++) {
+            if (t == tb) {
+                tb = group_range(p.T, t, nbw, L.seg);
+                compact_group<false>(p, i, t, tb, lane, nbw, L.nb, L.cnt, L.seg, p.fslot);
+                s0 = 0;
+            }
+            const int nv = group_type(L.cnt, t), pair = g.ti * p.T + t;
+            for (int k0 = 0; k0 < nv; k0 += TILE) {
+                int tp = pair;
+                asm volatile("" : "+v"(tp));
+                const int last = nv - k0 < TILE ? nv - k0 : TILE;      // live lanes of the tile
+                const bool live = n < last && s0 + k0 + n < nbw;
+                const float4 e = live ? L.nb[s0 + k0 + n] : make_float4(1.f, 0.f, 0.f, 0.f);
+                const int q = live ? __float_as_int(e.w) >> QSHIFT : 0;
+                const int64_t slot = ((i + q) * p.T + t) * (int64_t)p.mnl + (__float_as_int(e.w) & ((1 << QSHIFT) - 1));
+                // gather mode: the partner slot, loaded here so that its latency hides behind the tile
+                const int rs = (p.fslot && live && h == 0) ? p.rev[slot] : -1;
+                float Ri[4] = {0.f, 0.f, 0.f, 0.f};
+                float r = 1.f, s = 0.f, ds = 0.f;
+                if (live) ri_of(e, tinfo, p.rmin, p.rmax, p.iw, Ri, r, s, ds);
+                float dRi[4] = {0.f, 0.f, 0.f, 0.f};
+                float dsum = 0.0f;
+                const float *w1 = vec_ptr(p.vec, tp, V_W1, h);
+                floatx16 acc;
+                float dz[16], g1[16], g2[16];
+                {
+                    float G[16], t3[16];
+                    embed_fwd<E, BF16, false>(p.vec, mat, tp, lane, Ri[0], g1, g2, t3, G);
+                    // dG = dA Ri and dRi = dA G (this half's features) with the lane's own atom's dA
+                    const float4 *da = das + q * DA_STRIDE;
+#pragma unroll
+                    for (int rr = 0; rr < 16; rr++) {
+                        acc[rr] = 0.0f;
+                        dz[rr] = 0.0f;
+                        if (rr < NR) {
+                            const float4 d = da[feat(rr, h)];
+                            acc[rr] = d.x * Ri[0] + d.y * Ri[1] + d.z * Ri[2] + d.w * Ri[3];
+                            dRi[0] += d.x * G[rr];
+                            dRi[1] += d.y * G[rr];
+                            dRi[2] += d.z * G[rr];
+                            dRi[3] += d.w * G[rr];
+                            // layer 3: G = h2 + r3 t3 -> dh2 = dG + (W3 diag r3) (dG (1 - t3^2))
+                            dz[rr] = acc[rr] * (1.0f - t3[rr] * t3[rr]);
+                        }
+                    }
+                }
+                mfma_layer<BF16, false>(mat_ptr<BF16>(mat, tp, M_W3B), lane, dz, acc);
+                // layer 2: h2 = h1 + r2 t2 -> dh1 = dh2 + (W2 diag r2) (dh2 (1 - t2^2))
+#pragma unroll
+                for (int rr = 0; rr < 16; rr++) dz[rr] = rr < NR ? acc[rr] * (1.0f - g2[rr] * g2[rr]) : 0.0f;
+                mfma_layer<BF16, false>(mat_ptr<BF16>(mat, tp, M_W2B), lane, dz, acc);
+                // layer 1: h1 = tanh(s w1 + b1) -> ds = sum_f dh1 (1 - h1^2) w1
+#pragma unroll
+                for (int rr = 0; rr < NR; rr++) dsum += acc[rr] * (w1[rr] * (1.0f - g1[rr] * g1[rr]));
+                if constexpr (BF16) dsum *= 1.0f / TANH_K;     // w1 is stored pre-scaled
+                dRi[0] += dsum;
+                fold_halves2(dRi[0], dRi[1]);
+                fold_halves2(dRi[2], dRi[3]);
+                // force of this slot: f_a = sum_w dE/dRi_w * Ri_d[w][a], Ri_d = -dfeat/dstd
+                float f[3] = {0.f, 0.f, 0.f};
+                if (live && h == 0) {
+                    const float ir = __builtin_amdgcn_rcpf(r);
+                    const float x[3] = {e.x, e.y, e.z};
+                    float gw[4];
+#pragma unroll
+                    for (int w = 0; w < 4; w++) gw[w] = dRi[w] * tinfo[TI_ISTD + w];
+                    const float common = (ds - s * ir) * ir * ir;
+                    const float gx = gw[1] * x[0] + gw[2] * x[1] + gw[3] * x[2];
+                    const float cf = gw[0] * ds * ir + common * gx;
+#pragma unroll
+                    for (int a = 0; a < 3; a++) f[a] = -(x[a] * cf + gw[a + 1] * s * ir);
+                    if (p.fslot) {
+                        if (rs >= 0) p.fslot[rs] = make_float4(f[0], f[1], f[2], 0.f);
+                    } else {
+                        const int64_t j = (p.frame_start ? p.frame_start[g.frame] : 0) + p.list[slot] - 1;
+                        atomic_add(p.force + 3 * j, f[0]);
+                        atomic_add(p.force + 3 * j + 1, f[1]);
+                        atomic_add(p.force + 3 * j + 2, f[2]);
+                    }
+#pragma unroll
+                    for (int a = 0; a < 3; a++)
+#pragma unroll
+                        for (int c = 0; c < 3; c++) vf[3 * a + c] += f[a] * x[c];
+                }
+                // centre forces of the tile's atoms (its entries are sorted by atom; lanes of half 0 hold f)
+                const int q0 = __builtin_amdgcn_readfirstlane(q), q1 = __builtin_amdgcn_readlane(q, last - 1);
+                for (int x = q0; x <= q1; x++) {
+#pragma unroll
+                    for (int a = 0; a < 3; a++) {
+                        const float c = half_sum(q == x ? f[a] : 0.0f);
+                        if (lane == 0) cen[3 * x + a] -= c;
+                    }
+                }
+            }
+            s0 += nv;
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (lane < 3 * g.na) {
+            const float c = cen[lane];
+            if (p.fcenter) p.fcenter[3 * i + lane] = c;
+            else atomic_add(p.force + 3 * i + lane, c);
+        }
+#pragma unroll
+        for (int v = 0; v < 9; v++) {
+            vd[v] += (double)vf[v];
+            vf[v] = 0.0f;
+        }
+        __builtin_amdgcn_wave_barrier();
+        i += g.na;
+    }
+    // the last frame's sums: one set of atomics per block and frame
+#pragma unroll
+    for (int v = 0; v < 9; v++) {
+        const double x = wave_sum(vd[v]);
+        if (lane == 0) vsum[wid][v] = x;
+    }
+    if (lane == 0) vfr[wid] = vframe;
+    __syncthreads();
+    if (threadIdx.x < 9) {
+        double acc = 0.0;
+        int fr = -1;
+        for (int w = 0; w < FUSED_WAVES; w++) {
+            if (vfr[w] < 0) continue;
+            if (vfr[w] != fr) {
+                if (fr >= 0 && acc != 0.0) atomic_add(p.virial + 9 * fr + threadIdx.x, acc);
+                fr = vfr[w];
+                acc = 0.0;
+            }
+            acc += vsum[w][threadIdx.x];
+        }
+        if (fr >= 0 && acc != 0.0) atomic_add(p.virial + 9 * fr + threadIdx.x, acc);
+    }
+}
+
 // force[i] = fcenter[i] + sum over the used entries s of i's list of fslot[s]
 // (each written by the partner atom through the reverse slot map); one
 // wavefront per atom reading its own entries contiguously, fixed reduction
@@ -521,6 +831,21 @@ int launch_lw(FusedParams &p, bool fwd, hipStream_t st) {
     return check_launch("dp_fused_bwd_kernel");
 }
 
+// Net mode over groups of atoms (three types and more); returns 1 where the group's LDS does not fit.
+template <int E, bool BF16>
+int launch_group(FusedParams &p, bool fwd, hipStream_t st) {
+    const size_t extra = fwd ? (BF16 ? GROUP_BF16_BYTES : GROUP_F32_BYTES) : GROUP_DA_BYTES;
+    const size_t lds = FUSED_WAVES * (group_base_bytes(group_nbw(p)) + extra);
+    if (lds > 64 * 1024) return 1;
+    dp_group_shape(p);
+    const int64_t waves = (p.natoms + p.gchunk - 1) / p.gchunk, blocks = (waves + FUSED_WAVES - 1) / FUSED_WAVES;
+    const dim3 grid((unsigned)blocks), block(FUSED_WAVES * WAVE);
+    if (fwd && p.gbuf) hipLaunchKernelGGL((dp_group_fwd_kernel<E, BF16, true>), grid, block, lds, st, p);
+    else if (fwd) hipLaunchKernelGGL((dp_group_fwd_kernel<E, BF16, false>), grid, block, lds, st, p);
+    else hipLaunchKernelGGL((dp_group_bwd_kernel<E, BF16>), grid, block, lds, st, p);
+    return check_launch("dp_group_kernel");
+}
+
 // Net mode: weights in LDS or global memory, 2, 4 or 8 wavefronts per block.
 template <int E, bool BF16, bool GST>
 int launch_net(FusedParams &p, bool fwd, hipStream_t st, bool lw, int w) {
@@ -541,6 +866,11 @@ template <int E, bool BF16>
 int launch(FusedParams &p, bool fwd, hipStream_t st, int ck) {
     if (ck == 4) return launch_lw<E, BF16, false, 4>(p, fwd, st);
     if (ck == 6) return launch_lw<E, BF16, false, 6>(p, fwd, st);
+    // (the stored backward reads G atom by atom)
+    if ((fwd || !p.gbuf) && dp_group_wanted(p.T, p.mnl, p.natoms)) {
+        const int rc = launch_group<E, BF16>(p, fwd, st);
+        if (rc <= 0) return rc;
+    }
     const int mode = g_launch[fwd ? 0 : 1].lds_weights;
     // a wavefront count set for another workload whose neighbor tiles would exceed the LDS budget
     // here falls back to fewer wavefronts per block
