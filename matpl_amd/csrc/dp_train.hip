@@ -392,27 +392,59 @@ __device__ __forceinline__ void flush_pair(float *grad, int pair, int lane, floa
     }
 }
 
+// One pair's weights in this wavefront's LDS: [NVEC][2][16] floats, then the matrices in the chunked layout of
+// stage_weights.
+template <bool BF16>
+constexpr int EG_WEIGHT_BYTES = NVEC * 32 * 4 + NMAT * MatLayout<BF16>::BLK;
+
+template <bool BF16>
+__device__ __forceinline__ void stage_pair(const FusedParams &p, int pair, int lane, float *svec, unsigned char *smat) {
+    using ML = MatLayout<BF16>;
+    const float *v = p.vec + (size_t)pair * NVEC * 32;
+    for (int x = lane; x < NVEC * 32; x += WAVE) svec[x] = v[x];
+    const uint4 *g = reinterpret_cast<const uint4 *>(mat_ptr<BF16>(reinterpret_cast<const unsigned char *>(p.mat), pair, 0));
+    uint4 *l = reinterpret_cast<uint4 *>(smat);
+#pragma unroll
+    for (int m = 0; m < NMAT; m++)
+#pragma unroll
+        for (int c = 0; c < ML::CPL; c++) l[(m * ML::CPL + c) * 64 + lane] = g[(m * 64 + lane) * ML::CPL + c];
+    __builtin_amdgcn_wave_barrier();
+}
+
 template <int E, bool BF16>
-__global__ void __launch_bounds__(FUSED_WAVES * WAVE)
+__global__ void __launch_bounds__(WAVE, BF16 ? 2 : 1)
 dp_train_embgrad_kernel(TrainParams tp) {
     constexpr int NR = NReg<E>::value;
     static_assert(E < 32, "row E of the layer inputs carries the bias gradient");
     constexpr float IK = BF16 ? 1.0f / TANH_K : 1.0f;
     const FusedParams &p = tp.f;
     extern __shared__ float4 smem[];
-    const int lane = threadIdx.x & (WAVE - 1), wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int lane = threadIdx.x;
     const int h = lane >> 5, n = lane & 31;
     // per wave: the batch's compacted neighbors [NBW] (dx, dy, dz, atom of the batch), their
     // residual differences r_j - r_i [NBW], Ahat and Abar of the batch's atoms [EGA][32 features][4]
     constexpr int EGA = eg_atoms<BF16>();
     const int NBW = p.cap > WAVE ? p.cap : WAVE;
-    float4 *nb = smem + (size_t)wid * (2 * NBW + 2 * EGA * 32 + (BF16 ? 0 : EG_TFLOAT4));
+    float4 *nb = smem;
     float4 *us = nb + NBW;
     float4 *ahs = us + NBW, *abs = ahs + EGA * 32;
     float *tscr = reinterpret_cast<float *>(abs + EGA * 32);     // FP32 transpose tile
-    const int64_t wg = (int64_t)blockIdx.x * FUSED_WAVES + wid;
-    const int t = (int)(wg % p.T);
-    const int64_t i0 = (wg / p.T) * tp.chunk;
+    // the weights of the pair in hand: a wavefront's bucket type is fixed and its atoms change type rarely, so they
+    // are staged once per change instead of read through L2 by every tile. The addresses that this frees, and one
+    // outer product at a time, leave BF16 room for two wavefronts per SIMD; with that, single-wavefront blocks spread
+    // over the XCDs and the rows loaded ahead of the compaction, 73,742 atoms of four types take 1190 us (1452 with
+    // one wavefront per SIMD in blocks of one wavefront per bucket type), 7,000 in FP32 396 (433)
+    float *svec = tscr + (BF16 ? 0 : 4 * EG_TFLOAT4);
+    unsigned char *smat = reinterpret_cast<unsigned char *>(svec + NVEC * 32);
+    // (a wavefront per block: the bucket types' wavefronts differ several times in work, and a block of four would
+    // hold its SIMDs until the longest ends)
+    // Blocks go to the XCDs round-robin: eight chunks of one bucket type, then the same eight of the next, so that
+    // every XCD gets every type's share (with the type varying fastest the types with long buckets, half the work,
+    // would all fall to the same two of eight XCDs).
+    const int t = (int)(blockIdx.x / NXCD % p.T);
+    const int64_t chunk = blockIdx.x / (NXCD * (unsigned)p.T) * NXCD + blockIdx.x % NXCD;
+    const int64_t i0 = chunk * tp.chunk;
+    if (i0 >= p.natoms) return;
     int64_t i1 = i0 + tp.chunk;
     if (i1 > p.natoms) i1 = p.natoms;
     Transposer<BF16> tr;
@@ -452,6 +484,8 @@ dp_train_embgrad_kernel(TrainParams tp) {
         if (pair != cur) {
             if (cur >= 0) flush_pair<E>(tp.grad, cur, lane, g3, g2, w1s, b1s);
             cur = pair;
+            __builtin_amdgcn_wave_barrier();
+            stage_pair<BF16>(p, pair, lane, svec, smat);
         }
         if (tot == 0) {
             i += na;
@@ -461,16 +495,19 @@ dp_train_embgrad_kernel(TrainParams tp) {
         frame_type_mask(p, i, scale);
         const float *tinfo = p.tinfo + ti * NTI;
         const AtomGeo g0 = atom_geo(p, i);
-        // the batch's Ahat and Abar, scaled by c, feature-major
-        {
-            float *ahf = reinterpret_cast<float *>(ahs), *abf = reinterpret_cast<float *>(abs);
-            for (int x = lane; x < na * 128; x += WAVE) {
-                const int q = x >> 7, f = (x & 127) >> 2, w = x & 3;
+        // the batch's Ahat and Abar, scaled by c, feature-major: all loads go out before the compaction's, so that
+        // one wait covers both (a lane holds two of an atom's 128 padded values of each)
+        float ahv[EGA][2], abv[EGA][2];
+#pragma unroll
+        for (int q = 0; q < EGA; q++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int x = lane + u * WAVE, f = x >> 2, w = x & 3;
                 const size_t src = (size_t)(i + q) * 4 * E + w * E + f;
-                ahf[x] = f < E ? tp.ahat[src] * scale : 0.0f;
-                abf[x] = f < E ? tp.abar[src] * scale : 0.0f;
+                const bool in = q < na && f < E;
+                ahv[q][u] = in ? tp.ahat[src] : 0.0f;
+                abv[q][u] = in ? tp.abar[src] : 0.0f;
             }
-        }
         // in-cutoff neighbors of bucket t, atom by atom in order, with r_j - r_i (loaded with the
         // neighbor's position, so that the tiles below read nothing from global memory)
         int nv = 0;
@@ -502,6 +539,14 @@ dp_train_embgrad_kernel(TrainParams tp) {
             nv += __popcll(bal);
         }
         if (nv > NBW) nv = NBW;
+#pragma unroll
+        for (int q = 0; q < EGA; q++)
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+                if (q < na) {
+                    reinterpret_cast<float *>(ahs)[q * 128 + u * WAVE + lane] = ahv[q][u] * scale;
+                    reinterpret_cast<float *>(abs)[q * 128 + u * WAVE + lane] = abv[q][u] * scale;
+                }
         __builtin_amdgcn_wave_barrier();
         for (int k0 = 0; k0 < nv; k0 += TILE) {
             const int k = k0 + n;
@@ -517,9 +562,11 @@ dp_train_embgrad_kernel(TrainParams tp) {
                 ri_tangent(e, tinfo, r, s, ds, u, v);
                 qa = __float_as_int(e.w);
             }
-            const int pr = pair;
+            // (re-read the weights every tile instead of keeping them live across tiles)
+            int pr = 0;
+            asm volatile("" : "+v"(pr));
             EmbTan<E, BF16> et;
-            et.run(p.vec, reinterpret_cast<const unsigned char *>(p.mat), pr, lane, Ri[0]);
+            et.template run<true>(svec, smat, pr, lane, Ri[0]);
             // upstream of G: a = Ahat Ri - Abar v; of G': b = -v0 Abar Ri, with the rows of the lane's
             // own atom of the batch (FP32)
             floatx16 a, b;
@@ -553,15 +600,15 @@ dp_train_embgrad_kernel(TrainParams tp) {
                 if (feat(rr, h) == E) x[rr] = 1.0f;
             }
             {
-                const floatx16 xt = tr.apply(x), yt = tr.apply(zb), xdt = tr.apply(xd), ydt = tr.apply(zbd);
-                outer_acc<BF16>(xt, yt, g3);
-                outer_acc<BF16>(xdt, ydt, g3);
+                // (BF16: one product at a time, so that two wavefronts share a SIMD)
+                outer_acc<BF16>(tr.apply(x), tr.apply(zb), g3);
+                if constexpr (BF16) __builtin_amdgcn_sched_barrier(0);
+                outer_acc<BF16>(tr.apply(xd), tr.apply(zbd), g3);
+                if constexpr (BF16) __builtin_amdgcn_sched_barrier(0);
             }
             // h̄2 = a + W3 z̄3, ḣ̄2 = b + W3 ż̄3 (W3B: true weights)
-            mfma_layer<BF16, false>(mat_ptr<BF16>(reinterpret_cast<const unsigned char *>(p.mat), pr, M_W3B), lane,
-                                    zb, a);
-            mfma_layer<BF16, false>(mat_ptr<BF16>(reinterpret_cast<const unsigned char *>(p.mat), pr, M_W3B), lane,
-                                    zbd, b);
+            mfma_layer<BF16, true>(mat_ptr<BF16>(smat, pr, M_W3B), lane, zb, a);
+            mfma_layer<BF16, true>(mat_ptr<BF16>(smat, pr, M_W3B), lane, zbd, b);
             // layer 2 (h2 = h1 + t2, ḣ2 = ḣ1 + (1 - t2^2) ż2)
 #pragma unroll
             for (int rr = 0; rr < 16; rr++) {
@@ -573,17 +620,17 @@ dp_train_embgrad_kernel(TrainParams tp) {
                 if (feat(rr, h) == E) x[rr] = 1.0f;
             }
             {
-                const floatx16 xt = tr.apply(x), yt = tr.apply(zb), xdt = tr.apply(xd), ydt = tr.apply(zbd);
-                outer_acc<BF16>(xt, yt, g2);
-                outer_acc<BF16>(xdt, ydt, g2);
+                // (BF16: one product at a time, so that two wavefronts share a SIMD)
+                outer_acc<BF16>(tr.apply(x), tr.apply(zb), g2);
+                if constexpr (BF16) __builtin_amdgcn_sched_barrier(0);
+                outer_acc<BF16>(tr.apply(xd), tr.apply(zbd), g2);
+                if constexpr (BF16) __builtin_amdgcn_sched_barrier(0);
             }
-            mfma_layer<BF16, false>(mat_ptr<BF16>(reinterpret_cast<const unsigned char *>(p.mat), pr, M_W2B), lane,
-                                    zb, a);
-            mfma_layer<BF16, false>(mat_ptr<BF16>(reinterpret_cast<const unsigned char *>(p.mat), pr, M_W2B), lane,
-                                    zbd, b);
+            mfma_layer<BF16, true>(mat_ptr<BF16>(smat, pr, M_W2B), lane, zb, a);
+            mfma_layer<BF16, true>(mat_ptr<BF16>(smat, pr, M_W2B), lane, zbd, b);
             // layer 1 (h1 = tanh(x w1 + b1) with x = Ri[0] the normalized input, ḣ1 = (1 - h1^2) w1):
             // w̄1 += x z̄1 + ż̄1, b̄1 += z̄1
-            const float *w1 = vec_ptr(p.vec, pr, V_W1, h);
+            const float *w1 = vec_ptr(svec, pr, V_W1, h);
 #pragma unroll
             for (int rr = 0; rr < NR; rr++) {
                 const float q = 1.0f - et.h1[rr] * et.h1[rr];
@@ -623,14 +670,15 @@ int launch_train(TrainParams &tp, int which, hipStream_t st) {
         return check_launch("dp_train_tangent_kernel");
     }
     const size_t nbw = p.cap > WAVE ? p.cap : WAVE;
-    const size_t lds = sizeof(float4) * FUSED_WAVES * (2 * nbw + 2 * eg_atoms<BF16>() * 32 + (BF16 ? 0 : EG_TFLOAT4));
-    MATPL_CHECK_ARG(lds <= 64 * 1024, "dp_train_embgrad: list width too large for LDS (%zu bytes)", lds);
+    // (the list width's limit: that of four wavefronts' tiles in 64 KB)
+    const size_t tiles = sizeof(float4) * (2 * nbw + 2 * eg_atoms<BF16>() * 32 + (BF16 ? 0 : EG_TFLOAT4));
+    MATPL_CHECK_ARG(FUSED_WAVES * tiles <= 64 * 1024, "dp_train_embgrad: list width too large for LDS (%zu bytes)", tiles);
+    const size_t lds = tiles + EG_WEIGHT_BYTES<BF16>;
     const int64_t chunks = (p.natoms + tp.chunk - 1) / tp.chunk;
     const int64_t waves = chunks * p.T;
-    const int64_t blocks = (waves + FUSED_WAVES - 1) / FUSED_WAVES;
-    MATPL_CHECK_ARG(blocks <= (1 << 30), "dp_train_embgrad: too many chunks");
-    // waves beyond chunks * T find an empty atom range
-    hipLaunchKernelGGL((dp_train_embgrad_kernel<E, BF16>), dim3((unsigned)blocks), dim3(FUSED_WAVES * WAVE), lds, st, tp);
+    MATPL_CHECK_ARG(waves <= (1 << 30), "dp_train_embgrad: too many chunks");
+    hipLaunchKernelGGL((dp_train_embgrad_kernel<E, BF16>), dim3((unsigned)((chunks + NXCD - 1) / NXCD * NXCD * p.T)),
+                       dim3(WAVE), lds, st, tp);
     return check_launch("dp_train_embgrad_kernel");
 }
 
