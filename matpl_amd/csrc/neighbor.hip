@@ -391,22 +391,43 @@ cell_kernel(Lattice lat, Grid g, const double *__restrict__ fw, const int32_t *_
 // exact negation of dR_ij in the cutoff test; a missing partner (per-type
 // cutoffs that differ, or a tie in the nearest-image rule) sets status.
 //
-// Each pair of entries is matched once, by its owner: the entry of the atom with the smaller
-// index (for an atom's own images, the entry whose packed shift is the larger of the two). A
-// first pass sets every slot to -1; the owner then binary-searches j's bucket (sorted by
-// (j, image)) for its partner and writes both directions. Every load of the search touches a
-// different cache line per lane, so the kernel is bound by the number of such loads, which the
-// owner rule halves (a two-pass scan, every 16th entry then 15, took twice as long as the seven
-// or eight probes of a binary search: 807 against 386 us on a 99,636-atom list of 160 slots per
-// type, when every entry searched). An entry whose owner-side partner is missing sets status
-// directly; one missing on the other side stays -1, which reverse_check_kernel (a pass over the
-// used entries) turns into status.
+// Every entry searches its partner's bucket (sorted by (j, image)) by itself, four entries to a
+// load: the loads touch a different cache line per lane, so the kernel is bound by their number,
+// and four-wide ones halve a binary search's. The 8 XCDs take contiguous ranges of atoms, whose
+// neighbors' buckets share their L2. 230 us on a 99,636-atom list of 160 slots per type (105
+// neighbors an atom); matching each pair once, by the atom of smaller index, took 246 us with the
+// same search, as the partner's entry is a scattered store, plus 47 us of passes that set all
+// slots to -1 first and check them last (with a scalar binary search and no ranges: 288 + 47).
 constexpr int REV_WAVES = 4;
+constexpr int REV_XCDS = 8;
 
-__global__ void __launch_bounds__(256)
-reverse_init_kernel(int32_t *__restrict__ rev, int64_t nslots) {
-    for (int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s < nslots; s += (int64_t)gridDim.x * blockDim.x)
-        rev[s] = -1;
+struct __attribute__((packed, aligned(4))) Int4 { int32_t v[4]; };
+
+// The entry of row[0 .. cnt) (ascending) that names `target` with image `want`, or -1.
+__device__ __forceinline__ int find_entry(const int32_t *__restrict__ row, const int32_t *__restrict__ image, int cnt,
+                                          int target, int want) {
+    int lo = 0, hi = cnt, at = -1;
+    while (hi - lo > 4) {
+        const int mid = lo + ((hi - lo - 4) >> 1);
+        const Int4 x = *reinterpret_cast<const Int4 *>(row + mid);
+        if (x.v[3] < target) lo = mid + 4;
+        else if (x.v[0] > target) hi = mid;
+        else {
+            lo = mid + (x.v[0] < target) + (x.v[1] < target) + (x.v[2] < target);
+            const int32_t there = lo == mid ? x.v[0] : lo == mid + 1 ? x.v[1] : lo == mid + 2 ? x.v[2] : x.v[3];
+            at = there == target ? lo : -1;
+            hi = -1;
+        }
+    }
+    if (hi >= 0) {
+        while (lo < hi && row[lo] < target) lo++;
+        if (lo < hi && row[lo] == target) at = lo;
+    }
+    if (at < 0 || image[at] == want) return at;
+    while (at > 0 && row[at - 1] == target) at--;        // several images of one atom
+    for (; at < cnt && row[at] == target; at++)
+        if (image[at] == want) return at;
+    return -1;
 }
 
 __global__ void __launch_bounds__(REV_WAVES * WAVE)
@@ -415,58 +436,31 @@ reverse_kernel(const int32_t *__restrict__ list, const int32_t *__restrict__ shi
                const int64_t *__restrict__ frame_start, const int32_t *__restrict__ atom_frame, int T, int m,
                int64_t n, int32_t *__restrict__ rev, int32_t *__restrict__ status) {
     const int lane = threadIdx.x & (WAVE - 1);
-    for (int64_t i = (int64_t)blockIdx.x * REV_WAVES + threadIdx.x / WAVE; i < n;
-         i += (int64_t)gridDim.x * REV_WAVES) {
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int64_t per = (n + REV_XCDS - 1) / REV_XCDS;
+    const int64_t i0 = (blockIdx.x % REV_XCDS) * per, i1 = i0 + per < n ? i0 + per : n;
+    for (int64_t i = i0 + (int64_t)(blockIdx.x / REV_XCDS) * REV_WAVES + wid; i < i1;
+         i += (int64_t)(gridDim.x / REV_XCDS) * REV_WAVES) {
         const int64_t fb = frame_start ? frame_start[atom_frame[i]] : 0;
         const int ti = type_map[i];
         const int target = (int)(i - fb) + 1;
-        int total = 0;
-        for (int t = 0; t < T; t++) total += counts[i * T + t];
-        for (int e0 = 0; e0 < total; e0 += WAVE) {
-            const int e = e0 + lane;
-            if (e < total) {
-                int t = 0, k = e;
-                while (k >= counts[i * T + t]) k -= counts[i * T + t++];
-                const int64_t s = (i * T + t) * (int64_t)m + k;
-                const int64_t j = fb + list[s] - 1;
-                const int sh = shift[s];
-                const int want = pack_shift(-((sh & 255) - 128), -(((sh >> 8) & 255) - 128),
-                                            -(((sh >> 16) & 255) - 128));
-                if (i < j || (i == j && sh > want)) {
-                    const int64_t base = (j * T + ti) * (int64_t)m;
-                    const int cnt = counts[j * T + ti];
-                    int lo = 0, hi = cnt;          // first entry naming an atom >= i (buckets are sorted)
-                    while (lo < hi) {
-                        const int mid = (lo + hi) >> 1;
-                        if (list[base + mid] < target) lo = mid + 1; else hi = mid;
-                    }
-                    int found = -1;
-                    for (int q = lo; q < cnt && list[base + q] == target; q++)
-                        if (shift[base + q] == want) { found = q; break; }
-                    if (found < 0) {
-                        atomicCAS(status, 0, (int)(i + 1));
-                    } else {
-                        rev[s] = (int32_t)(base + found);
-                        rev[base + found] = (int32_t)s;
-                    }
-                }
-            }
-        }
-    }
-}
-
-// status = 1 + i for the first atom i with a used entry left without its partner (the owner's list
-// lacks it); one wavefront per atom over its used entries
-__global__ void __launch_bounds__(REV_WAVES * WAVE)
-reverse_check_kernel(const int32_t *__restrict__ counts, const int32_t *__restrict__ rev, int T, int m, int64_t n,
-                     int32_t *__restrict__ status) {
-    const int lane = threadIdx.x & (WAVE - 1);
-    for (int64_t i = (int64_t)blockIdx.x * REV_WAVES + threadIdx.x / WAVE; i < n;
-         i += (int64_t)gridDim.x * REV_WAVES) {
         bool bad = false;
         for (int t = 0; t < T; t++) {
             const int c = counts[i * T + t];
-            for (int k = lane; k < c; k += WAVE) bad |= rev[(i * T + t) * (int64_t)m + k] < 0;
+            const int64_t s0 = (i * T + t) * (int64_t)m;
+            for (int k = lane; k < m; k += WAVE) {
+                int r = -1;
+                if (k < c) {
+                    const int64_t j = fb + list[s0 + k] - 1;
+                    const int sh = shift[s0 + k];
+                    const int want = pack_shift(-((sh & 255) - 128), -(((sh >> 8) & 255) - 128),
+                                                -(((sh >> 16) & 255) - 128));
+                    const int64_t base = (j * T + ti) * (int64_t)m;
+                    const int f = find_entry(list + base, shift + base, counts[j * T + ti], target, want);
+                    if (f < 0) bad = true; else r = (int32_t)(base + f);
+                }
+                rev[s0 + k] = r;
+            }
         }
         if (__ballot(bad) != 0ull && lane == 0) atomicCAS(status, 0, (int)(i + 1));
     }
@@ -717,16 +711,11 @@ MATPL_EXPORT int matpl_dp_neighbor_reverse(const int32_t *list, const int32_t *s
     MATPL_CHECK_ARG((frame_start == nullptr) == (atom_frame == nullptr),
                     "dp_neighbor_reverse: frame_start and atom_frame go together");
     hipStream_t st = (hipStream_t)stream;
-    const int64_t nslots = n * ntypes * (int64_t)m;
-    hipLaunchKernelGGL(reverse_init_kernel, dim3(grid_cap(nslots)), dim3(256), 0, st, rev, nslots);
-    int rc = check_launch("reverse_init_kernel");
-    if (rc) return rc;
-    hipLaunchKernelGGL(reverse_kernel, dim3(grid_cap(n, REV_WAVES)), dim3(REV_WAVES * WAVE), 0, st, list, shift, counts,
-                       type_map, frame_start, atom_frame, ntypes, m, n, rev, status);
-    if ((rc = check_launch("reverse_kernel"))) return rc;
-    hipLaunchKernelGGL(reverse_check_kernel, dim3(grid_cap(n, REV_WAVES)), dim3(REV_WAVES * WAVE), 0, st, counts, rev,
-                       ntypes, m, n, status);
-    return check_launch("reverse_check_kernel");
+    // at least one block per XCD, a multiple of them
+    const unsigned grid = REV_XCDS * ((grid_cap(n, REV_WAVES) + REV_XCDS - 1) / REV_XCDS);
+    hipLaunchKernelGGL(reverse_kernel, dim3(grid), dim3(REV_WAVES * WAVE), 0, st, list, shift, counts, type_map,
+                       frame_start, atom_frame, ntypes, m, n, rev, status);
+    return check_launch("reverse_kernel");
 }
 
 MATPL_EXPORT int matpl_dp_lmp_neighdata(const double *x, const int32_t *type, const int32_t *type_to_model,
