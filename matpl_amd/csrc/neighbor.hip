@@ -21,8 +21,11 @@
 //   brute  : one wavefront per atom, j in 64-wide chunks, integer wave scans to
 //            place hits; any number of frames (batched training data).
 //   cell   : one large frame; atoms binned into a fractional cell grid with a
-//            counting sort, each wavefront scans the <=27 neighbor cells,
-//            appends hits to per-type LDS buckets, then ranks them by j.
+//            counting sort, each cell's atoms in ascending index. A block owns
+//            a cell: it merges the <=27 neighbor cells into one ascending list
+//            of candidates in LDS, and each wavefront runs one of the cell's
+//            atoms over it, so hits come in list order. Cells too sparse or too
+//            full for that are searched atom by atom (hits ranked by index).
 #include "common.h"
 
 #pragma clang fp contract(off)
@@ -63,6 +66,13 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
         if (lane >= off) v += u;
     }
     return v;
+}
+
+// LDS written by the wavefront's other lanes is visible after this.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // A non-finite coordinate has no cell and no image: status gets STATUS_NONFINITE (before any
@@ -206,16 +216,21 @@ struct Grid {
     int off[3][3];     // distinct offsets per dim
 };
 
+// A wrapped coordinate in [0, 1): fmod leaves one below -10 negative.
+__device__ __forceinline__ double cell_frac(double f) { return f < 0.0 ? f + 1.0 : f; }
+
+__device__ __forceinline__ int cell_of(double f, int nc) {
+    const int v = (int)(cell_frac(f) * nc);
+    return v < 0 ? 0 : (v >= nc ? nc - 1 : v);
+}
+
 __global__ void bin_kernel(const double *__restrict__ fw, int64_t n, Grid g, int32_t *__restrict__ atom_cell,
                            int32_t *__restrict__ cell_count) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x) {
         int c[3];
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-            int v = (int)(fw[3 * i + d] * g.nc[d]);
-            c[d] = v < 0 ? 0 : (v >= g.nc[d] ? g.nc[d] - 1 : v);
-        }
+        for (int d = 0; d < 3; d++) c[d] = cell_of(fw[3 * i + d], g.nc[d]);
         const int cell = (c[0] * g.nc[1] + c[1]) * g.nc[2] + c[2];
         atom_cell[i] = cell;
         atomicAdd(cell_count + cell, 1);
@@ -254,109 +269,166 @@ __global__ void fill_cells_kernel(const int32_t *__restrict__ atom_cell, int64_t
         cell_atoms[atomicAdd(cursor + atom_cell[i], 1)] = (int32_t)i;
 }
 
-constexpr int CELL_WAVES = 4;   // wavefronts (atoms) per block
+// The atoms of each cell and its neighbors along z (1 to 3 cells), in ascending order. A cell's
+// list starts where the counts of those before it end: whole columns give noff times their atoms,
+// and within a column the sums of the cells' counts shifted by -1, 0 and 1 telescope.
+struct ZRun { int64_t at; int count; };      // in the sorted array
 
-__global__ void __launch_bounds__(CELL_WAVES * WAVE)
-cell_kernel(Lattice lat, Grid g, const double *__restrict__ fw, const int32_t *__restrict__ atom_cell,
-            const int32_t *__restrict__ cell_start, const int32_t *__restrict__ cell_atoms,
-            const int32_t *__restrict__ type_map, const double *__restrict__ rc_type, int T, int m, double rc_m,
-            int64_t n, int32_t *__restrict__ list, double *__restrict__ dR, int32_t *__restrict__ counts,
-            int32_t *__restrict__ shift, int32_t *__restrict__ status) {
-    extern __shared__ int32_t smem[];
-    // wid is the same on every lane: the atom, its cell and the cells' ranges stay scalar
+__device__ __forceinline__ ZRun z_run(const int32_t *__restrict__ cell_start, const Grid &g, int cell) {
+    const int nz = g.nc[2], z = cell % nz, c0 = cell - z;
+    const int s0 = cell_start[c0], column = cell_start[c0 + nz] - s0;
+    if (nz < 3) return {(int64_t)nz * s0 + (int64_t)z * column, column};
+    auto upto = [&](int x) { return cell_start[c0 + x] - s0; };      // atoms of cells z < x
+    auto count = [&](int x) { return cell_start[c0 + x + 1] - cell_start[c0 + x]; };
+    const int below = z > 0 ? z - 1 : nz - 1, above = z + 1 < nz ? z + 1 : 0;
+    const int64_t at = z == 0 ? 0 : (int64_t)upto(z - 1) + count(nz - 1) + upto(z) + upto(z + 1) - upto(1);
+    return {3 * (int64_t)s0 + at, count(below) + count(z) + count(above)};
+}
+
+// One wavefront per cell; the rank of an atom is the number of smaller ones. A run longer than
+// `cap` is left out: a block that would need it has too many candidates for LDS.
+constexpr int SORT_WAVES = 4;
+__global__ void __launch_bounds__(SORT_WAVES * WAVE)
+sort_runs_kernel(const int32_t *__restrict__ cell_start, int ncells, Grid g, int cap,
+                 const int32_t *__restrict__ cell_atoms, int32_t *__restrict__ sorted) {
     const int lane = threadIdx.x & (WAVE - 1), wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    int32_t *bucket = smem + wid * (T * m + 2 * T);   // [T][m] hit indices
+    for (int c = blockIdx.x * SORT_WAVES + wid; c < ncells; c += gridDim.x * SORT_WAVES) {
+        const ZRun run = z_run(cell_start, g, c);
+        if (run.count > cap) continue;
+        const int nz = g.nc[2], z = c % nz, c0 = c - z;
+        // the run's atoms are those of [s0, s1) and, where the period splits it, of [s2, ..)
+        int s0, s1, s2 = 0;
+        if (nz <= 3) { s0 = cell_start[c0]; s1 = cell_start[c0 + nz]; }
+        else if (z == 0) { s0 = cell_start[c0]; s1 = cell_start[c0 + 2]; s2 = cell_start[c0 + nz - 1]; }
+        else if (z == nz - 1) { s0 = cell_start[c0 + z - 1]; s1 = cell_start[c0 + nz]; s2 = cell_start[c0]; }
+        else { s0 = cell_start[c0 + z - 1]; s1 = cell_start[c0 + z + 2]; }
+        const int n0 = s1 - s0;
+        auto atom = [&](int e) { return e < run.count ? cell_atoms[e < n0 ? s0 + e : s2 + e - n0] : 0x7fffffff; };
+        for (int e0 = 0; e0 < run.count; e0 += WAVE) {
+            const int j = atom(e0 + lane);
+            int rank = 0;
+            for (int q0 = 0; q0 < run.count; q0 += WAVE) {
+                const int other = atom(q0 + lane);
+                const int nq = run.count - q0 < WAVE ? run.count - q0 : WAVE;
+                for (int q = 0; q < nq; q++) rank += __builtin_amdgcn_readlane(other, q) < j;
+            }
+            if (e0 + lane < run.count) sorted[run.at + rank] = j;
+        }
+    }
+}
+
+struct CellArgs {
+    Lattice lat;
+    Grid g;
+    const double *fw;
+    const int32_t *atom_cell, *cell_start, *cell_atoms, *type_map;
+    const double *rc_type;
+    int T, m;
+    double rc_m;
+    int64_t n;
+    int32_t *list;
+    double *dR;
+    int32_t *counts, *shift, *status;
+    // cell_block_kernel only
+    const int32_t *sorted;      // ascending runs along z
+    double pitch[3];            // of the cells, in fractions
+    int32_t *overfull;          // [0] their number, then the cells with more candidates than LDS holds
+    float pre2;                 // squared radius of the FP32 preselection (infinity: none)
+    int cap, ncells, nparts;    // candidates in LDS, cells, blocks per cell
+};
+
+// The neighbors of atom i found by one wavefront alone, from the cells around it: hits go to
+// per-type LDS buckets ([T][m], then [T] stored and [T] counted at rc_m) and are ranked by index.
+__device__ void cell_scan_atom(const CellArgs &A, int64_t i, int32_t *bucket) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    const Grid &g = A.g;
+    const double *__restrict__ fw = A.fw;
+    const int T = A.T, m = A.m;
     int32_t *cnt = bucket + T * m;                    // [T] stored
     int32_t *cntM = cnt + T;                          // [T] counted at rc_m
-    const int64_t i = blockIdx.x * (int64_t)CELL_WAVES + wid;
-    const bool active = i < n;
     for (int t = lane; t < 2 * T; t += WAVE) cnt[t] = 0;
-    __syncthreads();
-    const double *L = lat.a;
-    const double rc2 = rc_m * rc_m;
-    double fi0 = 0, fi1 = 0, fi2 = 0, rci2 = 0;
-    int ci[3] = {0, 0, 0};
-    if (active) {
-        fi0 = fw[3 * i]; fi1 = fw[3 * i + 1]; fi2 = fw[3 * i + 2];
-        const double rci = rc_type[type_map[i]];
-        rci2 = rci * rci;
-        int c = atom_cell[i];
-        ci[2] = c % g.nc[2]; c /= g.nc[2];
-        ci[1] = c % g.nc[1]; ci[0] = c / g.nc[1];
-    }
-    if (active) {
-        // The z cells of one (x, y) column are contiguous in cell_atoms, so the column's 1-3 z
-        // offsets become at most two runs of consecutive cells (the periodic wrap splits one), and
-        // the lanes sweep each run in one pass rather than cell by cell (about 90 candidates per
-        // run against about 30 per cell: fewer, fuller passes of the FP64 distance test).
-        int zr0[3], zr1[3], nzr = 0;
-        {
-            int zs[3];
-            const int nzo = g.noff[2];
-            for (int c = 0; c < nzo; c++) zs[c] = (ci[2] + g.off[2][c] + g.nc[2]) % g.nc[2];
-            for (int x = 1; x < nzo; x++)
-                for (int y = x; y > 0 && zs[y - 1] > zs[y]; y--) {
-                    const int tmp = zs[y]; zs[y] = zs[y - 1]; zs[y - 1] = tmp;
-                }
-            for (int c = 0; c < nzo; c++) {
-                if (nzr > 0 && zs[c] == zr1[nzr - 1] + 1) zr1[nzr - 1] = zs[c];
-                else { zr0[nzr] = zs[c]; zr1[nzr] = zs[c]; nzr++; }
+    wave_sync();
+    const double *L = A.lat.a;
+    const double rc2 = A.rc_m * A.rc_m;
+    const double fi0 = fw[3 * i], fi1 = fw[3 * i + 1], fi2 = fw[3 * i + 2];
+    const double rci = A.rc_type[A.type_map[i]];
+    const double rci2 = rci * rci;
+    int c = A.atom_cell[i];
+    int ci[3];
+    ci[2] = c % g.nc[2]; c /= g.nc[2];
+    ci[1] = c % g.nc[1]; ci[0] = c / g.nc[1];
+    // The z cells of one (x, y) column are contiguous in cell_atoms, so the column's 1-3 z
+    // offsets become at most two runs of consecutive cells (the periodic wrap splits one), and
+    // the lanes sweep each run in one pass rather than cell by cell (about 90 candidates per
+    // run against about 30 per cell: fewer, fuller passes of the FP64 distance test).
+    int zr0[3], zr1[3], nzr = 0;
+    {
+        int zs[3];
+        const int nzo = g.noff[2];
+        for (int c = 0; c < nzo; c++) zs[c] = (ci[2] + g.off[2][c] + g.nc[2]) % g.nc[2];
+        for (int x = 1; x < nzo; x++)
+            for (int y = x; y > 0 && zs[y - 1] > zs[y]; y--) {
+                const int tmp = zs[y]; zs[y] = zs[y - 1]; zs[y - 1] = tmp;
             }
+        for (int c = 0; c < nzo; c++) {
+            if (nzr > 0 && zs[c] == zr1[nzr - 1] + 1) zr1[nzr - 1] = zs[c];
+            else { zr0[nzr] = zs[c]; zr1[nzr] = zs[c]; nzr++; }
         }
-        for (int a = 0; a < g.noff[0]; a++)
-        for (int b = 0; b < g.noff[1]; b++)
-        for (int c = 0; c < nzr; c++) {
-            const int cx = (ci[0] + g.off[0][a] + g.nc[0]) % g.nc[0];
-            const int cy = (ci[1] + g.off[1][b] + g.nc[1]) % g.nc[1];
-            const int col = (cx * g.nc[1] + cy) * g.nc[2];
-            const int s0 = cell_start[col + zr0[c]], s1 = cell_start[col + zr1[c] + 1];
-            // two candidates per lane per pass, both passes' loads issued before either is used
-            for (int p0 = s0; p0 < s1; p0 += 2 * WAVE) {
-                int jj[2];
-                double fj[2][3];
+    }
+    for (int a = 0; a < g.noff[0]; a++)
+    for (int b = 0; b < g.noff[1]; b++)
+    for (int c = 0; c < nzr; c++) {
+        const int cx = (ci[0] + g.off[0][a] + g.nc[0]) % g.nc[0];
+        const int cy = (ci[1] + g.off[1][b] + g.nc[1]) % g.nc[1];
+        const int col = (cx * g.nc[1] + cy) * g.nc[2];
+        const int s0 = A.cell_start[col + zr0[c]], s1 = A.cell_start[col + zr1[c] + 1];
+        // two candidates per lane per pass, both passes' loads issued before either is used
+        for (int p0 = s0; p0 < s1; p0 += 2 * WAVE) {
+            int jj[2];
+            double fj[2][3];
 #pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    const int p = p0 + u * WAVE + lane;
-                    jj[u] = p < s1 ? cell_atoms[p] : -1;
-                }
+            for (int u = 0; u < 2; u++) {
+                const int p = p0 + u * WAVE + lane;
+                jj[u] = p < s1 ? A.cell_atoms[p] : -1;
+            }
 #pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    const int j = jj[u] < 0 ? 0 : jj[u];
-                    fj[u][0] = fw[3 * j]; fj[u][1] = fw[3 * j + 1]; fj[u][2] = fw[3 * j + 2];
-                }
+            for (int u = 0; u < 2; u++) {
+                const int j = jj[u] < 0 ? 0 : jj[u];
+                fj[u][0] = fw[3 * j]; fj[u][1] = fw[3 * j + 1]; fj[u][2] = fw[3 * j + 2];
+            }
 #pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    const int j = jj[u];
-                    if (j < 0) continue;
-                    double dx1 = fj[u][0] - fi0, dx2 = fj[u][1] - fi1, dx3 = fj[u][2] - fi2;
-                    near_image(dx1); near_image(dx2); near_image(dx3);
-                    double dx, dy, dz;
-                    frac_to_cart(L, dx1, dx2, dx3, dx, dy, dz);
-                    const double dd = dx * dx + dy * dy + dz * dz;
-                    if (dd < rc2 && dd > 1e-8) {
-                        const int tj = type_map[j];
-                        atomicAdd(cntM + tj, 1);
-                        if (dd < rci2) {
-                            const int k = atomicAdd(cnt + tj, 1);
-                            if (k < m) bucket[tj * m + k] = j;
-                        }
+            for (int u = 0; u < 2; u++) {
+                const int j = jj[u];
+                if (j < 0) continue;
+                double dx1 = fj[u][0] - fi0, dx2 = fj[u][1] - fi1, dx3 = fj[u][2] - fi2;
+                near_image(dx1); near_image(dx2); near_image(dx3);
+                double dx, dy, dz;
+                frac_to_cart(L, dx1, dx2, dx3, dx, dy, dz);
+                const double dd = dx * dx + dy * dy + dz * dz;
+                if (dd < rc2 && dd > 1e-8) {
+                    const int tj = A.type_map[j];
+                    atomicAdd(cntM + tj, 1);
+                    if (dd < rci2) {
+                        const int k = atomicAdd(cnt + tj, 1);
+                        if (k < m) bucket[tj * m + k] = j;
                     }
                 }
             }
         }
     }
-    __syncthreads();
-    if (!active) return;
+    wave_sync();
     bool overflow = false;
     for (int t = 0; t < T; t++) overflow |= cntM[t] > m;
     if (overflow) {
-        if (lane == 0) atomicCAS(status, 0, (int)(i + 1));
-        for (int t = 0; t < T; t++) cnt[t] = 0;
+        if (lane == 0) atomicCAS(A.status, 0, (int)(i + 1));
+        wave_sync();
+        for (int t = lane; t < T; t += WAVE) cnt[t] = 0;
+        wave_sync();
     }
     const int64_t S = (int64_t)T * m;
-    int32_t *li = list + i * S;
-    double *di = dR ? dR + i * S * 3 : nullptr;
-    int32_t *si = shift ? shift + i * S : nullptr;
+    int32_t *li = A.list + i * S;
+    double *di = A.dR ? A.dR + i * S * 3 : nullptr;
+    int32_t *si = A.shift ? A.shift + i * S : nullptr;
     for (int t = 0; t < T; t++) {
         const int nt = cnt[t];
         const int32_t *bk = bucket + t * m;
@@ -381,7 +453,292 @@ cell_kernel(Lattice lat, Grid g, const double *__restrict__ fw, const int32_t *_
             if (di) { di[3 * slot] = 0.0; di[3 * slot + 1] = 0.0; di[3 * slot + 2] = 0.0; }
             if (si) si[slot] = pack_shift(0, 0, 0);
         }
-        if (counts && lane == 0) counts[i * T + t] = nt;
+        if (A.counts && lane == 0) A.counts[i * T + t] = nt;
+    }
+    wave_sync();                                      // the next atom reuses the buckets
+}
+
+constexpr int CELL_WAVES = 4;   // wavefronts (atoms) per block
+
+__global__ void __launch_bounds__(CELL_WAVES * WAVE) cell_kernel(CellArgs A) {
+    extern __shared__ int32_t smem[];
+    // wid is the same on every lane: the atom, its cell and the cells' ranges stay scalar
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int64_t i = blockIdx.x * (int64_t)CELL_WAVES + wid;
+    if (i < A.n) cell_scan_atom(A, i, smem + wid * (A.T * A.m + 2 * A.T));
+}
+
+// The cells that cell_block_kernel left: blockIdx.x strides over the cells, blockIdx.y over the atoms of one.
+constexpr int OVER_X = 256, OVER_Y = 8;
+__global__ void __launch_bounds__(CELL_WAVES * WAVE) cell_overfull_kernel(CellArgs A) {
+    extern __shared__ int32_t smem[];
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    int32_t *bucket = smem + wid * (A.T * A.m + 2 * A.T);
+    const int ncells = A.overfull[0];
+    for (int x = blockIdx.x; x < ncells; x += OVER_X) {
+        const int cell = A.overfull[1 + x];
+        const int p1 = A.cell_start[cell + 1];
+        for (int p = A.cell_start[cell] + blockIdx.y * CELL_WAVES + wid; p < p1; p += OVER_Y * CELL_WAVES)
+            cell_scan_atom(A, A.cell_atoms[p], bucket);
+    }
+}
+
+// One block per cell (or per part of a cell's atoms). All atoms of a cell have the same
+// candidates, the atoms of the <=27 cells around it, so the block puts these in ascending order
+// once: the runs along z are sorted already, and two rounds of merging (along y, then x; an
+// atom's place is its own rank plus its lower bounds in the one or two sibling runs) leave one
+// list. With it go FP32 Cartesian positions relative to the cell, so that a wavefront rejects 64
+// candidates with one 16-byte LDS read and seven FP32 operations; the survivors (about one in
+// seven) are queued, and 64 at a time take the exact FP64 test with all lanes busy and are stored
+// in list order by ballots: no ranking and no atomics.
+//
+// The preselection keeps every pair that the exact test can accept: with three or more cells in
+// every direction the image that a cell pair implies is the only one within rc. It is cut at
+// A.pre2, which covers the rounding of FP32 positions; with fewer cells it is off (infinity).
+//
+// Four atoms of a wavefront go over the candidates together, so that an LDS read serves four
+// tests (one atom a pass: 240 us; LDS reads were then the bound), and the queue holds places in the
+// list, not indices. 80 VGPRs (six wavefronts a SIMD): at 64 the compiler kept the four atoms'
+// positions in scalar registers and spilled (201 us).
+//
+// Bound: VALU issue (about 740 instructions an atom: 135 of the sweep over 807 candidates, 240 of
+// the exact tests, 160 of its share of the merging). 189 us, against 496 us of the search atom by
+// atom, on the 99,636-atom HfO2 list of 160 slots per type at 6.5 A (105 neighbors an atom, 255 MB
+// of list and shift stores).
+constexpr int CB_WAVES = 8;
+constexpr int CB_ATOMS = 4;     // atoms of a wavefront per pass over the candidates
+constexpr int CB_QUEUE = 2 * WAVE;
+constexpr int CB_MIN_ATOMS = 6;     // atoms per cell, and atoms, from which on this is the faster search
+constexpr int CB_MIN_TOTAL = 5000;
+constexpr int CB_MIN_BLOCKS = 512;
+
+__device__ __forceinline__ int lanes_below(unsigned long long mask) {
+    return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+}
+
+__device__ __forceinline__ float lane_value(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double lane_value(double v, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
+__global__ void __launch_bounds__(CB_WAVES * WAVE, 6)
+cell_block_kernel(CellArgs A) {
+    extern __shared__ __align__(16) int32_t smem[];
+    __shared__ int run_start[10];
+    __shared__ int64_t run_src[9];
+    // blocks go round-robin to the 8 XCDs: give each one a contiguous range of cells
+    const int nwork = A.ncells * A.nparts, per = (nwork + 7) >> 3;
+    const int work = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || work >= nwork) return;
+    const int cell = work / A.nparts, part = work - cell * A.nparts;
+    const int lane = threadIdx.x & (WAVE - 1), wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int own0 = A.cell_start[cell], nown = A.cell_start[cell + 1] - own0;
+    if (part * CB_WAVES >= nown) return;
+    const Grid &g = A.g;
+    const double *__restrict__ fw = A.fw;
+    int ci[3];
+    {
+        int c = cell;
+        ci[2] = c % g.nc[2]; c /= g.nc[2];
+        ci[1] = c % g.nc[1]; ci[0] = c / g.nc[1];
+    }
+    const int n0 = g.noff[0], n1 = g.noff[1], nrun = n0 * n1;
+    if (wid == 0) {
+        int64_t src = 0;
+        int cnt = 0;
+        if (lane < nrun) {
+            const int a = lane / n1, b = lane % n1;
+            const int cx = (ci[0] + a - (n0 == 3) + g.nc[0]) % g.nc[0];
+            const int cy = (ci[1] + b - (n1 == 3) + g.nc[1]) % g.nc[1];
+            const ZRun run = z_run(A.cell_start, g, (cx * g.nc[1] + cy) * g.nc[2] + ci[2]);
+            src = run.at;
+            cnt = run.count;
+        }
+        const int incl = wave_incl_scan(cnt);
+        if (lane < nrun) { run_start[lane + 1] = incl; run_src[lane] = src - (incl - cnt); }
+        if (lane == 0) run_start[0] = 0;
+    }
+    __syncthreads();
+    const int total = run_start[nrun];
+    if (total > A.cap) {        // cell_overfull_kernel searches these
+        if (part == 0 && threadIdx.x == 0) A.overfull[1 + atomicAdd(A.overfull, 1)] = cell;
+        return;
+    }
+    uint32_t *keyA = reinterpret_cast<uint32_t *>(smem);             // [cap], later the wavefronts' queues
+    float4 *pos = reinterpret_cast<float4 *>(smem + A.cap);          // [cap] (x, y, z, index)
+    uint32_t *keyB = reinterpret_cast<uint32_t *>(pos);              // [cap], before the positions
+    auto run_of = [&](int idx, int stride, int nr) {                 // last run that starts at or before idx
+        int lo = 0;
+        for (int r = 1; r < nr; r++) lo += run_start[r * stride] <= idx;
+        return lo;
+    };
+    for (int idx = threadIdx.x; idx < total; idx += CB_WAVES * WAVE)
+        keyA[idx] = (uint32_t)A.sorted[run_src[run_of(idx, 1, nrun)] + idx];
+    __syncthreads();
+#pragma unroll
+    for (int round = 0; round < 2; round++) {       // along y (runs of nrun), then x (runs of n0)
+        const uint32_t *in = round ? keyB : keyA;
+        uint32_t *out = round ? keyA : keyB;
+        const int gs = round ? n0 : n1, stride = round ? n1 : 1, nr = round ? n0 : nrun;
+        int longest = 0;
+        for (int r = 0; r < nr; r++) {
+            const int len = run_start[(r + 1) * stride] - run_start[r * stride];
+            longest = len > longest ? len : longest;
+        }
+        const int top = longest > 0 ? 1 << (31 - __clz(longest)) : 0;
+        for (int idx = threadIdx.x; idx < total; idx += CB_WAVES * WAVE) {
+            const uint32_t k = in[idx];
+            const int r = run_of(idx, stride, nr);
+            const int r0 = gs == 3 ? (r / 3) * 3 : (gs == 2 ? (r & ~1) : r);
+            int at = run_start[r0 * stride] + idx - run_start[r * stride];
+            // the sibling runs r1, r2 (r itself when there are fewer: an empty one)
+            const int r1 = gs > 1 ? (r + 1 < r0 + gs ? r + 1 : r + 1 - gs) : r;
+            const int r2 = gs > 2 ? (r + 2 < r0 + gs ? r + 2 : r + 2 - gs) : r;
+            const int lo1 = run_start[r1 * stride], lo2 = run_start[r2 * stride];
+            const int hi1 = gs > 1 ? run_start[(r1 + 1) * stride] : lo1, hi2 = gs > 2 ? run_start[(r2 + 1) * stride] : lo2;
+            // both lower bounds bit by bit; reads beyond a run (at most 2 * cap words in) are not used
+            int b1 = lo1, b2 = lo2;
+            for (int step = top; step > 0; step >>= 1) {
+                const uint32_t k1 = in[b1 + step - 1], k2 = in[b2 + step - 1];
+                b1 = b1 + step <= hi1 && k1 < k ? b1 + step : b1;
+                b2 = b2 + step <= hi2 && k2 < k ? b2 + step : b2;
+            }
+            out[at + (b1 - lo1) + (b2 - lo2)] = k;
+        }
+        __syncthreads();
+    }
+    // FP32 positions relative to the cell's corner, the image taken from the cells' distance
+    const double *L = A.lat.a;
+    const double corner[3] = {ci[0] * A.pitch[0], ci[1] * A.pitch[1], ci[2] * A.pitch[2]};
+    auto rel = [&](double f0, double f1, double f2, float o[3]) {
+        const double f[3] = {f0, f1, f2};
+        double u[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const int dc = cell_of(f[d], g.nc[d]) - ci[d];
+            const double s = dc > 1 ? -1.0 : (dc < -1 ? 1.0 : 0.0);
+            u[d] = (cell_frac(f[d]) + s) - corner[d];
+        }
+        double x, y, z;
+        frac_to_cart(L, u[0], u[1], u[2], x, y, z);
+        o[0] = (float)x; o[1] = (float)y; o[2] = (float)z;
+    };
+    const int padded = (total + WAVE - 1) & ~(WAVE - 1);             // to whole wavefronts with points at infinity
+    for (int idx = threadIdx.x; idx < padded; idx += CB_WAVES * WAVE) {
+        float o[3] = {INFINITY, INFINITY, INFINITY};
+        int64_t j = 0;
+        if (idx < total) {
+            j = keyA[idx];
+            rel(fw[3 * j], fw[3 * j + 1], fw[3 * j + 2], o);
+        }
+        pos[idx] = make_float4(o[0], o[1], o[2], __int_as_float((int)j));
+    }
+    __syncthreads();
+    const int T = A.T, m = A.m;
+    const double rc2 = A.rc_m * A.rc_m;
+    const int64_t S = (int64_t)T * m;
+    // [CB_ATOMS][CB_QUEUE] candidates (places in pos) of each atom of the wavefront, over keyA, which is spent
+    uint16_t *queue = reinterpret_cast<uint16_t *>(smem) + wid * (CB_ATOMS * CB_QUEUE);
+    const float pre2 = A.pre2;
+    const int first = part * CB_WAVES + wid, step = CB_WAVES * A.nparts;
+    for (int a0 = first; a0 < nown; a0 += step * CB_ATOMS) {
+        // lane 16 u + t serves the wavefront's u-th atom of this pass; its type-t entries stored and counted
+        const int mine = a0 + (lane >> 4) * step;
+        const int64_t my_atom = A.cell_atoms[own0 + (mine < nown ? mine : a0)];
+        const double my_f[3] = {fw[3 * my_atom], fw[3 * my_atom + 1], fw[3 * my_atom + 2]};
+        float my_pos[3];
+        rel(my_f[0], my_f[1], my_f[2], my_pos);
+        const double my_rc = A.rc_type[A.type_map[my_atom]];
+        const double my_rc2 = my_rc * my_rc;
+        int stored = 0, counted = 0;
+        float px[CB_ATOMS], py[CB_ATOMS], pz[CB_ATOMS];
+        int qn[CB_ATOMS];
+#pragma unroll
+        for (int u = 0; u < CB_ATOMS; u++) {
+            // one that is not there is at infinity: nothing is taken for it
+            px[u] = __shfl(mine < nown ? my_pos[0] : INFINITY, 16 * u, WAVE);
+            py[u] = __shfl(my_pos[1], 16 * u, WAVE);
+            pz[u] = __shfl(my_pos[2], 16 * u, WAVE);
+            qn[u] = 0;
+        }
+        for (int s0 = 0; s0 < padded; s0 += WAVE) {
+            const float4 c = pos[s0 + lane];
+            bool full = false;
+#pragma unroll
+            for (int u = 0; u < CB_ATOMS; u++) {
+                const float dx = c.x - px[u], dy = c.y - py[u], dz = c.z - pz[u];
+                const bool take = fmaf(dx, dx, fmaf(dy, dy, dz * dz)) < pre2;
+                const unsigned long long mask = __ballot(take);
+                if (take) queue[u * CB_QUEUE + qn[u] + lanes_below(mask)] = (uint16_t)(s0 + lane);
+                qn[u] += __popcll(mask);
+                full |= qn[u] >= WAVE;
+            }
+            const bool last = s0 + WAVE >= padded;
+            if (!full && !last) continue;
+            // the exact test on 64 queued candidates at a time, on what is left after the last ones
+            wave_sync();
+#pragma unroll 1
+            for (int u = 0; u < CB_ATOMS; u++) {
+                int left = u == 0 ? qn[0] : u == 1 ? qn[1] : u == 2 ? qn[2] : qn[3];
+                while (left >= (last ? 1 : WAVE)) {
+                    const int64_t i = __builtin_amdgcn_readlane((int)my_atom, 16 * u);
+                    const int q = queue[u * CB_QUEUE + lane], rest = queue[u * CB_QUEUE + WAVE + lane];
+                    const bool live = lane < left;
+                    const int64_t j = live ? __float_as_int(pos[q].w) : i;
+                    const int tj = A.type_map[j];
+                    double dx1 = fw[3 * j] - lane_value(my_f[0], 16 * u), dx2 = fw[3 * j + 1] - lane_value(my_f[1], 16 * u),
+                           dx3 = fw[3 * j + 2] - lane_value(my_f[2], 16 * u);
+                    const int s1 = near_image(dx1), s2 = near_image(dx2), s3 = near_image(dx3);
+                    double dx, dy, dz;
+                    frac_to_cart(L, dx1, dx2, dx3, dx, dy, dz);
+                    const double dd = dx * dx + dy * dy + dz * dz;
+                    const bool inM = live && dd < rc2 && dd > 1e-8;
+                    const bool in = inM && dd < lane_value(my_rc2, 16 * u);
+                    int k = 0;
+                    for (int t = 0; t < T; t++) {
+                        const unsigned long long mk = __ballot(in && tj == t), mkM = __ballot(inM && tj == t);
+                        const int b = __builtin_amdgcn_readlane(stored, 16 * u + t);
+                        if (tj == t) k = b + lanes_below(mk);
+                        if (lane == 16 * u + t) { stored += __popcll(mk); counted += __popcll(mkM); }
+                    }
+                    if (in && k < m) {
+                        const int64_t slot = i * S + (int64_t)tj * m + k;
+                        A.list[slot] = (int32_t)j + 1;
+                        if (A.dR) { A.dR[3 * slot] = dx; A.dR[3 * slot + 1] = dy; A.dR[3 * slot + 2] = dz; }
+                        if (A.shift) A.shift[slot] = pack_shift(s1, s2, s3);
+                    }
+                    left -= left < WAVE ? left : WAVE;
+                    wave_sync();
+                    if (lane < left) queue[u * CB_QUEUE + lane] = (uint16_t)rest;
+                    wave_sync();
+                }
+#pragma unroll
+                for (int v = 0; v < CB_ATOMS; v++)
+                    if (v == u) qn[v] = left;
+            }
+        }
+#pragma unroll 1
+        for (int u = 0; u < CB_ATOMS && a0 + u * step < nown; u++) {
+            const int64_t i = __builtin_amdgcn_readlane((int)my_atom, 16 * u);
+            if (__any((lane >> 4) == u && counted > m)) {
+                if (lane == 0) atomicCAS(A.status, 0, (int)(i + 1));
+                if ((lane >> 4) == u) stored = 0;
+                __threadfence();            // the zeros below go over entries already stored
+            }
+            for (int t = 0; t < T; t++) {
+                const int nt = __builtin_amdgcn_readlane(stored, 16 * u + t);
+                for (int k = nt + lane; k < m; k += WAVE) {
+                    const int64_t slot = i * S + (int64_t)t * m + k;
+                    A.list[slot] = 0;
+                    if (A.dR) { A.dR[3 * slot] = 0.0; A.dR[3 * slot + 1] = 0.0; A.dR[3 * slot + 2] = 0.0; }
+                    if (A.shift) A.shift[slot] = pack_shift(0, 0, 0);
+                }
+            }
+            if (A.counts && (lane >> 4) == u && (lane & 15) < T) A.counts[i * T + (lane & 15)] = stored;
+        }
     }
 }
 
@@ -626,8 +983,9 @@ using namespace matpl;
 MATPL_EXPORT int64_t matpl_dp_neighbor_cell_workspace_bytes(const double *lattice_host, double rc_m, int64_t n) {
     Grid g = make_grid(lattice_host, rc_m);
     const int64_t ncells = (int64_t)g.nc[0] * g.nc[1] * g.nc[2];
-    // atom_cell[n], cell_atoms[n], cell_count[ncells], cell_start[ncells+1], cursor[ncells]
-    return (int64_t)sizeof(int32_t) * (2 * n + 3 * ncells + 1 + 64);
+    // atom_cell[n], cell_atoms[n], sorted[3n], cell_count[ncells], overfull[ncells+1], cell_start[ncells+1],
+    // cursor[ncells]
+    return (int64_t)sizeof(int32_t) * (5 * n + 4 * ncells + 2 + 64);
 }
 
 MATPL_EXPORT int matpl_dp_neighbor_is_small_box(const double *lattice_host, double rc_m) {
@@ -679,24 +1037,68 @@ MATPL_EXPORT int matpl_dp_neighbor_cell(const double *lattice_host, const double
     int32_t *ws = (int32_t *)workspace;
     int32_t *atom_cell = ws;
     int32_t *cell_atoms = atom_cell + n;
-    int32_t *cell_count = cell_atoms + n;
-    int32_t *cell_start = cell_count + ncells;
+    int32_t *sorted = cell_atoms + n;
+    int32_t *cell_count = sorted + 3 * n;               // zeroed, with the word after it
+    int32_t *overfull = cell_count + ncells;
+    int32_t *cell_start = overfull + 1 + ncells;
     int32_t *cursor = cell_start + ncells + 1;
     Lattice lat;
     for (int k = 0; k < 9; k++) lat.a[k] = lattice_host[k];
     int rc;
     hipLaunchKernelGGL(wrap_kernel, dim3(grid_cap(n * 3)), dim3(256), 0, st, frac, frac_wrapped, n * 3, status);
     if ((rc = check_launch("wrap_kernel"))) return rc;
-    if ((rc = fill_async<int32_t>(cell_count, 0, ncells, st))) return rc;
+    if ((rc = fill_async<int32_t>(cell_count, 0, ncells + 1, st))) return rc;
     hipLaunchKernelGGL(bin_kernel, dim3(grid_cap(n)), dim3(256), 0, st, frac_wrapped, n, g, atom_cell, cell_count);
     if ((rc = check_launch("bin_kernel"))) return rc;
     hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, st, cell_count, cell_start, cursor, ncells);
     if ((rc = check_launch("scan_kernel"))) return rc;
     hipLaunchKernelGGL(fill_cells_kernel, dim3(grid_cap(n)), dim3(256), 0, st, atom_cell, n, cursor, cell_atoms);
     if ((rc = check_launch("fill_cells_kernel"))) return rc;
-    hipLaunchKernelGGL(cell_kernel, dim3(ceil_div(n, CELL_WAVES)), dim3(CELL_WAVES * WAVE), lds, st, lat, g,
-                       frac_wrapped, atom_cell, cell_start, cell_atoms, type_map, rc_type, ntypes, m, rc_m, n, list,
-                       dR, counts, shift, status);
+    CellArgs A{};
+    A.lat = lat; A.g = g; A.fw = frac_wrapped; A.atom_cell = atom_cell; A.cell_start = cell_start;
+    A.cell_atoms = cell_atoms; A.type_map = type_map; A.rc_type = rc_type; A.T = ntypes; A.m = m; A.rc_m = rc_m;
+    A.n = n; A.list = list; A.dR = dR; A.counts = counts; A.shift = shift; A.status = status;
+    // A block per cell shares its candidates among the cell's atoms; with few atoms to a cell (a
+    // cluster or a slab in vacuum) its wavefronts idle, and with few atoms in all the chip has too
+    // few blocks to hide the merging. Whole searches at a cutoff of 6.5 A, by cells' blocks against
+    // atom by atom: 20,000 atoms at 4 a cell 100 and 90 us, at 8 a cell 80 and 95, at 16 a cell 91
+    // and 119; at a solid's density (0.09 per A^3) 3,000 atoms 82 and 69 us, 6,000 70 and 79,
+    // 12,000 89 and 126, 40,000 136 and 264.
+    if (n >= CB_MIN_TOTAL && n >= (int64_t)CB_MIN_ATOMS * ncells) {
+        // Candidates in LDS (20 bytes each): 2048, which a cell pitch of 6.5 to 9 A needs at the
+        // density of a solid, or 4096 where the average cell is fuller; fuller blocks search atom
+        // by atom.
+        const double avg = (double)n / ncells * (g.noff[0] * g.noff[1] * g.noff[2]);
+        A.cap = 1.5 * avg > 2048.0 ? 4096 : 2048;
+        hipLaunchKernelGGL(sort_runs_kernel, dim3(grid_cap(ncells, SORT_WAVES)), dim3(SORT_WAVES * WAVE), 0, st,
+                           cell_start, ncells, g, A.cap, cell_atoms, sorted);
+        if ((rc = check_launch("sort_runs_kernel"))) return rc;
+        A.sorted = sorted;
+        A.ncells = ncells;
+        // enough blocks for the chip, as long as each wavefront has an atom
+        const int most = (int)((n / ncells + CB_WAVES - 1) / CB_WAVES);
+        int parts = (CB_MIN_BLOCKS + ncells - 1) / ncells;
+        A.nparts = parts < 1 ? 1 : (parts > most ? (most > 0 ? most : 1) : parts);
+        // FP32 positions span at most three cells, R; each coordinate of a difference is wrong by
+        // at most 4 R 2^-24 (two roundings of positions, one of the difference) and the squared
+        // length by 4 of its ulps: |d| by less than 6e-7 R + 3e-7 rc.
+        double R = 0.0;
+        for (int d = 0; d < 3; d++)
+            R += 3.0 / g.nc[d] * sqrt(lattice_host[3 * d] * lattice_host[3 * d] +
+                                      lattice_host[3 * d + 1] * lattice_host[3 * d + 1] +
+                                      lattice_host[3 * d + 2] * lattice_host[3 * d + 2]);
+        const double pre = rc_m + 1e-6 * R + 1e-6 * rc_m;
+        A.pre2 = g.nc[0] >= 3 && g.nc[1] >= 3 && g.nc[2] >= 3 ? (float)(pre * pre * (1.0 + 1e-6)) : INFINITY;
+        for (int d = 0; d < 3; d++) A.pitch[d] = 1.0 / g.nc[d];
+        A.overfull = overfull;
+        const int64_t nwork = (int64_t)ncells * A.nparts;
+        hipLaunchKernelGGL(cell_block_kernel, dim3((unsigned)(8 * ((nwork + 7) / 8))), dim3(CB_WAVES * WAVE),
+                           (size_t)A.cap * 20, st, A);
+        if ((rc = check_launch("cell_block_kernel"))) return rc;
+        hipLaunchKernelGGL(cell_overfull_kernel, dim3(OVER_X, OVER_Y), dim3(CELL_WAVES * WAVE), lds, st, A);
+        return check_launch("cell_overfull_kernel");
+    }
+    hipLaunchKernelGGL(cell_kernel, dim3(ceil_div(n, CELL_WAVES)), dim3(CELL_WAVES * WAVE), lds, st, A);
     return check_launch("cell_kernel");
 }
 

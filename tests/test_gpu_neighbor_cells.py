@@ -1,4 +1,7 @@
-"""The reverse map against its definition."""
+"""The cell search against the brute-force one, bit for bit, over the forms its dispatch tells apart: cells with
+enough atoms for a block each, few atoms or sparse cells (atom by atom), cells with more candidates than LDS
+holds, fewer than three cells in a direction (no preselection), one block or several per cell, triclinic boxes,
+cutoffs per type, coordinates outside [0, 1). The reverse map against its definition."""
 import numpy as np
 import pytest
 import torch
@@ -14,6 +17,58 @@ def dev():
 
 
 CUBE = np.eye(3)
+TRI = np.array([[1.0, 0.1, 0.0], [-0.2, 1.1, 0.15], [0.05, -0.1, 0.95]])
+
+# name, lattice (A), atoms, types, cutoff, slots per type, cutoffs per type, spread (1: fills the box), offset
+CASES = [
+    ("blocks", 39.5 * CUBE, 5200, 2, 6.5, 160, None, 1.0, 0.0),
+    ("blocks_tri", 42.0 * TRI, 5100, 3, 6.0, 128, (6.0, 5.0, 5.5), 1.0, 0.0),
+    ("by_atom", 33.0 * CUBE, 3000, 2, 6.5, 160, None, 1.0, 0.0),
+    ("three_cells", 20.0 * CUBE, 5001, 1, 6.5, 900, None, 1.0, 0.0),
+    ("two_cells", np.diag([14.0, 35.0, 49.0]), 5123, 4, 6.9, 400, None, 1.0, 0.0),
+    ("one_cell", 30.0 * np.array([[1.0, 0, 0], [0.9, 0.5, 0], [0, 0, 1.0]]), 5000, 2, 8.0, 600, None, 1.0, 0.0),
+    ("sparse", 80.0 * CUBE, 5500, 2, 6.5, 64, (6.5, 4.0), 1.0, 0.0),
+    ("overfull", 60.0 * CUBE, 6000, 2, 6.0, 1400, None, 0.28, 0.0),
+    ("fuller_lds", 30.0 * CUBE, 5000, 5, 9.0, 300, None, 0.96, 0.0),
+    ("outside", 39.5 * CUBE, 5200, 2, 6.5, 160, None, 1.0, -13.0),
+    ("edge_cells", 39.2 * CUBE, 65 * 216, 16, 6.5, 100, None, 1.0, 0.0),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+@pytest.mark.parametrize("want_dR", [False, True])
+def test_cell_search_is_the_brute_force_one(dev, case, want_dR):
+    from matpl_amd.neighbor import find_neighbore_gpu
+    name, lat, n, T, rc, m, rct, spread, offset = case
+    rng = np.random.Generator(np.random.PCG64([len(name), n]))
+    frac = rng.random((n, 3)) * spread
+    if offset:
+        frac[::3] += offset
+        frac[1::3] += 7.0
+    types = rng.integers(0, T, n)
+    kw = dict(rc_type=rct, want_dR=want_dR, want_shift=True, device=dev)
+    print(f"{name} n={n} T={T}", flush=True)
+    a = find_neighbore_gpu(lat, frac, types, T, m, rc, **kw)
+    b = find_neighbore_gpu(lat, frac, types, T, m, rc, force_brute=True, **kw)
+    assert int(b.counts.sum()) > 0
+    for k in ("counts", "list", "shift", "frac_wrapped") + (("dR",) if want_dR else ()):
+        assert torch.equal(getattr(a, k), getattr(b, k)), k
+
+
+def test_cell_search_overflow_zeroes_the_row(dev):
+    from matpl_amd.neighbor import find_neighbore_gpu
+    rng = np.random.Generator(np.random.PCG64(5))
+    frac, types = rng.random((5200, 3)), rng.integers(0, 2, 5200)
+    frac[:80] = 0.5 + 0.02 * rng.random((80, 3))
+    kw = dict(want_dR=False, want_shift=True, device=dev, check=False)
+    a = find_neighbore_gpu(39.5 * CUBE, frac, types, 2, 60, 6.0, **kw)
+    b = find_neighbore_gpu(39.5 * CUBE, frac, types, 2, 60, 6.0, force_brute=True, **kw)
+    over = (b.counts.sum(1) == 0)
+    assert int(over.sum()) >= 80 and not bool(over.all())
+    assert int(a.status) > 0 and bool(over[int(a.status) - 1])
+    assert torch.equal(a.counts, b.counts)
+    assert torch.equal(a.list[~over], b.list[~over])
+    assert int(a.list[over].abs().sum()) == 0
 
 
 @pytest.mark.parametrize("lat,n,m", [(39.5 * CUBE, 1601, 27), (13.2 * CUBE, 130, 130), (8.0 * CUBE, 37, 150)])
