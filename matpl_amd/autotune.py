@@ -31,6 +31,7 @@ from . import _lib
 
 BLOCK_CAPS = (512, 768, 1024, 1536, 2048, 3072, 4096, 8192, 16384)
 WAVES = (2, 4, 8)
+# the shape that leaves the choice to the library (by size, types and precision)
 DEFAULT = {"max_blocks": 4096, "lds_weights": -1, "xcd": 0, "waves": 4}
 
 

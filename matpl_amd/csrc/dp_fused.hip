@@ -59,7 +59,8 @@ struct LaunchCfg {
     int xcd;
     int waves;          // wavefronts per block: 2, 4 or 8 (net mode; table mode always 4)
 };
-LaunchCfg g_launch[2] = {{4096, -1, 0, FUSED_WAVES}, {4096, -1, 0, FUSED_WAVES}};
+constexpr LaunchCfg LAUNCH_DEFAULT = {4096, -1, 0, FUSED_WAVES};
+LaunchCfg g_launch[2] = {LAUNCH_DEFAULT, LAUNCH_DEFAULT};
 
 template <int E, bool BF16, bool LW, int CK, bool GST, int W>
 __global__ void __launch_bounds__(W * WAVE)
@@ -807,12 +808,11 @@ gather_kernel(const int32_t *__restrict__ counts, const float4 *__restrict__ fsl
 }
 
 template <int E, bool BF16, bool LW, int CK = 0, bool GST = false, int W = FUSED_WAVES>
-int launch_lw(FusedParams &p, bool fwd, hipStream_t st) {
+int launch_lw(FusedParams &p, bool fwd, hipStream_t st, const LaunchCfg &cfg) {
     const size_t lds =
         fwd ? fused_lds_bytes<BF16, LW, false>(p.T, p.cap, W) : fused_lds_bytes<BF16, LW, true>(p.T, p.cap, W);
     MATPL_CHECK_ARG(lds <= 64 * 1024, "dp_fused: T*mnl too large for LDS (%zu bytes, %d waves per block)", lds, W);
     // persistent-style grid: a few blocks per CU, each strides over atoms
-    const LaunchCfg &cfg = g_launch[fwd ? 0 : 1];
     int64_t blocks = (p.natoms + W - 1) / W;
     if (blocks > cfg.max_blocks) blocks = cfg.max_blocks;
     p.xcd = 0;
@@ -848,15 +848,37 @@ int launch_group(FusedParams &p, bool fwd, hipStream_t st) {
 
 // Net mode: weights in LDS or global memory, 2, 4 or 8 wavefronts per block.
 template <int E, bool BF16, bool GST>
-int launch_net(FusedParams &p, bool fwd, hipStream_t st, bool lw, int w) {
+int launch_net(FusedParams &p, bool fwd, hipStream_t st, const LaunchCfg &cfg, bool lw, int w) {
     if (lw) {
-        if (w == 2) return launch_lw<E, BF16, true, 0, GST, 2>(p, fwd, st);
-        if (w == 8) return launch_lw<E, BF16, true, 0, GST, 8>(p, fwd, st);
-        return launch_lw<E, BF16, true, 0, GST, 4>(p, fwd, st);
+        if (w == 2) return launch_lw<E, BF16, true, 0, GST, 2>(p, fwd, st, cfg);
+        if (w == 8) return launch_lw<E, BF16, true, 0, GST, 8>(p, fwd, st, cfg);
+        return launch_lw<E, BF16, true, 0, GST, 4>(p, fwd, st, cfg);
     }
-    if (w == 2) return launch_lw<E, BF16, false, 0, GST, 2>(p, fwd, st);
-    if (w == 8) return launch_lw<E, BF16, false, 0, GST, 8>(p, fwd, st);
-    return launch_lw<E, BF16, false, 0, GST, 4>(p, fwd, st);
+    if (w == 2) return launch_lw<E, BF16, false, 0, GST, 2>(p, fwd, st, cfg);
+    if (w == 8) return launch_lw<E, BF16, false, 0, GST, 8>(p, fwd, st, cfg);
+    return launch_lw<E, BF16, false, 0, GST, 4>(p, fwd, st, cfg);
+}
+
+// The net-mode launch where the caller has set none, from LAUNCH_ATOMS atoms on. Times of a whole
+// evaluation, HfO2 (two types) and Cu (one), the plain launch (4096 blocks of 4, plain order) first:
+//   backward, weights in LDS: 512 blocks stage them once for many atoms, in contiguous ranges per
+//   XCD whose slot stores stay in one L2. BF16 11,880 HfO2 atoms 248 -> 199 us, 32,928: 498 -> 431,
+//   99,636: 1299 -> 1227; Cu 32,000: 398 -> 346, FP32 1014 -> 975. At 1,500 and 2,916 atoms the
+//   two are within 3 us or 7 us of each other, either way.
+//   forward, BF16 with two types: the four pairs' weights cost LDS, so wavefronts, and reading them
+//   through the caches with 8 wavefronts a block is faster: 248 -> 229, 498 -> 439, 1299 -> 1196.
+//   One type's (Cu) are better in LDS (398 -> 402 us without), and FP32's are read through the
+//   caches already.
+constexpr int64_t LAUNCH_ATOMS = 8192;
+
+LaunchCfg launch_cfg(const FusedParams &p, bool fwd, bool bf16, bool lds_fits) {
+    const LaunchCfg set = g_launch[fwd ? 0 : 1];
+    const bool unset = set.max_blocks == LAUNCH_DEFAULT.max_blocks && set.lds_weights == LAUNCH_DEFAULT.lds_weights &&
+                       set.xcd == LAUNCH_DEFAULT.xcd && set.waves == LAUNCH_DEFAULT.waves;
+    if (!unset || p.gbuf || p.natoms < LAUNCH_ATOMS) return set;
+    if (!fwd && lds_fits) return LaunchCfg{512, -1, 1, FUSED_WAVES};
+    if (fwd && bf16 && p.T == 2) return LaunchCfg{16384, 0, 1, 8};
+    return set;
 }
 
 // Weights go to LDS when they and the neighbor tiles fit in 64 KB per block
@@ -864,26 +886,30 @@ int launch_net(FusedParams &p, bool fwd, hipStream_t st, bool lw, int w) {
 // Table mode (ck = 4 or 6 coefficients) reads no net weights.
 template <int E, bool BF16>
 int launch(FusedParams &p, bool fwd, hipStream_t st, int ck) {
-    if (ck == 4) return launch_lw<E, BF16, false, 4>(p, fwd, st);
-    if (ck == 6) return launch_lw<E, BF16, false, 6>(p, fwd, st);
+    if (ck == 4) return launch_lw<E, BF16, false, 4>(p, fwd, st, g_launch[fwd ? 0 : 1]);
+    if (ck == 6) return launch_lw<E, BF16, false, 6>(p, fwd, st, g_launch[fwd ? 0 : 1]);
     // (the stored backward reads G atom by atom)
     if ((fwd || !p.gbuf) && dp_group_wanted(p.T, p.mnl, p.natoms)) {
         const int rc = launch_group<E, BF16>(p, fwd, st);
         if (rc <= 0) return rc;
     }
-    const int mode = g_launch[fwd ? 0 : 1].lds_weights;
+    auto lds_fits = [&](int w) {
+        return (fwd ? fused_lds_bytes<BF16, true, false>(p.T, p.cap, w)
+                    : fused_lds_bytes<BF16, true, true>(p.T, p.cap, w)) <= 64 * 1024;
+    };
+    const LaunchCfg cfg = launch_cfg(p, fwd, BF16, lds_fits(FUSED_WAVES));
+    const int mode = cfg.lds_weights;
     // a wavefront count set for another workload whose neighbor tiles would exceed the LDS budget
     // here falls back to fewer wavefronts per block
-    int w = g_launch[fwd ? 0 : 1].waves;
+    int w = cfg.waves;
     while (w > 2 && (fwd ? fused_lds_bytes<BF16, false, false>(p.T, p.cap, w)
                          : fused_lds_bytes<BF16, false, true>(p.T, p.cap, w)) > 64 * 1024)
         w /= 2;
-    const bool fits = (fwd ? fused_lds_bytes<BF16, true, false>(p.T, p.cap, w)
-                           : fused_lds_bytes<BF16, true, true>(p.T, p.cap, w)) <= 64 * 1024;
+    const bool fits = lds_fits(w);
     MATPL_CHECK_ARG(mode != 1 || fits, "dp_fused: weights do not fit in LDS for this T and list width");
     const bool lw = mode == 1 || (mode < 0 && fits);
-    if (p.gbuf) return launch_net<E, BF16, true>(p, fwd, st, lw, w);
-    return launch_net<E, BF16, false>(p, fwd, st, lw, w);
+    if (p.gbuf) return launch_net<E, BF16, true>(p, fwd, st, cfg, lw, w);
+    return launch_net<E, BF16, false>(p, fwd, st, cfg, lw, w);
 }
 
 int dispatch(FusedParams &p, int E, int bf16, bool fwd, hipStream_t st, int ck = 0) {
