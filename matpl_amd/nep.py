@@ -3,12 +3,15 @@
 Mirrors src/model/nep_net.py:293-648 (device != cpu): features from
 CalcOps_cuda.calculateNepFeat / calculateNepMbFeat, per-type fitting nets,
 dE = dEtot/dRi by autograd (create_graph, so force losses train the
-parameters), forces and virial returned negated as the reference does. The
+parameters), forces and virial returned negated as the reference does. Where
+the fitting nets run on their kernel, the descriptor of both lists is one
+call (nep_ops.NepDescriptor) and forces and frame virials come from dE/dq in
+another (nep_ops.NepModelForces), with no dE/dRi in between. Otherwise the
 reference's sequence per list (Ri_d from [r, x, y, z], nep_net.py:440-468;
 the centre force by a batched torch.matmul, nep_net.py:608;
-calculateNepForce; the frame virial of calculateNepVirial) runs here as one
+calculateNepForce; the frame virial of calculateNepVirial) runs as one
 kernel that forms Ri_d in registers (nep_ops.nep_force_virial), with its
-backward in one kernel too; the reference's operators themselves stay
+backward in one kernel too. The reference's operators themselves stay
 available with their own signatures (nep_ops / calcops).
 Fitting-layer products run tall-by-small or split over atoms (_TallMM), at
 every derivative order.
