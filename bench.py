@@ -589,7 +589,9 @@ def main():
     roofline = None
     traffic = None
     if reps == REPS and args.precision == "bf16":
-        traffic = BWD_TRAFFIC_BYTES["xcd" if launch and launch["backward"]["xcd"] else "plain"]
+        # the default shape is the library's own choice, the XCD order at this size
+        shape = launch["backward"] if launch else autotune.DEFAULT
+        traffic = BWD_TRAFFIC_BYTES["xcd" if shape["xcd"] or shape == autotune.DEFAULT else "plain"]
     if bwd_ms and nvalid:
         kt = float(np.mean(bwd_ms)) * 1e-3
         flops = flops_per_neighbor_bwd(w.cfg.emb_out) * nvalid
