@@ -24,8 +24,9 @@
 //            counting sort, each cell's atoms in ascending index. A block owns
 //            a cell: it merges the <=27 neighbor cells into one ascending list
 //            of candidates in LDS, and each wavefront runs one of the cell's
-//            atoms over it, so hits come in list order. Cells too sparse or too
-//            full for that are searched atom by atom (hits ranked by index).
+//            atoms over it, so hits come in list order. Systems of few or sparse
+//            cells, and cells too full for that, are searched atom by atom (hits
+//            ranked by index).
 #include "common.h"
 
 #pragma clang fp contract(off)
@@ -269,15 +270,14 @@ __global__ void fill_cells_kernel(const int32_t *__restrict__ atom_cell, int64_t
         cell_atoms[atomicAdd(cursor + atom_cell[i], 1)] = (int32_t)i;
 }
 
-// The atoms of each cell and its neighbors along z (1 to 3 cells), in ascending order. A cell's
-// list starts where the counts of those before it end: whole columns give noff times their atoms,
-// and within a column the sums of the cells' counts shifted by -1, 0 and 1 telescope.
+// The atoms of each cell and its two neighbors along z (a grid of three or more), in ascending order.
+// A cell's list starts where the counts of those before it end: whole columns give three times their
+// atoms, and within a column the sums of the cells' counts shifted by -1, 0 and 1 telescope.
 struct ZRun { int64_t at; int count; };      // in the sorted array
 
 __device__ __forceinline__ ZRun z_run(const int32_t *__restrict__ cell_start, const Grid &g, int cell) {
     const int nz = g.nc[2], z = cell % nz, c0 = cell - z;
-    const int s0 = cell_start[c0], column = cell_start[c0 + nz] - s0;
-    if (nz < 3) return {(int64_t)nz * s0 + (int64_t)z * column, column};
+    const int s0 = cell_start[c0];
     auto upto = [&](int x) { return cell_start[c0 + x] - s0; };      // atoms of cells z < x
     auto count = [&](int x) { return cell_start[c0 + x + 1] - cell_start[c0 + x]; };
     const int below = z > 0 ? z - 1 : nz - 1, above = z + 1 < nz ? z + 1 : 0;
@@ -286,19 +286,20 @@ __device__ __forceinline__ ZRun z_run(const int32_t *__restrict__ cell_start, co
 }
 
 // One wavefront per cell; the rank of an atom is the number of smaller ones. A run longer than
-// `cap` is left out: a block that would need it has too many candidates for LDS.
+// `longest` is left out (the ranking takes its square): a block that would need it leaves its atoms
+// to cell_overfull_kernel.
 constexpr int SORT_WAVES = 4;
 __global__ void __launch_bounds__(SORT_WAVES * WAVE)
-sort_runs_kernel(const int32_t *__restrict__ cell_start, int ncells, Grid g, int cap,
+sort_runs_kernel(const int32_t *__restrict__ cell_start, int ncells, Grid g, int longest,
                  const int32_t *__restrict__ cell_atoms, int32_t *__restrict__ sorted) {
     const int lane = threadIdx.x & (WAVE - 1), wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     for (int c = blockIdx.x * SORT_WAVES + wid; c < ncells; c += gridDim.x * SORT_WAVES) {
         const ZRun run = z_run(cell_start, g, c);
-        if (run.count > cap) continue;
+        if (run.count > longest) continue;
         const int nz = g.nc[2], z = c % nz, c0 = c - z;
         // the run's atoms are those of [s0, s1) and, where the period splits it, of [s2, ..)
         int s0, s1, s2 = 0;
-        if (nz <= 3) { s0 = cell_start[c0]; s1 = cell_start[c0 + nz]; }
+        if (nz == 3) { s0 = cell_start[c0]; s1 = cell_start[c0 + 3]; }
         else if (z == 0) { s0 = cell_start[c0]; s1 = cell_start[c0 + 2]; s2 = cell_start[c0 + nz - 1]; }
         else if (z == nz - 1) { s0 = cell_start[c0 + z - 1]; s1 = cell_start[c0 + nz]; s2 = cell_start[c0]; }
         else { s0 = cell_start[c0 + z - 1]; s1 = cell_start[c0 + z + 2]; }
@@ -332,8 +333,8 @@ struct CellArgs {
     // cell_block_kernel only
     const int32_t *sorted;      // ascending runs along z
     double pitch[3];            // of the cells, in fractions
-    int32_t *overfull;          // [0] their number, then the cells with more candidates than LDS holds
-    float pre2;                 // squared radius of the FP32 preselection (infinity: none)
+    int32_t *overfull;          // [0] their number, then the atoms of cells with too many candidates
+    float pre2;                 // squared radius of the FP32 preselection
     int cap, ncells, nparts;    // candidates in LDS, cells, blocks per cell
 };
 
@@ -468,33 +469,29 @@ __global__ void __launch_bounds__(CELL_WAVES * WAVE) cell_kernel(CellArgs A) {
     if (i < A.n) cell_scan_atom(A, i, smem + wid * (A.T * A.m + 2 * A.T));
 }
 
-// The cells that cell_block_kernel left: blockIdx.x strides over the cells, blockIdx.y over the atoms of one.
-constexpr int OVER_X = 256, OVER_Y = 8;
+// The atoms that cell_block_kernel left, a wavefront each: as many wavefronts as it has work for, whether
+// they come from a few crowded cells or from many.
 __global__ void __launch_bounds__(CELL_WAVES * WAVE) cell_overfull_kernel(CellArgs A) {
     extern __shared__ int32_t smem[];
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     int32_t *bucket = smem + wid * (A.T * A.m + 2 * A.T);
-    const int ncells = A.overfull[0];
-    for (int x = blockIdx.x; x < ncells; x += OVER_X) {
-        const int cell = A.overfull[1 + x];
-        const int p1 = A.cell_start[cell + 1];
-        for (int p = A.cell_start[cell] + blockIdx.y * CELL_WAVES + wid; p < p1; p += OVER_Y * CELL_WAVES)
-            cell_scan_atom(A, A.cell_atoms[p], bucket);
-    }
+    const int left = A.overfull[0];
+    for (int x = blockIdx.x * CELL_WAVES + wid; x < left; x += gridDim.x * CELL_WAVES)
+        cell_scan_atom(A, A.overfull[1 + x], bucket);
 }
 
-// One block per cell (or per part of a cell's atoms). All atoms of a cell have the same
-// candidates, the atoms of the <=27 cells around it, so the block puts these in ascending order
-// once: the runs along z are sorted already, and two rounds of merging (along y, then x; an
-// atom's place is its own rank plus its lower bounds in the one or two sibling runs) leave one
-// list. With it go FP32 Cartesian positions relative to the cell, so that a wavefront rejects 64
+// One block per cell (or per part of a cell's atoms), on a grid of three or more cells in every
+// direction. All atoms of a cell have the same candidates, the atoms of the 27 cells around it, so
+// the block puts these in ascending order once: the nine runs along z are sorted already, and two
+// rounds of merging (along y, then x; an atom's place is its own rank plus its lower bounds in the
+// two sibling runs) leave one list. With it go FP32 Cartesian positions relative to the cell, so that a wavefront rejects 64
 // candidates with one 16-byte LDS read and seven FP32 operations; the survivors (about one in
 // seven) are queued, and 64 at a time take the exact FP64 test with all lanes busy and are stored
 // in list order by ballots: no ranking and no atomics.
 //
 // The preselection keeps every pair that the exact test can accept: with three or more cells in
 // every direction the image that a cell pair implies is the only one within rc. It is cut at
-// A.pre2, which covers the rounding of FP32 positions; with fewer cells it is off (infinity).
+// A.pre2, which covers the rounding of FP32 positions.
 //
 // Four atoms of a wavefront go over the candidates together, so that an LDS read serves four
 // tests (one atom a pass: 240 us; LDS reads were then the bound), and the queue holds places in the
@@ -511,6 +508,8 @@ constexpr int CB_QUEUE = 2 * WAVE;
 constexpr int CB_MIN_ATOMS = 6;     // atoms per cell, and atoms, from which on this is the faster search
 constexpr int CB_MIN_TOTAL = 5000;
 constexpr int CB_MIN_BLOCKS = 512;
+constexpr int CB_MAX_CAND = 4096;   // candidates of a block, at most
+constexpr int CB_RUN_SHARE = 4;     // of its nine runs, each at most this part (a ninth where the density is even)
 
 __device__ __forceinline__ int lanes_below(unsigned long long mask) {
     return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
@@ -545,26 +544,30 @@ cell_block_kernel(CellArgs A) {
         ci[2] = c % g.nc[2]; c /= g.nc[2];
         ci[1] = c % g.nc[1]; ci[0] = c / g.nc[1];
     }
-    const int n0 = g.noff[0], n1 = g.noff[1], nrun = n0 * n1;
     if (wid == 0) {
         int64_t src = 0;
         int cnt = 0;
-        if (lane < nrun) {
-            const int a = lane / n1, b = lane % n1;
-            const int cx = (ci[0] + a - (n0 == 3) + g.nc[0]) % g.nc[0];
-            const int cy = (ci[1] + b - (n1 == 3) + g.nc[1]) % g.nc[1];
+        if (lane < 9) {
+            const int cx = (ci[0] + lane / 3 - 1 + g.nc[0]) % g.nc[0];
+            const int cy = (ci[1] + lane % 3 - 1 + g.nc[1]) % g.nc[1];
             const ZRun run = z_run(A.cell_start, g, (cx * g.nc[1] + cy) * g.nc[2] + ci[2]);
             src = run.at;
             cnt = run.count;
         }
         const int incl = wave_incl_scan(cnt);
-        if (lane < nrun) { run_start[lane + 1] = incl; run_src[lane] = src - (incl - cnt); }
+        const bool crowded = __any(cnt > A.cap / CB_RUN_SHARE);
+        if (lane < 9) { run_start[lane + 1] = lane == 8 && crowded ? A.cap + 1 : incl; run_src[lane] = src - (incl - cnt); }
         if (lane == 0) run_start[0] = 0;
     }
     __syncthreads();
-    const int total = run_start[nrun];
-    if (total > A.cap) {        // cell_overfull_kernel searches these
-        if (part == 0 && threadIdx.x == 0) A.overfull[1 + atomicAdd(A.overfull, 1)] = cell;
+    const int total = run_start[9];
+    if (total > A.cap) {        // cell_overfull_kernel searches this cell's atoms
+        if (part == 0) {
+            __shared__ int at;
+            if (threadIdx.x == 0) at = atomicAdd(A.overfull, nown);
+            __syncthreads();
+            for (int e = threadIdx.x; e < nown; e += CB_WAVES * WAVE) A.overfull[1 + at + e] = A.cell_atoms[own0 + e];
+        }
         return;
     }
     uint32_t *keyA = reinterpret_cast<uint32_t *>(smem);             // [cap], later the wavefronts' queues
@@ -576,13 +579,13 @@ cell_block_kernel(CellArgs A) {
         return lo;
     };
     for (int idx = threadIdx.x; idx < total; idx += CB_WAVES * WAVE)
-        keyA[idx] = (uint32_t)A.sorted[run_src[run_of(idx, 1, nrun)] + idx];
+        keyA[idx] = (uint32_t)A.sorted[run_src[run_of(idx, 1, 9)] + idx];
     __syncthreads();
 #pragma unroll
-    for (int round = 0; round < 2; round++) {       // along y (runs of nrun), then x (runs of n0)
+    for (int round = 0; round < 2; round++) {       // along y (nine runs), then x (three)
         const uint32_t *in = round ? keyB : keyA;
         uint32_t *out = round ? keyA : keyB;
-        const int gs = round ? n0 : n1, stride = round ? n1 : 1, nr = round ? n0 : nrun;
+        const int stride = round ? 3 : 1, nr = round ? 3 : 9;
         int longest = 0;
         for (int r = 0; r < nr; r++) {
             const int len = run_start[(r + 1) * stride] - run_start[r * stride];
@@ -592,13 +595,12 @@ cell_block_kernel(CellArgs A) {
         for (int idx = threadIdx.x; idx < total; idx += CB_WAVES * WAVE) {
             const uint32_t k = in[idx];
             const int r = run_of(idx, stride, nr);
-            const int r0 = gs == 3 ? (r / 3) * 3 : (gs == 2 ? (r & ~1) : r);
-            int at = run_start[r0 * stride] + idx - run_start[r * stride];
-            // the sibling runs r1, r2 (r itself when there are fewer: an empty one)
-            const int r1 = gs > 1 ? (r + 1 < r0 + gs ? r + 1 : r + 1 - gs) : r;
-            const int r2 = gs > 2 ? (r + 2 < r0 + gs ? r + 2 : r + 2 - gs) : r;
+            const int r0 = (r / 3) * 3;
+            const int at = run_start[r0 * stride] + idx - run_start[r * stride];
+            // the sibling runs r1, r2
+            const int r1 = r + 1 < r0 + 3 ? r + 1 : r0, r2 = r + 2 < r0 + 3 ? r + 2 : r - 1;
             const int lo1 = run_start[r1 * stride], lo2 = run_start[r2 * stride];
-            const int hi1 = gs > 1 ? run_start[(r1 + 1) * stride] : lo1, hi2 = gs > 2 ? run_start[(r2 + 1) * stride] : lo2;
+            const int hi1 = run_start[(r1 + 1) * stride], hi2 = run_start[(r2 + 1) * stride];
             // both lower bounds bit by bit; reads beyond a run (at most 2 * cap words in) are not used
             int b1 = lo1, b2 = lo2;
             for (int step = top; step > 0; step >>= 1) {
@@ -983,9 +985,9 @@ using namespace matpl;
 MATPL_EXPORT int64_t matpl_dp_neighbor_cell_workspace_bytes(const double *lattice_host, double rc_m, int64_t n) {
     Grid g = make_grid(lattice_host, rc_m);
     const int64_t ncells = (int64_t)g.nc[0] * g.nc[1] * g.nc[2];
-    // atom_cell[n], cell_atoms[n], sorted[3n], cell_count[ncells], overfull[ncells+1], cell_start[ncells+1],
+    // atom_cell[n], cell_atoms[n], sorted[3n], cell_count[ncells], overfull[n+1], cell_start[ncells+1],
     // cursor[ncells]
-    return (int64_t)sizeof(int32_t) * (5 * n + 4 * ncells + 2 + 64);
+    return (int64_t)sizeof(int32_t) * (6 * n + 3 * ncells + 2 + 64);
 }
 
 MATPL_EXPORT int matpl_dp_neighbor_is_small_box(const double *lattice_host, double rc_m) {
@@ -1040,7 +1042,7 @@ MATPL_EXPORT int matpl_dp_neighbor_cell(const double *lattice_host, const double
     int32_t *sorted = cell_atoms + n;
     int32_t *cell_count = sorted + 3 * n;               // zeroed, with the word after it
     int32_t *overfull = cell_count + ncells;
-    int32_t *cell_start = overfull + 1 + ncells;
+    int32_t *cell_start = overfull + 1 + n;
     int32_t *cursor = cell_start + ncells + 1;
     Lattice lat;
     for (int k = 0; k < 9; k++) lat.a[k] = lattice_host[k];
@@ -1064,14 +1066,18 @@ MATPL_EXPORT int matpl_dp_neighbor_cell(const double *lattice_host, const double
     // atom by atom: 20,000 atoms at 4 a cell 100 and 90 us, at 8 a cell 80 and 95, at 16 a cell 91
     // and 119; at a solid's density (0.09 per A^3) 3,000 atoms 82 and 69 us, 6,000 70 and 79,
     // 12,000 89 and 126, 40,000 136 and 264.
-    if (n >= CB_MIN_TOTAL && n >= (int64_t)CB_MIN_ATOMS * ncells) {
-        // Candidates in LDS (20 bytes each): 2048, which a cell pitch of 6.5 to 9 A needs at the
-        // density of a solid, or 4096 where the average cell is fuller; fuller blocks search atom
-        // by atom.
-        const double avg = (double)n / ncells * (g.noff[0] * g.noff[1] * g.noff[2]);
-        A.cap = 1.5 * avg > 2048.0 ? 4096 : 2048;
+    // With fewer than three cells in a direction nothing can be preselected, and every candidate takes
+    // the exact test here as there: 14 x 35 x 49 A, 5,123 atoms 177 and 120 us; 13.2 x 13.2 x 400 A,
+    // 6,000 atoms 63 and 48. Candidates in LDS (20 bytes each): 2048, which a cell pitch of 6.5 to 9 A
+    // needs at the density of a solid, or 4096 where the average cell is fuller; where even that is too
+    // small for the average cell (with 8 % for the spread of random positions, some 5 deviations), every
+    // block would only find so.
+    const double avg = (double)n / ncells * 27.0;
+    const bool grid3 = g.nc[0] >= 3 && g.nc[1] >= 3 && g.nc[2] >= 3;
+    if (grid3 && n >= CB_MIN_TOTAL && n >= (int64_t)CB_MIN_ATOMS * ncells && 1.08 * avg <= CB_MAX_CAND) {
+        A.cap = 1.5 * avg > 2048.0 ? CB_MAX_CAND : 2048;
         hipLaunchKernelGGL(sort_runs_kernel, dim3(grid_cap(ncells, SORT_WAVES)), dim3(SORT_WAVES * WAVE), 0, st,
-                           cell_start, ncells, g, A.cap, cell_atoms, sorted);
+                           cell_start, ncells, g, A.cap / CB_RUN_SHARE, cell_atoms, sorted);
         if ((rc = check_launch("sort_runs_kernel"))) return rc;
         A.sorted = sorted;
         A.ncells = ncells;
@@ -1088,14 +1094,14 @@ MATPL_EXPORT int matpl_dp_neighbor_cell(const double *lattice_host, const double
                                       lattice_host[3 * d + 1] * lattice_host[3 * d + 1] +
                                       lattice_host[3 * d + 2] * lattice_host[3 * d + 2]);
         const double pre = rc_m + 1e-6 * R + 1e-6 * rc_m;
-        A.pre2 = g.nc[0] >= 3 && g.nc[1] >= 3 && g.nc[2] >= 3 ? (float)(pre * pre * (1.0 + 1e-6)) : INFINITY;
+        A.pre2 = (float)(pre * pre * (1.0 + 1e-6));
         for (int d = 0; d < 3; d++) A.pitch[d] = 1.0 / g.nc[d];
         A.overfull = overfull;
         const int64_t nwork = (int64_t)ncells * A.nparts;
         hipLaunchKernelGGL(cell_block_kernel, dim3((unsigned)(8 * ((nwork + 7) / 8))), dim3(CB_WAVES * WAVE),
                            (size_t)A.cap * 20, st, A);
         if ((rc = check_launch("cell_block_kernel"))) return rc;
-        hipLaunchKernelGGL(cell_overfull_kernel, dim3(OVER_X, OVER_Y), dim3(CELL_WAVES * WAVE), lds, st, A);
+        hipLaunchKernelGGL(cell_overfull_kernel, dim3(grid_cap(n, CELL_WAVES)), dim3(CELL_WAVES * WAVE), lds, st, A);
         return check_launch("cell_overfull_kernel");
     }
     hipLaunchKernelGGL(cell_kernel, dim3(ceil_div(n, CELL_WAVES)), dim3(CELL_WAVES * WAVE), lds, st, A);

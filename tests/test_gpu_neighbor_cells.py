@@ -1,7 +1,9 @@
 """The cell search against the brute-force one, bit for bit, over the forms its dispatch tells apart: cells with
-enough atoms for a block each, few atoms or sparse cells (atom by atom), cells with more candidates than LDS
-holds, fewer than three cells in a direction (no preselection), one block or several per cell, triclinic boxes,
-cutoffs per type, coordinates outside [0, 1). The reverse map against its definition."""
+enough atoms for a block each (up to 2,048 candidates, up to 4,096, three cells in one direction or more), few
+atoms, sparse cells, fewer than three cells in a direction or more candidates than LDS holds in the average cell
+(atom by atom), single cells with more than that, one block or several per cell, triclinic boxes, cutoffs per
+type, coordinates outside [0, 1). _form restates the dispatch, so that each case is known to reach what it is
+for. The reverse map against its definition."""
 import numpy as np
 import pytest
 import torch
@@ -19,6 +21,27 @@ def dev():
 CUBE = np.eye(3)
 TRI = np.array([[1.0, 0.1, 0.0], [-0.2, 1.1, 0.15], [0.05, -0.1, 0.95]])
 
+def _cells(lat, frac, rc):
+    """(cells per direction, candidates of every occupied cell): the atoms of the 27 cells around it."""
+    vol = abs(np.linalg.det(lat))
+    nc = [max(1, int(np.floor(vol / np.linalg.norm(np.cross(lat[(d + 1) % 3], lat[(d + 2) % 3])) / rc))) for d in range(3)]
+    own = np.zeros(nc)
+    np.add.at(own, tuple(np.minimum((np.mod(frac, 1.0) * nc).astype(int), np.array(nc) - 1).T), 1)
+    tot = sum(np.roll(own, s, (0, 1, 2)) for s in np.ndindex(3, 3, 3)) if min(nc) >= 3 else None
+    return nc, None if tot is None else tot[own > 0]
+
+
+def _form(lat, frac, rc):
+    """The search that a call takes: atom by atom, or cells' blocks of a capacity and which cells exceed it."""
+    nc, tot = _cells(lat, frac, rc)
+    n, ncells = len(frac), int(np.prod(nc))
+    avg = n / ncells * 27.0
+    if min(nc) < 3 or n < 5000 or n < 6 * ncells or 1.08 * avg > 4096:
+        return "by_atom"
+    cap = 4096 if 1.5 * avg > 2048 else 2048
+    return f"blocks_{cap}" + ("" if tot.max() <= cap else "_overfull")
+
+
 # name, lattice (A), atoms, types, cutoff, slots per type, cutoffs per type, spread (1: fills the box), offset
 CASES = [
     ("blocks", 39.5 * CUBE, 5200, 2, 6.5, 160, None, 1.0, 0.0),
@@ -32,7 +55,15 @@ CASES = [
     ("fuller_lds", 30.0 * CUBE, 5000, 5, 9.0, 300, None, 0.96, 0.0),
     ("outside", 39.5 * CUBE, 5200, 2, 6.5, 160, None, 1.0, -13.0),
     ("edge_cells", 39.2 * CUBE, 65 * 216, 16, 6.5, 100, None, 1.0, 0.0),
+    ("three_along_x", np.diag([20.0, 41.0, 41.0]), 5400, 2, 6.5, 250, None, 1.0, 0.0),
+    ("three_along_y_z", np.diag([81.0, 20.0, 20.5]), 5100, 3, 6.5, 190, (6.5, 6.0, 5.0), 1.0, 0.0),
+    ("three_tri", np.diag([24.0, 44.0, 24.0]) @ TRI, 6100, 2, 6.5, 260, None, 1.0, -13.0),
+    ("upper_half", 39.5 * CUBE, 27200, 2, 6.5, 340, None, 1.0, 0.0),
 ]
+FORMS = dict(blocks="blocks_2048", blocks_tri="blocks_2048", by_atom="by_atom", three_cells="by_atom",
+             two_cells="by_atom", one_cell="by_atom", sparse="by_atom", overfull="blocks_2048_overfull",
+             fuller_lds="by_atom", outside="blocks_2048", edge_cells="blocks_4096", three_along_x="blocks_2048",
+             three_along_y_z="blocks_2048", three_tri="blocks_4096", upper_half="blocks_4096")
 
 
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
@@ -46,6 +77,11 @@ def test_cell_search_is_the_brute_force_one(dev, case, want_dR):
         frac[::3] += offset
         frac[1::3] += 7.0
     types = rng.integers(0, T, n)
+    assert _form(lat, frac, rc) == FORMS[name]
+    if name.startswith("three_a") or name == "three_tri":
+        assert min(_cells(lat, frac, rc)[0]) == 3
+    if name == "upper_half":
+        assert (_cells(lat, frac, rc)[1] > 2048).all()
     kw = dict(rc_type=rct, want_dR=want_dR, want_shift=True, device=dev)
     print(f"{name} n={n} T={T}", flush=True)
     a = find_neighbore_gpu(lat, frac, types, T, m, rc, **kw)
