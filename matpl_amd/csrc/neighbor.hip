@@ -750,24 +750,29 @@ cell_block_kernel(CellArgs A) {
 // exact negation of dR_ij in the cutoff test; a missing partner (per-type
 // cutoffs that differ, or a tie in the nearest-image rule) sets status.
 //
-// Every entry searches its partner's bucket (sorted by (j, image)) by itself, four entries to a
-// load: the loads touch a different cache line per lane, so the kernel is bound by their number,
-// and four-wide ones halve a binary search's. The 8 XCDs take contiguous ranges of atoms, whose
-// neighbors' buckets share their L2. 230 us on a 99,636-atom list of 160 slots per type (105
-// neighbors an atom); matching each pair once, by the atom of smaller index, took 246 us with the
-// same search, as the partner's entry is a scattered store, plus 47 us of passes that set all
-// slots to -1 first and check them last (with a scalar binary search and no ranges: 288 + 47).
+// Every entry searches its partner's bucket (sorted by (j, image)) by itself, four entries to a load. The loads
+// touch a different cache line per lane, so what bounds the kernel is their number and where they hit. The
+// 8 XCDs take contiguous ranges of atoms: where neighbors in space are near in index, the buckets of a range's
+// neighbors share its L2, and bisecting the bucket is cheapest. Where the atoms are in no spatial order
+// (scattered_order) every line comes from beyond the L2s; but then the entries of a bucket are spread evenly,
+// so that the partner's place follows from its index, and the search starts there: one line, not two or three.
+// 99,636 HfO2 atoms (160 slots per type, 105 neighbors an atom) 218 us, shuffled 510 (bisected 651);
+// 40,000 atoms of 255 neighbors in random order 367 (675), 30,000 of 104 112 (151). A kernel in which one atom
+// of each pair searches and stores both directions, between passes that set all slots to -1 and look for
+// those left, takes 307, 479, 422 and 114 us.
 constexpr int REV_WAVES = 4;
 constexpr int REV_XCDS = 8;
 
 struct __attribute__((packed, aligned(4))) Int4 { int32_t v[4]; };
 
-// The entry of row[0 .. cnt) (ascending) that names `target` with image `want`, or -1.
+// The entry of row[0 .. cnt) (ascending) that names `target` with image `want`, or -1. guess >= 0: where it is
+// likely to be (the search goes outward from there), else the row is bisected.
 __device__ __forceinline__ int find_entry(const int32_t *__restrict__ row, const int32_t *__restrict__ image, int cnt,
-                                          int target, int want) {
-    int lo = 0, hi = cnt, at = -1;
+                                          int target, int want, int guess) {
+    int lo = 0, hi = cnt, at = -1, step = 0;
+    int g = guess >= 0 ? guess - 1 : (cnt - 4) >> 1;
     while (hi - lo > 4) {
-        const int mid = lo + ((hi - lo - 4) >> 1);
+        const int mid = g < lo ? lo : (g > hi - 4 ? hi - 4 : g);
         const Int4 x = *reinterpret_cast<const Int4 *>(row + mid);
         if (x.v[3] < target) lo = mid + 4;
         else if (x.v[0] > target) hi = mid;
@@ -776,6 +781,12 @@ __device__ __forceinline__ int find_entry(const int32_t *__restrict__ row, const
             const int32_t there = lo == mid ? x.v[0] : lo == mid + 1 ? x.v[1] : lo == mid + 2 ? x.v[2] : x.v[3];
             at = there == target ? lo : -1;
             hi = -1;
+        }
+        if (guess >= 0 && (lo == 0 || hi == cnt)) {
+            g = lo > 0 ? lo + step : hi - 4 - step;
+            step = 2 * step + 4;
+        } else {
+            g = lo + ((hi - lo - 4) >> 1);
         }
     }
     if (hi >= 0) {
@@ -789,6 +800,31 @@ __device__ __forceinline__ int find_entry(const int32_t *__restrict__ row, const
     return -1;
 }
 
+// Whether neighbors in space are far apart in index (one frame): the buckets of an atom then span most of the
+// indices, each on its own (types mixed) or together (atoms sorted by type). Asked of four atoms, since the
+// buckets of one at the period's edge span the frame in any order; only the search's start depends on it.
+__device__ __forceinline__ bool scattered_order(const int32_t *__restrict__ list, const int32_t *__restrict__ counts,
+                                                int T, int m, int64_t n) {
+    const int lane = threadIdx.x & (WAVE - 1), t = lane & 15;           // 16 lanes, one per type, to an atom
+    const int64_t bucket = (2 * (lane >> 4) + 1) * n / 8 * T + t, row = bucket * m;
+    const int c = t < T ? min(counts[bucket], m) : 0;
+    int64_t f = n, l = 0, sum = 0;
+    if (c > 0) {
+        f = list[row];
+        l = list[row + c - 1];
+        sum = l - f;
+    }
+    int lo = (int)f, hi = (int)l;
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) {
+        sum += __shfl_xor(sum, o, WAVE);
+        lo = min(lo, __shfl_xor(lo, o, WAVE));
+        hi = max(hi, __shfl_xor(hi, o, WAVE));
+    }
+    const bool wide = 4 * (sum < hi - lo ? sum : hi - lo) > 3 * n;
+    return __popcll(__ballot(wide && t == 0)) >= 3;
+}
+
 __global__ void __launch_bounds__(REV_WAVES * WAVE)
 reverse_kernel(const int32_t *__restrict__ list, const int32_t *__restrict__ shift,
                const int32_t *__restrict__ counts, const int32_t *__restrict__ type_map,
@@ -798,28 +834,43 @@ reverse_kernel(const int32_t *__restrict__ list, const int32_t *__restrict__ shi
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int64_t per = (n + REV_XCDS - 1) / REV_XCDS;
     const int64_t i0 = (blockIdx.x % REV_XCDS) * per, i1 = i0 + per < n ? i0 + per : n;
+    const bool wide = !frame_start && scattered_order(list, counts, T, m, n);
     for (int64_t i = i0 + (int64_t)(blockIdx.x / REV_XCDS) * REV_WAVES + wid; i < i1;
          i += (int64_t)(gridDim.x / REV_XCDS) * REV_WAVES) {
         const int64_t fb = frame_start ? frame_start[atom_frame[i]] : 0;
         const int ti = type_map[i];
         const int target = (int)(i - fb) + 1;
         bool bad = false;
+        float at = 0.0f;
+        if (wide) {
+            const int own = min(counts[i * T + ti], m);
+            const int64_t row = (i * T + ti) * (int64_t)m;
+            const int f = own > 0 ? list[row] : target, l = own > 0 ? list[row + own - 1] : target;
+            at = fminf(fmaxf((float)(target - f) / (float)(l - f + 1), 0.0f), 1.0f);
+        }
+        // the entries of all buckets as one sequence: fuller wavefronts, fewer rounds of waiting
+        int total = 0;
         for (int t = 0; t < T; t++) {
-            const int c = counts[i * T + t];
-            const int64_t s0 = (i * T + t) * (int64_t)m;
-            for (int k = lane; k < m; k += WAVE) {
-                int r = -1;
-                if (k < c) {
-                    const int64_t j = fb + list[s0 + k] - 1;
-                    const int sh = shift[s0 + k];
-                    const int want = pack_shift(-((sh & 255) - 128), -(((sh >> 8) & 255) - 128),
-                                                -(((sh >> 16) & 255) - 128));
-                    const int64_t base = (j * T + ti) * (int64_t)m;
-                    const int f = find_entry(list + base, shift + base, counts[j * T + ti], target, want);
-                    if (f < 0) bad = true; else r = (int32_t)(base + f);
-                }
-                rev[s0 + k] = r;
+            const int c = min(counts[i * T + t], m);
+            for (int k = c + lane; k < m; k += WAVE) __builtin_nontemporal_store(-1, rev + (i * T + t) * (int64_t)m + k);
+            total += c;
+        }
+        for (int e = lane; e < total; e += WAVE) {
+            int t = 0, k = e;
+            for (int u = 0; u + 1 < T; u++) {
+                const int c = min(counts[i * T + u], m);
+                if (t == u && k >= c) { k -= c; t++; }
             }
+            const int64_t s = (i * T + t) * (int64_t)m + k;
+            const int64_t j = fb + list[s] - 1;
+            const int sh = shift[s];
+            const int want = pack_shift(-((sh & 255) - 128), -(((sh >> 8) & 255) - 128), -(((sh >> 16) & 255) - 128));
+            const int64_t base = (j * T + ti) * (int64_t)m;
+            const int cnt = min(counts[j * T + ti], m);
+            const int f = find_entry(list + base, shift + base, cnt, target, want, wide ? (int)(at * cnt) : -1);
+            if (f < 0) bad = true;
+            const int32_t r = f < 0 ? -1 : (int32_t)(base + f);
+            __builtin_nontemporal_store(r, rev + s);
         }
         if (__ballot(bad) != 0ull && lane == 0) atomicCAS(status, 0, (int)(i + 1));
     }

@@ -137,3 +137,40 @@ def test_reverse_map_names_the_partner(dev, lat, n, m):
     nl2 = type(nl)(nl.list, None, c, nl.shift, nl.frac_wrapped, nl.status)
     rev2, status2 = reverse_map(nl2, tm, m)
     assert int(status2) > 0
+
+
+@pytest.mark.parametrize("order,scattered", [("space", False), ("type_space", False), ("random", True),
+                                             ("type_random", True)])
+def test_reverse_map_in_any_order(dev, order, scattered):
+    """The search starts at the bucket's middle, or where atoms in no spatial order put the partner."""
+    from matpl_amd.neighbor import find_neighbore_gpu, reverse_map
+    rng = np.random.Generator(np.random.PCG64(17))
+    n, T, m, L = 9001, 2, 121, 62.0
+    frac, types = rng.random((n, 3)), rng.integers(0, T, n)
+    if "space" in order:
+        o = np.argsort(frac[:, 0])
+        frac, types = frac[o], types[o]
+    if "type" in order:
+        o = np.argsort(types, kind="stable")
+        frac, types = frac[o], types[o]
+    tm = torch.as_tensor(types, dtype=torch.int32, device=dev)
+    nl = find_neighbore_gpu(L * CUBE, frac, tm, T, m, 6.0, want_dR=False, want_shift=True, device=dev)
+    lst, cnt = nl.list.cpu().numpy().reshape(n, T, m), nl.counts.cpu().numpy()
+    span = []
+    for a in (n // 8, 3 * n // 8, 5 * n // 8, 7 * n // 8):
+        f, l = lst[a, :, 0], lst[a, np.arange(T), cnt[a] - 1]
+        assert (cnt[a] > 4).all()
+        span.append(min((l - f).sum(), l.max() - f.min()))
+    assert (sum(4 * x > 3 * n for x in span) >= 3) == scattered
+    rev, status = reverse_map(nl, tm, m)
+    assert int(status) == 0
+    rv, sh = rev.cpu().numpy().reshape(-1), nl.shift.cpu().numpy().reshape(-1)
+    lst = lst.reshape(-1)
+    slots = np.nonzero(lst > 0)[0]
+    partner = rv[slots]
+    assert (rv[lst == 0] == -1).all() and (partner >= 0).all()
+    assert np.array_equal(rv[partner], slots)
+    assert np.array_equal(partner // (T * m), lst[slots] - 1)
+    assert np.array_equal(lst[partner], slots // (T * m) + 1)
+    image = lambda p: np.stack([(p >> k & 255) - 128 for k in (0, 8, 16)])
+    assert np.array_equal(image(sh[partner]), -image(sh[slots]))
