@@ -60,6 +60,7 @@ struct FitArgs {
     void *part;              // [ntiles][PW]     backward: per-tile parameter-gradient rows
     int D, H, TA;
     int per;                 // forward: atoms per block (divides TA)
+    int part_rows;           // forward: rows of W0 in LDS at a time
 };
 
 // Orders a wavefront's own LDS writes before its lanes' reads of each other's values.
@@ -78,23 +79,30 @@ __device__ __forceinline__ float tanh_t<float>(float z) { return tanhf(z); }
 template <>
 __device__ __forceinline__ double tanh_t<double>(double z) { return tanh(z); }
 
-// Forward: 32 lanes per atom, 8 atoms of a block at a time; lanes over the hidden units, then over the features.
-// With WL the type's W0 sits in LDS (rows of odd stride, read along both axes without conflicts), otherwise it is
-// read from global memory. Each half-wave only reads the rows it wrote, so no block barrier follows the staging.
+// Forward: G lanes per R atoms, 256 R / G atoms of a block at a time; lanes over the hidden units, then over the
+// features. The type's W0 sits in LDS (rows of odd stride, read along both axes without conflicts), in parts of
+// `part` rows where it is larger than FWD_W_LDS; without that the features' sums would read it from global memory
+// across its rows, a cache line per lane.
 // What bounds it: at thousands of atoms the serial chain of two D x H products on few wavefronts (a block per 64
-// atoms, a thread per atom and strided units: 1,728 atoms 23 us, with a block per 8 atoms 5 us); at 62,713
-// atoms LDS reads (37 -> 34 us).
-constexpr int FIT_GROUP = 32, FIT_ATOMS = FIT_THREADS / FIT_GROUP;
+// atoms, a thread per atom and strided units: 1,728 atoms 23 us, with a block per 8 atoms 5 us); at tens of
+// thousands LDS reads, one of W0 per product, hence R atoms to a read. 60,000 atoms, thread per atom / one atom
+// per 32 lanes / now: D 30, H 30 float 38 / 23 / 21 us, double 69 / 40 / 33; D 5, H 10 double 19 / 24 / 13;
+// D 56, H 100 float 113 / 118 / 88, double 250 / 370 / 195.
+constexpr int FIT_GROUP = 32, FIT_GROUP_FEW = 8;     // lanes per atom; of nets with few hidden units
+constexpr int FIT_FEW = 16;
+constexpr int FIT_ATOMS = FIT_THREADS / FIT_GROUP;
+constexpr size_t FWD_W_LDS = 46 * 1024;      // three blocks in a CU's 160 KB
 
-template <typename T, bool WL>
+template <typename T, int G, int R, bool WHOLE>
 __global__ void __launch_bounds__(FIT_THREADS) nep_fit_fwd_kernel(FitArgs a) {
     extern __shared__ unsigned char smem_raw[];
-    const int D = a.D, H = a.H, nsub = a.TA / a.per;
+    constexpr int NA = FIT_THREADS / G;
+    const int D = a.D, H = a.H, nsub = a.TA / a.per, DP = WHOLE ? D : a.part_rows;
     const int sd = odd(D), sh = odd(H);
-    const int l = threadIdx.x % FIT_GROUP, grp = threadIdx.x / FIT_GROUP;
-    T *x = reinterpret_cast<T *>(smem_raw) + grp * (sd + sh);      // [D] this atom's x
-    T *u = x + sd;                                                 // [H]
-    T *ws = reinterpret_cast<T *>(smem_raw) + FIT_ATOMS * (sd + sh);   // [D][sh] (WL)
+    const int l = threadIdx.x % G, grp = threadIdx.x / G;
+    T *x = reinterpret_cast<T *>(smem_raw) + grp * R * (sd + sh);      // [R][D] these atoms' x
+    T *u = x + R * sd;                                                 // [R][H] z, then w1 (1 - h^2)
+    T *ws = reinterpret_cast<T *>(smem_raw) + NA * R * (sd + sh);   // [DP][sh]
     const int *tile = a.tiles + 3 * (blockIdx.x / nsub);
     const int ty = tile[0], r0 = (blockIdx.x % nsub) * a.per;
     const int first = tile[1] + r0, cnt = tile[2] - r0 < a.per ? tile[2] - r0 : a.per;
@@ -103,36 +111,77 @@ __global__ void __launch_bounds__(FIT_THREADS) nep_fit_fwd_kernel(FitArgs a) {
     const T *qs = reinterpret_cast<const T *>(a.qs);
     const T *W0, *b0, *w1, *b1;
     a.w.of<T>(ty, D, H, W0, b0, w1, b1);
-    if constexpr (WL) {
-        for (int e = threadIdx.x; e < D * H; e += FIT_THREADS) ws[(e / H) * sh + e % H] = W0[e];
+    // rows [d0, d1) of W0
+    auto stage = [&](int d0, int d1) {
+        if (!WHOLE) __syncthreads();
+        for (int e = threadIdx.x; e < (d1 - d0) * H; e += FIT_THREADS) ws[(e / H) * sh + e % H] = W0[(size_t)d0 * H + e];
         __syncthreads();
-    }
-    const T *W = WL ? ws : W0;
-    const int sw = WL ? sh : H;
-    for (int r = grp; r < cnt; r += FIT_ATOMS) {
-        const size_t at = (size_t)a.perm[first + r];
-        for (int d = l; d < D; d += FIT_GROUP) x[d] = q[at * D + d] * qs[d];
+    };
+    if (WHOLE) stage(0, D);
+    for (int rb = 0; rb < cnt; rb += NA * R) {       // the same rounds in every group: parts have barriers
+        size_t at[R];
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            const int r = rb + k * NA + grp;
+            at[k] = (size_t)a.perm[first + (r < cnt ? r : cnt - 1)];
+            for (int d = l; d < D; d += G) x[k * sd + d] = q[at[k] * D + d] * qs[d];
+        }
         wave_sync();
-        T e = T(0);
-        for (int j = l; j < H; j += FIT_GROUP) {
-            T z = b0[j];
+        T e[R];
+#pragma unroll
+        for (int k = 0; k < R; k++) e[k] = T(0);
+        for (int d0 = 0; d0 < D; d0 += DP) {
+            const int nd = D - d0 < DP ? D - d0 : DP;
+            if (!WHOLE) stage(d0, d0 + nd);
+            for (int j = l; j < H; j += G) {
+                T z[R];
+#pragma unroll
+                for (int k = 0; k < R; k++) z[k] = WHOLE || d0 == 0 ? b0[j] : u[k * sh + j];
 #pragma unroll 10
-            for (int d = 0; d < D; d++) z += x[d] * W[d * sw + j];
-            const T h = tanh_t(z);
-            e += w1[j] * h;
-            u[j] = w1[j] * (T(1) - h * h);
+                for (int d = 0; d < nd; d++) {
+                    const T w = ws[d * sh + j];
+#pragma unroll
+                    for (int k = 0; k < R; k++) z[k] += x[k * sd + d0 + d] * w;
+                }
+                const bool last = WHOLE || d0 + nd == D;
+                const T w1j = w1[j];
+#pragma unroll
+                for (int k = 0; k < R; k++) {
+                    if (last) {
+                        const T h = tanh_t(z[k]);
+                        e[k] += w1j * h;
+                        z[k] = w1j * (T(1) - h * h);
+                    }
+                    u[k * sh + j] = z[k];
+                }
+            }
         }
         wave_sync();
 #pragma unroll
-        for (int o = FIT_GROUP / 2; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
-        if (l == 0) reinterpret_cast<T *>(a.Ei)[at] = e + b1[0];
+        for (int k = 0; k < R; k++) {
+#pragma unroll
+            for (int o = G / 2; o > 0; o >>= 1) e[k] += __shfl_xor(e[k], o, 64);
+            if (l == 0 && rb + k * NA + grp < cnt) reinterpret_cast<T *>(a.Ei)[at[k]] = e[k] + b1[0];
+        }
         if (a.g) {
             T *g = reinterpret_cast<T *>(a.g);
-            for (int d = l; d < D; d += FIT_GROUP) {
-                T s = T(0);
+            for (int d0 = 0; d0 < D; d0 += DP) {
+                const int nd = D - d0 < DP ? D - d0 : DP;
+                if (!WHOLE) stage(d0, d0 + nd);
+                for (int d = l; d < nd; d += G) {
+                    T s[R];
+#pragma unroll
+                    for (int k = 0; k < R; k++) s[k] = T(0);
 #pragma unroll 10
-                for (int j = 0; j < H; j++) s += W[d * sw + j] * u[j];
-                g[at * D + d] = s * qs[d];
+                    for (int j = 0; j < H; j++) {
+                        const T w = ws[d * sh + j];
+#pragma unroll
+                        for (int k = 0; k < R; k++) s[k] += w * u[k * sh + j];
+                    }
+#pragma unroll
+                    for (int k = 0; k < R; k++)
+                        if (rb + k * NA + grp < cnt) g[at[k] * D + d0 + d] = s[k] * qs[d0 + d];
+                }
             }
         }
         wave_sync();
@@ -244,11 +293,35 @@ nep_fit_reduce_kernel(const T *part, const int32_t *tstart, int PW, int D, int H
     else db1[t] = s;
 }
 
-size_t fwd_lds(int D, int H, bool wl, size_t es) {
-    return es * ((size_t)FIT_ATOMS * (odd(D) + odd(H)) + (wl ? (size_t)D * odd(H) : 0));
+size_t fwd_lds(int D, int H, int rows, int atoms, size_t es) {
+    return es * ((size_t)atoms * (odd(D) + odd(H)) + (size_t)rows * odd(H));
 }
 size_t bwd_lds(int D, int H, int TA, size_t es) {
     return es * (2 * (size_t)TA * odd(D) + 3 * (size_t)TA * odd(H) + (size_t)TA);
+}
+
+template <typename T, int G, int R>
+int fwd_launch_r(FitArgs &a, int ntiles, hipStream_t st) {
+    constexpr size_t LDS_MAX = 64 * 1024;
+    constexpr int NA = FIT_THREADS / G * R;
+    const size_t row = (size_t)odd(a.H) * sizeof(T);
+    a.part_rows = a.D * row <= FWD_W_LDS ? a.D : (int)(FWD_W_LDS / 2 / row);
+    if (fwd_lds(a.D, a.H, a.part_rows, NA, sizeof(T)) > LDS_MAX) {
+        if constexpr (R > 1) return fwd_launch_r<T, G, R / 2>(a, ntiles, st);
+        if constexpr (G != FIT_GROUP) return fwd_launch_r<T, FIT_GROUP, 1>(a, ntiles, st);
+        // (the atoms' rows of the widest nets, at most half of it, and what is left for W0)
+        a.part_rows = (int)((LDS_MAX - fwd_lds(a.D, a.H, 0, NA, sizeof(T))) / row);
+    }
+    const size_t lds = fwd_lds(a.D, a.H, a.part_rows, NA, sizeof(T));
+    const dim3 grid((unsigned)ntiles * (unsigned)(a.TA / a.per)), block(FIT_THREADS);
+    if (a.part_rows == a.D) {
+        hipLaunchKernelGGL((nep_fit_fwd_kernel<T, G, R, true>), grid, block, lds, st, a);
+    } else if constexpr (G != FIT_GROUP) {
+        return fwd_launch_r<T, FIT_GROUP, 1>(a, ntiles, st);
+    } else {
+        hipLaunchKernelGGL((nep_fit_fwd_kernel<T, G, R, false>), grid, block, lds, st, a);
+    }
+    return check_launch("nep_fit_fwd_kernel");
 }
 
 template <typename T>
@@ -256,13 +329,11 @@ int fwd_launch(FitArgs &a, int ntiles, hipStream_t st) {
     // fewer atoms per block while that leaves the chip short of blocks (four per CU), down to one per half-wave
     a.per = a.TA;
     while (a.per > FIT_ATOMS && (int64_t)ntiles * (a.TA / a.per) < 1024) a.per /= 2;
-    const dim3 grid((unsigned)ntiles * (unsigned)(a.TA / a.per)), block(FIT_THREADS);
-    // W0 in LDS up to 24 KB: blocks of several types share a CU's 160 KB
-    if ((size_t)a.D * odd(a.H) * sizeof(T) <= 24 * 1024)
-        hipLaunchKernelGGL((nep_fit_fwd_kernel<T, true>), grid, block, fwd_lds(a.D, a.H, true, sizeof(T)), st, a);
-    else
-        hipLaunchKernelGGL((nep_fit_fwd_kernel<T, false>), grid, block, fwd_lds(a.D, a.H, false, sizeof(T)), st, a);
-    return check_launch("nep_fit_fwd_kernel");
+    // 32 lanes per atom leave most idle with few hidden units, where the atoms are enough without
+    if (a.H <= FIT_FEW && a.per >= FIT_THREADS / FIT_GROUP_FEW) return fwd_launch_r<T, FIT_GROUP_FEW, 1>(a, ntiles, st);
+    if (a.per >= 4 * FIT_ATOMS) return fwd_launch_r<T, FIT_GROUP, 4>(a, ntiles, st);
+    if (a.per >= 2 * FIT_ATOMS) return fwd_launch_r<T, FIT_GROUP, 2>(a, ntiles, st);
+    return fwd_launch_r<T, FIT_GROUP, 1>(a, ntiles, st);
 }
 
 int set_stacked(FitArgs &a, const void *W0, const void *b0, const void *w1, const void *b1) {

@@ -1,7 +1,10 @@
 """The NEP fitting kernels with one weight pointer per type (matpl_nep_fit_forward_nets / _backward_nets), forward
 and first and second derivative, against float64 torch autograd: atoms counts around the block's 8 and the tile's 64,
-weights above the forward's LDS budget (D = 35, H = 100 in double: 28 KB), an empty type. Tolerances as
-tests/test_gpu_nep_fit.py: float64 1e-12, float32 2e-5 of the largest entry."""
+enough atoms for two and four at a time (20,000 and 40,000) with remainders, weights that the forward stages in parts
+(D = 56, H = 120 in double: 54 KB; D = 480, H = 8, whose rows leave less room), an empty type. Tolerances as
+tests/test_gpu_nep_fit.py: float64 1e-12, float32 2e-5 of the largest entry. A parameter gradient is a sum of N terms
+of order one, whose partial sums reach sqrt(N) whatever the total is; it takes at most 64 additions in a tile, N / 512
+over tiles and 8 over groups, about 150 roundings of half an ulp of sqrt(N)."""
 import numpy as np
 import pytest
 import torch
@@ -11,7 +14,7 @@ from matpl_amd import nep as mn
 pytestmark = pytest.mark.gpu
 
 CASES = [(1, 1, 30, 30), (8, 1, 5, 3), (9, 2, 30, 30), (64, 1, 33, 31), (65, 3, 30, 32), (1000, 4, 35, 100),
-         (20000, 2, 30, 30)]
+         (20000, 2, 30, 30), (40003, 3, 5, 10), (36001, 2, 56, 120), (700, 2, 480, 8), (9001, 1, 56, 64)]
 
 
 @pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-12), (torch.float32, 2e-5)])
@@ -42,4 +45,5 @@ def test_nets_entry(dev, dtype, tol, N, T, D, H):
         a = a.detach().double()
         b = torch.zeros_like(a) if b is None else b.detach()
         err = float((a - b).abs().max())
-        assert err <= tol * max(float(b.abs().max()), 1.0), (k, err)
+        summed = 75 * torch.finfo(dtype).eps * N ** 0.5 if k >= 3 else 0.0
+        assert err <= tol * max(float(b.abs().max()), 1.0) + summed, (k, err)
