@@ -38,6 +38,8 @@
 // gradient).
 #include "dp_group.h"
 
+#include <type_traits>
+
 namespace matpl {
 namespace {
 
@@ -411,38 +413,45 @@ __device__ __forceinline__ void stage_pair(const FusedParams &p, int pair, int l
     __builtin_amdgcn_wave_barrier();
 }
 
-template <int E, bool BF16>
-__global__ void __launch_bounds__(WAVE, BF16 ? 2 : 1)
+// The kernel's two forms. With no more wavefronts than SIMDs (OCC 1) each may have a SIMD's registers to itself:
+// the transposes of both outer products at a time, and in FP32 at E = 25 one wavefront to a block with the pair's
+// weights in LDS instead of read through L2 by every tile. With more, two wavefronts share a SIMD: one product at
+// a time and, at E = 25, 37 (BF16) or 62 (FP32) registers spilled, which the second wavefront outweighs. Four
+// wavefronts to a block there, the bucket types of a chunk side by side: blocks of one wavefront fill the SIMDs
+// unevenly where two fit one. us, one per SIMD / two, in blocks of four / two, in blocks of one: 28,800 atoms of
+// four types BF16 E = 25 551 / 345 / 447, FP32 1289 / 1005 / 1153, FP32 E = 16 (two fit either way) 743 in blocks
+// of four, 893 of one; 1,800 atoms (900 wavefronts) BF16 53 / 61 / 67, FP32 110 / 142 / 168.
+template <int E, bool BF16, int OCC>
+struct EgForm {
+    static constexpr bool LW = !BF16 && E > 16 && OCC == 1;          // the pair's weights in LDS
+    static constexpr int W = LW ? 1 : FUSED_WAVES;         // wavefronts per block
+};
+constexpr int64_t EG_SIMDS = 1024;
+
+template <int E, bool BF16, int OCC>
+__global__ void __launch_bounds__((EgForm<E, BF16, OCC>::W * WAVE), OCC)
 dp_train_embgrad_kernel(TrainParams tp) {
+    constexpr bool LW = EgForm<E, BF16, OCC>::LW;
+    constexpr int W = EgForm<E, BF16, OCC>::W;
     constexpr int NR = NReg<E>::value;
     static_assert(E < 32, "row E of the layer inputs carries the bias gradient");
     constexpr float IK = BF16 ? 1.0f / TANH_K : 1.0f;
     const FusedParams &p = tp.f;
     extern __shared__ float4 smem[];
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & (WAVE - 1), wid = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) : 0;
     const int h = lane >> 5, n = lane & 31;
     // per wave: the batch's compacted neighbors [NBW] (dx, dy, dz, atom of the batch), their
     // residual differences r_j - r_i [NBW], Ahat and Abar of the batch's atoms [EGA][32 features][4]
     constexpr int EGA = eg_atoms<BF16>();
     const int NBW = p.cap > WAVE ? p.cap : WAVE;
-    float4 *nb = smem;
+    float4 *nb = smem + (size_t)wid * (2 * NBW + 2 * EGA * 32 + (BF16 ? 0 : EG_TFLOAT4));
     float4 *us = nb + NBW;
     float4 *ahs = us + NBW, *abs = ahs + EGA * 32;
     float *tscr = reinterpret_cast<float *>(abs + EGA * 32);     // FP32 transpose tile
-    // the weights of the pair in hand: a wavefront's bucket type is fixed and its atoms change type rarely, so they
-    // are staged once per change instead of read through L2 by every tile. The addresses that this frees, and one
-    // outer product at a time, leave BF16 room for two wavefronts per SIMD; with that, single-wavefront blocks spread
-    // over the XCDs and the rows loaded ahead of the compaction, 73,742 atoms of four types take 1190 us (1452 with
-    // one wavefront per SIMD in blocks of one wavefront per bucket type), 7,000 in FP32 396 (433)
     float *svec = tscr + (BF16 ? 0 : 4 * EG_TFLOAT4);
     unsigned char *smat = reinterpret_cast<unsigned char *>(svec + NVEC * 32);
-    // (a wavefront per block: the bucket types' wavefronts differ several times in work, and a block of four would
-    // hold its SIMDs until the longest ends)
-    // Blocks go to the XCDs round-robin: eight chunks of one bucket type, then the same eight of the next, so that
-    // every XCD gets every type's share (with the type varying fastest the types with long buckets, half the work,
-    // would all fall to the same two of eight XCDs).
-    const int t = (int)(blockIdx.x / NXCD % p.T);
-    const int64_t chunk = blockIdx.x / (NXCD * (unsigned)p.T) * NXCD + blockIdx.x % NXCD;
+    const int64_t wg = (int64_t)blockIdx.x * W + wid, chunk = wg / p.T;
+    const int t = (int)(wg % p.T);
     const int64_t i0 = chunk * tp.chunk;
     if (i0 >= p.natoms) return;
     int64_t i1 = i0 + tp.chunk;
@@ -485,7 +494,7 @@ dp_train_embgrad_kernel(TrainParams tp) {
             if (cur >= 0) flush_pair<E>(tp.grad, cur, lane, g3, g2, w1s, b1s);
             cur = pair;
             __builtin_amdgcn_wave_barrier();
-            stage_pair<BF16>(p, pair, lane, svec, smat);
+            if constexpr (LW) stage_pair<BF16>(p, pair, lane, svec, smat);
         }
         if (tot == 0) {
             i += na;
@@ -563,10 +572,12 @@ dp_train_embgrad_kernel(TrainParams tp) {
                 qa = __float_as_int(e.w);
             }
             // (re-read the weights every tile instead of keeping them live across tiles)
-            int pr = 0;
+            int pr = LW ? 0 : pair;
             asm volatile("" : "+v"(pr));
+            const float *vecb = LW ? svec : p.vec;
+            const unsigned char *matb = LW ? smat : reinterpret_cast<const unsigned char *>(p.mat);
             EmbTan<E, BF16> et;
-            et.template run<true>(svec, smat, pr, lane, Ri[0]);
+            et.template run<LW>(vecb, matb, pr, lane, Ri[0]);
             // upstream of G: a = Ahat Ri - Abar v; of G': b = -v0 Abar Ri, with the rows of the lane's
             // own atom of the batch (FP32)
             floatx16 a, b;
@@ -600,15 +611,20 @@ dp_train_embgrad_kernel(TrainParams tp) {
                 if (feat(rr, h) == E) x[rr] = 1.0f;
             }
             {
-                // (BF16: one product at a time, so that two wavefronts share a SIMD)
-                outer_acc<BF16>(tr.apply(x), tr.apply(zb), g3);
-                if constexpr (BF16) __builtin_amdgcn_sched_barrier(0);
-                outer_acc<BF16>(tr.apply(xd), tr.apply(zbd), g3);
-                if constexpr (BF16) __builtin_amdgcn_sched_barrier(0);
+                if constexpr (OCC == 1) {
+                    const floatx16 xt = tr.apply(x), yt = tr.apply(zb), xdt = tr.apply(xd), ydt = tr.apply(zbd);
+                    outer_acc<BF16>(xt, yt, g3);
+                    outer_acc<BF16>(xdt, ydt, g3);
+                } else {
+                    outer_acc<BF16>(tr.apply(x), tr.apply(zb), g3);
+                    __builtin_amdgcn_sched_barrier(0);
+                    outer_acc<BF16>(tr.apply(xd), tr.apply(zbd), g3);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
             // h̄2 = a + W3 z̄3, ḣ̄2 = b + W3 ż̄3 (W3B: true weights)
-            mfma_layer<BF16, true>(mat_ptr<BF16>(smat, pr, M_W3B), lane, zb, a);
-            mfma_layer<BF16, true>(mat_ptr<BF16>(smat, pr, M_W3B), lane, zbd, b);
+            mfma_layer<BF16, LW>(mat_ptr<BF16>(matb, pr, M_W3B), lane, zb, a);
+            mfma_layer<BF16, LW>(mat_ptr<BF16>(matb, pr, M_W3B), lane, zbd, b);
             // layer 2 (h2 = h1 + t2, ḣ2 = ḣ1 + (1 - t2^2) ż2)
 #pragma unroll
             for (int rr = 0; rr < 16; rr++) {
@@ -620,17 +636,22 @@ dp_train_embgrad_kernel(TrainParams tp) {
                 if (feat(rr, h) == E) x[rr] = 1.0f;
             }
             {
-                // (BF16: one product at a time, so that two wavefronts share a SIMD)
-                outer_acc<BF16>(tr.apply(x), tr.apply(zb), g2);
-                if constexpr (BF16) __builtin_amdgcn_sched_barrier(0);
-                outer_acc<BF16>(tr.apply(xd), tr.apply(zbd), g2);
-                if constexpr (BF16) __builtin_amdgcn_sched_barrier(0);
+                if constexpr (OCC == 1) {
+                    const floatx16 xt = tr.apply(x), yt = tr.apply(zb), xdt = tr.apply(xd), ydt = tr.apply(zbd);
+                    outer_acc<BF16>(xt, yt, g2);
+                    outer_acc<BF16>(xdt, ydt, g2);
+                } else {
+                    outer_acc<BF16>(tr.apply(x), tr.apply(zb), g2);
+                    __builtin_amdgcn_sched_barrier(0);
+                    outer_acc<BF16>(tr.apply(xd), tr.apply(zbd), g2);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
-            mfma_layer<BF16, true>(mat_ptr<BF16>(smat, pr, M_W2B), lane, zb, a);
-            mfma_layer<BF16, true>(mat_ptr<BF16>(smat, pr, M_W2B), lane, zbd, b);
+            mfma_layer<BF16, LW>(mat_ptr<BF16>(matb, pr, M_W2B), lane, zb, a);
+            mfma_layer<BF16, LW>(mat_ptr<BF16>(matb, pr, M_W2B), lane, zbd, b);
             // layer 1 (h1 = tanh(x w1 + b1) with x = Ri[0] the normalized input, ḣ1 = (1 - h1^2) w1):
             // w̄1 += x z̄1 + ż̄1, b̄1 += z̄1
-            const float *w1 = vec_ptr(svec, pr, V_W1, h);
+            const float *w1 = vec_ptr(vecb, pr, V_W1, h);
 #pragma unroll
             for (int rr = 0; rr < NR; rr++) {
                 const float q = 1.0f - et.h1[rr] * et.h1[rr];
@@ -673,13 +694,19 @@ int launch_train(TrainParams &tp, int which, hipStream_t st) {
     // (the list width's limit: that of four wavefronts' tiles in 64 KB)
     const size_t tiles = sizeof(float4) * (2 * nbw + 2 * eg_atoms<BF16>() * 32 + (BF16 ? 0 : EG_TFLOAT4));
     MATPL_CHECK_ARG(FUSED_WAVES * tiles <= 64 * 1024, "dp_train_embgrad: list width too large for LDS (%zu bytes)", tiles);
-    const size_t lds = tiles + EG_WEIGHT_BYTES<BF16>;
     const int64_t chunks = (p.natoms + tp.chunk - 1) / tp.chunk;
     const int64_t waves = chunks * p.T;
     MATPL_CHECK_ARG(waves <= (1 << 30), "dp_train_embgrad: too many chunks");
-    hipLaunchKernelGGL((dp_train_embgrad_kernel<E, BF16>), dim3((unsigned)((chunks + NXCD - 1) / NXCD * NXCD * p.T)),
-                       dim3(WAVE), lds, st, tp);
-    return check_launch("dp_train_embgrad_kernel");
+    // waves beyond chunks * T find an empty atom range
+    auto run = [&](auto occ) {
+        constexpr int OCC = decltype(occ)::value;
+        using Form = EgForm<E, BF16, OCC>;
+        const size_t lds = Form::W * tiles + (Form::LW ? EG_WEIGHT_BYTES<BF16> : 0);
+        hipLaunchKernelGGL((dp_train_embgrad_kernel<E, BF16, OCC>), dim3(ceil_div(waves, Form::W)),
+                           dim3(Form::W * WAVE), lds, st, tp);
+        return check_launch("dp_train_embgrad_kernel");
+    };
+    return waves <= EG_SIMDS ? run(std::integral_constant<int, 1>()) : run(std::integral_constant<int, 2>());
 }
 
 int train_dispatch(TrainParams &tp, int E, int bf16, int which, hipStream_t st) {

@@ -2,7 +2,7 @@
 their edges: frames of 1 and 2 atoms, types in no order, atoms without neighbors, buckets of more than a tile and
 atoms whose lists exceed a wavefront's buffer (256 entries), against the FP64 oracle frame by frame; and a training
 step on a batch large enough for whole groups against the sum of its parts, which are small enough to run atom by
-atom. Tolerances: as tests/test_gpu_dp_fused.py (FP32 1e-5 eV/A per force component, 1e-6 relative energy; BF16
+atom. The embedding gradients' two forms (no more wavefronts than SIMDs, and more) against each other. Tolerances: as tests/test_gpu_dp_fused.py (FP32 1e-5 eV/A per force component, 1e-6 relative energy; BF16
 force RMSE 1e-3 eV/A); gradients in FP32 are sums of ~1e6 products added in another order, 2e-5 of their norm."""
 import numpy as np
 import pytest
@@ -37,8 +37,8 @@ def _frames(T, sort, dense, seed):
     return out
 
 
-def _weights(T, m, seed):
-    cfg = DPConfig(ntypes=T, m=m)
+def _weights(T, m, seed, E=25):
+    cfg = DPConfig(ntypes=T, m=m, emb_sizes=[E] * 3)
     davg = np.tile([0.05, 0, 0, 0], (T, 1))
     dstd = np.tile([0.1, 0.07, 0.07, 0.07], (T, 1))
     return DPWeights.random(cfg, seed=seed, davg=davg, dstd=dstd)
@@ -114,3 +114,25 @@ def test_group_training_step_equals_its_parts(dev):
         assert (x is None) == (y is None)
         if x is not None:
             assert float((x.double() - y).norm()) <= 2e-5 * float(y.norm()) + 1e-12
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+@pytest.mark.parametrize("E", [25, 16])
+def test_gradient_kernel_forms_agree(dev, E, precision):
+    """One batch by atoms per wavefront: 1 (some 3,500 wavefronts) and 40 (fewer than SIMDs). Both round the same operands,
+    so that in BF16 too only the order of the sums differs."""
+    frames = _frames(4, True, False, 3)[:7]
+    n = sum(f.natoms for f in frames)
+    print(f"case embedding gradient forms E={E} {precision} atoms={n}", flush=True)
+    model = DPTrainFused(_weights(4, 60, 9, E), precision, dev)
+    batch = pack_fused_batch(frames, model.cfg, dev, seed=4)
+    got = []
+    for chunk in (1, 40):
+        assert (-(-n // chunk) * 4 > 1024) == (chunk == 1)
+        model.chunk = chunk
+        got.append(model.loss_and_grads(batch)[1])
+    assert sum(x is not None for x in got[0]) > 0
+    for x, y in zip(*got):
+        assert (x is None) == (y is None)
+        if x is not None:
+            assert float((x - y).norm()) <= 2e-5 * float(y.norm()) + 1e-12
