@@ -195,7 +195,10 @@ int matpl_bsmm(int f64, int mode, const void *P1, const void *P2, void *out, int
  * (list/shift [N][T][mnl], counts [N][T], positions pos [N][3] float64,
  * lattice [F][9] device, atom_frame [N] / frame_start [F+1] or NULL for one
  * frame) give the normalized Ri (FP32), the embedding net output G on the
- * matrix cores (bf16 != 0: BF16 in / FP32 accumulate; 0: FP32), and
+ * matrix cores (bf16 != 0: BF16 in / FP32 accumulate; 0: FP32; either with
+ * 0x100 added: the caller expects short buckets, so that from 4,096 atoms on
+ * models of three types and more run several atoms per wavefront, with the
+ * same results up to the order of sums; also in matpl_dp_train_tangent), and
  * A[i] = scale * (sum Ri^T G + empty-slot term) [N][4][E], E in {16,25,32}.
  * frame_types [F] (uint32, or NULL): bit t set when type t is in the frame's
  * atom_type list. Only those types' buckets add an empty-slot term, and the

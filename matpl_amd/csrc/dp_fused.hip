@@ -470,7 +470,7 @@ dp_group_fwd_kernel(FusedParams p) {
     const int h = lane >> 5, n = lane & 31, nbw = group_nbw(p);
     const GroupLds L = group_lds(reinterpret_cast<unsigned char *>(smem), wid, nbw, BF16 ? GROUP_BF16_BYTES : GROUP_F32_BYTES);
     const unsigned char *mat = reinterpret_cast<const unsigned char *>(p.mat);
-    const int64_t i0 = ((int64_t)blockIdx.x * FUSED_WAVES + wid) * p.gchunk;
+    const int64_t i0 = (logical_block(1) * FUSED_WAVES + wid) * p.gchunk;
     const int64_t i1 = i0 + p.gchunk < p.natoms ? i0 + p.gchunk : p.natoms;
     for (int64_t i = i0; i < i1;) {
         int first;
@@ -598,7 +598,7 @@ dp_group_bwd_kernel(FusedParams p) {
     double vd[9];
 #pragma unroll
     for (int v = 0; v < 9; v++) { vf[v] = 0.0f; vd[v] = 0.0; }
-    const int64_t i0 = ((int64_t)blockIdx.x * FUSED_WAVES + wid) * p.gchunk;
+    const int64_t i0 = (logical_block(1) * FUSED_WAVES + wid) * p.gchunk;
     const int64_t i1 = i0 + p.gchunk < p.natoms ? i0 + p.gchunk : p.natoms;
     for (int64_t i = i0; i < i1;) {
         int first;
@@ -831,18 +831,20 @@ int launch_lw(FusedParams &p, bool fwd, hipStream_t st, const LaunchCfg &cfg) {
     return check_launch("dp_fused_bwd_kernel");
 }
 
+template <int E, bool BF16>
+constexpr bool GROUP_BWD = !(E == 32 && BF16);
+
 // Net mode over groups of atoms (three types and more); returns 1 where the group's LDS does not fit.
 template <int E, bool BF16>
 int launch_group(FusedParams &p, bool fwd, hipStream_t st) {
     const size_t extra = fwd ? (BF16 ? GROUP_BF16_BYTES : GROUP_F32_BYTES) : GROUP_DA_BYTES;
     const size_t lds = FUSED_WAVES * (group_base_bytes(group_nbw(p)) + extra);
     if (lds > 64 * 1024) return 1;
-    dp_group_shape(p);
-    const int64_t waves = (p.natoms + p.gchunk - 1) / p.gchunk, blocks = (waves + FUSED_WAVES - 1) / FUSED_WAVES;
-    const dim3 grid((unsigned)blocks), block(FUSED_WAVES * WAVE);
+    dp_group_shape(p, fwd ? 3 : 2);
+    const dim3 grid(dp_group_blocks(p)), block(FUSED_WAVES * WAVE);
     if (fwd && p.gbuf) hipLaunchKernelGGL((dp_group_fwd_kernel<E, BF16, true>), grid, block, lds, st, p);
     else if (fwd) hipLaunchKernelGGL((dp_group_fwd_kernel<E, BF16, false>), grid, block, lds, st, p);
-    else hipLaunchKernelGGL((dp_group_bwd_kernel<E, BF16>), grid, block, lds, st, p);
+    else if constexpr (GROUP_BWD<E, BF16>) hipLaunchKernelGGL((dp_group_bwd_kernel<E, BF16>), grid, block, lds, st, p);
     return check_launch("dp_group_kernel");
 }
 
@@ -889,7 +891,7 @@ int launch(FusedParams &p, bool fwd, hipStream_t st, int ck) {
     if (ck == 4) return launch_lw<E, BF16, false, 4>(p, fwd, st, g_launch[fwd ? 0 : 1]);
     if (ck == 6) return launch_lw<E, BF16, false, 6>(p, fwd, st, g_launch[fwd ? 0 : 1]);
     // (the stored backward reads G atom by atom)
-    if ((fwd || !p.gbuf) && dp_group_wanted(p.T, p.mnl, p.natoms)) {
+    if ((fwd || (GROUP_BWD<E, BF16> && !p.gbuf)) && dp_group_wanted(p)) {
         const int rc = launch_group<E, BF16>(p, fwd, st);
         if (rc <= 0) return rc;
     }
@@ -913,6 +915,8 @@ int launch(FusedParams &p, bool fwd, hipStream_t st, int ck) {
 }
 
 int dispatch(FusedParams &p, int E, int bf16, bool fwd, hipStream_t st, int ck = 0) {
+    p.group = bf16 & DP_GROUP;
+    bf16 &= ~DP_GROUP;
     MATPL_CHECK_ARG(p.T >= 1 && p.T <= MAXT, "dp_fused: ntypes must be in [1,%d]", MAXT);
     MATPL_CHECK_ARG(p.mnl >= 1 && p.m >= 1, "dp_fused: bad bucket sizes");
     p.cap = p.m < p.mnl ? p.m : p.mnl;

@@ -69,7 +69,8 @@ struct FusedParams {
     float rmin, rmax, scale;    // scale = 1 / (m * T), used when frame_types is null
     float iw;                   // 1 / (rmax - rmin)
     int xcd;                    // 1: XCD-aware block order (grid a multiple of NXCD)
-    int ga, gchunk;             // group kernels (dp_group.h): atoms per group, atoms per wavefront
+    int group;                  // the caller's word that buckets are short (dp_group.h)
+    int ga, gchunk;             // group kernels: atoms per group, atoms per wavefront
     // compressed embedding (table mode): G(s) by piecewise polynomials, K coefficients per
     // feature and interval, highest power first, laid out [T*T][rows][32 features][K], so that
     // the 32 lanes of a half-wave read one interval's row in one coalesced load

@@ -1,7 +1,7 @@
 // Group passes of the fused DP kernels: one wavefront takes up to GA consecutive atoms of one frame and one type
 // together, so that their in-cutoff neighbors of each type share 32-lane tiles. A four-type system holds ~2 to 25
 // neighbors per bucket (48 of 128 tile lanes filled atom by atom); four atoms together fill ~80 %. Used for
-// ntypes >= 3 (dp_group_wanted): with one or two types a bucket fills its tiles by itself (HfO2 27 and 55, Cu 78),
+// three types and more (dp_group_wanted): with one or two a bucket fills its tiles by itself (HfO2 27 and 55, Cu 78),
 // and the per-lane atom selects below would only cost.
 #pragma once
 #include "dp_fused_common.h"
@@ -16,14 +16,40 @@ constexpr int GT_STRIDE = 33;                  // FP32 G tile [32 neighbors][33]
 constexpr int QSHIFT = 24;                     // atom of an entry's packed (bucket slot | atom << 24)
 constexpr int JSHIFT = 29;                     // atom of an entry's packed (neighbor | atom << 29)
 
-inline bool dp_group_wanted(int T, int mnl, int64_t n) { return T >= 3 && mnl < (1 << QSHIFT) && n < (1ll << JSHIFT); }
+// Where the passes are taken. The caller says whether buckets are short (DP_GROUP in its precision argument), since
+// the lists themselves are on the device: matpl_amd.dp_fused.short_buckets, by the mix of types. us of a whole
+// evaluation, an atom per wavefront against groups, four-type models in BF16:
+//   60,000 atoms of four types (40, 4, 8 and 48 %) 865 and 660; 55,296 HfO2 atoms 726 and 769, 8,640 191 and 222;
+//   of few atoms each wavefront takes one (500 atoms 81 and 84, 4,000 126 and 133; 4,500 143 and 120).
+// The backward at E = 32 in BF16 needs all registers for groups (one wavefront per SIMD: 20,000 atoms 204 and 245).
+constexpr int DP_GROUP = 0x100;
+constexpr int64_t GROUP_ATOMS = 4096;
 
-// Atoms per group and wavefront: fewer where whole groups would leave the chip short of wavefronts.
-inline void dp_group_shape(FusedParams &p) {
-    const int64_t g = p.natoms / 2048;
-    p.ga = (int)(g < 1 ? 1 : (g > GA ? GA : g));
+inline bool dp_group_wanted(const FusedParams &p) {
+    return p.group && p.T >= 3 && p.natoms >= GROUP_ATOMS && p.natoms < (1ll << JSHIFT) && p.mnl < (1 << QSHIFT);
+}
+
+// Atoms per group and wavefront of a kernel that runs `occ` wavefronts on each of the 1,024 SIMDs: those whose
+// rounds of wavefronts take the least, a group of g atoms costing about g + 1 (a last round that is nearly empty costs
+// as much as a full one: 8,640 atoms in groups of four are 2,160 wavefronts, of 2,048 that run at once). With
+// many rounds, whole groups, and several per wavefront.
+inline void dp_group_shape(FusedParams &p, int occ) {
+    int64_t best = 0;
+    for (int g = GA; g >= 2; g--) {
+        const int64_t waves = (p.natoms + g - 1) / g, rounds = (waves + 1024 * occ - 1) / (1024 * occ);
+        if (g == GA || rounds * (g + 1) < best) {
+            best = rounds * (g + 1);
+            p.ga = g;
+        }
+    }
     const int64_t per = p.natoms / (8192 * (int64_t)p.ga);          // whole groups per wavefront
     p.gchunk = p.ga * (int)(per < 1 ? 1 : per);
+}
+
+// Blocks of a group kernel: a multiple of the XCDs, which take contiguous ranges of atoms (logical_block).
+inline unsigned dp_group_blocks(const FusedParams &p) {
+    const int64_t per = FUSED_WAVES * (int64_t)p.gchunk, blocks = (p.natoms + per - 1) / per;
+    return (unsigned)((blocks + NXCD - 1) / NXCD * NXCD);
 }
 
 struct Group {

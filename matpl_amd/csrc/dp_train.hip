@@ -222,7 +222,7 @@ dp_group_tangent_kernel(TrainParams tp) {
     const int n = lane & 31, nbw = group_nbw(p);
     const GroupLds L = group_lds(reinterpret_cast<unsigned char *>(smem), wid, nbw, GROUP_F32_BYTES);
     float *xs = reinterpret_cast<float *>(L.rest), *gt = xs + 32 * 5;
-    const int64_t i0 = ((int64_t)blockIdx.x * FUSED_WAVES + wid) * p.gchunk;
+    const int64_t i0 = (logical_block(1) * FUSED_WAVES + wid) * p.gchunk;
     const int64_t i1 = i0 + p.gchunk < p.natoms ? i0 + p.gchunk : p.natoms;
     for (int64_t i = i0; i < i1;) {
         int first;
@@ -670,13 +670,12 @@ dp_train_embgrad_kernel(TrainParams tp) {
 template <int E, bool BF16>
 int launch_train(TrainParams &tp, int which, hipStream_t st) {
     FusedParams &p = tp.f;
-    if (which == 0 && dp_group_wanted(p.T, p.mnl, p.natoms)) {
+    if (which == 0 && dp_group_wanted(p)) {
         const size_t lds = FUSED_WAVES * (group_base_bytes(group_nbw(p)) + GROUP_F32_BYTES);
         if (lds <= 64 * 1024) {
-            dp_group_shape(p);
-            const int64_t waves = (p.natoms + p.gchunk - 1) / p.gchunk;
-            hipLaunchKernelGGL((dp_group_tangent_kernel<E, BF16>), dim3(ceil_div(waves, FUSED_WAVES)),
-                               dim3(FUSED_WAVES * WAVE), lds, st, tp);
+            dp_group_shape(p, 3);
+            hipLaunchKernelGGL((dp_group_tangent_kernel<E, BF16>), dim3(dp_group_blocks(p)), dim3(FUSED_WAVES * WAVE),
+                               lds, st, tp);
             return check_launch("dp_group_tangent_kernel");
         }
     }
@@ -711,6 +710,8 @@ int launch_train(TrainParams &tp, int which, hipStream_t st) {
 
 int train_dispatch(TrainParams &tp, int E, int bf16, int which, hipStream_t st) {
     FusedParams &p = tp.f;
+    p.group = bf16 & DP_GROUP;
+    bf16 &= ~DP_GROUP;
     MATPL_CHECK_ARG(p.T >= 1 && p.T <= MAXT, "dp_train: ntypes must be in [1,%d]", MAXT);
     MATPL_CHECK_ARG(p.mnl >= 1 && p.m >= 1, "dp_train: bad bucket sizes");
     p.cap = p.m < p.mnl ? p.m : p.mnl;

@@ -219,6 +219,18 @@ def type_masks(type_present, nframes: int, ntypes: int) -> np.ndarray:
     return masks
 
 
+# of the kernels' precision argument: neighbor buckets are short, so that several atoms share a wavefront
+DP_GROUP = 0x100
+
+
+def short_buckets(type_counts) -> bool:
+    """Whether atoms in these numbers per type leave the neighbor buckets short: they are spread over three types or
+    more. The effective number of types, 1 / sum of squared fractions, is 1.8 for HfO2 on a model of any number of
+    types, whose buckets fill the kernels' tiles atom by atom, and 2.5 for Li10GeP2S12 (csrc/dp_group.h has times)."""
+    n = np.asarray(type_counts, np.float64)
+    return float(n.sum()) ** 2 >= 2.3 * float((n * n).sum()) > 0.0
+
+
 class FusedDP:
     """DP E/F/V for one (or a batch of) frame(s) given a neighbor list.
 
@@ -261,6 +273,7 @@ class FusedDP:
         self.fit = _Fitting(w, self.device)
         self.fitting = fitting
         self._mfma_fit = {}
+        self._short = {}        # short_buckets of the type runs seen
         self.precision = precision
         self.events = None      # when a list: (start, end) HIP events around each backward launch
         self._masks = {}        # checked per-frame type masks on the device, by content and atoms
@@ -284,13 +297,20 @@ class FusedDP:
         dev = pos.device
         if type_ranges is None:
             type_ranges = type_runs(type_map.cpu().numpy())
+        key = tuple(segments(type_ranges))
+        if key not in self._short:
+            counts = [0] * T
+            for t, a, b in key:
+                counts[t] += b - a
+            self._short[key] = short_buckets(counts)
+        precision = int(self.fw.bf16) | (DP_GROUP if self._short[key] else 0)
         scale = 1.0 / (cfg.m * T)
         masks = None if type_present is None else self._type_masks(type_present, type_map, atom_frame, nframes)
         A = torch.empty((N, 4, self.fw.E), dtype=torch.float32, device=dev)
         status = torch.zeros(1, dtype=torch.int32, device=dev)
         head = (_ptr(pos), _ptr(lattice), _ptr(atom_frame), _ptr(frame_start), _ptr(masks), _ptr(nl_list),
                 _ptr(nl_shift), _ptr(nl_counts), _ptr(type_map), _ptr(self.fw.vec))
-        tail = (_ptr(self.fw.tinfo), N, T, mnl, cfg.m, self.fw.E, int(self.fw.bf16), float(cfg.rcut),
+        tail = (_ptr(self.fw.tinfo), N, T, mnl, cfg.m, self.fw.E, precision, float(cfg.rcut),
                 float(cfg.rcut_smooth), scale)
         if self.table is None:
             args, sfx = head + (_ptr(self.fw.mat),) + tail, ""
@@ -309,7 +329,6 @@ class FusedDP:
         else:
             _lib.call("matpl_dp_fused_forward" + sfx, *args, _ptr(A), _ptr(status), _stream())
         if self.fitting == "mfma":
-            key = tuple(segments(type_ranges))
             if key not in self._mfma_fit:
                 self._mfma_fit[key] = FittingMFMA(self.w, type_ranges, self.precision, dev)
             Ei, dA = self._mfma_fit[key](A)

@@ -35,8 +35,8 @@ import torch
 from . import _lib
 from .calcops import _ptr, _stream
 from .dp import _Net
-from .dp_fused import M_W2B, M_W2F, M_W3B, M_W3F, NMAT, NTI, NVEC, TANH_K, V_B1, V_B2, V_B3, V_GPAD, V_R2, V_R3, \
-    V_W1, feat, type_masks
+from .dp_fused import DP_GROUP, M_W2B, M_W2F, M_W3B, M_W3F, NMAT, NTI, NVEC, TANH_K, V_B1, V_B2, V_B3, V_GPAD, \
+    V_R2, V_R3, V_W1, feat, short_buckets, type_masks
 from .dpnet import DPWeights
 from .neighbor import find_neighbore_batch, reverse_map
 
@@ -61,6 +61,7 @@ class FusedBatch:
     rev: torch.Tensor            # [N, T*m] int32 partner slot
     E_label: torch.Tensor        # [F] float64
     F_label: torch.Tensor        # [N, 3] float64
+    short: bool = False          # short neighbor buckets (dp_fused.short_buckets) in most frames, by atoms
 
 
 def pack_fused_batch(frames, cfg, device="cuda", seed=0, type_present=None) -> FusedBatch:
@@ -97,7 +98,8 @@ def pack_fused_batch(frames, cfg, device="cuda", seed=0, type_present=None) -> F
     return FusedBatch(len(frames), N, pos, lat, tm, af, fs, torch.as_tensor(sizes, dtype=torch.float64, device=device),
                       torch.as_tensor(type_masks(tp, len(frames), T).view(np.int32), device=device),
                       torch.as_tensor(tp, device=device), [torch.nonzero(tm64 == t).reshape(-1) for t in range(T)],
-                      nl.list, nl.shift, nl.counts, rev, E_label, F_label)
+                      nl.list, nl.shift, nl.counts, rev, E_label, F_label,
+                      2 * sum(f.natoms for f in frames if short_buckets(np.bincount(f.types))) > N)
 
 
 class _EmbPack:
@@ -354,7 +356,8 @@ class DPTrainFused(torch.nn.Module):
 
     def _tail(self, b: FusedBatch, mnl: int):
         cfg = self.cfg
-        return (_ptr(self.tinfo), b.natoms, cfg.ntypes, mnl, cfg.m, self.E, int(self.bf16), float(cfg.rcut),
+        return (_ptr(self.tinfo), b.natoms, cfg.ntypes, mnl, cfg.m, self.E,
+                int(self.bf16) | (DP_GROUP if b.short else 0), float(cfg.rcut),
                 float(cfg.rcut_smooth), 1.0 / (cfg.m * cfg.ntypes))
 
     def _listed_any(self, b: FusedBatch):
