@@ -331,7 +331,9 @@ int matpl_dp_train_grad_size(int E);
  * or LDS when they fit (-1, default), and the XCD-aware block order (1) or
  * plain order (0, default). With all of these and the wavefronts per block at
  * their defaults, large workloads get a shape by size, type count and
- * precision. Results do not depend on the shape except through
+ * precision. They are of the kernels that run an atom per
+ * wavefront; short buckets in groups (below) take their own shape, and only
+ * where none is set. Results do not depend on the shape except through
  * the virial's FP64 summation order. No counterpart in the reference: it is
  * the knob the launch autotuner (matpl_amd/autotune.py) turns.
  */

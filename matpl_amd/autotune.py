@@ -1,8 +1,9 @@
 """Launch-shape autotuner for the fused DP kernels.
 
 The fused forward and backward kernels (csrc/dp_fused.hip) run a persistent
-grid, one atom per wavefront. Four launch choices change their speed but not
-their results:
+grid, one atom per wavefront, unless short neighbor buckets put several atoms
+on one (dp_fused.short_buckets), where no shape is set. Four launch choices
+change their speed but not their results:
   * the wavefronts per block (2, 4 or 8 atoms sharing one block's staged
     weights and LDS; each is a separate instantiation of the kernels);
   * the grid's block cap (how many blocks stride over the atoms);
@@ -31,7 +32,7 @@ from . import _lib
 
 BLOCK_CAPS = (512, 768, 1024, 1536, 2048, 3072, 4096, 8192, 16384)
 WAVES = (2, 4, 8)
-# the shape that leaves the choice to the library (by size, types and precision)
+# the shape that leaves the choice to the library (by size, types and precision, groups of atoms included)
 DEFAULT = {"max_blocks": 4096, "lds_weights": -1, "xcd": 0, "waves": 4}
 
 

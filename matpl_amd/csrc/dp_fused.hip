@@ -873,11 +873,15 @@ int launch_net(FusedParams &p, bool fwd, hipStream_t st, const LaunchCfg &cfg, b
 //   caches already.
 constexpr int64_t LAUNCH_ATOMS = 8192;
 
+bool launch_unset(bool fwd) {
+    const LaunchCfg &set = g_launch[fwd ? 0 : 1];
+    return set.max_blocks == LAUNCH_DEFAULT.max_blocks && set.lds_weights == LAUNCH_DEFAULT.lds_weights &&
+           set.xcd == LAUNCH_DEFAULT.xcd && set.waves == LAUNCH_DEFAULT.waves;
+}
+
 LaunchCfg launch_cfg(const FusedParams &p, bool fwd, bool bf16, bool lds_fits) {
     const LaunchCfg set = g_launch[fwd ? 0 : 1];
-    const bool unset = set.max_blocks == LAUNCH_DEFAULT.max_blocks && set.lds_weights == LAUNCH_DEFAULT.lds_weights &&
-                       set.xcd == LAUNCH_DEFAULT.xcd && set.waves == LAUNCH_DEFAULT.waves;
-    if (!unset || p.gbuf || p.natoms < LAUNCH_ATOMS) return set;
+    if (!launch_unset(fwd) || p.gbuf || p.natoms < LAUNCH_ATOMS) return set;
     if (!fwd && lds_fits) return LaunchCfg{512, -1, 1, FUSED_WAVES};
     if (fwd && bf16 && p.T == 2) return LaunchCfg{16384, 0, 1, 8};
     return set;
@@ -890,8 +894,8 @@ template <int E, bool BF16>
 int launch(FusedParams &p, bool fwd, hipStream_t st, int ck) {
     if (ck == 4) return launch_lw<E, BF16, false, 4>(p, fwd, st, g_launch[fwd ? 0 : 1]);
     if (ck == 6) return launch_lw<E, BF16, false, 6>(p, fwd, st, g_launch[fwd ? 0 : 1]);
-    // (the stored backward reads G atom by atom)
-    if ((fwd || (GROUP_BWD<E, BF16> && !p.gbuf)) && dp_group_wanted(p)) {
+    // A shape that the caller has set is of the atom-by-atom kernels. The stored backward reads G atom by atom.
+    if (launch_unset(fwd) && (fwd || (GROUP_BWD<E, BF16> && !p.gbuf)) && dp_group_wanted(p)) {
         const int rc = launch_group<E, BF16>(p, fwd, st);
         if (rc <= 0) return rc;
     }
