@@ -105,6 +105,43 @@ struct RowSums {
 };
 static_assert(SUM_ROWS == 1 << (32 - 23), "the hash keeps the top bits");
 
+// A block's few slots in small frames cost less added directly than a table's clearing and flushing.
+// Force and virial, double, us: 4,000 frames of one atom with 4 slots 40 directly, 53 by tables; 2,000 of one
+// with 40 slots 58 and 37.
+constexpr int SUM_MIN_SLOTS = 17;
+
+// The terms of one slot: f_c, or f_a r_b.
+template <typename T, bool VIRIAL>
+__device__ __forceinline__ void slot_terms(const T *__restrict__ dE, const T *__restrict__ Rij,
+                                           const T *__restrict__ Ri_d, int64_t s, T v[VIRIAL ? 9 : 3]) {
+    T f[3];
+    slot_force(dE, Ri_d, s, f);
+    if constexpr (VIRIAL) {
+        const T r[3] = {Rij[3 * s], Rij[3 * s + 1], Rij[3 * s + 2]};
+#pragma unroll
+        for (int c = 0; c < 9; c++) v[c] = f[c / 3] * r[c % 3];
+    } else {
+#pragma unroll
+        for (int c = 0; c < 3; c++) v[c] = f[c];
+    }
+}
+
+template <typename T, bool VIRIAL>
+__global__ void __launch_bounds__(SUM_THREADS)
+slot_direct_kernel(const int32_t *__restrict__ nlist, const T *__restrict__ dE, const T *__restrict__ Rij,
+                   const T *__restrict__ Ri_d, T *__restrict__ out, int64_t per_frame, int64_t NA, int64_t nslots) {
+    constexpr int W = VIRIAL ? 9 : 3;
+    for (int64_t s = blockIdx.x * (int64_t)SUM_THREADS + threadIdx.x; s < nslots; s += (int64_t)gridDim.x * SUM_THREADS) {
+        const int j = nlist[s];
+        if (j < 0) continue;
+        T v[W];
+        slot_terms<T, VIRIAL>(dE, Rij, Ri_d, s, v);
+        T *o = out + (s / per_frame * NA + j) * W;
+#pragma unroll
+        for (int c = 0; c < W; c++) atomic_add(o + c, v[c]);
+    }
+}
+
 // Blocks (chunk of SUM_CENTRES atoms, frame); the grid strides over both.
 template <typename T, bool VIRIAL>
 __global__ void __launch_bounds__(SUM_THREADS)
@@ -121,16 +158,8 @@ slot_scatter_kernel(const int32_t *__restrict__ nlist, const T *__restrict__ dE,
         for (int64_t s = (b * N + i0) * S + threadIdx.x; s < (b * N + i1) * S; s += SUM_THREADS) {
             const int j = nlist[s];
             if (j < 0) continue;
-            T f[3], v[W];
-            slot_force(dE, Ri_d, s, f);
-            if constexpr (VIRIAL) {
-                const T r[3] = {Rij[3 * s], Rij[3 * s + 1], Rij[3 * s + 2]};
-#pragma unroll
-                for (int c = 0; c < 9; c++) v[c] = f[c / 3] * r[c % 3];
-            } else {
-#pragma unroll
-                for (int c = 0; c < 3; c++) v[c] = f[c];
-            }
+            T v[W];
+            slot_terms<T, VIRIAL>(dE, Rij, Ri_d, s, v);
             const int x = rows.place(j);
             if (x >= 0) {
 #pragma unroll
@@ -253,6 +282,11 @@ inline unsigned grid_for(int64_t n) {
 template <typename T, bool VIRIAL>
 int launch_scatter(const int32_t *nlist, const T *dE, const T *Rij, const T *Ri_d, T *out, int64_t B, int64_t N,
                    int64_t S, int64_t NA, hipStream_t st) {
+    if ((N < SUM_CENTRES ? N : SUM_CENTRES) * S < SUM_MIN_SLOTS) {
+        hipLaunchKernelGGL((slot_direct_kernel<T, VIRIAL>), dim3(grid_for(B * N * S)), dim3(SUM_THREADS), 0, st, nlist, dE,
+                           Rij, Ri_d, out, N * S, NA, B * N * S);
+        return check_launch("slot_direct_kernel");
+    }
     const int64_t nchunk = (N + SUM_CENTRES - 1) / SUM_CENTRES, nwork = B * nchunk;
     hipLaunchKernelGGL((slot_scatter_kernel<T, VIRIAL>), dim3((unsigned)(nwork < 8192 ? nwork : 8192)),
                        dim3(SUM_THREADS), 0, st, nlist, dE, Rij, Ri_d, out, N, S, NA, nchunk, nwork);

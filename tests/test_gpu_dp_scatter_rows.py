@@ -11,6 +11,7 @@ pytestmark = pytest.mark.gpu
     (1, 700, 130, 40, 740),         # about 1040 slots a block over 740 rows: the table overflows
     (1, 4000, 70, 0, 4000),         # hardly any row twice in a block
     (1, 20, 300, 0, 1),             # every slot the same row
+    (300, 2, 8, 1, 3), (77, 1, 17, 0, 1),       # frames of few slots: directly up to 16 a block, by the table from 17 on
 ])
 def test_scatter_row_sums(B, N, S, ng, rows, dtype):
     if not torch.cuda.is_available():
