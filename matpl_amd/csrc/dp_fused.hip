@@ -871,6 +871,8 @@ int launch_net(FusedParams &p, bool fwd, hipStream_t st, const LaunchCfg &cfg, b
 //   through the caches with 8 wavefronts a block is faster: 248 -> 229, 498 -> 439, 1299 -> 1196.
 //   One type's (Cu) are better in LDS (398 -> 402 us without), and FP32's are read through the
 //   caches already.
+// Not at E = 16 in FP32 with one type, where more than 512 blocks run at once (backward of 57,600 Cu atoms 638
+// us plain, 726 in the shape), and not the forward at E = 32 (99,636 HfO2 atoms 467 and 498).
 constexpr int64_t LAUNCH_ATOMS = 8192;
 
 bool launch_unset(bool fwd) {
@@ -879,11 +881,11 @@ bool launch_unset(bool fwd) {
            set.xcd == LAUNCH_DEFAULT.xcd && set.waves == LAUNCH_DEFAULT.waves;
 }
 
-LaunchCfg launch_cfg(const FusedParams &p, bool fwd, bool bf16, bool lds_fits) {
+LaunchCfg launch_cfg(const FusedParams &p, int E, bool fwd, bool bf16, bool lds_fits) {
     const LaunchCfg set = g_launch[fwd ? 0 : 1];
     if (!launch_unset(fwd) || p.gbuf || p.natoms < LAUNCH_ATOMS) return set;
-    if (!fwd && lds_fits) return LaunchCfg{512, -1, 1, FUSED_WAVES};
-    if (fwd && bf16 && p.T == 2) return LaunchCfg{16384, 0, 1, 8};
+    if (!fwd && lds_fits && (bf16 || E > 16)) return LaunchCfg{512, -1, 1, FUSED_WAVES};
+    if (fwd && bf16 && E < 32 && p.T == 2) return LaunchCfg{16384, 0, 1, 8};
     return set;
 }
 
@@ -903,7 +905,7 @@ int launch(FusedParams &p, bool fwd, hipStream_t st, int ck) {
         return (fwd ? fused_lds_bytes<BF16, true, false>(p.T, p.cap, w)
                     : fused_lds_bytes<BF16, true, true>(p.T, p.cap, w)) <= 64 * 1024;
     };
-    const LaunchCfg cfg = launch_cfg(p, fwd, BF16, lds_fits(FUSED_WAVES));
+    const LaunchCfg cfg = launch_cfg(p, E, fwd, BF16, lds_fits(FUSED_WAVES));
     const int mode = cfg.lds_weights;
     // a wavefront count set for another workload whose neighbor tiles would exceed the LDS budget
     // here falls back to fewer wavefronts per block
