@@ -1046,18 +1046,20 @@ nep_angular_bwd2_kernel(FeatArgs a) {
 // CalcOps.cpp:75-158; the frame sum of calculateNepVirial, CalcOps.cpp:239-328), with the model's signs
 // (nep_net.py negates both): F[i] += f, F[j] -= f, V[frame] -= f (x) x. No [N][S][4] gradient is written or read.
 // A block takes windows of `ch` consecutive atoms, frame by frame (a segment); neighbor terms go to an LDS copy
-// of F over the segment's frame (n <= rcap atoms), written once to the segment's row of `part`, since device
-// atomics are carried out beyond the per-XCD L2 caches here; nep_force_final_kernel adds the rows. The copy is in
+// of F over the segment's frame (n <= rcap atoms), written once to the segment's row in `part`, since device
+// atomics are carried out beyond the per-XCD L2 caches here; nep_force_final_kernel adds the rows. A frame's rows
+// (as long as the frame, one per window that it touches, at most force_rows) lie together, from 3 force_rows times
+// its first atom on: the buffer grows with the atoms, whatever the sizes of the other frames. The copy is in
 // double in both precisions: LDS adds of floats take several times those of doubles here (62,713-atom float
 // batch: 276 us with a float copy, 181 with this one; the position gradients, two force kernels and their
 // reductions that this kernel stands for took 590 us). Segment
-// (window b, frame f) has row b + f: consecutive segments advance b or f. Larger frames (rcap = 0), and any
+// (window b, frame f) has virial row b + f: consecutive segments advance b or f. Larger frames (rcap = 0), and any
 // entry naming an atom of another frame, use global atomics.
 struct ForceArgs {
     FeatArgs r, a;                // radial / angular: c, Ri, NL, atom_map, gfeat, save, sizes
     const int64_t *frame_start;   // [F + 1]
     const int32_t *atom_frame;    // [N]
-    void *F, *part;               // [N][3] (zeroed), [segments][3 rcap]
+    void *F, *part;               // [N][3] (zeroed), the frames' rows
     double *vpart;                // [segments][9]
     int64_t rcap;
     int ch;
@@ -1081,8 +1083,11 @@ __device__ __forceinline__ T fold16(T v[16], int lane) {
     return x;
 }
 
-// (141 float and 256 double VGPRs: 3 and 2 wavefronts per SIMD, which blocks of 4 wavefronts fill; of 8, one
-// float block fits a CU)
+// Rows of a frame of at most rcap atoms: the windows of ch that it touches.
+__host__ __device__ inline int64_t force_rows(int64_t rcap, int ch) { return rcap > 0 ? (rcap - 1) / ch + 2 : 0; }
+
+// (153 float and 256 double VGPRs: 3 and 2 wavefronts per SIMD, which blocks of 4 wavefronts fill; of 8, one
+// float block fits a CU; in double 4 registers spill, in the general sizes' form 32)
 constexpr int FORCE_WAVES = 4;
 
 template <typename T>
@@ -1231,7 +1236,7 @@ nep_force_kernel(ForceArgs p) {
             p.vpart[seg * 9 + threadIdx.x] = v;
         }
         if (lds) {
-            T *o = reinterpret_cast<T *>(p.part) + seg * 3 * p.rcap;
+            T *o = reinterpret_cast<T *>(p.part) + 3 * (fs * force_rows(p.rcap, p.ch) + (i0 / p.ch - fs / p.ch) * (fe - fs));
             for (int64_t x = threadIdx.x; x < 3 * (fe - fs); x += blockDim.x) o[x] = (T)acc[x];
         }
         __syncthreads();
@@ -1272,10 +1277,10 @@ nep_force_final_kernel(const int64_t *__restrict__ frame_start, const int32_t *_
         const int64_t fs = frame_start[f], fe = frame_start[f + 1];
         any = fe - fs <= rcap;
         if (any) {
-            const T *q = part + (e - 3 * fs);
-            const int64_t b1 = (fe - 1) / ch;
+            const T *q = part + 3 * fs * force_rows(rcap, ch) + (e - 3 * fs);
+            const int64_t nw = (fe - 1) / ch - fs / ch + 1;
 #pragma unroll 4
-            for (int64_t b = fs / ch + g; b <= b1; b += 4) s += q[(b + f) * 3 * rcap];
+            for (int64_t b = g; b < nw; b += 4) s += q[b * 3 * (fe - fs)];
         }
     }
     redT[threadIdx.x] = s;
@@ -1449,14 +1454,14 @@ MATPL_EXPORT int matpl_nep_descriptor(int f64, int angular, int mode, const void
     return feat_run(a, f64, angular != 0, what[mode], (hipStream_t)stream);
 }
 
-// Bytes of the work buffer of matpl_nep_model_forces (segment rows of F, then of the virial).
+// Bytes of the work buffer of matpl_nep_model_forces (the segments' virials, then the frames' rows of F).
 MATPL_EXPORT int64_t matpl_nep_model_forces_work(int f64, int64_t N, int64_t nframes, int64_t max_frame, int ntypes,
                                                  int na, int nbr) {
     if (N <= 0 || nframes < 1 || max_frame < 1 || ntypes < 1 || na < 0 || nbr < 1) return 0;
     const ForcePlan pl = f64 ? force_plan<double>(N, max_frame, ntypes, na, nbr)
                              : force_plan<float>(N, max_frame, ntypes, na, nbr);
     const int64_t seg = ceil_div(N, pl.ch) + nframes;
-    return seg * (9 * (int64_t)sizeof(double) + 3 * pl.rcap * (f64 ? 8 : 4));
+    return seg * 9 * (int64_t)sizeof(double) + 3 * N * force_rows(pl.rcap, pl.ch) * (f64 ? 8 : 4);
 }
 
 MATPL_EXPORT int matpl_nep_model_forces(int f64, const void *c2, const void *c3, const void *Ri_r, const int64_t *NL_r,

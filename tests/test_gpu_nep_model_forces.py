@@ -47,7 +47,8 @@ def _by_ops(model, nb, p):
 CASES = [([1, 2, 3, 70, 64, 5, 1, 130], 3, 4, 12, [4, 2, 0]),       # many frames in a window
          ([2500], 2, 4, 12, [4, 2, 0]),                              # above the LDS copy in double
          ([40, 9, 300], 2, 3, 7, [4, 2, 1]),                         # other sizes, 5-body
-         ([50, 20], 5, 4, 12, [0, 0, 0])]                            # radial only
+         ([50, 20], 5, 4, 12, [0, 0, 0]),                            # radial only
+         ([3] * 40 + [1900] + [2] * 30, 2, 4, 12, [4, 2, 0])]        # one large frame among many tiny ones
 
 
 @pytest.mark.parametrize("sizes,T,n_max,basis,l_max", CASES)
@@ -87,3 +88,13 @@ def test_model_path_equals_operator_sequence(dev, sizes, T, n_max, basis, l_max)
             x = F if wx is wF else V
             gs = torch.autograd.grad((x * wx).sum(), params, allow_unused=True)
             assert all(torch.isfinite(q).all() for q in gs if q is not None)
+
+
+def test_work_buffer_grows_with_the_atoms():
+    """100,000 frames of 10 atoms and one of 2,000: rows of 2,000 for each frame would be gigabytes."""
+    from matpl_amd import _lib
+    small = _lib.query("matpl_nep_model_forces_work", 0, 1_000_000, 100_000, 10, 4, 5, 13)
+    mixed = _lib.query("matpl_nep_model_forces_work", 0, 1_002_000, 100_001, 2000, 4, 5, 13)
+    # three floats an atom and window of its frame, 72 bytes for each window and frame
+    assert small <= 1_000_000 * 12 * 2 + 72 * (1_000_000 // 64 + 100_001)
+    assert mixed <= 1_002_000 * 12 * (2000 // 64 + 2) + 72 * (1_002_000 // 64 + 100_002)
