@@ -358,8 +358,8 @@ class NEPTorch(torch.nn.Module):
         Ri_r = Ri_r.to(self.dtype).detach()
         Ri_a = Ri_a.to(self.dtype).detach()
         if self.fit_kernel:
-            lists = nep_ops.nep_lists(self.c2, self.c3, Ri_r, NL_r, Ri_a, NL_a, atom_type_map, num_atom,
-                                      cfg.rcut_radial, cfg.rcut_angular, cfg.l_max)
+            lists = nep_ops.nep_lists(self.c2, self.c3, Ri_r, NL_r, Ri_a, NL_a, atom_type_map,
+                                      num_atom if is_calc_f else None, cfg.rcut_radial, cfg.rcut_angular, cfg.l_max)
             q, s = nep_ops.NepDescriptor.apply(self.c2, self.c3, lists)
             Ei, gq = self.energies_and_grad(q, atom_type_map, type_index)
             Etot = self._frame_sum(Ei, num_atom)

@@ -442,19 +442,23 @@ class NepLists:
 
 
 def nep_lists(c2, c3, Ri_r, NL_r, Ri_a, NL_a, atom_map, num_atom, rc_r, rc_a, l) -> NepLists:
+    """num_atom None: no frames (the descriptor alone, as for energies, asks nothing of them)."""
     c2, Ri_r, NL_r, am = _prep(c2.detach(), Ri_r, NL_r, atom_map)
     if l[0] > 0:
         c3, Ri_a, NL_a, am = _prep(c3.detach(), Ri_a, NL_a, atom_map)
         if NL_a.shape[0] != NL_r.shape[0]:
             raise ValueError("NEP model: the radial and angular lists have different atom counts")
     N = NL_r.shape[0]
-    if _STATIC is not None and num_atom is _STATIC.num_atom:
-        maxf = _STATIC.max_frame
-    else:
-        if _int_sum(num_atom) != N:
-            raise ValueError(f"NEP model: num_atom sums to {_int_sum(num_atom)}, list has {N} atoms")
-        maxf = max(_int_max(num_atom), 1)
-    start, af = _frame_index(num_atom, Ri_r.device)
+    start = af = None
+    maxf = 0
+    if num_atom is not None:
+        if _STATIC is not None and num_atom is _STATIC.num_atom:
+            maxf = _STATIC.max_frame
+        else:
+            if _int_sum(num_atom) != N:
+                raise ValueError(f"NEP model: num_atom sums to {_int_sum(num_atom)}, list has {N} atoms")
+            maxf = max(_int_max(num_atom), 1)
+        start, af = _frame_index(num_atom, Ri_r.device)
     return NepLists(c2, c3.detach(), Ri_r, NL_r, Ri_a, NL_a, am, float(rc_r), float(rc_a), tuple(int(x) for x in l),
                     start, af, maxf)
 

@@ -98,3 +98,20 @@ def test_work_buffer_grows_with_the_atoms():
     # three floats an atom and window of its frame, 72 bytes for each window and frame
     assert small <= 1_000_000 * 12 * 2 + 72 * (1_000_000 // 64 + 100_001)
     assert mixed <= 1_002_000 * 12 * (2000 // 64 + 2) + 72 * (1_002_000 // 64 + 100_002)
+
+
+def test_energies_ask_nothing_of_the_frames(dev):
+    """One frame whose num_atom is not the list's atom count: energies as for the whole list, forces refused."""
+    cfg = NEPConfig(ntypes=2)
+    w = NEPWeights.random(cfg, seed=3, q_scaler=np.full(cfg.nfeat, 0.3))
+    p = mn.pack_frames(_frames([40], 2, 6), cfg.rcut_radial, dev)
+    nb = mn.neighbors(p, cfg.rcut_radial, cfg.rcut_angular, 2)
+    model = mn.NEPTorch(w, torch.float64, dev)
+    args = (nb["NN_r"], nb["NL_r"], nb["Ri_r"], nb["NN_a"], nb["NL_a"], nb["Ri_a"])
+    E0, Ei0, _, _ = model(*args, p["num_atoms"], p["atom_type_map"])
+    E, Ei, F, V = model(*args, torch.ones_like(p["num_atoms"]), p["atom_type_map"], is_calc_f=False)
+    assert torch.equal(E, E0) and torch.equal(Ei, Ei0) and F is None and V is None
+    (g,) = torch.autograd.grad(E.sum(), [model.c2])
+    assert torch.isfinite(g).all()
+    with pytest.raises(ValueError):
+        model(*args, torch.ones_like(p["num_atoms"]), p["atom_type_map"])
