@@ -64,7 +64,10 @@ def test_model_path_equals_operator_sequence(dev, sizes, T, n_max, basis, l_max)
     wE, wF, wV = (torch.randn(*s, dtype=torch.float64, device=dev, generator=g) for s in ((nf, 1), (n, 3), (nf, 9)))
     ref = mn.NEPTorch(w, torch.float64, dev)
     want = _by_ops(ref, nb, p)
+    names = [k for k, q in ref.named_parameters() if l_max[0] > 0 or q is not ref.c3]
     params = [q for q in ref.parameters() if l_max[0] > 0 or q is not ref.c3]
+    partial = {k: [torch.zeros_like(q) if g is None else g for q, g in zip(params, torch.autograd.grad(
+        (x * wx).sum(), params, retain_graph=True, allow_unused=True))] for k, x, wx in ((2, want[1], wF), (3, want[2], wV))}
     want += torch.autograd.grad((want[0] * wE).sum() + (want[1] * wF).sum() + 0.1 * (want[2] * wV).sum(), params)
     for dtype, tol in ((torch.float64, 1e-11), (torch.float32, 2e-4)):
         model = mn.NEPTorch(w, dtype, dev)
@@ -82,12 +85,16 @@ def test_model_path_equals_operator_sequence(dev, sizes, T, n_max, basis, l_max)
         E1, _, F1, V1 = model(*args, create_graph=False)
         assert not F1.requires_grad and not V1.requires_grad
         assert float((F1 - F.detach()).abs().max()) <= tol * float(F.detach().abs().max().clamp_min(1e-2))
-        # only the forces, or only the virials, in the loss
-        for x, wx in ((F, wF), (V, wV)):
-            E, _, F, V = model(*args, create_graph=True)
-            x = F if wx is wF else V
+        # only the forces, or only the virials, in the loss: a bias b1 of the nets (the last tensor of each) reaches
+        # neither
+        for k, wx in ((2, wF), (3, wV)):
+            x = model(*args, create_graph=True)[k]
             gs = torch.autograd.grad((x * wx).sum(), params, allow_unused=True)
-            assert all(torch.isfinite(q).all() for q in gs if q is not None)
+            for q, a, b in zip(names, gs, partial[k]):
+                a = torch.zeros_like(b) if a is None else a.double()
+                assert a.abs().max() > 0 or q.endswith("b.1"), q
+                err = float((a - b).abs().max())
+                assert err <= tol * max(float(b.abs().max()), 1e-2), (dtype, k, q, err, float(b.abs().max()))
 
 
 def test_work_buffer_grows_with_the_atoms():
