@@ -520,17 +520,16 @@ int matpl_nep_feat(int f64, int angular, int mode, const void *c, const void *Ri
  * The descriptor kernels of matpl_nep_feat with each derivative on its own (a model that knows which it
  * needs): arguments as there, save [N][nm*24] the angular sums s or [N][T*nb] the radial basis sums.
  *  mode 0: feats and save (radial: save may be null);
- *  mode 1: gRi only, for gfeat (angular: reads save);
- *  mode 2: second order: ggfeat and gc, for gg or, if gg is null, for the upstream gradients gF [N][3] and
- *          gV [frames][9] (either may be null) of matpl_nep_model_forces' outputs; angular: the gradient of s
- *          goes to gsave [N][nm*24] instead of into gc, for the caller's mode 3 to add (gs there);
- *  mode 3: gc only, from gfeat and save (angular: gs, if not null, is added to dL/ds; gfeat may then be null).
+ *  mode 1: second order: ggfeat and gc, for the upstream gradients gF [N][3] and gV [frames][9] (one may be
+ *          null) of matpl_nep_model_forces' outputs; angular: the gradient of s goes to gsave [N][nm*24]
+ *          instead of into gc, for the caller's mode 2 to add (gs there);
+ *  mode 2: gc only, from gfeat and save (angular: gs, if not null, is added to dL/ds; gfeat may then be null).
  */
 int matpl_nep_descriptor(int f64, int angular, int mode, const void *c, const void *Ri, const int64_t *NL,
                          const int64_t *atom_map, int64_t N, int S, int T, int nm, int nb, int ld, int col0, int l3,
                          int l4, int l5, double rc, void *feats, void *save, const void *gfeat, const void *gs,
-                         const void *gg, const void *gF, const void *gV, const int32_t *atom_frame, void *gRi,
-                         void *gc, void *ggfeat, void *gsave, void *stream);
+                         const void *gF, const void *gV, const int32_t *atom_frame, void *gc, void *ggfeat,
+                         void *gsave, void *stream);
 
 /*
  * Forces F [N][3] and frame virials V [frames][9] of the NEP model (its own signs, src/model/nep_net.py:600-648)

@@ -76,7 +76,7 @@ SIGNATURES = {
     "matpl_nep_neighbor": (I32, [P] * 7 + [F64, F64, I64, I64, I64, I32, I32, I32] + [P] * 8),
     "matpl_nep_neighbor_ri32": (I32, [P] * 6 + [F64, F64, I64, I64, I64, I32] + [P] * 8),
     "matpl_nep_feat": (I32, [I32, I32, I32, P, P, P, P, I64] + [I32] * 9 + [F64] + [P] * 8),
-    "matpl_nep_descriptor": (I32, [I32, I32, I32, P, P, P, P, I64] + [I32] * 9 + [F64] + [P] * 13),
+    "matpl_nep_descriptor": (I32, [I32, I32, I32, P, P, P, P, I64] + [I32] * 9 + [F64] + [P] * 11),
     "matpl_nep_model_forces_work": (I64, [I32, I64, I64, I64, I32, I32, I32]),
     "matpl_nep_model_forces": (I32, [I32] + [P] * 9 + [I64, I64, I64] + [I32] * 11 + [F64, F64] + [P] * 5 + [I64, P]),
     "matpl_nep_force": (I32, [I32, P, P, P, P, I64, I32, P]),

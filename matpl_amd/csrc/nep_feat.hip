@@ -293,8 +293,7 @@ __device__ __forceinline__ int sort_by_type(bool live, int tj, int T, int lane, 
 // ------------------------------------------------------------------ radial kernels
 // One wavefront per atom, lanes over slots. WHAT is a set of:
 constexpr int R_FEAT = 1;      // feats (and the basis sums F into save, if given)
-constexpr int R_GRI = 2;       // gRi
-constexpr int R_GC = 4;        // gc from F summed here
+constexpr int R_1ST = 2;       // first derivatives: gRi, and gc from F summed here
 constexpr int R_GCF = 8;       // gc from the F of an earlier pass (save): no slots are read
 constexpr int R_2ND = 16;      // ggfeat and gc of the second-order pass (V[t][k] = sum gg f'_k in F's place)
 // A slot's basis values go to its row in LDS, at its position sorted by neighbor type; lanes over (type, k)
@@ -312,7 +311,7 @@ template <typename T, int NMC, int NBC, int WHAT>
 __global__ void __launch_bounds__(RAD_WAVES * WAVE)
 nep_radial_kernel(FeatArgs a) {
     extern __shared__ unsigned char smem_raw[];
-    constexpr bool TAB = (WHAT & (R_GC | R_GCF | R_2ND)) != 0, SUM = (WHAT & (R_FEAT | R_GC | R_2ND)) != 0;
+    constexpr bool TAB = (WHAT & (R_1ST | R_GCF | R_2ND)) != 0, SUM = (WHAT & (R_FEAT | R_1ST | R_2ND)) != 0;
     constexpr bool GRAD = (WHAT & ~R_FEAT) != 0;
     const int nm = NMC ? NMC : a.nm, nb = NBC ? NBC : a.nb;
     const int lane = threadIdx.x & (WAVE - 1), wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
@@ -321,7 +320,7 @@ nep_radial_kernel(FeatArgs a) {
     T *gcl = reinterpret_cast<T *>(smem_raw);
     T *gtab = gcl + (ntab > 1 ? wid : 0) * ncoef;
     T *rows = gcl + (size_t)ntab * ncoef + (size_t)wid * WAVE * st;                               // SUM
-    T *wt = gcl + (size_t)ntab * ncoef + (SUM ? (size_t)waves * WAVE * st : 0) + (size_t)wid * tb;   // R_GRI
+    T *wt = gcl + (size_t)ntab * ncoef + (SUM ? (size_t)waves * WAVE * st : 0) + (size_t)wid * tb;   // R_1ST
     if constexpr (TAB) {
         for (int x = threadIdx.x; x < ntab * ncoef; x += blockDim.x) gcl[x] = T(0);
         __syncthreads();
@@ -340,7 +339,7 @@ nep_radial_kernel(FeatArgs a) {
         T acc[NPASS];
 #pragma unroll
         for (int p = 0; p < NPASS; p++) acc[p] = T(0);
-        if constexpr ((WHAT & R_GRI) != 0) {
+        if constexpr ((WHAT & R_1ST) != 0) {
             // w[t][k] = sum_n g_n c[ti][t][n][k]
             for (int o = lane; o < tb; o += WAVE) {
                 const int t = o / nb, q = o - t * nb;
@@ -376,13 +375,13 @@ nep_radial_kernel(FeatArgs a) {
 #pragma unroll
                     for (int q = 0; q < (NBC ? NBC : NB_MAX); q++) {
                         if (NBC == 0 && q >= nb) continue;
-                        if constexpr ((WHAT & (R_FEAT | R_GC)) != 0) row[q] = bs.value();
+                        if constexpr ((WHAT & (R_FEAT | R_1ST)) != 0) row[q] = bs.value();
                         if constexpr ((WHAT & R_2ND) != 0) row[q] = gg * bs.slope();
-                        if constexpr ((WHAT & R_GRI) != 0) d += w[q] * bs.slope();
+                        if constexpr ((WHAT & R_1ST) != 0) d += w[q] * bs.slope();
                         bs.step();
                     }
-                    if constexpr ((WHAT & R_GRI) != 0) store4<T>(reinterpret_cast<T *>(a.gRi) + s * 4, d, T(0), T(0), T(0));
-                } else if constexpr ((WHAT & R_GRI) != 0) {
+                    if constexpr ((WHAT & R_1ST) != 0) store4<T>(reinterpret_cast<T *>(a.gRi) + s * 4, d, T(0), T(0), T(0));
+                } else if constexpr ((WHAT & R_1ST) != 0) {
                     if (k < a.S) store4<T>(reinterpret_cast<T *>(a.gRi) + s * 4, T(0), T(0), T(0), T(0));
                 }
                 if constexpr (SUM) {
@@ -398,7 +397,7 @@ nep_radial_kernel(FeatArgs a) {
                     wave_sync();
                 }
                 if (end) {
-                    if constexpr ((WHAT & R_GRI) != 0)
+                    if constexpr ((WHAT & R_1ST) != 0)
                         for (int kk = k + WAVE; kk < a.S; kk += WAVE)
                             store4<T>(reinterpret_cast<T *>(a.gRi) + (i * a.S + kk) * 4, T(0), T(0), T(0), T(0));
                     break;
@@ -748,14 +747,12 @@ nep_angular_fwd_kernel(FeatArgs a) {
 }
 
 // ------------------------------------------------------------------ angular first derivative
-// GRI: gRi = sum_nm D_nm d(g_n b_m)/dRi of every slot; GC: dc[ti][tj][n][q] = f_q (D b)_n (mode 1: both;
-// alone: the position gradient of a force pass, or the coefficient gradient of a training step with gs, the
-// second-order pass's gradient of s, added to D).
-__host__ __device__ inline int angb_wave_elems(int nm, int nb, bool gc) {
-    return ANG_AB * nm * NLM + (gc ? WAVE * ((nm + nb) | 1) : 0);
-}
+// dc[ti][tj][n][q] = f_q (D b)_n, and with GRI gRi = sum_nm D_nm d(g_n b_m)/dRi of every slot (mode 1 of
+// matpl_nep_feat; without, the coefficient gradient of a training step with gs, the second-order pass's gradient
+// of s, added to D).
+__host__ __device__ inline int angb_wave_elems(int nm, int nb) { return ANG_AB * nm * NLM + WAVE * ((nm + nb) | 1); }
 
-template <typename T, int NMC, int NBC, bool GRI, bool GC>
+template <typename T, int NMC, int NBC, bool GRI>
 __global__ void __launch_bounds__(ANG_WAVES * WAVE)
 nep_angular_bwd_kernel(FeatArgs a) {
     extern __shared__ unsigned char smem_raw[];
@@ -763,16 +760,14 @@ nep_angular_bwd_kernel(FeatArgs a) {
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int nm = NMC ? NMC : a.nm, nb = NBC ? NBC : a.nb, per = nm * NLM, st = (nm + nb) | 1;
     const int ncoef = a.T * a.T * nm * nb;
-    const int waves = blockDim.x / WAVE, ntab = GC ? (a.pw ? waves : 1) : 0;
+    const int waves = blockDim.x / WAVE, ntab = a.pw ? waves : 1;
     // the D rows first: their 16-byte alignment lets a slot read them four or two values at a time
     T *Bq = reinterpret_cast<T *>(smem_raw) + (size_t)wid * ANG_AB * per;                   // [AB][nm][24]
     T *rows = reinterpret_cast<T *>(smem_raw) + (size_t)waves * ANG_AB * per + (size_t)wid * WAVE * st;
-    T *gcl = reinterpret_cast<T *>(smem_raw) + (size_t)waves * angb_wave_elems(nm, nb, GC);   // [ntab][ncoef]
+    T *gcl = reinterpret_cast<T *>(smem_raw) + (size_t)waves * angb_wave_elems(nm, nb);   // [ntab][ncoef]
     T *gtab = gcl + (ntab > 1 ? wid : 0) * ncoef;
-    if constexpr (GC) {
-        for (int x = threadIdx.x; x < ntab * ncoef; x += blockDim.x) gcl[x] = T(0);
-        __syncthreads();
-    }
+    for (int x = threadIdx.x; x < ntab * ncoef; x += blockDim.x) gcl[x] = T(0);
+    __syncthreads();
     const T *c = reinterpret_cast<const T *>(a.c);
     const T *Ri = reinterpret_cast<const T *>(a.Ri);
     T *gRiA = reinterpret_cast<T *>(a.gRi);
@@ -796,8 +791,8 @@ nep_angular_bwd_kernel(FeatArgs a) {
             const int e = e0 + (live ? lane : 0), q = b.atom(e);
             const int64_t s = (i + q) * a.S + (e - b.first(q));
             const int tj = (int)a.atom_map[a.NL[s]];
-            int start = 0, pos = 0;
-            if constexpr (GC) pos = sort_by_type(live, tj, a.T, lane, start);
+            int start;
+            const int pos = sort_by_type(live, tj, a.T, lane, start);
             if (live) {
                 const Row4<T> er = load4(Ri + s * 4);
                 const T ir = T(1) / er.v[0];
@@ -806,9 +801,7 @@ nep_angular_bwd_kernel(FeatArgs a) {
                 T gn[NM_MAX], gp[NM_MAX];
                 if constexpr (GRI) {
                     radial_fn<T, NMC, NBC, true>(c + (int64_t)(b.ti * a.T + tj) * nm * nb, er.v[0], (T)a.rc, nm, nb,
-                                                 gn, gp, [&](int qb, T f, T) {
-                                                     if constexpr (GC) row[nm + qb] = f;
-                                                 });
+                                                 gn, gp, [&](int qb, T f, T) { row[nm + qb] = f; });
                 } else {
                     Basis<T> bs(er.v[0], (T)a.rc);
 #pragma unroll
@@ -820,23 +813,19 @@ nep_angular_bwd_kernel(FeatArgs a) {
                 }
                 T Db[NM_MAX], d[4];
                 angular_slot<T, NMC, GRI>(Bq + q * per, nm, ux, uy, uz, ir, gn, gp, Db, d);
-                if constexpr (GC) {
 #pragma unroll
-                    for (int n = 0; n < (NMC ? NMC : NM_MAX); n++)
-                        if (n < nm) row[n] = Db[n];
-                }
+                for (int n = 0; n < (NMC ? NMC : NM_MAX); n++)
+                    if (n < nm) row[n] = Db[n];
                 if constexpr (GRI) store4<T>(gRiA + s * 4, d[0], d[1], d[2], d[3]);
             }
-            if constexpr (GC) {
-                wave_sync();
-                add_dc<T, 1>(rows, st, 0, nm, nm, nb, a.T, start, gtab + b.ti * a.T * nm * nb, ntab > 1, lane);
-                wave_sync();
-            }
+            wave_sync();
+            add_dc<T, 1>(rows, st, 0, nm, nm, nb, a.T, start, gtab + b.ti * a.T * nm * nb, ntab > 1, lane);
+            wave_sync();
         }
         wave_sync();
         i += b.na;
     }
-    if constexpr (GC) block_flush_add(gcl, reinterpret_cast<T *>(a.gc), ncoef, ntab);
+    block_flush_add(gcl, reinterpret_cast<T *>(a.gc), ncoef, ntab);
 }
 
 // ------------------------------------------------------------------ angular second order (mode 2)
@@ -1041,7 +1030,7 @@ nep_angular_bwd2_kernel(FeatArgs a) {
 
 // ------------------------------------------------------------------ model forces
 // F [N][3] and the frame virials V [F][9] of the NEP model straight from dE/dq: the radial and angular slot
-// derivatives (nep_radial_kernel R_GRI, nep_angular_bwd_kernel GRI) and the force terms of each slot,
+// derivatives (nep_radial_kernel R_1ST, nep_angular_bwd_kernel GRI) and the force terms of each slot,
 // f = dE[s][0] (x, y, z)/r + dE[s][1:4] (src/model/nep_net.py:440-468 and :608; calculateNepForce,
 // CalcOps.cpp:75-158; the frame sum of calculateNepVirial, CalcOps.cpp:239-328), with the model's signs
 // (nep_net.py negates both): F[i] += f, F[j] -= f, V[frame] -= f (x) x. No [N][S][4] gradient is written or read.
@@ -1322,26 +1311,26 @@ int force_launch(ForceArgs &p, const ForcePlan &pl, int64_t nframes, T *V, hipSt
 }
 
 // ------------------------------------------------------------------ launch
-enum FeatWhat { W_FEAT, W_GRI, W_GRI_GC, W_GC, W_2ND, W_2ND_GS };
+enum FeatWhat { W_FEAT, W_1ST, W_GC, W_2ND, W_2ND_GS };
 
 template <typename T, int NMC, int NBC>
 int feat_launch(FeatArgs &a, bool angular, FeatWhat what, hipStream_t st) {
     if (!angular && what == W_2ND_GS) what = W_2ND;
     const size_t ncoef = (size_t)a.T * a.T * a.nm * a.nb, tb = (size_t)a.T * a.nb;
-    const bool table = what == W_GRI_GC || what == W_GC || what == W_2ND || what == W_2ND_GS;
+    const bool table = what == W_1ST || what == W_GC || what == W_2ND || what == W_2ND_GS;
     int waves = angular ? ANG_WAVES : RAD_WAVES;
     // LDS of a block of w wavefronts with ntab coefficient-gradient tables
     auto lds_of = [&](int w, size_t ntab) -> size_t {
         size_t e = table ? ntab * ncoef : 0;
         if (!angular) {
-            const bool sum = what == W_FEAT || what == W_GRI_GC || what == W_2ND;
-            e += (size_t)w * ((sum ? WAVE * rad_stride<NBC>(a.nb) : 0) + (what == W_GRI || what == W_GRI_GC ? tb : 0));
+            const bool sum = what == W_FEAT || what == W_1ST || what == W_2ND;
+            e += (size_t)w * ((sum ? WAVE * rad_stride<NBC>(a.nb) : 0) + (what == W_1ST ? tb : 0));
         } else if (what == W_FEAT) {
             e += (size_t)w * angf_wave_elems(a.nm);
         } else if (what == W_2ND || what == W_2ND_GS) {
             e += (size_t)w * ang2_wave_elems<T>(a.nm, a.nb);
         } else {
-            e += (size_t)w * angb_wave_elems(a.nm, a.nb, table);
+            e += (size_t)w * angb_wave_elems(a.nm, a.nb);
         }
         return e * sizeof(T);
     };
@@ -1363,8 +1352,7 @@ int feat_launch(FeatArgs &a, bool angular, FeatWhat what, hipStream_t st) {
     if (!angular) {
         switch (what) {
         case W_FEAT: hipLaunchKernelGGL((nep_radial_kernel<T, NMC, NBC, R_FEAT>), grid, block, lds, st, a); break;
-        case W_GRI: hipLaunchKernelGGL((nep_radial_kernel<T, NMC, NBC, R_GRI>), grid, block, lds, st, a); break;
-        case W_GRI_GC: hipLaunchKernelGGL((nep_radial_kernel<T, NMC, NBC, R_GRI | R_GC>), grid, block, lds, st, a); break;
+        case W_1ST: hipLaunchKernelGGL((nep_radial_kernel<T, NMC, NBC, R_1ST>), grid, block, lds, st, a); break;
         case W_GC: hipLaunchKernelGGL((nep_radial_kernel<T, NMC, NBC, R_GCF>), grid, block, lds, st, a); break;
         default: hipLaunchKernelGGL((nep_radial_kernel<T, NMC, NBC, R_2ND>), grid, block, lds, st, a); break;
         }
@@ -1372,9 +1360,8 @@ int feat_launch(FeatArgs &a, bool angular, FeatWhat what, hipStream_t st) {
     }
     switch (what) {
     case W_FEAT: hipLaunchKernelGGL((nep_angular_fwd_kernel<T, NMC, NBC>), grid, block, lds, st, a); break;
-    case W_GRI: hipLaunchKernelGGL((nep_angular_bwd_kernel<T, NMC, NBC, true, false>), grid, block, lds, st, a); break;
-    case W_GRI_GC: hipLaunchKernelGGL((nep_angular_bwd_kernel<T, NMC, NBC, true, true>), grid, block, lds, st, a); break;
-    case W_GC: hipLaunchKernelGGL((nep_angular_bwd_kernel<T, NMC, NBC, false, true>), grid, block, lds, st, a); break;
+    case W_1ST: hipLaunchKernelGGL((nep_angular_bwd_kernel<T, NMC, NBC, true>), grid, block, lds, st, a); break;
+    case W_GC: hipLaunchKernelGGL((nep_angular_bwd_kernel<T, NMC, NBC, false>), grid, block, lds, st, a); break;
     case W_2ND: hipLaunchKernelGGL((nep_angular_bwd2_kernel<T, NMC, NBC, false>), grid, block, lds, st, a); break;
     default: hipLaunchKernelGGL((nep_angular_bwd2_kernel<T, NMC, NBC, true>), grid, block, lds, st, a); break;
     }
@@ -1424,33 +1411,30 @@ MATPL_EXPORT int matpl_nep_feat(int f64, int angular, int mode, const void *c, c
     MATPL_CHECK_ARG(mode != 1 || N == 0 || (gfeat && gRi && gc && (!angular || s_save)), "nep_feat: null grad io");
     MATPL_CHECK_ARG(mode != 2 || N == 0 || (gfeat && gg && gc && ggfeat && (!angular || s_save)),
                     "nep_feat: null 2nd-order io");
-    return feat_run(a, f64, angular != 0, mode == 0 ? W_FEAT : (mode == 1 ? W_GRI_GC : W_2ND), (hipStream_t)stream);
+    return feat_run(a, f64, angular != 0, mode == 0 ? W_FEAT : (mode == 1 ? W_1ST : W_2ND), (hipStream_t)stream);
 }
 
 MATPL_EXPORT int matpl_nep_descriptor(int f64, int angular, int mode, const void *c, const void *Ri, const int64_t *NL,
                                       const int64_t *atom_map, int64_t N, int S, int T, int nm, int nb, int ld,
                                       int col0, int l3, int l4, int l5, double rc, void *feats, void *save,
-                                      const void *gfeat, const void *gs, const void *gg, const void *gF,
-                                      const void *gV, const int32_t *atom_frame, void *gRi, void *gc, void *ggfeat,
-                                      void *gsave, void *stream) {
+                                      const void *gfeat, const void *gs, const void *gF, const void *gV,
+                                      const int32_t *atom_frame, void *gc, void *ggfeat, void *gsave, void *stream) {
     FeatArgs a{};
     a.c = c; a.Ri = Ri; a.NL = NL; a.atom_map = atom_map; a.feats = feats; a.save = save;
-    a.gfeat = gfeat; a.gs = angular ? gs : nullptr; a.gg = gg; a.gRi = gRi; a.gc = gc; a.ggfeat = ggfeat; a.gsave = gsave;
+    a.gfeat = gfeat; a.gs = angular ? gs : nullptr; a.gc = gc; a.ggfeat = ggfeat; a.gsave = gsave;
     a.gF = gF; a.gV = gV; a.atom_frame = atom_frame;
     a.N = N; a.S = S; a.T = T; a.nm = nm; a.nb = nb; a.ld = ld; a.col0 = col0; a.l3 = l3; a.l4 = l4; a.l5 = l5;
     a.rc = rc;
-    MATPL_CHECK_ARG(mode >= 0 && mode <= 3, "nep_descriptor: bad mode");
+    MATPL_CHECK_ARG(mode >= 0 && mode <= 2, "nep_descriptor: bad mode");
     MATPL_CHECK_ARG(N >= 0 && S >= 0 && ld >= 1 && col0 >= 0, "nep_descriptor: bad sizes");
     MATPL_CHECK_ARG(N == 0 || (c && Ri && NL && atom_map), "nep_descriptor: null input");
     MATPL_CHECK_ARG(mode != 0 || N == 0 || (feats && (!angular || save)), "nep_descriptor: null output");
-    MATPL_CHECK_ARG(mode != 1 || N == 0 || (gfeat && gRi && (!angular || save)), "nep_descriptor: null gradient io");
-    MATPL_CHECK_ARG(mode != 2 || N == 0 || (gfeat && gc && ggfeat && (!angular || (save && gsave))),
+    MATPL_CHECK_ARG(mode != 1 || N == 0 || (gfeat && gc && ggfeat && (gF || gV) && (!gV || atom_frame) &&
+                                            (!angular || (save && gsave))),
                     "nep_descriptor: null 2nd-order io");
-    MATPL_CHECK_ARG(mode != 2 || N == 0 || gg || ((gF || gV) && (!gV || atom_frame)),
-                    "nep_descriptor: second order needs gg, or gF / gV with atom_frame");
-    MATPL_CHECK_ARG(mode != 3 || N == 0 || (gc && save && (gfeat || (angular && gs))),
+    MATPL_CHECK_ARG(mode != 2 || N == 0 || (gc && save && (gfeat || (angular && gs))),
                     "nep_descriptor: null coefficient-gradient io");
-    static const FeatWhat what[4] = {W_FEAT, W_GRI, W_2ND_GS, W_GC};
+    static const FeatWhat what[3] = {W_FEAT, W_2ND_GS, W_GC};
     return feat_run(a, f64, angular != 0, what[mode], (hipStream_t)stream);
 }
 

@@ -408,8 +408,8 @@ def _desc_call(mode, angular, a, feats=None, save=None, gfeat=None, gs=None, gF=
     N, S = NL.shape
     T, _, nm, nb = c.shape
     _lib.call("matpl_nep_descriptor", _f64(Ri), int(angular), mode, _ptr(c), _ptr(Ri), _ptr(NL), _ptr(a.atom_map), N, S,
-              T, nm, nb, width, col0, *l, rc, _ptr(feats), _ptr(save), _ptr(gfeat), _ptr(gs), None, _ptr(gF), _ptr(gV),
-              _ptr(a.af), None, _ptr(gc), _ptr(ggfeat), _ptr(gsave), _stream())
+              T, nm, nb, width, col0, *l, rc, _ptr(feats), _ptr(save), _ptr(gfeat), _ptr(gs), _ptr(gF), _ptr(gV),
+              _ptr(a.af), _ptr(gc), _ptr(ggfeat), _ptr(gsave), _stream())
 
 
 @dataclass
@@ -496,10 +496,10 @@ class NepDescriptor(torch.autograd.Function):
         g2 = g3 = None
         if ctx.needs_input_grad[0] and gq is not None:
             g2 = torch.zeros_like(a.c2)
-            _desc_call(3, False, a, save=F, gfeat=gq, gc=g2, width=a.width)
+            _desc_call(2, False, a, save=F, gfeat=gq, gc=g2, width=a.width)
         if ctx.needs_input_grad[1] and a.l[0] > 0 and (gq is not None or gs is not None):
             g3 = torch.zeros_like(a.c3)
-            _desc_call(3, True, a, save=s, gfeat=gq, gs=gs, gc=g3, width=a.width)
+            _desc_call(2, True, a, save=s, gfeat=gq, gs=gs, gc=g3, width=a.width)
         return g2, g3, None
 
 
@@ -540,11 +540,11 @@ class NepModelForces(torch.autograd.Function):
         gV = None if gV is None else gV.to(dt).contiguous()
         ggq = torch.empty_like(g)
         g2 = torch.zeros_like(a.c2)
-        _desc_call(2, False, a, gfeat=g, gF=gF, gV=gV, gc=g2, ggfeat=ggq, width=a.width)
+        _desc_call(1, False, a, gfeat=g, gF=gF, gV=gV, gc=g2, ggfeat=ggq, width=a.width)
         g3 = gs = None
         if a.l[0] > 0:
             g3, gs = torch.zeros_like(a.c3), torch.empty_like(s)
-            _desc_call(2, True, a, save=s, gfeat=g, gF=gF, gV=gV, gc=g3, ggfeat=ggq, gsave=gs, width=a.width)
+            _desc_call(1, True, a, save=s, gfeat=g, gF=gF, gV=gV, gc=g3, ggfeat=ggq, gsave=gs, width=a.width)
         return ggq, gs, g2, g3, None
 
 

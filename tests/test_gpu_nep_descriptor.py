@@ -77,12 +77,20 @@ def test_descriptor_modes(dev, dtype, angular, T, nm, nb, l, S, counts):
     gc1, gRi = torch.autograd.grad(q, [c_, Ri_], gq_, create_graph=True)
     valid = torch.as_tensor(NL >= 0).unsqueeze(-1)
     gRi = torch.where(valid, gRi, torch.zeros_like(gRi))
-    ggq, gc2 = torch.autograd.grad((gRi * gg_).sum(), [gq_, c_])
+    ggq, gc2 = torch.autograd.grad((gRi * gg_).sum(), [gq_, c_], retain_graph=True)
+    # the same for gradients of model forces and of two frames' virials: q = gF[i] - gF[j] - gV x, gg = [q . u, q]
+    gF, gV = f32(rng.normal(size=(N, 3))), f32(rng.normal(size=(2, 9)))
+    frame = (torch.arange(N) >= N // 2).to(torch.int32)
+    x, r = Ri_.detach()[..., 1:], Ri_.detach()[..., :1]
+    qf = gF[:, None] - gF[torch.as_tensor(NL).clamp(min=0)] - (gV.view(2, 1, 3, 3)[frame.long()] @ x[..., None])[..., 0]
+    ggf_ = torch.where(valid, torch.cat([(qf * x).sum(-1, keepdim=True) / torch.where(valid, r, 1.0), qf], -1), 0.0)
+    ggq_f, gc2_f = torch.autograd.grad((gRi * ggf_).sum(), [gq_, c_])
 
     d = lambda a: torch.as_tensor(np.ascontiguousarray(a), device=dev).to(dtype).contiguous()
     cd, Rd, gqd, ggd = d(c), d(Ri), torch.zeros((N, ld), dtype=dtype, device=dev), d(gg)
     gqd[:, col0:col0 + nf] = d(gq)
     NLd, amd = torch.as_tensor(NL, device=dev), torch.as_tensor(am, device=dev)
+    gFd, gVd, frame = gF.to(dtype).to(dev), gV.to(dtype).to(dev), frame.to(dev)
     f64 = int(dtype == torch.float64)
     new = lambda *s: torch.full(s, float("nan"), dtype=dtype, device=dev)
     save = new(N, nm * 24 if angular else T * nb)
@@ -106,21 +114,18 @@ def test_descriptor_modes(dev, dtype, angular, T, nm, nb, l, S, counts):
             _close(cut(ggf), ggq, dtype, "ggfeat")
             _close(gc, gc2, dtype, "gc second order")
         else:
-            call(name, 0, feats, save, *[None] * 10)
+            call(name, 0, feats, save, *[None] * 8)
             _close(cut(feats), q, dtype, "feats")
             assert torch.isnan(feats[:, :col0]).all() and torch.isnan(feats[:, col0 + nf:]).all()
-            g = new(N, S, 4)
-            call(name, 1, None, save, gqd, *[None] * 5, g, None, None, None)
-            _close(g, gRi, dtype, "gRi")
             gc, ggf, gs = torch.zeros_like(cd), new(N, ld), new(N, nm * 24)
-            call(name, 2, None, save, gqd, None, ggd, *[None] * 4, gc, ggf, gs if angular else None)
-            _close(cut(ggf), ggq, dtype, "ggfeat")
+            call(name, 1, None, save, gqd, None, gFd, gVd, frame, gc, ggf, gs if angular else None)
+            _close(cut(ggf), ggq_f, dtype, "ggfeat")
             # the second order's rest and the first order in one coefficient pass
-            call(name, 3, None, save, gqd, gs if angular else None, *[None] * 5, gc, None, None)
-            _close(gc, gc1 + gc2, dtype, "gc of both orders")
+            call(name, 2, None, save, gqd, gs if angular else None, *[None] * 3, gc, None, None)
+            _close(gc, gc1 + gc2_f, dtype, "gc of both orders")
             if angular:
                 gc = torch.zeros_like(cd)
-                call(name, 3, None, save, None, gs, *[None] * 5, gc, None, None)
+                call(name, 2, None, save, None, gs, *[None] * 3, gc, None, None)
                 gc3 = torch.zeros_like(cd)
-                call(name, 3, None, save, gqd, gs, *[None] * 5, gc3, None, None)
+                call(name, 2, None, save, gqd, gs, *[None] * 3, gc3, None, None)
                 _close(gc3 - gc, gc1, dtype, "gc without gs")
