@@ -46,6 +46,13 @@ inline unsigned grid_cap(int64_t n, int threads = 256) {
 __device__ __forceinline__ void atomic_add(float *p, float v) { unsafeAtomicAdd(p, v); }
 __device__ __forceinline__ void atomic_add(double *p, double v) { unsafeAtomicAdd(p, v); }
 
+// Orders a wavefront's own LDS writes before its lanes' reads of each other's values.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Wavefront (64-lane) sum via cross-lane shuffles.
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {

@@ -69,13 +69,6 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
     return v;
 }
 
-// LDS written by the wavefront's other lanes is visible after this.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // A non-finite coordinate has no cell and no image: status gets STATUS_NONFINITE (before any
 // search kernel can record an overflow) and the coordinate is searched as 0, so that every index
 // the search forms stays in range.

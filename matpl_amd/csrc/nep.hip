@@ -87,13 +87,6 @@ __device__ __forceinline__ void put_row(int64_t *NL, R *Ri, int64_t idx, int w, 
     }
 }
 
-// Orders a wavefront's own LDS writes before its lanes' reads of each other's values.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // MODE 0: lists; 1: counts; 2: per-type counts. One wavefront per atom n1, lanes over the frame's
 // atoms n2, each with its replicas (ia, ib, ic) in the reference's order; a list holds the hits in
 // (n2, replica) order. With one replica (the box is at least 2 rc thick) a lane has at most one hit

@@ -200,13 +200,6 @@ struct FeatArgs {
     double rc;
 };
 
-// Orders a wavefront's own LDS writes before its lanes' reads of each other's values.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Rows of four values at the element type's own alignment.
 template <typename T>
 struct __attribute__((packed, aligned(sizeof(T)))) Row4 {

@@ -63,13 +63,6 @@ struct FitArgs {
     int part_rows;           // forward: rows of W0 in LDS at a time
 };
 
-// Orders a wavefront's own LDS writes before its lanes' reads of each other's values.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __host__ __device__ inline int odd(int n) { return n | 1; }     // LDS row stride (odd: fewer bank conflicts)
 
 template <typename T>
