@@ -117,3 +117,30 @@ def test_model_kernel_path_equals_torch_layers(dev, dtype, tol):
     assert _rel(E1, E2) < tol and _rel(F1, F2) < tol and _rel(V1, V2) < tol
     for a, b in zip(g1, g2):
         assert _rel(a, b) < 10 * tol
+
+
+@pytest.mark.parametrize("T", [16, 17])
+@pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-11), (torch.float32, 1e-4)])
+def test_energies_up_to_and_past_the_pointer_tables(dev, T, dtype, tol):
+    """NEPTorch.energies_and_grad at 16 types (the fitting kernels' pointer tables, each net's own tensors) and 17
+    (stacked parameters): energies, dEi/dq and their parameter gradients equal the per-type torch layers."""
+    from matpl_amd.nepnet import NEPConfig, NEPWeights
+    cfg = NEPConfig(ntypes=T)
+    model = mn.NEPTorch(NEPWeights.random(cfg, seed=T), dtype, dev)
+    assert model.fit_kernel
+    D = model.fit[0].W[0].shape[0]
+    g = torch.Generator().manual_seed(T)
+    N = 200
+    feats = torch.randn((N, D), generator=g, dtype=torch.float64).to(dtype).to(dev)
+    tm = torch.randint(0, T, (N,), generator=g).to(dev)
+    up_e, up_g = (torch.randn(s, generator=g, dtype=torch.float64).to(dtype).to(dev) for s in ((N,), (N, D)))
+    params = [p for n in model.fit for p in n.parameters()]
+    Ei, dq = model.energies_and_grad(feats, tm)
+    res = [(Ei, dq, *torch.autograd.grad((Ei * up_e).sum() + (dq * up_g).sum(), params))]
+    model.fit_kernel = False
+    f = feats.clone().requires_grad_()
+    Ei = model.energies(f, tm)
+    dq, = torch.autograd.grad(Ei.sum(), f, create_graph=True)
+    res.append((Ei, dq, *torch.autograd.grad((Ei * up_e).sum() + (dq * up_g).sum(), params)))
+    for a, b in zip(*res):
+        assert _rel(a, b) < tol
