@@ -1043,7 +1043,7 @@ struct ForceArgs {
     const int32_t *atom_frame;    // [N]
     void *F, *part;               // [N][3] (zeroed), the frames' rows
     double *vpart;                // [segments][9]
-    int64_t rcap;
+    int64_t rcap, rows;           // atoms of the LDS copy, rows kept per frame (force_rows)
     int ch;
 };
 
@@ -1065,8 +1065,9 @@ __device__ __forceinline__ T fold16(T v[16], int lane) {
     return x;
 }
 
+// (Atom numbers fit 32 bits wherever they are divided by ch: a grid of a block per window holds fewer.)
 // Rows of a frame of at most rcap atoms: the windows of ch that it touches.
-__host__ __device__ inline int64_t force_rows(int64_t rcap, int ch) { return rcap > 0 ? (rcap - 1) / ch + 2 : 0; }
+inline int64_t force_rows(int64_t rcap, int ch) { return rcap > 0 ? (rcap - 1) / ch + 2 : 0; }
 
 // (153 float and 256 double VGPRs: 3 and 2 wavefronts per SIMD, which blocks of 4 wavefronts fill; of 8, one
 // float block fits a CU; in double 4 registers spill, in the general sizes' form 32)
@@ -1218,7 +1219,8 @@ nep_force_kernel(ForceArgs p) {
             p.vpart[seg * 9 + threadIdx.x] = v;
         }
         if (lds) {
-            T *o = reinterpret_cast<T *>(p.part) + 3 * (fs * force_rows(p.rcap, p.ch) + (i0 / p.ch - fs / p.ch) * (fe - fs));
+            const unsigned row = blockIdx.x - (unsigned)fs / (unsigned)p.ch;
+            T *o = reinterpret_cast<T *>(p.part) + 3 * (fs * p.rows + row * (fe - fs));
             for (int64_t x = threadIdx.x; x < 3 * (fe - fs); x += blockDim.x) o[x] = (T)acc[x];
         }
         __syncthreads();
@@ -1230,7 +1232,7 @@ nep_force_kernel(ForceArgs p) {
 template <typename T>
 __global__ void __launch_bounds__(256)
 nep_force_final_kernel(const int64_t *__restrict__ frame_start, const int32_t *__restrict__ atom_frame, int64_t N,
-                       int ch, int64_t rcap, const T *__restrict__ part, const double *__restrict__ vpart,
+                       int ch, int64_t rcap, int64_t rows, const T *__restrict__ part, const double *__restrict__ vpart,
                        T *__restrict__ F, T *__restrict__ V, int64_t fblocks) {
     __shared__ double red[256];
     if ((int64_t)blockIdx.x >= fblocks) {
@@ -1259,10 +1261,11 @@ nep_force_final_kernel(const int64_t *__restrict__ frame_start, const int32_t *_
         const int64_t fs = frame_start[f], fe = frame_start[f + 1];
         any = fe - fs <= rcap;
         if (any) {
-            const T *q = part + 3 * fs * force_rows(rcap, ch) + (e - 3 * fs);
-            const int64_t nw = (fe - 1) / ch - fs / ch + 1;
+            const T *q = part + 3 * fs * rows + (e - 3 * fs);
+            const unsigned w = (unsigned)ch, nw = (unsigned)(fe - 1) / w - (unsigned)fs / w + 1;
+            const unsigned pitch = 3 * (unsigned)(fe - fs);          // nw pitch < 2^22: the LDS copy bounds the frame
 #pragma unroll 4
-            for (int64_t b = g; b < nw; b += 4) s += q[b * 3 * (fe - fs)];
+            for (unsigned b = g; b < nw; b += 4) s += q[b * pitch];
         }
     }
     redT[threadIdx.x] = s;
@@ -1292,13 +1295,14 @@ int force_launch(ForceArgs &p, const ForcePlan &pl, int64_t nframes, T *V, hipSt
     const int64_t N = p.r.N, blocks = ceil_div(N, pl.ch);
     p.ch = pl.ch;
     p.rcap = pl.rcap;
+    p.rows = force_rows(pl.rcap, pl.ch);
     hipLaunchKernelGGL((nep_force_kernel<T, NMC, NBC>), dim3((unsigned)blocks), dim3(FORCE_WAVES * WAVE), pl.lds, st,
                        p);
     int rc = check_launch("nep_force_kernel");
     if (rc) return rc;
     const int64_t fblocks = pl.rcap > 0 ? ceil_div(3 * N, 64) : 0;
     hipLaunchKernelGGL(nep_force_final_kernel<T>, dim3((unsigned)(fblocks + nframes)), dim3(256), 0, st, p.frame_start,
-                       p.atom_frame, N, pl.ch, pl.rcap, reinterpret_cast<const T *>(p.part), p.vpart,
+                       p.atom_frame, N, pl.ch, pl.rcap, p.rows, reinterpret_cast<const T *>(p.part), p.vpart,
                        reinterpret_cast<T *>(p.F), V, fblocks);
     return check_launch("nep_force_final_kernel");
 }
