@@ -459,8 +459,8 @@ dp_fused_bwd_kernel(FusedParams p) {
 // ------------------------------------------------------------------ group passes (dp_group.h)
 // The forward of up to GA atoms at once: the same tiles and net as dp_fused_fwd_kernel over the group's neighbors;
 // the contraction's rows are (atom, component), of which a neighbor fills its own atom's four (BF16 as there, FP32
-// by contract_group). Measured against an atom per wavefront: 73,742 atoms of four types in BF16 395 -> 248 us,
-// 7,000 in FP32 151 -> 106.
+// by contract_group). Measured against an atom per wavefront: 73,742 atoms of four types in BF16 395 -> 243 us,
+// 7,000 in FP32 151 -> 111.
 template <int E, bool BF16, bool GST>
 __global__ void __launch_bounds__(FUSED_WAVES * WAVE)
 dp_group_fwd_kernel(FusedParams p) {
@@ -578,7 +578,7 @@ dp_group_fwd_kernel(FusedParams p) {
 
 // The backward of up to GA atoms at once: dp_fused_bwd_kernel's tile with the dA rows of the lane's own atom (read
 // once for dG and dRi), centre forces summed per atom of the tile. Measured against an
-// atom per wavefront: 73,742 atoms of four types in BF16 786 -> 495 us, 7,000 in FP32 212 -> 184.
+// atom per wavefront: 73,742 atoms of four types in BF16 786 -> 485 us, 7,000 in FP32 212 -> 152.
 template <int E, bool BF16>
 __global__ void __launch_bounds__(FUSED_WAVES * WAVE)
 dp_group_bwd_kernel(FusedParams p) {

@@ -211,7 +211,8 @@ dp_train_tangent_kernel(TrainParams tp) {
 
 // The tangent of up to GA atoms at once (dp_group.h): the same tiles over the group's neighbors, the two
 // contractions v (x) G and Ri (x) v0 G' in FP32 on the matrix cores (contract_group). Measured
-// against an atom per wavefront: 73,742 atoms of four types in BF16 672 -> 365 us, 7,000 in FP32 187 -> 137.
+// against an atom per wavefront: 73,742 atoms of four types in BF16 672 -> 363 us, 7,000 in FP32 187 -> 138
+// (FP32 spills 4 registers at three wavefronts per SIMD).
 template <int E, bool BF16>
 __global__ void __launch_bounds__(FUSED_WAVES * WAVE, 3)
 dp_group_tangent_kernel(TrainParams tp) {

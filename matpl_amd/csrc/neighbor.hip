@@ -492,7 +492,7 @@ __global__ void __launch_bounds__(CELL_WAVES * WAVE) cell_overfull_kernel(CellAr
 // positions in scalar registers and spilled (201 us).
 //
 // Bound: VALU issue (about 740 instructions an atom: 135 of the sweep over 807 candidates, 240 of
-// the exact tests, 160 of its share of the merging). 189 us, against 496 us of the search atom by
+// the exact tests, 160 of its share of the merging). 178 us, against 496 us of the search atom by
 // atom, on the 99,636-atom HfO2 list of 160 slots per type at 6.5 A (105 neighbors an atom, 255 MB
 // of list and shift stores).
 constexpr int CB_WAVES = 8;

@@ -292,8 +292,8 @@ constexpr int R_2ND = 16;      // ggfeat and gc of the second-order pass (V[t][k
 // A slot's basis values go to its row in LDS, at its position sorted by neighbor type; lanes over (type, k)
 // then add only their own type's rows. What bounds it: the LDS reads of that sum and, with few atoms, the
 // chain list -> type -> basis -> sum. Measured on the 62,713-atom four-type float batch, against nm nb
-// multiply-adds a slot with gathered coefficients and a scan of all rows per (type, k): features 190 -> 56 us,
-// gRi and gc 357 -> 105, second order 373 -> 102; 1,728 atoms, gRi and gc: 32 -> 15.
+// multiply-adds a slot with gathered coefficients and a scan of all rows per (type, k): features 190 -> 57 us,
+// gRi and gc 357 -> 105, second order 373 -> 109; 1,728 atoms, gRi and gc: 32 -> 15, features 16 -> 8.
 constexpr int RAD_WAVES = 4;
 constexpr int NPASS = (NT_MAX * NB_MAX + WAVE - 1) / WAVE;   // (type, k) pairs per lane at most
 
@@ -451,8 +451,10 @@ nep_radial_kernel(FeatArgs a) {
 // What bounds the angular kernels: VALU work per slot (basis, harmonics, the D contractions) and the LDS
 // traffic of the slot sums, which as lanes over outputs read every row from every lane and, for dc, read and
 // wrote a table entry per slot; as 16x16x4 products each row is read once per 16 outputs and the table once per
-// type and batch. Same batch, float: features 136 -> 65 us, first derivative 375 -> 129, second order
-// 1020 -> 357; double on 16 frames: 65 -> 32, 96 -> 44, 264 -> 183.
+// type and batch. Same batch, float: features 136 -> 63 us, first derivative 375 -> 129, second order 1020 -> 357
+// with its coefficient gradient, 263 without (the first derivative's pass, 143, then forms both); double on 16
+// frames: 65 -> 31, 96 -> 44, 264 -> 183 (142). The second order in double holds 256 VGPRs and 58 AGPRs (104 at
+// the general sizes), which is one wavefront per SIMD.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 template <typename T> struct Acc;
@@ -1375,7 +1377,12 @@ int feat_check(const FeatArgs &a, bool angular) {
 }
 
 // The reference's default sizes (n_max 4, basis_size 12: nm = 5, nb = 13) have kernels of their own, whose
-// loops over n and k unroll and keep their values in registers; other sizes run the general ones.
+// loops over n and k unroll and keep their values in registers; other sizes run the general ones. At 5 and 13, these
+// against the general ones: 62,713-atom float batch, second order 263 us (434), forces 181 (339), angular features
+// 63 (133), radial 57 (106) and its second order 109 (244); double on 16 frames 142 (231), 49 (84), 31 (58),
+// 18 (39), 30 (48); 1,728 atoms, float: forces 18 (29). At other sizes the training gradient takes 1.6 to 2.3 times
+// less than with nm nb multiply-adds a slot (32 frames, n_max 7, basis_size 12, l_max (4, 2, 1): float
+// 2228 -> 1106 us, double 2506 -> 1383; n_max 6, basis_size 8: 1851 -> 1020, 2050 -> 1261).
 template <typename T>
 int feat_sizes(FeatArgs &a, bool angular, FeatWhat what, hipStream_t st) {
     if (a.nm == 5 && a.nb == 13) return feat_launch<T, 5, 13>(a, angular, what, st);
