@@ -227,8 +227,8 @@ def short_buckets(type_counts) -> bool:
     """Whether atoms in these numbers per type leave the neighbor buckets short: they are spread over three types or
     more. The effective number of types, 1 / sum of squared fractions, is 1.8 for HfO2 on a model of any number of
     types, whose buckets fill the kernels' tiles atom by atom, and 2.5 for Li10GeP2S12 (csrc/dp_group.h has times)."""
-    n = np.asarray(type_counts, np.float64)
-    return float(n.sum()) ** 2 >= 2.3 * float((n * n).sum()) > 0.0
+    n = [float(c) for c in type_counts]
+    return sum(n) ** 2 >= 2.3 * sum(c * c for c in n) > 0.0
 
 
 class FusedDP:
@@ -273,7 +273,6 @@ class FusedDP:
         self.fit = _Fitting(w, self.device)
         self.fitting = fitting
         self._mfma_fit = {}
-        self._short = {}        # short_buckets of the type runs seen
         self.precision = precision
         self.events = None      # when a list: (start, end) HIP events around each backward launch
         self._masks = {}        # checked per-frame type masks on the device, by content and atoms
@@ -298,12 +297,10 @@ class FusedDP:
         if type_ranges is None:
             type_ranges = type_runs(type_map.cpu().numpy())
         key = tuple(segments(type_ranges))
-        if key not in self._short:
-            counts = [0] * T
-            for t, a, b in key:
-                counts[t] += b - a
-            self._short[key] = short_buckets(counts)
-        precision = int(self.fw.bf16) | (DP_GROUP if self._short[key] else 0)
+        counts = [0] * T
+        for t, a, b in key:
+            counts[t] += b - a
+        precision = int(self.fw.bf16) | (DP_GROUP if short_buckets(counts) else 0)
         scale = 1.0 / (cfg.m * T)
         masks = None if type_present is None else self._type_masks(type_present, type_map, atom_frame, nframes)
         A = torch.empty((N, 4, self.fw.E), dtype=torch.float32, device=dev)
